@@ -127,29 +127,29 @@ __device__ __forceinline__ float kf_expf(float x)
     if (k < -126) { y = y * 5.421010862427522e-20f; k += 64; }
     return y * __int_as_float((k + 127) << 23);
 }
-// kf_expf for x <= 0 or NaN (the bilateral weights, -a - b with a, b >= 0):
-// the overflow branches of kf_expf are never taken there, so the same
-// operations without them give the same bits.  Its scaling by 2^k is one
-// rounding of y * 2^k (for k < -126 the first step, by 2^-64, is exact, and
-// y in [0.7, 1.5] keeps it normal), which is what v_ldexp_f32 computes.
+// kf_expf for the bilateral weights (x <= 0): the same bits in 16 instructions
+// (checked against kf_expf for every float in [-inf, -0]).  The argument is
+// clamped to -105 instead of tested: exp(-105) is below 2^-151, which rounds
+// to the 0 that kf_expf returns below -104.  fk * 0.693359375 is exact (at
+// most 17 bits), so the subtraction is one fused multiply-add; the scaling by
+// 2^k is one rounding of y * 2^k, which is what v_ldexp_f32 computes.  A NaN
+// argument comes from a tap that is not finite, and gives 0 here: the caller's
+// 0 * tap is then NaN, as with kf_expf's NaN.
 __device__ __forceinline__ float kf_expf_nonpos(float x)
 {
-    if (!(x == x)) return x;
-    if (x < -104.0f) return 0.0f;
-    float fk = floorf(x * 1.44269504088896341f + 0.5f);
-    int k = (int)fk;
-    float r = x - fk * 0.693359375f;  // exact product (9-bit constant)
+    x = fmaxf(x, -105.0f);
+    const float fk = floorf(x * 1.44269504088896341f + 0.5f);
+    float r = fmaf(fk, -0.693359375f, x);
     r = fmaf(fk, 2.12194440e-4f, r);
-    float z = r * r;
+    const float z = r * r;
     float p = 1.9875691500e-4f;
     p = fmaf(p, r, 1.3981999507e-3f);
     p = fmaf(p, r, 8.3334519073e-3f);
     p = fmaf(p, r, 4.1665795894e-2f);
     p = fmaf(p, r, 1.6666665459e-1f);
     p = fmaf(p, r, 5.0000001201e-1f);
-    float y = fmaf(p, z, r);
-    y = y + 1.0f;
-    return __builtin_amdgcn_ldexpf(y, k);
+    const float y = fmaf(p, z, r) + 1.0f;
+    return __builtin_amdgcn_ldexpf(y, (int)fk);
 }
 
 // Live normal at (i,j) of a vertex map (device_helper.cuh:81-110).

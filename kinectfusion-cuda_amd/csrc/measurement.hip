@@ -38,25 +38,46 @@ typedef float BilateralTile[kTile + 6][kTile + 6 + 1];
 // of two; 16 id overflows exactly when the product does), so it is one
 // rounding of c - 16 id with c = -(x^2 + y^2) / 16 exact, i.e. one fused
 // multiply-add on a per-tap constant.
+//
+// Bound: the vector ALU, 49 weights of 22 instructions (exp 16, argument 3,
+// sums 3) and one LDS read per pixel; the 22x22 window costs under 2 reads and
+// conversions per pixel.
+//
+// One column of taps.  CENTRE: the column holding the pixel itself, whose tap
+// has weight exp(0) = 1; 0 * centre makes it NaN for a centre that is not
+// finite, as its inf - inf would.
+template <bool CENTRE>
+__device__ __forceinline__ void bilateral_column(const BilateralTile& tile, int tx, int ty, int x, float center,
+                                                 float& norm, float& acc)
+{
+    const float cx = (float)(x * x) * -0.0625f;
+#pragma unroll
+    for (int y = -3; y <= 3; ++y) {
+        if (CENTRE && y == 0) {
+            const float f = fmaf(center, 0.0f, 1.0f);
+            norm = norm + f;
+            acc = acc + f * center;
+            continue;
+        }
+        const float cur = tile[ty + 3 + y][tx + 3 + x];
+        float id = center - cur;
+        id = id * id;
+        const float f = kf_expf_nonpos(fmaf(id, -16.0f, cx + (float)(y * y) * -0.0625f));
+        norm = norm + f;
+        acc = acc + f * cur;
+    }
+}
 __device__ __forceinline__ float bilateral_at(const BilateralTile& tile, int tx, int ty)
 {
-    float center = tile[ty + 3][tx + 3];
+    const float center = tile[ty + 3][tx + 3];
     float norm = 0.0f, acc = 0.0f;
-    // the outer loop stays rolled: unrolled, all 49 taps' tile reads were held
-    // at once (106 VGPRs, 4 waves per SIMD); rolled, 27 VGPRs and 8 waves
+    // the loops over columns stay rolled: unrolled, all 49 taps' tile reads were
+    // held at once (106 VGPRs, 4 waves per SIMD); rolled, under 32 and 8 waves
 #pragma unroll 1
-    for (int x = -3; x <= 3; ++x) {
-        const float cx = (float)(x * x) * -0.0625f;
-#pragma unroll
-        for (int y = -3; y <= 3; ++y) {
-            float cur = tile[ty + 3 + y][tx + 3 + x];
-            float id = center - cur;
-            id = id * id;
-            float f = kf_expf_nonpos(fmaf(id, -16.0f, cx + (float)(y * y) * -0.0625f));
-            norm = norm + f;
-            acc = acc + f * cur;
-        }
-    }
+    for (int x = -3; x < 0; ++x) bilateral_column<false>(tile, tx, ty, x, center, norm, acc);
+    bilateral_column<true>(tile, tx, ty, 0, center, norm, acc);
+#pragma unroll 1
+    for (int x = 1; x <= 3; ++x) bilateral_column<false>(tile, tx, ty, x, center, norm, acc);
     return acc / norm;
 }
 
