@@ -12,9 +12,6 @@ int launch_bilateral(const float* in, float* out, int w, int h, hipStream_t s);
 int launch_down_sample(const float* in, int w_in, int h_in, float* out, hipStream_t s);
 int launch_vertex_map(const float* depth, float4* out, int w, int h, const float* inv_k, hipStream_t s);
 int launch_normal_map(const float4* v, float4* out, int w, int h, hipStream_t s);
-int launch_preprocess(const uint16_t* raw, int w, int h, float scale, int unmirror, int levels,
-                      const float (*inv_k)[9], float* depth_m, float* const* dpyr, float4* const* vpyr,
-                      float4* const* npyr, hipStream_t s);
 
 // ---- batch ticks (batch.hip): one table per tick in device memory, a header
 // followed by the job arrays of every stage.  Counts are per tick; the fuse
@@ -36,23 +33,26 @@ struct BatchHeader {
 };
 
 // Preprocess of one session: raw codes -> metres (fuse input), bilateral L0,
-// pyramid and vertex maps at 3 levels.
+// pyramid and vertex maps of `levels` levels, normal maps on request.
 struct PreJob {
     const uint16_t* raw;
     float* depth_m;
     float* d0;         // bilateral-filtered level 0
-    float* dmax;       // tile-max maps of depth_m (FuseArgs::dmax layout)
+    float* dmax;       // tile-max maps of depth_m (FuseArgs::dmax layout; optional)
     float4* v[3];      // camera-space vertex maps
-    float* d12[2];     // filtered depth of levels 1 and 2 (optional)
+    float4* n[3];      // camera-space normal maps (all levels or none)
+    float* d12[2];     // one session: filtered depth of levels 1 and 2 (optional)
     int w, h;
+    int levels;        // one session: 1..3, w and h divisible by 2^(levels - 1); a batch tick's jobs have 3
+    int unmirror;      // one session: nonzero reads row j of the frame right to left
     float scale;
     float Kinv[3][9];
     int tile0, tiles_x;    // level-0 16x16 tiles of this job
-    int ptile0, ptiles_x;  // level-2 16x16 tiles of this job
+    int ptile0, ptiles_x;  // batch ticks: level-2 16x16 tiles of this job
 };
 int launch_preprocess_batch(const BatchHeader* hd, const PreJob* jobs, unsigned blocks, hipStream_t s);
-// The same two passes for one session (w, h divisible by 4; no mirror).
-int launch_measure(const PreJob& J, hipStream_t s);
+// The measurement of one session (fills in J.tiles_x).
+int launch_measure(PreJob& J, hipStream_t s);
 
 // ---- TSDF (tsdf.hip)
 constexpr unsigned kFuseBlocks = 2048;  // fuse workgroups: 256 CUs x 8 resident workgroups of 4 waves

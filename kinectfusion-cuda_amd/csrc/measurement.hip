@@ -5,6 +5,8 @@
 // validity in .w).  Every kernel is one thread per output pixel over 16x16
 // tiles (4 waves of 64), with bounds checks, so any frame size works (the
 // reference launches w/8 x h/8 blocks and skips the remainder).
+#include <string.h>
+
 #include "kf_device.hpp"
 #include "kf_kernels.hpp"
 
@@ -146,8 +148,10 @@ __global__ __launch_bounds__(256) void vertex_kernel(const float* __restrict__ d
 
 // ---- the measurement step in two launches (one session or many).
 // Pass 1, per level-0 16x16 tile lt of job J: raw codes -> metres in LDS (the
-// fuse input is written back, with the tile's max valid depth), bilateral
-// filter, level-0 vertex map.
+// fuse input is written back, with the tile's max valid depth when J.dmax is
+// set), bilateral filter, level-0 vertex map.
+// UNMIRROR: row j of the frame is read right to left (measurement.cu:22-25).
+template <bool UNMIRROR>
 __device__ __forceinline__ void measure_tile(const PreJob& J, int lt, BilateralTile& tile, float* wave_max)
 {
     const int t = threadIdx.y * kTile + threadIdx.x;
@@ -156,6 +160,7 @@ __device__ __forceinline__ void measure_tile(const PreJob& J, int lt, BilateralT
     for (int q = t; q < (kTile + 6) * (kTile + 6); q += kTile * kTile) {
         int ly = q / (kTile + 6), lx = q % (kTile + 6);
         int gi = clampi(i0 + lx, 0, J.w - 1), gj = clampi(j0 + ly, 0, J.h - 1);
+        if (UNMIRROR) gi = J.w - 1 - gi;
         tile[ly][lx] = half_rne(J.raw[(int64_t)gj * J.w + gi]) * J.scale;
     }
     __syncthreads();
@@ -170,55 +175,163 @@ __device__ __forceinline__ void measure_tile(const PreJob& J, int lt, BilateralT
         J.d0[q] = d;
         J.v[0][q] = vertex_at(d, i, j, J.Kinv[0]);
     }
+    if (!J.dmax) return;
     dv = kf::wave_max(dv);  // (wave_max below is the LDS array)
     if ((t & 63) == 0) wave_max[t >> 6] = dv;
     __syncthreads();
     if (t == 0) J.dmax[lt] = fmaxf(fmaxf(wave_max[0], wave_max[1]), fmaxf(wave_max[2], wave_max[3]));
 }
 
-// Pass 2, one thread per level-2 pixel of level-2 tile lt: its 4x4 level-0
-// block gives 4 level-1 depths (downSample) and those the level-2 depth; vertex
-// maps of both levels (and the depths, when J.d12 is set).  A workgroup covers
-// a 64x64 level-0 region and also writes its max valid depth.
+// The max valid depth of 64x64 level-0 region (rx, ry) from its 16x16 tiles',
+// by one wave (each row of 16 lanes reads the 16 tiles; past the last tile row
+// or column they repeat it).
+__device__ __forceinline__ void region_max(const PreJob& J, int rx, int ry)
+{
+    const int lane = (threadIdx.y * kTile + threadIdx.x) & 63;
+    const int tx16 = J.tiles_x, ty16 = (J.h + 15) / 16;
+    const int qx = min(rx * 4 + (lane & 3), tx16 - 1), qy = min(ry * 4 + ((lane >> 2) & 3), ty16 - 1);
+    float m = J.dmax[qy * tx16 + qx];
+    m = fmaxf(m, dpp_partner<kDppRowMirror>(m));
+    m = fmaxf(m, dpp_partner<kDppRowHalfMirror>(m));
+    m = fmaxf(m, dpp_partner<kDppXor2>(m));
+    m = fmaxf(m, dpp_partner<kDppXor1>(m));
+    if (lane == 0) J.dmax[tx16 * ty16 + ry * ((J.w + 63) / 64) + rx] = m;
+}
+
+// Pass 2 of many sessions (3 levels, no normals), one thread per level-2 pixel
+// of level-2 tile lt: its 4x4 level-0 block (the frame's width is a multiple of
+// 4, so each row is one 16-byte load) gives 4 level-1 depths (downSample) and
+// those the level-2 depth; vertex maps of both levels.  A workgroup covers a
+// 64x64 level-0 region and also writes its max valid depth.  Bound: HBM.
 __device__ __forceinline__ void pyramid_tile(const PreJob& J, int lt)
 {
-    if (threadIdx.x == 0 && threadIdx.y == 0) {
-        const int tx16 = J.tiles_x, ty16 = (J.h + 15) / 16;
-        const int rx = lt % J.ptiles_x, ry = lt / J.ptiles_x;
-        float m = 0.0f;
-        for (int qy = ry * 4; qy < min(ry * 4 + 4, ty16); ++qy)
-            for (int qx = rx * 4; qx < min(rx * 4 + 4, tx16); ++qx) m = fmaxf(m, J.dmax[qy * tx16 + qx]);
-        J.dmax[tx16 * ty16 + lt] = m;
-    }
-    const int i2 = (lt % J.ptiles_x) * kTile + threadIdx.x, j2 = (lt / J.ptiles_x) * kTile + threadIdx.y;
+    const int t = threadIdx.y * kTile + threadIdx.x;
+    const int rx = lt % J.ptiles_x, ry = lt / J.ptiles_x;
+    if (t < 64) region_max(J, rx, ry);
+    const int i2 = rx * kTile + threadIdx.x, j2 = ry * kTile + threadIdx.y;
     const int w1 = J.w >> 1, w2 = J.w >> 2;
     if (i2 >= w2 || j2 >= (J.h >> 2)) return;
+    float4 r[4];
+#pragma unroll
+    for (int y = 0; y < 4; ++y) r[y] = *reinterpret_cast<const float4*>(J.d0 + (int64_t)(4 * j2 + y) * J.w + 4 * i2);
     float l1[2][2];
 #pragma unroll
-    for (int dy = 0; dy < 2; ++dy)
+    for (int dy = 0; dy < 2; ++dy) {
+        const float4 a = r[2 * dy], b = r[2 * dy + 1];
+        l1[dy][0] = down4(a.x, a.y, b.x, b.y);
+        l1[dy][1] = down4(a.z, a.w, b.z, b.w);
 #pragma unroll
         for (int dx = 0; dx < 2; ++dx) {
             const int i1 = 2 * i2 + dx, j1 = 2 * j2 + dy;
-            const float* r0 = J.d0 + (int64_t)(2 * j1) * J.w + 2 * i1;
-            const float* r1 = r0 + J.w;
-            const float d = down4(r0[0], r0[1], r1[0], r1[1]);
-            l1[dy][dx] = d;
-            J.v[1][(int64_t)j1 * w1 + i1] = vertex_at(d, i1, j1, J.Kinv[1]);
-            if (J.d12[0]) J.d12[0][(int64_t)j1 * w1 + i1] = d;
+            J.v[1][(int64_t)j1 * w1 + i1] = vertex_at(l1[dy][dx], i1, j1, J.Kinv[1]);
         }
+    }
     const float d2 = down4(l1[0][0], l1[0][1], l1[1][0], l1[1][1]);
     J.v[2][(int64_t)j2 * w2 + i2] = vertex_at(d2, i2, j2, J.Kinv[2]);
-    if (J.d12[1]) J.d12[1][(int64_t)j2 * w2 + i2] = d2;
+}
+
+// Pass 2 of one session, per 32x32 level-0 region lt: the depths of levels 1 and 2
+// (downSample), their vertex maps and, when J.n is set, the normals of every
+// level, all from the region's filtered depths in LDS.  A normal needs its right
+// and lower neighbour (device_helper.cuh:81-110): one more column and row per
+// level, so 36x36 level-0 depths feed 18x18 of level 1 and 9x9 of level 2, and
+// the neighbours' vertices are formed again from those depths (15 operations)
+// instead of read back (48 bytes).  Depths outside the image are 0 here, which
+// makes their vertices invalid as device_helper.cuh:43-50 has it.
+//
+// Bound: launch and memory latency.  32x32 regions give a 640x480 frame 300
+// workgroups; the 64x64 ones above (80) leave most of the chip idle.  Many
+// sessions fill the chip either way, and there the regions' barriers cost: 64
+// frames of 640x480 took 109 us by regions, 50 us by the form above (73 us with
+// its depths read one by one).  Measured
+// against one launch per level and map: kf_preprocess with normals 160x120
+// 30.9 -> 12.2 us, 640x480 30.0 -> 18.5 us, 1276x716 53.8 -> 33.7 us.
+constexpr int kRegion = 32;
+struct PyramidTile {
+    float d0[kRegion + 4][kRegion + 5];
+    float d1[kRegion / 2 + 2][kRegion / 2 + 3];
+    float d2[kRegion / 4 + 1][kRegion / 4 + 1];
+};
+template <class Row>
+__device__ __forceinline__ float4 normal_from_depths(const Row& d, int x, int y, int i, int j, const float* ki)
+{
+    NormalStencil s;
+    s.c = vertex_at(d[y][x], i, j, ki);
+    s.r = vertex_at(d[y][x + 1], i + 1, j, ki);
+    s.d = vertex_at(d[y + 1][x], i, j + 1, ki);
+    return normal_of(s);
+}
+
+__device__ __forceinline__ void pyramid_region(const PreJob& J, int lt, PyramidTile& T)
+{
+    const int t = threadIdx.y * kTile + threadIdx.x;
+    const int rtx = (J.w + kRegion - 1) / kRegion, rx = lt % rtx, ry = lt / rtx;
+    const int x0 = rx * kRegion, y0 = ry * kRegion;
+    const bool normals = J.n[0] != nullptr;
+    const int halo = normals ? 4 : 0, e0 = kRegion + halo;
+    for (int q = t; q < e0 * e0; q += kTile * kTile) {
+        const int y = q / e0, x = q - y * e0;
+        const bool in = x0 + x < J.w && y0 + y < J.h;
+        T.d0[y][x] = in ? J.d0[(int64_t)(y0 + y) * J.w + (x0 + x)] : 0.0f;
+    }
+    if (J.dmax && !(rx & 1) && !(ry & 1) && t >= 192) region_max(J, rx >> 1, ry >> 1);
+    __syncthreads();
+    if (normals) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int x = t & 31, y = (t >> 5) + 8 * q, i = x0 + x, j = y0 + y;
+            if (i < J.w && j < J.h) J.n[0][(int64_t)j * J.w + i] = normal_from_depths(T.d0, x, y, i, j, J.Kinv[0]);
+        }
+    }
+    if (J.levels < 2) return;  // uniform
+    const int w1 = J.w >> 1, h1 = J.h >> 1, e1 = kRegion / 2 + (normals ? 2 : 0);
+    for (int q = t; q < e1 * e1; q += kTile * kTile) {
+        const int y = q / e1, x = q - y * e1;
+        T.d1[y][x] = down4(T.d0[2 * y][2 * x], T.d0[2 * y][2 * x + 1], T.d0[2 * y + 1][2 * x], T.d0[2 * y + 1][2 * x + 1]);
+    }
+    __syncthreads();
+    {
+        const int x = threadIdx.x, y = threadIdx.y, i = x0 / 2 + x, j = y0 / 2 + y;
+        if (i < w1 && j < h1) {
+            const int64_t q = (int64_t)j * w1 + i;
+            const float d = T.d1[y][x];
+            J.v[1][q] = vertex_at(d, i, j, J.Kinv[1]);
+            if (J.d12[0]) J.d12[0][q] = d;
+            if (normals) J.n[1][q] = normal_from_depths(T.d1, x, y, i, j, J.Kinv[1]);
+        }
+    }
+    if (J.levels < 3) return;
+    const int w2 = J.w >> 2, h2 = J.h >> 2, e2 = kRegion / 4 + (normals ? 1 : 0);
+    if (t < e2 * e2) {
+        const int y = t / e2, x = t - y * e2;
+        T.d2[y][x] = down4(T.d1[2 * y][2 * x], T.d1[2 * y][2 * x + 1], T.d1[2 * y + 1][2 * x], T.d1[2 * y + 1][2 * x + 1]);
+    }
+    __syncthreads();
+    if (t < 64) {
+        const int x = t & 7, y = t >> 3, i = x0 / 4 + x, j = y0 / 4 + y;
+        if (i < w2 && j < h2) {
+            const int64_t q = (int64_t)j * w2 + i;
+            const float d = T.d2[y][x];
+            J.v[2][q] = vertex_at(d, i, j, J.Kinv[2]);
+            if (J.d12[1]) J.d12[1][q] = d;
+            if (normals) J.n[2][q] = normal_from_depths(T.d2, x, y, i, j, J.Kinv[2]);
+        }
+    }
 }
 
 // One session: one workgroup per tile, the job by value.
+template <bool UNMIRROR>
 __global__ __launch_bounds__(256) void measure_kernel(PreJob J)
 {
     __shared__ BilateralTile tile;
     __shared__ float wave_max[4];
-    measure_tile(J, blockIdx.x, tile, wave_max);
+    measure_tile<UNMIRROR>(J, blockIdx.x, tile, wave_max);
 }
-__global__ __launch_bounds__(256) void pyramid_kernel(PreJob J) { pyramid_tile(J, blockIdx.x); }
+__global__ __launch_bounds__(256) void pyramid_kernel(PreJob J)
+{
+    __shared__ PyramidTile T;
+    pyramid_region(J, blockIdx.x, T);
+}
 
 // Many sessions per launch (batch ticks), persistent over the tick's tiles.
 // The first kernel also clears the tick's fuse-list counter and raycast tile
@@ -235,7 +348,7 @@ __global__ __launch_bounds__(256) void measure_batch_kernel(const BatchHeader* h
     const int tiles = hd->pre_tiles, njobs = hd->n_pre;
     for (int tl = blockIdx.x; tl < tiles; tl += gridDim.x) {
         const PreJob& J = jobs[job_of(jobs, njobs, tl, [](const PreJob& x) { return x.tile0; })];
-        measure_tile(J, tl - J.tile0, tile, wave_max);
+        measure_tile<false>(J, tl - J.tile0, tile, wave_max);
     }
 }
 
@@ -293,13 +406,19 @@ int launch_normal_map(const float4* v, float4* out, int w, int h, hipStream_t s)
     return KF_OK;
 }
 
-int launch_measure(const PreJob& J, hipStream_t s)
+int launch_measure(PreJob& J, hipStream_t s)
 {
-    const int tiles = J.tiles_x * ((J.h + 15) / 16), ptiles = J.ptiles_x * ((J.h / 4 + 15) / 16);
-    measure_kernel<<<(unsigned)tiles, dim3(kTile, kTile), 0, s>>>(J);
+    J.tiles_x = (J.w + kTile - 1) / kTile;
+    const unsigned tiles = (unsigned)(J.tiles_x * ((J.h + kTile - 1) / kTile));
+    if (J.unmirror) measure_kernel<true><<<tiles, dim3(kTile, kTile), 0, s>>>(J);
+    else measure_kernel<false><<<tiles, dim3(kTile, kTile), 0, s>>>(J);
     KF_LAUNCHED("measure_kernel");
-    pyramid_kernel<<<(unsigned)ptiles, dim3(kTile, kTile), 0, s>>>(J);
-    KF_LAUNCHED("pyramid_kernel");
+    // pass 2 has work for a pyramid, normals or the 64x64 tile maxima
+    if (J.levels > 1 || J.n[0] || J.dmax) {
+        const int regions = ((J.w + kRegion - 1) / kRegion) * ((J.h + kRegion - 1) / kRegion);
+        pyramid_kernel<<<(unsigned)regions, dim3(kTile, kTile), 0, s>>>(J);
+        KF_LAUNCHED("pyramid_kernel");
+    }
     return KF_OK;
 }
 
@@ -309,24 +428,6 @@ int launch_preprocess_batch(const BatchHeader* hd, const PreJob* jobs, unsigned 
     KF_LAUNCHED("measure_batch_kernel");
     pyramid_batch_kernel<<<blocks, dim3(kTile, kTile), 0, s>>>(hd, jobs);
     KF_LAUNCHED("pyramid_batch_kernel");
-    return KF_OK;
-}
-
-int launch_preprocess(const uint16_t* raw, int w, int h, float scale, int unmirror, int levels,
-                      const float (*inv_k)[9], float* depth_m, float* const* dpyr, float4* const* vpyr,
-                      float4* const* npyr, hipStream_t s)
-{
-    int st;
-    if ((st = launch_convert(raw, depth_m, w, h, scale, unmirror, s))) return st;
-    if ((st = launch_bilateral(depth_m, dpyr[0], w, h, s))) return st;
-    if ((st = launch_vertex_map(dpyr[0], vpyr[0], w, h, inv_k[0], s))) return st;
-    for (int l = 1; l < levels; ++l) {
-        if ((st = launch_down_sample(dpyr[l - 1], w >> (l - 1), h >> (l - 1), dpyr[l], s))) return st;
-        if ((st = launch_vertex_map(dpyr[l], vpyr[l], w >> l, h >> l, inv_k[l], s))) return st;
-    }
-    if (npyr)
-        for (int l = 0; l < levels; ++l)
-            if ((st = launch_normal_map(vpyr[l], npyr[l], w >> l, h >> l, s))) return st;
     return KF_OK;
 }
 
@@ -409,16 +510,24 @@ int kf_preprocess(const uint16_t* raw, int w, int h, float scale, int unmirror, 
         return kf::fail(KF_ERR_DIMS, "Can't construct pyramid. Dimensions must be divisible by 2^(m_n_layers - 1).");
     hipStream_t s = kf::stream_of(stream);
     kf::CallTimer t(elapsed_ms, s);
-    float4* vp[3] = {nullptr, nullptr, nullptr};
-    float4* np[3] = {nullptr, nullptr, nullptr};
+    kf::PreJob J;
+    memset(&J, 0, sizeof(J));
+    J.raw = raw;
+    J.depth_m = depth_m;
+    J.d0 = depth_pyr[0];
     for (int l = 0; l < levels; ++l) {
-        vp[l] = reinterpret_cast<float4*>(vertex_pyr[l]);
-        if (normal_pyr) np[l] = reinterpret_cast<float4*>(normal_pyr[l]);
+        J.v[l] = reinterpret_cast<float4*>(vertex_pyr[l]);
+        if (normal_pyr) J.n[l] = reinterpret_cast<float4*>(normal_pyr[l]);
+        if (l > 0) J.d12[l - 1] = depth_pyr[l];
+        memcpy(J.Kinv[l], inv_k[l], sizeof(J.Kinv[l]));
     }
+    J.w = w;
+    J.h = h;
+    J.levels = levels;
+    J.unmirror = unmirror;
+    J.scale = scale;
     int st;
-    if ((st = t.start()) || (st = kf::launch_preprocess(raw, w, h, scale, unmirror, levels, inv_k, depth_m, depth_pyr,
-                                                        vp, normal_pyr ? np : nullptr, s)))
-        return st;
+    if ((st = t.start()) || (st = kf::launch_measure(J, s))) return st;
     return t.finish();
 }
 

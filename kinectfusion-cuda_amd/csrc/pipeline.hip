@@ -170,47 +170,36 @@ int kf_pipeline_frame(kf_pipeline* p, const uint16_t* raw)
     }
     int st;
     kf::PoseState* state = p->icp->state;
-    // the fused two-pass measurement (metres, bilateral, pyramid, vertex maps and
-    // the fuse's tile-max maps) when the frame allows it; else the stage kernels
-    const bool fused = !p->cfg.unmirror && p->levels == 3 && w % 4 == 0 && h % 4 == 0;
-    if (fused) {
-        kf::PreJob J;
-        memset(&J, 0, sizeof(J));
-        J.raw = raw;
-        J.depth_m = p->depth_m;
-        J.d0 = p->dpyr[0];
-        J.dmax = kf::volume_depth_max(p->vol, w, h, s);
-        if (!J.dmax) return kf::fail(KF_ERR_OOM, "kf_pipeline_frame: depth tile-max maps");
-        for (int l = 0; l < 3; ++l) J.v[l] = p->vpyr[l];
-        J.d12[0] = p->dpyr[1];
-        J.d12[1] = p->dpyr[2];
-        J.w = w;
-        J.h = h;
-        J.scale = p->cfg.depth_scale;
-        memcpy(J.Kinv, p->Ki, sizeof(J.Kinv));
-        J.tiles_x = (w + 15) / 16;
-        J.ptiles_x = (w / 4 + 15) / 16;
-        if ((st = kf::launch_measure(J, s))) return st;
-        p->normals_fresh = false;
-    }
+    // the two-pass measurement: metres, bilateral, pyramid, vertex maps and the
+    // fuse's tile-max maps (depthFrameToVertexPyramid, kinect_fusion.cpp:116-135).
+    // ICP computes the live normals itself, so the normal pyramid is only built
+    // when a caller asks for it.
+    kf::PreJob J;
+    memset(&J, 0, sizeof(J));
+    J.raw = raw;
+    J.depth_m = p->depth_m;
+    J.d0 = p->dpyr[0];
+    J.dmax = kf::volume_depth_max(p->vol, w, h, s);
+    if (!J.dmax) return kf::fail(KF_ERR_OOM, "kf_pipeline_frame: depth tile-max maps");
+    for (int l = 0; l < p->levels; ++l) J.v[l] = p->vpyr[l];
+    J.d12[0] = p->dpyr[1];
+    J.d12[1] = p->dpyr[2];
+    J.w = w;
+    J.h = h;
+    J.levels = p->levels;
+    J.unmirror = p->cfg.unmirror;
+    J.scale = p->cfg.depth_scale;
+    memcpy(J.Kinv, p->Ki, sizeof(J.Kinv));
+    if ((st = kf::launch_measure(J, s))) return st;
+    p->normals_fresh = false;
     if (p->frame == 0) {
-        // initializeTracking (kinect_fusion.cpp:75-94): convert and fuse at the initial pose
-        if (!fused && (st = kf::launch_convert(raw, p->depth_m, w, h, p->cfg.depth_scale, p->cfg.unmirror, s)))
-            return st;
+        // initializeTracking (kinect_fusion.cpp:75-94): fuse at the initial pose
         if (p->timing) {
             KF_HIP(hipEventRecord(ev[1], s));
             KF_HIP(hipEventRecord(ev[2], s));
             KF_HIP(hipEventRecord(ev[3], s));
         }
     } else {
-        // depthFrameToVertexPyramid (kinect_fusion.cpp:116-135); ICP computes the live
-        // normals itself, so the normal pyramid is only built when a caller asks for it
-        if (!fused) {
-            if ((st = kf::launch_preprocess(raw, w, h, p->cfg.depth_scale, p->cfg.unmirror, p->levels, p->Ki,
-                                            p->depth_m, p->dpyr, p->vpyr, nullptr, s)))
-                return st;
-            p->normals_fresh = false;
-        }
         if (p->timing) KF_HIP(hipEventRecord(ev[1], s));
         // raycastTsdf (kinect_fusion.cpp:137-144) at the previous pose
         if ((st = kf::launch_raycast_levels(p->vol, nullptr, state, p->levels, p->Ki, p->pv, p->pn, w, h, s)))
@@ -228,7 +217,7 @@ int kf_pipeline_frame(kf_pipeline* p, const uint16_t* raw)
     }
     // fuseCurrentDepthToTSDF (kinect_fusion.cpp:179-183): unfiltered metres at the new pose
     if ((st = kf::launch_fuse(p->depth_m, w, h, p->vol, p->K[0], nullptr, state, s, p->timing ? ev + 5 : nullptr,
-                              fused)))
+                              true)))
         return st;
     if (p->timing) KF_HIP(hipEventRecord(ev[4], s));
     // the visualisation volume takes the same depth at the same pose (kinect_fusion.cpp:179-183)

@@ -1,0 +1,60 @@
+"""Edges of the kernels' tiles and dispatch rules, against the oracle."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from gpu_util import announce, small_sequence
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def kf():
+    import kfusion
+    kfusion.init()
+    return kfusion
+
+
+def same(got, ref, what):
+    """The same bits, any NaN for a NaN (its sign and payload are the platform's)."""
+    nan = np.isnan(ref)
+    np.testing.assert_array_equal(np.isnan(got), nan, err_msg=what)
+    np.testing.assert_array_equal(np.where(nan, 0, got.view(np.uint32)), np.where(nan, 0, ref.view(np.uint32)),
+                                  err_msg=what)
+
+
+# (w, h, levels): one pixel, under and over the 16-pixel tile and the 32-pixel region, odd sizes, and
+# sizes whose last region holds one coarse pixel
+@pytest.mark.parametrize("w,h,levels", [(1, 1, 1), (15, 17, 1), (33, 31, 1), (2, 2, 2), (34, 62, 2), (66, 18, 2),
+                                        (4, 4, 3), (28, 32, 3), (36, 68, 3), (132, 100, 3)])
+@pytest.mark.parametrize("mirrored", [0, 1])
+@pytest.mark.parametrize("normals", [0, 1])
+def test_preprocess_edges_bit_exact(kf, oracle32, w, h, levels, mirrored, normals):
+    announce(f"kf_preprocess {w}x{h}, {levels} levels, mirrored {mirrored}, normals {normals}")
+    rng = np.random.default_rng(100 * w + h)
+    raw_h = (1500 + 400 * rng.random((h, w))).astype(np.uint16)
+    raw_h[rng.random((h, w)) < 0.05] = 0       # holes
+    raw_h[rng.random((h, w)) < 0.02] = 65535   # +inf codes
+    raw = kf.DeviceArray.from_host(raw_h)
+    dm = kf.GridMap(w, h)
+    dp = [kf.GridMap(w >> l, h >> l) for l in range(levels)]
+    vp = [kf.GridMap(w >> l, h >> l, 4) for l in range(levels)]
+    npm = [kf.GridMap(w >> l, h >> l, 4) for l in range(levels)]
+    Ks = [oracle32.intrinsics(525.0, 525.0, w / 2 - 0.5, h / 2 - 0.5, l) for l in range(3)]
+    kinv = np.ascontiguousarray(np.stack([k[1] for k in Ks]))
+    arr = lambda maps: (C.c_void_p * levels)(*[m.ptr.value for m in maps])  # noqa: E731
+    kf.check(kf.lib().kf_preprocess(raw.ptr, w, h, 1e-3, mirrored, levels, kinv.ctypes.data_as(C.c_void_p), dm.ptr,
+                                    arr(dp), arr(vp), arr(npm) if normals else None, None, None), "kf_preprocess")
+    kf.check(kf.lib().kf_device_synchronize())
+    ref = oracle32.convert_to_depth_meters(raw_h, 1e-3, bool(mirrored))
+    same(dm.download(), ref, "metres")
+    d = oracle32.apply_bilateral_filter(ref)
+    for l in range(levels):
+        if l:
+            d = oracle32.down_sample(d)
+        v = oracle32.create_vertex_map(d, Ks[l][1])
+        same(dp[l].download(), d, f"depth L{l}")
+        same(vp[l].download(), v, f"vertex L{l}")
+        if normals:
+            same(npm[l].download(), oracle32.create_normal_map(v), f"normal L{l}")
