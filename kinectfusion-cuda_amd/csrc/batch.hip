@@ -145,9 +145,9 @@ int alloc(void** p, size_t bytes, size_t* acc)
 
 size_t volume_meta_bytes(int n)
 {
-    const size_t nb = (size_t)n / 8, ns = (nb + 7) / 8;
+    const size_t nb = (size_t)n / 8;
     return (sizeof(float) + sizeof(float4)) * n + sizeof(unsigned long long) * kf::kFuseBlocks +
-           nb * nb * nb * (sizeof(int) + sizeof(int)) + ns * ns * ns * sizeof(int) + 2 * sizeof(unsigned);
+           nb * nb * nb * (sizeof(int) + 1) + sizeof(unsigned long long) * kf::free_words(n / 8) + 2 * sizeof(unsigned);
 }
 
 size_t maps_bytes(int w, int h)
@@ -603,6 +603,7 @@ int kf_batch_tick(kf_batch* b, int n, const int* ids, const uint16_t* const* raw
     int ray_tiles = 0, pre_tiles = 0, pyr_tiles = 0;
     int icp_blocks[3] = {0, 0, 0};
     unsigned bricks = 0;
+    int dist_tiles = 0;
     int n_ray = 0, n_icp = 0;
     for (int k = 0; k < n; ++k) {
         Session& q = b->sess[ids[k]];
@@ -655,6 +656,8 @@ int kf_batch_tick(kf_batch* b, int n, const int* ids, const uint16_t* const* raw
         F.a = kf::fuse_args(q.depth_m, w, h, q.vol, q.K[0], nullptr, q.st);
         F.a.dmax = q.dmax;
         F.brick0 = bricks;
+        F.dist_tile0 = dist_tiles;
+        dist_tiles += kf::dist_tiles(q.cfg.volume_n / 8);
         const unsigned nb = (unsigned)(q.cfg.volume_n / 8);
         bricks += nb * nb * nb;
     }
@@ -695,6 +698,7 @@ int kf_batch_tick(kf_batch* b, int n, const int* ids, const uint16_t* const* raw
     for (int l = 0; l < 3; ++l) hd->icp_blocks[l] = icp_blocks[l];
     hd->n_fuse = n;
     hd->fuse_bricks = bricks;
+    hd->dist_tiles = dist_tiles;
 
     // ---- launch
     if (b->tuning) {

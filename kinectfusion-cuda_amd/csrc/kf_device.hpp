@@ -286,31 +286,43 @@ __device__ __forceinline__ uint32_t brick_oz(int nb, int k)
 {
     return __umul24((uint32_t)(k >> 3), ((uint32_t)nb * (uint32_t)nb) << 9) + (uint32_t)(k & 7);
 }
-// Linear index of cell (x, y, z) of an m^3 grid (bricks or super-bricks:
-// m <= 128), in 24-bit multiplies.
+// Linear index of cell (x, y, z) of an m^3 grid of bricks (m <= 128), in 24-bit
+// multiplies.
 __device__ __forceinline__ int grid_index(int x, int y, int z, int m)
 {
     return (int)(__umul24(__umul24((uint32_t)z, (uint32_t)m) + (uint32_t)y, (uint32_t)m) + (uint32_t)x);
 }
 
-// Brick bounds (raycast skipping): brick (bi, bj, bk) keeps a lower bound of F
-// over its halo, the voxels [8bi, 8bi + 8] x [8bj, 8bj + 8] x [8bk, 8bk + 8]
-// clamped to the volume: its own 512 voxels and the first voxel plane of its
-// +x, +y and +z neighbours.  A trilinear stencil spans (i0, i0 + 1) per axis
-// (clamped), so the bound of the brick holding its first corner (i0, j0, k0)
-// covers all 8 corners, also where the stencil crosses into the next brick.
-// Several waves lower one bound in a fuse (the brick's own and those of the
-// bricks whose halo reaches into it), so it is kept as an ordered integer key
-// (order_key) and lowered with an integer atomicMin.
-// Super-bricks: 8x8x8 bricks (64^3 voxels) carry a lower bound of F over their
-// own voxels too, in the same key form.
-constexpr int kSuper = 64;
-__device__ __forceinline__ int order_key(float f)
+// Free bricks (raycast skipping): brick (bi, bj, bk) keeps two bits about F over
+// its halo, the voxels [8bi, 8bi + 8] x [8bj, 8bj + 8] x [8bk, 8bk + 8] clamped
+// to the volume: its own 512 voxels and the first voxel plane of its +x, +y and
+// +z neighbours.  A trilinear stencil spans (i0, i0 + 1) per axis (clamped), so
+// the halo of the brick holding its first corner (i0, j0, k0) covers all 8
+// corners, also where the stencil crosses into the next brick.  The first bit
+// says that every value there has been at least kSkipBound, the second that
+// every one has been non-negative; a fuse clears them (atomicAnd: several waves
+// may clear bits of one word), only a new start or an upload sets them.
+// A sample matters to a march on a large step only when it may be below 0.99: a
+// stencil of values >= 0.991 is above it (convex weights; 1e-3 covers the
+// rounding of the three lerp levels).  On a small step only a negative sample
+// matters: non-negative corners and weights give a non-negative value in any
+// rounding.
+//
+// Free distances: from these bits every fuse forms, per brick and kind of step,
+// how many bricks (Chebyshev) it is away from the nearest brick that is not
+// free, at most kDistMax.  With distance D >= 1 every brick within D - 1 of this
+// one is free, so the box of bricks around it holds no first corner of a stencil
+// that matters (outside the volume counts as free: stencils clamp into the edge
+// bricks).
+constexpr float kSkipBound = 0.991f;
+constexpr int kDistRadius = 8, kDistMax = kDistRadius + 1;  // in a byte, low 4 bits: large steps, high 4: small
+// The word of bit x & 63 of brick (x, y, z), kind h (0: large steps, 1: small):
+// rows of bricks along x, one or two words per kind.
+__host__ __device__ __forceinline__ size_t free_word(int nb, int x, int y, int z, int h)
 {
-    int b = __float_as_int(f);
-    return b >= 0 ? b : (b ^ 0x7fffffff);
+    const int W = nb > 64 ? 2 : 1;
+    return (((size_t)z * nb + y) * 2 + h) * W + (x >> 6);
 }
-__device__ __forceinline__ float order_value(int k) { return __int_as_float(k >= 0 ? k : (k ^ 0x7fffffff)); }
 
 // snorm16 TSDF codes (precision form): f = q / 32767 with q in [-32767, 32767];
 // the code snorm16 leaves unused, -32768, holds the unobserved value 2 of
@@ -328,6 +340,17 @@ __device__ __forceinline__ int16_t snorm_encode(float f)
     float s = f * kSnormScale;
     s = fminf(fmaxf(s, -kSnormScale), kSnormScale);
     return (int16_t)rintf(s);
+}
+
+// x / b rounded to nearest from y = RN(1/b): q = RN(x*y), r = x - b*q (exact by
+// the fused multiply-add), RN(q + r*y) is RN(x/b) for every x and b whose
+// quotient and residual neither overflow nor underflow (Markstein's theorem;
+// checked on the CPU over the operand ranges: tests/test_exact_division.py).
+__device__ __forceinline__ float div_by_exact_reciprocal(float x, float b, float y)
+{
+    const float q = x * y;
+    const float r = fmaf(-q, b, x);
+    return fmaf(r, y, q);
 }
 
 // Rank of workgroup g among G such that the ranks on one XCD (workgroups are

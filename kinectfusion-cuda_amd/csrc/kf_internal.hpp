@@ -79,9 +79,8 @@ struct kf_volume {
     float* zk = nullptr;      // z coordinate of each k slice (repeated addition, tsdf.cu:27-31)
     float4* zt = nullptr;     // per fuse: the inverse pose's z terms of each k slice (FuseArgs::zt)
     unsigned long long* touched = nullptr;  // per-workgroup counts of fused voxels (summed on read)
-    int* brick_key = nullptr;               // per-brick halo lower bound of F, order_key form (raycast skipping)
-    int* super_key = nullptr;               // per-super-brick lower bound of F (order_key)
-    int ns = 0;                             // super-bricks per axis (ceil(nb / 8))
+    unsigned long long* free_bits = nullptr;  // per-brick free bits (raycast skipping)
+    uint8_t* dist = nullptr;                  // per-brick free distances, formed from free_bits
     int* brick_list = nullptr;              // visible bricks of the current fuse
     unsigned int* list_count = nullptr;     // list lengths, double-buffered by launch parity
     float* dmax = nullptr;                  // max valid depth per 16x16 and per 64x64 pixel tile

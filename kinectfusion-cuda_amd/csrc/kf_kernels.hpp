@@ -23,6 +23,7 @@ struct BatchHeader {
     int n_icp, icp_blocks[3];         // ICP sessions, blocks per level
     int n_fuse;                       // fuse jobs
     unsigned fuse_bricks;             // bricks over all fuse jobs
+    int dist_tiles;                   // free-distance tiles over all fuse jobs
     unsigned* fuse_count;
     unsigned long long* fuse_list;    // job << 32 | brick of the job's volume
     unsigned long long* touched;
@@ -71,9 +72,8 @@ struct FuseArgs {
     void* f;
     void* wt;
     unsigned long long* touched;
-    int* brick_key;
-    int* super_key;
-    int ns;
+    unsigned long long* free_bits;  // per-brick free bits (kf_device.hpp)
+    uint8_t* dist;  // per-brick free distances, formed from free_bits after the sweep
     int cull;     // 1 when K is a plain pinhole matrix (culling planes valid)
     // lengths of the culling planes' normals |(fx, cx)|, |(fx, w - cx)|, |(fy, cy)|,
     // |(fy, h - cy)|, rounded up (they scale the bounding-sphere radius)
@@ -92,7 +92,11 @@ inline size_t depth_max_floats(int w, int h)
 struct FuseJob {
     FuseArgs a;       // a.dyn set: the session's committed pose
     unsigned brick0;  // first global brick index of this job
+    int dist_tile0;   // first 8x8-row tile of this job's free distances
 };
+// Workgroups of one volume's free distances: one per 8x8 rows of bricks.
+inline size_t free_words(int nb) { return (size_t)nb * nb * 2 * (nb > 64 ? 2 : 1); }
+inline int dist_tiles(int nb) { return ((nb + 7) / 8) * ((nb + 7) / 8); }
 FuseArgs fuse_args(const float* depth, int w, int h, const kf_volume* v, const float* K, const float* inv_pose,
                    const PoseState* dyn_state);
 // mid (optional): an event recorded between the brick cull and the sweep.
@@ -114,11 +118,10 @@ int volume_create(int n, float width_m, float mue_m, int format, hipStream_t s, 
 // ---- raycast (raycast.hip)
 struct RaycastVolume {
     const void* f;
-    const int* brick_key;    // per-brick halo lower bound of F, order_key form (null: no skipping)
-    const int* super_key;    // per-super-brick lower bound of F, order_key form
-    int n, nb, ns, format;
+    const uint8_t* dist;     // per-brick free distances (kf_device.hpp)
+    int n, nb, format;
     float width, mue;
-    float inv_width;  // 1 / width when width is a power of two (then x * inv_width == x / width), else 0
+    float inv_width;  // 1 / width correctly rounded
     int p2;           // width and n are powers of two (the march's texel coordinates are then exact)
 };
 struct RaycastLevel {
@@ -128,13 +131,12 @@ struct RaycastLevel {
     int w, h, tiles_x, tile0;  // tile0: first global tile of this level
 };
 // A ray the per-lane march handed to the finishing pass: its march state
-// before the sample at t (that sample already counted in guard).
+// before the sample at t.
 struct DeferredRay {
     int job;    // pyramid level (single launch) or raycast job (batch)
     int px;     // j * w + i
-    int guard;  // samples counted, the one at t included
     int flags;  // bit 0: the last sample was skipped (prev comes from prev_t), bit 1: small steps
-    float t, prev, prev_t, pad;
+    float t, prev, prev_t, pad[2];
 };
 // One (session, level) of a batched raycast; lives in device memory.
 struct RaycastJob {

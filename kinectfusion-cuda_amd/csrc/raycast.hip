@@ -21,27 +21,16 @@ namespace kf {
 
 namespace {
 
-constexpr int kMaxMarchSteps = 1 << 20;
-// Skipping: a brick's bound covers every stencil whose first corner lies in it
-// (its halo, kf_device.hpp), a super-brick's the stencils inside it.  On a
-// large step a sample whose bound is at least kSkipBound is >= 0.99 (convex
-// weights; 1e-3 of margin covers the rounding of the three lerp levels), so
-// it can neither end the march nor shorten the step.  On a small step only a
-// negative sample changes the march (the step is already small), and a sample
-// whose bound is >= 0 is >= 0 (non-negative corners and weights give a
-// non-negative value in any rounding), so kSmallSkipBound = 0 applies there.
-// A skipped sample only sets prev_t; its value is computed if and when the
-// zero-crossing formula needs it.
-constexpr float kSkipBound = 0.991f;
-constexpr float kSmallSkipBound = 0.0f;
-
-
-// The fast skip test works on texel coordinates computed with a reciprocal
-// instead of the exact division (a few 1e-5 voxel apart): a sample counts as
-// inside a region only when its coordinate is at least kMargin voxel inside it,
-// so its exact stencil is inside that region too.
+// Skipping: a sample is skipped when its stencil certainly lies in the box of
+// free bricks around its brick (the free distances, kf_device.hpp): it can then
+// neither end the march nor change its step.  A skipped sample only sets prev_t;
+// its value is computed if and when the zero-crossing formula needs it.
+//
+// The test works on texel coordinates computed with a reciprocal instead of
+// the exact division (a few 1e-5 voxel apart): a sample counts as inside a box
+// only when its coordinate is at least kMargin voxel inside it, so its exact
+// stencil is inside the box too.
 constexpr float kMargin = 0.01f;
-
 
 // Dispatch order of the first pass.  Workgroup g of a level runs on XCD
 // g % 8 and takes the (g / 8)-th tile of its level's band on that XCD; which
@@ -74,14 +63,12 @@ struct RaycastArgs {
 };
 
 
-// Normalized texture coordinate x / width + 1/2 of a world coordinate.  For a
-// power-of-two width the quotient is the product with the exact reciprocal
-// (the same real number, so the same rounding), which skips the division; the
-// product is exact (or far below the half's ulp), so fusing it with the
-// addition rounds the same way.
+// Normalized texture coordinate x / width + 1/2 of a world coordinate, the
+// quotient from the exact reciprocal (three operations; x / width in every
+// bit: for an x so small that its residual underflows the sum is 1/2 either way).
 __device__ __forceinline__ float tex(const RaycastVolume& a, float x)
 {
-    return a.inv_width != 0.0f ? fmaf(x, a.inv_width, 0.5f) : x / a.width + 0.5f;
+    return div_by_exact_reciprocal(x, a.width, a.inv_width) + 0.5f;
 }
 
 // Approximate texel coordinate of a world coordinate for the skip tests only
@@ -154,20 +141,23 @@ __device__ __forceinline__ void cell_offsets(int nb, const Stencil& t, uint32_t*
     o[7] = x1 + y1z1;
 }
 
+__device__ __forceinline__ float lerp_cell(const float* v, float a, float b, float c)
+{
+    const float e00 = (1.0f - a) * v[0] + a * v[1], e10 = (1.0f - a) * v[2] + a * v[3];
+    const float e01 = (1.0f - a) * v[4] + a * v[5], e11 = (1.0f - a) * v[6] + a * v[7];
+    const float g0 = (1.0f - b) * e00 + b * e10, g1 = (1.0f - b) * e01 + b * e11;
+    return (1.0f - c) * g0 + c * g1;
+}
+
 template <int FMT>
 __device__ __forceinline__ float trilinear(const void* F, int nb, const Stencil& t)
 {
     uint32_t o[8];
+    float v[8];
     cell_offsets(nb, t, o);
-    float c000 = voxel_at<FMT>(F, o[0]), c100 = voxel_at<FMT>(F, o[1]);
-    float c010 = voxel_at<FMT>(F, o[2]), c110 = voxel_at<FMT>(F, o[3]);
-    float c001 = voxel_at<FMT>(F, o[4]), c101 = voxel_at<FMT>(F, o[5]);
-    float c011 = voxel_at<FMT>(F, o[6]), c111 = voxel_at<FMT>(F, o[7]);
-    const float a = t.a, b = t.b, c = t.c;
-    float e00 = (1.0f - a) * c000 + a * c100, e10 = (1.0f - a) * c010 + a * c110;
-    float e01 = (1.0f - a) * c001 + a * c101, e11 = (1.0f - a) * c011 + a * c111;
-    float g0 = (1.0f - b) * e00 + b * e10, g1 = (1.0f - b) * e01 + b * e11;
-    return (1.0f - c) * g0 + c * g1;
+#pragma unroll
+    for (int q = 0; q < 8; ++q) v[q] = voxel_at<FMT>(F, o[q]);
+    return lerp_cell(v, t.a, t.b, t.c);
 }
 
 template <int FMT, bool P2>
@@ -176,182 +166,80 @@ __device__ __forceinline__ float sample_tsdf(const void* F, int n, int nb, float
     return trilinear<FMT>(F, nb, stencil<P2>(n, u, v, s));
 }
 
-// Brick holding the stencil's first corner (its halo bound covers the stencil).
-__device__ __forceinline__ int stencil_brick(const RaycastVolume& a, const Stencil& t)
-{
-    return grid_index(t.i0 >> 3, t.j0 >> 3, t.k0 >> 3, a.nb);
-}
-
-// True when the sample's bound is >= thr (the exact stencil), through the
-// brick cache (ck, cbk).
-__device__ __forceinline__ bool skippable(const RaycastVolume& a, const Stencil& t, float thr, int& ck, float& cbk)
-{
-    if (!a.brick_key) return false;
-    const int b0 = stencil_brick(a, t);
-    if (b0 != ck) {
-        ck = b0;
-        cbk = order_value(a.brick_key[b0]);
-    }
-    return cbk >= thr;
-}
-
-// Conservative skip test on approximate texel coordinates (xa, ya, za).
-// Returns 1 when the exact stencil lies inside one super-brick, or has its
-// first corner in one brick, whose bound of F is >= thr, 0 when its first
-// corner is in one brick whose bound is below it (so skippable() would say
-// no), -1 when the margins leave it open.  The last super-brick's and brick's
-// bounds are cached in (cs, cb) and (ck, cbk), so a march through free space,
-// or along a brick, reads no memory.  (A stencil inside a free super-brick whose
-// brick's halo reaches into a neighbour with a lower bound is then evaluated
-// when that brick is the cached one: conservative.)
-__device__ __forceinline__ int fast_skip(const RaycastVolume& a, float xa, float ya, float za, float thr, int& cs,
-                                         float& cb, int& ck, float& cbk)
-{
-    const float hi = (float)a.n - 1.0f - kMargin;
-    if (!(xa >= kMargin && ya >= kMargin && za >= kMargin && xa < hi && ya < hi && za < hi)) return -1;
-    const int xi = (int)xa, yi = (int)ya, zi = (int)za;
-    // the exact first corner is in brick (bx, by, bz) when the coordinate is
-    // kMargin inside the brick's [0, 8) span on every axis
-    const int bx = xi >> 3, by = yi >> 3, bz = zi >> 3;
-    const float vx = xa - (float)(bx * kBrick), vy = ya - (float)(by * kBrick), vz = za - (float)(bz * kBrick);
-    const float bhi = (float)kBrick - kMargin;
-    const bool in_brick = vx >= kMargin && vy >= kMargin && vz >= kMargin && vx < bhi && vy < bhi && vz < bhi;
-    const int bidx = grid_index(bx, by, bz, a.nb);
-    // the cached brick decides first (along a brick or near a surface, where the
-    // super-brick test rarely passes): no memory read and no super-brick test
-    if (in_brick && bidx == ck) return cbk >= thr ? 1 : 0;
-    const int sx = xi >> 6, sy = yi >> 6, sz = zi >> 6;
-    const float ux = xa - (float)(sx * kSuper), uy = ya - (float)(sy * kSuper), uz = za - (float)(sz * kSuper);
-    const float shi = (float)(kSuper - 1) - kMargin;
-    if (ux >= kMargin && uy >= kMargin && uz >= kMargin && ux < shi && uy < shi && uz < shi) {
-        const int sidx = grid_index(sx, sy, sz, a.ns);
-        if (sidx != cs) {
-            cs = sidx;
-            cb = order_value(a.super_key[sidx]);
-        }
-        if (cb >= thr) return 1;
-    }
-    if (in_brick) {
-        ck = bidx;
-        cbk = order_value(a.brick_key[bidx]);
-        return cbk >= thr ? 1 : 0;
-    }
-    return -1;
-}
-
-// Samples after the one at t (same step, t + k*step by repeated addition)
-// whose stencils certainly stay in the texel region [lo, hi] per axis (the
-// first corner at most hi - 1).  The march's approximate texel coordinates are
-// linear in t up to rounding: t stays below 6 m, so each addition is off by at
-// most 2^-22 m, and k of them by k * 2^-22 m * (texels per metre); k is capped
-// so that this stays below kMargin / 2, the coordinates' own rounding is a few
-// 1e-4 texel.  A sample whose linear coordinate is 2 kMargin inside the region
-// thus has a computed coordinate kMargin inside it, and fast_skip's tests hold
-// for it.  The step count is formed with the hardware reciprocal: a relative
-// error of a few 1e-7 on at most 64 texels of distance moves the last counted
-// sample by under 1e-4 texel, far inside the kMargin / 2 left for it.  -1 when
-// the sample at t itself is not 2 kMargin inside.
-__device__ __forceinline__ int region_run(v3 o, v3 dir, float t, float step, float invw, float nf, const int* lo,
-                                          const int* hi)
-{
-    const v3 p = add3(o, mul3s(dir, t));
-    const float pos[3] = {approx_texel(p.x, invw, nf), approx_texel(p.y, invw, nf), approx_texel(p.z, invw, nf)};
-    const float d[3] = {dir.x, dir.y, dir.z};
-    const float m2 = 2.0f * kMargin;
-    float kmax = 20000.0f / (nf * invw);  // k * 2^-22 * texels per metre <= kMargin / 2
-#pragma unroll
-    for (int ax = 0; ax < 3; ++ax) {
-        const float l = (float)lo[ax] + m2, h = (float)hi[ax] - m2;
-        if (!(pos[ax] >= l && pos[ax] <= h)) return -1;
-        const float rate = d[ax] * invw * nf * step;  // texels per step
-        const float inv = __builtin_amdgcn_rcpf(rate);
-        if (rate > 0.0f) kmax = fminf(kmax, (h - pos[ax]) * inv);
-        else if (rate < 0.0f) kmax = fminf(kmax, (l - pos[ax]) * inv);
-    }
-    return (int)kmax;
-}
-
-// Samples after the one at t inside the cached super-brick, which covers
-// stencils inside it; 0 when its bound is below thr or the sample at t is
-// near its faces.  The super-brick's coordinates are those of the sample's
-// position when its index is the cached one (region_run checks the margins).
-__device__ __forceinline__ int super_run(const RaycastVolume& a, v3 o, v3 dir, float t, float step, float invw,
-                                         float nf, float thr, int cs, float cb)
-{
-    if (cs < 0 || !(cb >= thr)) return 0;
-    const v3 p = add3(o, mul3s(dir, t));
-    const int sc[3] = {(int)approx_texel(p.x, invw, nf) / kSuper, (int)approx_texel(p.y, invw, nf) / kSuper,
-                       (int)approx_texel(p.z, invw, nf) / kSuper};
-    if (sc[0] < 0 || sc[1] < 0 || sc[2] < 0 || grid_index(sc[0], sc[1], sc[2], a.ns) != cs) return 0;
-    int lo[3], hi[3];
-#pragma unroll
-    for (int ax = 0; ax < 3; ++ax) {
-        lo[ax] = sc[ax] * kSuper;
-        hi[ax] = min(sc[ax] * kSuper + kSuper - 1, a.n - 1);
-    }
-    const int k = region_run(o, dir, t, step, invw, nf, lo, hi);
-    return k > 0 ? k : 0;
-}
-
-// The corner values of the last trilinear cell a march read: consecutive small
-// steps (0.1 mue) often stay in one cell, and then need no loads.
-struct CellCache {
-    int ki = -1, kj = -1, kk = -1;  // (i0 | i1 << 16) per axis
-    float c[8];
+// The ray of a march in texel space, for the skip test.
+struct RaySpeed {
+    float ix, iy, iz;  // large steps per texel along each axis, signed, at most 1e9
+    float cap;         // most steps a run may take (see free_run)
 };
-
-template <int FMT>
-__device__ __forceinline__ float trilinear_cached(const void* F, int nb, const Stencil& t, CellCache& cc)
+__device__ __forceinline__ RaySpeed ray_speed(v3 dir, float large, float invw, float nf)
 {
-    const int ki = t.i0 | (t.i1 << 16), kj = t.j0 | (t.j1 << 16), kk = t.k0 | (t.k1 << 16);
-    if (ki != cc.ki || kj != cc.kj || kk != cc.kk) {
-        cc.ki = ki;
-        cc.kj = kj;
-        cc.kk = kk;
-        uint32_t o[8];
-        cell_offsets(nb, t, o);
-#pragma unroll
-        for (int q = 0; q < 8; ++q) cc.c[q] = voxel_at<FMT>(F, o[q]);
-    }
-    const float a = t.a, b = t.b, c = t.c;
-    float e00 = (1.0f - a) * cc.c[0] + a * cc.c[1], e10 = (1.0f - a) * cc.c[2] + a * cc.c[3];
-    float e01 = (1.0f - a) * cc.c[4] + a * cc.c[5], e11 = (1.0f - a) * cc.c[6] + a * cc.c[7];
-    float g0 = (1.0f - b) * e00 + b * e10, g1 = (1.0f - b) * e01 + b * e11;
-    return (1.0f - c) * g0 + c * g1;
+    // 1 / 0 is held at 1e9: such an axis never bounds a run
+    const float k = invw * nf * large;
+    RaySpeed r;
+    r.ix = __builtin_amdgcn_fmed3f(__builtin_amdgcn_rcpf(dir.x * k), -1e9f, 1e9f);
+    r.iy = __builtin_amdgcn_fmed3f(__builtin_amdgcn_rcpf(dir.y * k), -1e9f, 1e9f);
+    r.iz = __builtin_amdgcn_fmed3f(__builtin_amdgcn_rcpf(dir.z * k), -1e9f, 1e9f);
+    r.cap = 20000.0f / (nf * invw);
+    return r;
 }
 
-// A lane marches at most kLaneBudget samples of its ray unless it took at most
-// kWorkFloor trips of the march loop for them (a ray crossing free space skips
-// many samples per trip and stays); a longer ray (about 1 in 40 grazes a
-// surface and takes hundreds of small steps) is appended to a list that a second pass
-// finishes with a whole wave per ray, so no wave of the first pass waits on
-// one long ray.
-// The single-session first pass (its waves' tail bounds the frame) hands rays
-// over after 40 samples; the batch's persistent pass (throughput-bound) after 48.
-constexpr int kLaneBudget = 40;
-constexpr int kBatchLaneBudget = 48;
-constexpr int kWorkFloor = 16;
-
-// One trilinear evaluation of the march at t: 1 = skipped (the sample's bound
-// is >= thr: kSkipBound on a large step, kSmallSkipBound on a small one),
-// 0 = evaluated into f.  With P2 (power-of-two width and n: invw is the exact
-// reciprocal, and tex then x = u*n - 1/2 round like the two fused
-// multiply-adds of approx_texel) the skip test's texel coordinates are the
-// stencil's.
-template <int FMT, bool P2>
-__device__ __forceinline__ int march_sample(const RaycastVolume& a, v3 o, v3 dir, float t, float width, float invw,
-                                            float nf, float thr, int& cs, float& cb, int& ck, float& cbk,
-                                            CellCache& cc, float& f)
+// The brick of a sample from its approximate texel coordinates: its index and
+// its centre plane coordinates (8 b + 4) per axis.
+struct BrickAt {
+    int index;
+    float cx, cy, cz;
+};
+__device__ __forceinline__ BrickAt brick_at(const RaycastVolume& a, float xa, float ya, float za)
 {
-    const v3 p = add3(o, mul3s(dir, t));
-    const float xa = approx_texel(p.x, invw, nf), ya = approx_texel(p.y, invw, nf), za = approx_texel(p.z, invw, nf);
-    const int fs = a.brick_key ? fast_skip(a, xa, ya, za, thr, cs, cb, ck, cbk) : 0;
-    if (fs == 1) return 1;
-    const Stencil st = P2 ? stencil_texel(a.n, xa, ya, za) : stencil<false>(a.n, tex(a, p.x), tex(a, p.y), tex(a, p.z));
-    if (fs < 0 && skippable(a, st, thr, ck, cbk)) return 1;
-    f = trilinear_cached<FMT>(a.f, a.nb, st, cc);
-    return 0;
+    const int top = a.n - 1;
+    const int x = clampi((int)xa, 0, top), y = clampi((int)ya, 0, top), z = clampi((int)za, 0, top);
+    BrickAt b;
+    b.index = grid_index(x >> 3, y >> 3, z >> 3, a.nb);
+    b.cx = (float)((x & ~7) | 4);
+    b.cy = (float)((y & ~7) | 4);
+    b.cz = (float)((z & ~7) | 4);
+    return b;
 }
+
+// Half the side of the box of free bricks around a brick of distance D, less
+// 2 kMargin; negative for D = 0 (no sample is inside).
+__device__ __forceinline__ float free_extent(int D) { return (float)(8 * D) - (4.0f + 2.0f * kMargin); }
+
+__device__ __forceinline__ bool inside_box(const BrickAt& b, float xa, float ya, float za, float E)
+{
+    return fmaxf(fmaxf(fabsf(xa - b.cx), fabsf(ya - b.cy)), fabsf(za - b.cz)) <= E;
+}
+
+// Steps after a sample inside the box (scale: large steps 1, small steps
+// large / small) whose samples certainly stay in it.  The march's approximate
+// texel coordinates are linear in t up to rounding: t stays below 6 m, so each
+// addition is off by at most 2^-22 m, and k of them by k * 2^-22 m * (texels
+// per metre); cap keeps k below kMargin / 2 of that.  The reciprocals'
+// relative error of a few 1e-7 on at most 140 texels moves the last counted
+// sample by under 1e-4 texel.  So a counted sample, 2 kMargin inside the box by
+// the linear form, has a computed coordinate kMargin inside it.
+__device__ __forceinline__ int free_run(const BrickAt& b, float xa, float ya, float za, float E, const RaySpeed& r,
+                                        float scale)
+{
+    const float kx = fmaf(b.cx - xa, r.ix, E * fabsf(r.ix));
+    const float ky = fmaf(b.cy - ya, r.iy, E * fabsf(r.iy));
+    const float kz = fmaf(b.cz - za, r.iz, E * fabsf(r.iz));
+    return (int)fminf(fminf(fminf(kx, ky), kz) * scale, r.cap);
+}
+
+// A lane takes at most this many trips in the large-step part of its march and
+// in the small-step part (a trip skips a run of samples or evaluates one); a
+// longer ray (about 1 in 40 grazes a surface and takes hundreds of small steps)
+// is appended to a list that a second pass finishes with a whole wave per ray,
+// so no wave of the first pass waits on one long ray.  The single-session
+// pass's tail bounds the frame; the batch's persistent pass is throughput-bound.
+// Large/small trips, first + finishing pass: one 640x480 frame into 512^3 (three
+// levels) 12/12 82 + 90 us, 16/16 87 + 24, 20/16 86 + 17, 24/24 103 + 15, 32/32
+// 120 + 14; 64 such frames in a tick (small trips) 12 3.26 + 2.10 ms, 16 3.06 +
+// 0.61, 24 3.11 + 0.54, 32 3.14 + 0.28, 40 3.18 + 0.21.
+constexpr int kLargeTrips = 20;
+constexpr int kSmallTrips = 16;
+constexpr int kBatchSmallTrips = 32;
 
 __device__ __forceinline__ float lane_bcast(float v, int lane)
 {
@@ -469,100 +357,167 @@ struct RayQueue {
     DeferredRay* rays;
     unsigned* count;
     unsigned cap;
-    int budget;  // samples a lane marches before it may hand its ray over
+    int small_trips;  // small-step trips of a lane before it may hand its ray over
 };
+
+// t and prev_t after the sample at t and `run` more samples have been skipped,
+// by the march's own repeated additions.
+__device__ __forceinline__ void advance(float& t, float& prev_t, float step, int run)
+{
+    for (int k = 0; k < run; ++k) t = t + step;
+    prev_t = t;
+    t = t + step;
+}
 
 // raycast.cu:44-145 for pixel (i, j) of one level map, one lane per pixel,
 // called by all 64 lanes of a wave together (in_image false past the map's
-// edge).  A ray still marching after its budget of samples is appended to q with
-// its exact march state and left to the finishing pass (when q is full it
-// marches on here).  A skipped sample only sets prev_t; its value is computed
-// if and when the zero-crossing formula needs it.
+// edge).  The march takes large steps up to the first sample below 0.99, and
+// small ones from there on, so it is two loops, each with the code of its step
+// only.  A ray still marching after its trips is appended to rq with its exact
+// march state and left to the finishing pass (when rq is full it marches on
+// here); the lanes of a wave take their slots with one atomic (per-lane
+// atomics on the launch's single counter serialise).
+//
+// Bound: the vector ALU and, in a launch that does not fill the chip, the
+// chain of dependent reads of the longest ray.  With one loop for both steps and
+// a skip test on one brick or one 64^3 super-brick at a time a lane took 20 trips
+// of both steps' code; the boxes of free bricks leave 8 large-step and 7
+// small-step ones.  First + finishing pass: 64 frames of 640x480 from 512^3
+// snorm16 volumes 3.98 + 0.45 -> 3.14 + 0.28 ms, one frame from 512^3 FP32 105 + 22
+// -> 86 + 17 us, its coarsest level alone (160x120) 52 -> 30 us.
 template <int FMT, bool P2>
 __device__ __forceinline__ void raycast_pixel(const RaycastVolume& a, const float* pose, const RaycastLevel& L, int i,
                                               int j, bool in_image, const RayQueue& rq, int job)
 {
     const RayGeom g = ray_geom(a, pose, L, i, j, in_image);
     const v3 o = g.o, dir = g.dir;
-    const float nearv = g.nearv, farv = g.farv;
     const float width = a.width, mue = a.mue;
     const float large = mue * 1.99f, small = mue * 0.1f;
     const float invw = 1.0f / width, nf = (float)a.n;
-    float step = large, prev = 0.0f, tstar = 0.0f, prev_t = 0.0f, t = nearv;
-    bool prev_skipped = false, can_defer = true;
-    int work = 0;  // trips of the march loop so far (each a skip test or an evaluation)
-    int cs = -1, ck = -1;
-    float cb = 0.0f, cbk = 0.0f;
-    CellCache cc;
-    int guard = 0;  // never binds for mue >= 1e-4 m (kf_volume_create enforces it)
-    if (!g.active) return;
+    const RaySpeed speed = ray_speed(dir, large, invw, nf);
+    float t = g.nearv, prev = 0.0f, prev_t = 0.0f, fhit = 0.0f;
+    bool prev_skipped = false, hit = false, can_defer = true;
+    enum { kLarge, kSmall, kDone, kHandedOver };
+    int phase = g.active ? kLarge : kDone;
     for (;;) {
-        if (!(t < farv)) break;
-        if (++guard > kMaxMarchSteps) break;
-        // the lanes handing their rays over in this trip take their slots with one
-        // atomic per wave (one counter for the whole launch: per-lane atomics on it
-        // serialise)
-        const bool defer = can_defer && ++work > kWorkFloor && guard > rq.budget;
-        const uint64_t dm = __ballot(defer);
-        if (dm) {
-            const int leader = __ffsll((unsigned long long)dm) - 1;
-            unsigned base = 0u;
-            if ((int)(threadIdx.x & 63) == leader) base = atomicAdd(rq.count, (unsigned)__popcll(dm));
-            base = (unsigned)__builtin_amdgcn_readlane((int)base, leader);
-            const unsigned slot = base + (unsigned)__popcll(dm & ((1ull << (threadIdx.x & 63)) - 1ull));
-            if (defer && slot < rq.cap) {
-                DeferredRay d;
-                d.job = job;
-                d.px = j * L.w + i;
-                d.guard = guard;
-                d.flags = (prev_skipped ? 1 : 0) | (step == small ? 2 : 0);
-                d.t = t;
-                d.prev = prev;
-                d.prev_t = prev_t;
-                d.pad = 0.0f;
-                rq.rays[slot] = d;
-                return;
+        bool defer = false;
+        int trips = 0;
+        while (phase == kLarge) {
+            if (!(t < g.farv)) {
+                phase = kDone;
+                break;
             }
-            if (defer) can_defer = false;
-        }
-        // one sample per trip on either step: large and small steps share the code,
-        // so lanes of a wave in different phases of their march do not run two paths
-        const bool lg = step == large;
-        float f = 0.0f;
-        if (march_sample<FMT, P2>(a, o, dir, t, width, invw, nf, lg ? kSkipBound : kSmallSkipBound, cs, cb, ck, cbk, cc,
-                              f)) {
-            // a skipped large step, and the following ones inside the same free
-            // super-brick: positions by the same additions, no coordinates computed
-            int run = lg ? super_run(a, o, dir, t, step, invw, nf, kSkipBound, cs, cb) : 0;
-            prev_skipped = true;
-            prev_t = t;
-            t = t + step;
-            for (; run > 0 && t < farv && guard < kMaxMarchSteps; --run) {
-                ++guard;
-                prev_t = t;
-                t = t + step;
+            if (++trips > kLargeTrips && can_defer) {
+                defer = true;
+                break;
             }
-            continue;
-        }
-        if (f < 0.0f) {
-            if (t == nearv) break;
-            if (lg) {
-                t = t - mue;  // back off and march on with small steps
-                step = small;
-                t = t + step;
+            const v3 p = add3(o, mul3s(dir, t));
+            const float xa = approx_texel(p.x, invw, nf), ya = approx_texel(p.y, invw, nf),
+                        za = approx_texel(p.z, invw, nf);
+            const BrickAt b = brick_at(a, xa, ya, za);
+            const float E = free_extent(a.dist[b.index] & 15);
+            if (inside_box(b, xa, ya, za, E)) {
+                prev_skipped = true;
+                advance(t, prev_t, large, free_run(b, xa, ya, za, E, speed, 1.0f));
                 continue;
             }
-            if (prev_skipped) {
-                const v3 pp = add3(o, mul3s(dir, prev_t));
-                prev = sample_tsdf<FMT, P2>(a.f, a.n, a.nb, tex(a, pp.x), tex(a, pp.y), tex(a, pp.z));
+            const float f = trilinear<FMT>(
+                a.f, a.nb, P2 ? stencil_texel(a.n, xa, ya, za) : stencil<false>(a.n, tex(a, p.x), tex(a, p.y), tex(a, p.z)));
+            if (f < 0.0f) {
+                if (t == g.nearv) {
+                    phase = kDone;
+                    break;
+                }
+                t = t - mue;  // back off and march on with small steps
+                t = t + small;
+                phase = kSmall;
+                break;
             }
-            tstar = t - small * prev / (f - prev);
-            break;
+            prev = f;
+            prev_skipped = false;
+            if (f < 0.99f) {
+                t = t + small;
+                phase = kSmall;
+                break;
+            }
+            t = t + large;
         }
-        if (lg && f < 0.99f) step = small;
-        prev = f;
-        prev_skipped = false;
-        t = t + step;
+        trips = 0;
+        // the corner values of the last cell (small steps often stay in one)
+        float fi = -1e9f, fj = -1e9f, fk = -1e9f, c[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+        while (phase == kSmall && !defer) {
+            if (!(t < g.farv)) {
+                phase = kDone;
+                break;
+            }
+            if (++trips > rq.small_trips && can_defer) {
+                defer = true;
+                break;
+            }
+            const v3 p = add3(o, mul3s(dir, t));
+            const float xa = approx_texel(p.x, invw, nf), ya = approx_texel(p.y, invw, nf),
+                        za = approx_texel(p.z, invw, nf);
+            const float x = P2 ? xa : tex(a, p.x) * nf - 0.5f, y = P2 ? ya : tex(a, p.y) * nf - 0.5f,
+                        z = P2 ? za : tex(a, p.z) * nf - 0.5f;
+            const float fx = floorf(x), fy = floorf(y), fz = floorf(z);
+            if (fx != fi || fy != fj || fz != fk) {
+                const BrickAt b = brick_at(a, xa, ya, za);
+                const float E = free_extent(a.dist[b.index] >> 4);
+                if (inside_box(b, xa, ya, za, E)) {
+                    prev_skipped = true;
+                    advance(t, prev_t, small, free_run(b, xa, ya, za, E, speed, 19.9f));
+                    continue;
+                }
+                fi = fx;
+                fj = fy;
+                fk = fz;
+                uint32_t q[8];
+                cell_offsets(a.nb, stencil_texel(a.n, x, y, z), q);
+#pragma unroll
+                for (int k = 0; k < 8; ++k) c[k] = voxel_at<FMT>(a.f, q[k]);
+            }
+            const float f = lerp_cell(c, x - fx, y - fy, z - fz);
+            if (f < 0.0f) {
+                hit = t != g.nearv;
+                fhit = f;
+                phase = kDone;
+                break;
+            }
+            prev = f;
+            prev_skipped = false;
+            t = t + small;
+        }
+        const uint64_t dm = __ballot(defer);
+        if (!dm) break;
+        const int leader = __ffsll((unsigned long long)dm) - 1;
+        unsigned base = 0u;
+        if ((int)(threadIdx.x & 63) == leader) base = atomicAdd(rq.count, (unsigned)__popcll(dm));
+        base = (unsigned)__builtin_amdgcn_readlane((int)base, leader);
+        const unsigned slot = base + (unsigned)__popcll(dm & ((1ull << (threadIdx.x & 63)) - 1ull));
+        if (defer && slot < rq.cap) {
+            DeferredRay d;
+            d.job = job;
+            d.px = j * L.w + i;
+            d.flags = (prev_skipped ? 1 : 0) | (phase == kSmall ? 2 : 0);
+            d.t = t;
+            d.prev = prev;
+            d.prev_t = prev_t;
+            d.pad[0] = d.pad[1] = 0.0f;
+            rq.rays[slot] = d;
+            phase = kHandedOver;
+        } else if (defer) {
+            can_defer = false;
+        }
+        if (!__ballot(phase == kLarge || phase == kSmall)) break;
+    }
+    if (!g.active || phase == kHandedOver) return;
+    float tstar = 0.0f;
+    if (hit) {
+        if (prev_skipped) {
+            const v3 pp = add3(o, mul3s(dir, prev_t));
+            prev = sample_tsdf<FMT, P2>(a.f, a.n, a.nb, tex(a, pp.x), tex(a, pp.y), tex(a, pp.z));
+        }
+        tstar = t - small * prev / (fhit - prev);
     }
     write_surface<FMT, P2>(a, L, i, j, g, tstar);
 }
@@ -599,7 +554,7 @@ __device__ __forceinline__ float chunk_position(float t, float step, int lane)
 // The finishing pass for one handed-over ray: the wave marches it 64 samples
 // at a time, lane k taking sample k of the chunk (its position by the same
 // repeated additions t = t + step, chunk_position), and a ballot finds the first sample that
-// ends the ray or changes the march (end of the interval or the guard, f < 0,
+// ends the ray or changes the march (end of the interval, f < 0,
 // or f < 0.99 on a large step).  The samples before it are consumed as the
 // single-lane march would (prev from the last of them), the ones after it are
 // discarded, so every sample position, value and decision is the sequential
@@ -617,19 +572,23 @@ __device__ __forceinline__ void finish_ray(const RaycastVolume& a, const float* 
     float step = (r.flags & 2) ? small : large;
     float t = r.t, pv = r.prev, pt = r.prev_t;
     bool psk = (r.flags & 1) != 0;
-    int gb = r.guard;
-    int cs = -1, ck = -1;
-    float cb = 0.0f, cbk = 0.0f;
-    CellCache cc;
     float tstar = 0.0f;
     for (;;) {
         const float tk = chunk_position(t, step, lane);
-        const bool end = !(tk < g.farv) || gb + lane > kMaxMarchSteps;
+        const bool end = !(tk < g.farv);
         float f = 0.0f;
         int sk = 1;
-        if (!end)
-            sk = march_sample<FMT, P2>(a, g.o, g.dir, tk, width, invw, nf, step == large ? kSkipBound : kSmallSkipBound,
-                                   cs, cb, ck, cbk, cc, f);
+        if (!end) {
+            const v3 p = add3(g.o, mul3s(g.dir, tk));
+            const float xa = approx_texel(p.x, invw, nf), ya = approx_texel(p.y, invw, nf),
+                        za = approx_texel(p.z, invw, nf);
+            const BrickAt b = brick_at(a, xa, ya, za);
+            const int d = a.dist[b.index];
+            sk = inside_box(b, xa, ya, za, free_extent(step == large ? d & 15 : d >> 4)) ? 1 : 0;
+            if (!sk)
+                f = trilinear<FMT>(a.f, a.nb, P2 ? stencil_texel(a.n, xa, ya, za)
+                                                 : stencil<false>(a.n, tex(a, p.x), tex(a, p.y), tex(a, p.z)));
+        }
         const bool neg = !end && !sk && f < 0.0f;
         const bool slow = !end && !sk && step == large && f < 0.99f;
         const uint64_t evm = __ballot(end || neg || slow);
@@ -646,7 +605,6 @@ __device__ __forceinline__ void finish_ray(const RaycastVolume& a, const float* 
         }
         if (k == 64) {
             t = lane_bcast(tk, 63) + step;
-            gb += 64;
             continue;
         }
         const float tkk = lane_bcast(tk, k), fk = lane_bcast(f, k);
@@ -657,7 +615,6 @@ __device__ __forceinline__ void finish_ray(const RaycastVolume& a, const float* 
                 t = tkk - mue;  // back off and march on with small steps
                 step = small;
                 t = t + step;
-                gb = gb + k + 1;
                 continue;
             }
             float pk = pv;
@@ -673,7 +630,6 @@ __device__ __forceinline__ void finish_ray(const RaycastVolume& a, const float* 
         pv = fk;
         psk = false;
         t = tkk + step;
-        gb = gb + k + 1;
     }
     write_surface_wave<FMT, P2>(a, L, i, j, g, tstar);
 }
@@ -749,7 +705,7 @@ __global__ __launch_bounds__(64, 5) void raycast_kernel(RaycastArgs a)
         const RaycastLevel& L = a.lv[l];
         const int i = (lt % L.tiles_x) * 8 + (threadIdx.x & 7);
         const int j = (lt / L.tiles_x) * 8 + (threadIdx.x >> 3);
-        const RayQueue rq{a.rays, a.count, a.cap, kLaneBudget};
+        const RayQueue rq{a.rays, a.count, a.cap, kSmallTrips};
         const float* pose = a.dyn ? a.dyn->pose : a.pose;
         if (a.vol.p2) raycast_pixel<FMT, true>(a.vol, pose, L, i, j, i < L.w && j < L.h, rq, l);
         else raycast_pixel<FMT, false>(a.vol, pose, L, i, j, i < L.w && j < L.h, rq, l);
@@ -785,7 +741,6 @@ __global__ __launch_bounds__(64 * kFinishPer) void raycast_finish_kernel(Raycast
         DeferredRay d;
         d.job = cr.job;
         d.px = cr.px;
-        d.guard = cr.guard;
         d.flags = cr.flags;
         d.t = cr.t;
         d.prev = cr.prev;
@@ -800,11 +755,9 @@ template <class CJ>
 __device__ __forceinline__ void copy_job(const CJ& j, RaycastVolume& vol, RaycastLevel& L)
 {
     vol.f = j.vol.f;
-    vol.brick_key = j.vol.brick_key;
-    vol.super_key = j.vol.super_key;
+    vol.dist = j.vol.dist;
     vol.n = j.vol.n;
     vol.nb = j.vol.nb;
-    vol.ns = j.vol.ns;
     vol.format = j.vol.format;
     vol.width = j.vol.width;
     vol.mue = j.vol.mue;
@@ -833,7 +786,7 @@ template <int FMT>
 __global__ __launch_bounds__(64) void raycast_batch_kernel(const BatchHeader* hd, const RaycastJob* jobs)
 {
     const RayQueue rq{hd->ray_list + (FMT == KF_VOXEL_F32 ? 0u : hd->ray_list_cap),
-                      hd->ray_next + (FMT == KF_VOXEL_F32 ? 16 : 17), hd->ray_list_cap, kBatchLaneBudget};
+                      hd->ray_next + (FMT == KF_VOXEL_F32 ? 16 : 17), hd->ray_list_cap, kBatchSmallTrips};
     const int nf = hd->n_ray_f32, tf = hd->ray_tiles_f32;
     const int j0 = FMT == KF_VOXEL_F32 ? 0 : nf, j1 = FMT == KF_VOXEL_F32 ? nf : hd->n_ray;
     const int t0 = FMT == KF_VOXEL_F32 ? 0 : tf, t1 = FMT == KF_VOXEL_F32 ? tf : hd->ray_tiles;
@@ -898,7 +851,6 @@ __global__ __launch_bounds__(64 * kFinishPer) void raycast_batch_finish_kernel(c
         DeferredRay d;
         d.job = rays[r].job;
         d.px = rays[r].px;
-        d.guard = rays[r].guard;
         d.flags = rays[r].flags;
         d.t = rays[r].t;
         d.prev = rays[r].prev;
@@ -917,17 +869,15 @@ RaycastVolume raycast_volume(const kf_volume* v)
 {
     RaycastVolume r{};
     r.f = v->f;
-    r.brick_key = v->brick_key;
-    r.super_key = v->super_key;
+    r.dist = v->dist;
     r.n = v->n;
     r.nb = v->nb;
-    r.ns = v->ns;
     r.format = v->format;
     r.width = v->width;
     r.mue = v->mue;
     int e = 0;
-    r.inv_width = frexpf(v->width, &e) == 0.5f ? 1.0f / v->width : 0.0f;
-    r.p2 = r.inv_width != 0.0f && (v->n & (v->n - 1)) == 0 ? 1 : 0;
+    r.inv_width = 1.0f / v->width;
+    r.p2 = frexpf(v->width, &e) == 0.5f && (v->n & (v->n - 1)) == 0 ? 1 : 0;
     return r;
 }
 

@@ -130,19 +130,6 @@ __global__ __launch_bounds__(256) void depth_max_kernel(const float* __restrict_
     }
 }
 
-// x / b rounded to nearest from y = RN(1/b): q = RN(x*y), r = x - b*q (exact by
-// the fused multiply-add), RN(q + r*y) is RN(x/b) for every x and b whose
-// quotient and residual neither overflow nor underflow (Markstein's theorem;
-// checked exhaustively on the CPU for every x in [-mue, mue] at several mue
-// and for every divisor 1..129 of the count update).  The fuse's operands
-// (|x| >= 2^-25 or 0, b in [1e-4, 129]) stay far from both ranges.
-__device__ __forceinline__ float div_by_exact_reciprocal(float x, float b, float y)
-{
-    const float q = x * y;
-    const float r = fmaf(-q, b, x);
-    return fmaf(r, y, q);
-}
-
 // True when x may lie within a few ulp of an integer (0 and the image size
 // included): x*rcp(z) is within 2^-22 |x/z| of the rounded quotient x/z
 // (v_rcp_f32 is within 1 ulp), so outside a band of half-width band =
@@ -409,51 +396,53 @@ __global__ __launch_bounds__(kCullThreads) void fuse_cull_kernel(FuseArgs a, int
 
 constexpr int kFuseWaves = 4;
 
-// The bounds a fused brick may lower (kf_device.hpp): bound l < 8 belongs to
-// brick (bi - (l & 1), bj - (l >> 1 & 1), bk - (l >> 2)), the brick itself and
-// the 7 below it whose halos reach into it; bound 8 is the super-brick's.
-// Lane l <= 8 loads bound l at the brick's start (-inf for a brick outside
-// the volume: never lowered), so the load shares the column loads' round trip.
-__device__ __forceinline__ float load_bound(const FuseArgs& a, int bi, int bj, int bk, int lane)
+// The free bits a fused brick may clear (kf_device.hpp): lane l < 8 loads those
+// of brick (bi - (l & 1), bj - (l >> 1 & 1), bk - (l >> 2)), the brick itself
+// and the 7 below it whose halos reach into it (bit 0: large steps, bit 1: small;
+// 0 for a brick outside the volume), at the brick's start, so that the load
+// shares the column loads' round trip.
+__device__ __forceinline__ int load_free(const FuseArgs& a, int bi, int bj, int bk, int lane)
 {
-    float b = -__int_as_float(0x7f800000);
+    int b = 0;
     if (lane < 8) {
         const int ni = bi - (lane & 1), nj = bj - ((lane >> 1) & 1), nk = bk - (lane >> 2);
-        if (ni >= 0 && nj >= 0 && nk >= 0) b = order_value(a.brick_key[((int64_t)nk * a.nb + nj) * a.nb + ni]);
-    } else if (lane == 8) {
-        b = order_value(a.super_key[((bk >> 3) * a.ns + (bj >> 3)) * a.ns + (bi >> 3)]);
+        if (ni >= 0 && nj >= 0 && nk >= 0) {
+            const unsigned long long* r = a.free_bits + free_word(a.nb, ni, nj, nk, 0);
+            const unsigned long long large = r[0], small = r[a.nb > 64 ? 2 : 1];
+            b = (int)((large >> (ni & 63)) & 1ull) | (int)((small >> (ni & 63)) & 1ull) << 1;
+        }
     }
     return b;
 }
 
-// Lowers the bounds the brick's written values fall below: every value lowers
-// its brick's and super-brick's bound, values on the local i = 0 plane (lanes
-// with i == 0) the -x neighbour's, on j = 0 (lanes with j == 0) the -y
-// neighbour's, on k = 0 (each lane's first voxel) the -z neighbour's, and the
-// values on two or three of these planes the diagonal neighbours'.  A lane
-// issues an atomicMin only where its own smallest value on the set is below
-// the bound loaded at the start; bounds are only ever lowered, so a value not
-// below the loaded bound is not below the current one either.  Once the model
-// has settled, no value is below its bounds and no atomic is issued.
-__device__ __forceinline__ void lower_bounds(const FuseArgs& a, int bi, int bj, int bk, int lane, float bound,
-                                             float lane_min, float lane_k0)
+// Clears the free bits the brick's written values end: every value counts for
+// its brick, values on the local i = 0 plane (lanes with i == 0) for the -x
+// neighbour too, on j = 0 (lanes with j == 0) for the -y neighbour, on k = 0
+// (each lane's first voxel) for the -z neighbour, and the values on two or three
+// of these planes for the diagonal neighbours.  A brick in front of the surface
+// has no value below kSkipBound, and once the model has settled the bits at the
+// surface are clear already: then no atomic is issued.
+__device__ __forceinline__ void clear_free(const FuseArgs& a, int bi, int bj, int bk, int lane, int free,
+                                           float lane_min, float lane_k0)
 {
-    float b[9];
-#pragma unroll
-    for (int l = 0; l < 9; ++l) b[l] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(bound), l));
+    if (!__ballot(lane_min < kSkipBound) || !__ballot(free != 0)) return;
     const bool i0 = (lane & 7) == 0, j0 = (lane >> 3) == 0;
 #pragma unroll
     for (int l = 0; l < 8; ++l) {
+        const int b = __builtin_amdgcn_readlane(free, l);
+        if (b == 0) continue;  // uniform
         const int dx = l & 1, dy = (l >> 1) & 1, dz = l >> 2;
-        const float v = dz ? lane_k0 : lane_min;
-        if ((!dx || i0) && (!dy || j0) && v < b[l])
-            atomicMin(&a.brick_key[((int64_t)(bk - dz) * a.nb + (bj - dy)) * a.nb + (bi - dx)], order_key(v));
+        const float v = ((!dx || i0) && (!dy || j0)) ? (dz ? lane_k0 : lane_min) : 1.0f;
+        const bool large = (b & 1) && __ballot(v < kSkipBound), small = (b & 2) && __ballot(v < 0.0f);
+        if (lane < 2 && (lane == 0 ? large : small)) {
+            const int x = bi - dx;
+            atomicAnd(&a.free_bits[free_word(a.nb, x, bj - dy, bk - dz, lane)], ~(1ull << (x & 63)));
+        }
     }
-    if (lane_min < b[8]) atomicMin(&a.super_key[((bk >> 3) * a.ns + (bj >> 3)) * a.ns + (bi >> 3)], order_key(lane_min));
 }
 
 // One wave fuses brick (bi, bj, bk) (lane = (j, i) inside the brick, its
-// column of 8 voxels along z) and lowers the bounds of F it reaches.  Returns
+// column of 8 voxels along z) and clears the free bits it ends.  Returns
 // the lane's count of updated voxels.
 //
 // The brick's z terms are uniform: they are read through the constant address
@@ -477,10 +466,10 @@ __device__ __forceinline__ int fuse_brick(const FuseArgs& a, const float* ip, un
     const int i = bi * 8 + (lane & 7), j = bj * 8 + (lane >> 3);
     const float x = a.half + (float)i * a.res, y = a.half + (float)j * a.res;
     const v3 col = mk3(ip[0] * x + ip[4] * y, ip[1] * x + ip[5] * y, ip[2] * x + ip[6] * y);
-    const float bound = load_bound(a, bi, bj, bk, lane);
+    const int free = load_free(a, bi, bj, bk, lane);
     float fmin = __int_as_float(0x7f800000), fk0 = fmin;
     const int cnt = fuse_column<FMT>(a, col, zt, brick * kBrickVoxels + lane * 8, fmin, fk0, inv_count);
-    lower_bounds(a, bi, bj, bk, lane, bound, fmin, fk0);
+    clear_free(a, bi, bj, bk, lane, free, fmin, fk0);
     return cnt;
 }
 
@@ -641,9 +630,7 @@ __device__ __forceinline__ void load_fuse_args(const CJ& j, FuseArgs& a)
     a.band = j.a.band;
     a.f = j.a.f;
     a.wt = j.a.wt;
-    a.brick_key = j.a.brick_key;
-    a.super_key = j.a.super_key;
-    a.ns = j.a.ns;
+    a.free_bits = j.a.free_bits;
     a.cull = j.a.cull;
     a.format = j.a.format;
 }
@@ -702,13 +689,17 @@ __global__ __launch_bounds__(64 * kFuseWaves, 8) void fuse_batch_list_kernel(con
 
 template <int FMT>
 __global__ __launch_bounds__(256) void init_kernel(void* f, void* wt, int64_t count, float f0, float w0,
-                                                   int* brick_key, int64_t nbricks, int* super_key, int nsuper)
+                                                   unsigned long long* free_bits, uint8_t* dist, int nb)
 {
     int64_t q = (int64_t)blockIdx.x * 256 + threadIdx.x;
     int64_t stride = (int64_t)gridDim.x * 256;
     const float fb = (FMT == KF_VOXEL_F32) ? f0 : snorm_decode(snorm_encode(f0));
-    for (int64_t b = q; b < nbricks; b += stride) brick_key[b] = order_key(fb);
-    for (int64_t b = q; b < nsuper; b += stride) super_key[b] = order_key(fb);
+    const bool large = fb >= kSkipBound, small = fb >= 0.0f;
+    const int W = nb > 64 ? 2 : 1;
+    for (int64_t r = q; r < (int64_t)nb * nb * 2 * W; r += stride)
+        free_bits[r] = ((r / W) & 1 ? small : large) ? ~0ull : 0ull;
+    const uint8_t db = (uint8_t)((large ? kDistMax : 0) | (small ? kDistMax << 4 : 0));
+    for (int64_t b = q; b < (int64_t)nb * nb * nb; b += stride) dist[b] = db;
     for (; q < count; q += stride) {
         if (FMT == KF_VOXEL_F32) {
             static_cast<float*>(f)[q] = f0;
@@ -759,18 +750,18 @@ __global__ __launch_bounds__(256) void volume_to_slab(float* __restrict__ slab, 
     }
 }
 
-__global__ void super_reset_kernel(int* super_key, int nsuper)
+// Every free bit set (before free_bits_kernel clears the others).
+__global__ void free_reset_kernel(unsigned long long* free_bits, int64_t words)
 {
-    int q = blockIdx.x * 256 + threadIdx.x;
-    if (q < nsuper) super_key[q] = 0x7f800000;  // order_key(+inf)
+    const int64_t q = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (q < words) free_bits[q] = ~0ull;
 }
 
-// Exact halo minimum of F per brick (after an upload): one wave per brick
-// takes the 9^3 voxels [8b, 8b + 8] per axis that lie in the volume; the
-// super-brick's bound takes the smallest of its bricks'.
+// Free bits from the voxels (after an upload): one wave per brick takes the 9^3
+// voxels [8b, 8b + 8] per axis that lie in the volume.
 template <int FMT>
-__global__ __launch_bounds__(256) void brick_bound_kernel(const void* f, int* brick_key, int64_t nbricks, int n,
-                                                          int nb, int ns, int* super_key)
+__global__ __launch_bounds__(256) void free_bits_kernel(const void* f, unsigned long long* free_bits, int64_t nbricks,
+                                                        int n, int nb)
 {
     const int64_t brick = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
     if (brick >= nbricks) return;
@@ -786,10 +777,145 @@ __global__ __launch_bounds__(256) void brick_bound_kernel(const void* f, int* br
         m = fminf(m, v);
     }
     m = wave_min(m);
-    if (lane == 0) {
-        brick_key[brick] = order_key(m);
-        atomicMin(&super_key[((bk >> 3) * ns + (bj >> 3)) * ns + (bi >> 3)], order_key(m));
+    if (lane < 2 && m < (lane == 0 ? kSkipBound : 0.0f))
+        atomicAnd(&free_bits[free_word(nb, bi, bj, bk, lane)], ~(1ull << (bi & 63)));
+}
+
+// ---- free distances (kf_device.hpp) from the free bits.
+// One workgroup per 8 x 8 rows of bricks along x, one lane per row of the
+// 24 x 24 window its distances depend on.  A row's free bits are one or two words
+// (W) per kind of step, and a step of the distance is an erosion by one brick: two
+// shifts along x, then the neighbouring rows along y and z through LDS.  A
+// brick's distance is the number of steps it stays free, counted in four
+// bit-sliced planes per row.  Rows past the window count as free; what they
+// get wrong moves in one row per step and ends outside the 8 x 8 rows.
+//
+// Bound: latency (64 workgroups for 512^3): one load per lane, then kDistRadius
+// steps of two barriers: 7.5 us for one 512^3 volume, 0.13 ms for 64 of them.
+constexpr int kDistWin = 8 + 2 * kDistRadius;
+constexpr int kDistThreads = kDistWin * kDistWin;
+static_assert(kDistThreads % 64 == 0 && kDistMax < 16, "whole waves; distances fit four bits");
+// Two words per row and exchange: both kinds of step at once for one-word rows,
+// one kind after the other for two-word rows (their registers at once, 148,
+// left room for one workgroup per CU).
+template <int W>
+struct DistRows {
+    uint64_t a[kDistThreads][2], b[kDistThreads][2];
+    uint64_t planes[64][2][4][W];
+};
+template <int W>
+__device__ __forceinline__ void erode_x(uint64_t* m)
+{
+    if (W == 1) {
+        m[0] &= ((m[0] >> 1) | (1ull << 63)) & ((m[0] << 1) | 1ull);
+    } else {
+        const uint64_t lo = m[0], hi = m[W - 1];
+        m[0] = lo & ((lo >> 1) | (hi << 63)) & ((lo << 1) | 1ull);
+        m[W - 1] = hi & ((hi >> 1) | (1ull << 63)) & ((hi << 1) | (lo >> 63));
     }
+}
+template <int W>
+__device__ void brick_dist_tile(const unsigned long long* free_bits, uint8_t* dist, int nb, int tile, DistRows<W>& S)
+{
+    const int tid = threadIdx.x, tiles = (nb + 7) / 8, ty = tile % tiles, tz = tile / tiles;
+    const int y = tid % kDistWin, z = tid / kDistWin;
+    const int gy = ty * 8 - kDistRadius + y, gz = tz * 8 - kDistRadius + z;
+    const bool in = gy >= 0 && gy < nb && gz >= 0 && gz < nb;
+    const unsigned long long* r = free_bits + free_word(nb, 0, clampi(gy, 0, nb - 1), clampi(gz, 0, nb - 1), 0);
+    const int ym = tid - (y > 0), yp = tid + (y < kDistWin - 1);
+    const int zm = z > 0 ? tid - kDistWin : tid, zp = z < kDistWin - 1 ? tid + kDistWin : tid;
+    constexpr int kKinds = 2 / W;  // kinds of step at once
+    for (int h0 = 0; h0 < 2; h0 += kKinds) {
+        uint64_t m[2], c[2][4];  // [kind][word], kKinds x W
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            m[q] = r[h0 * W + q];
+            // bricks past the volume are free
+            const int valid = nb - 64 * (q % W);
+            if (valid < 64) m[q] |= ~0ull << valid;
+            if (!in) m[q] = ~0ull;
+            c[q][0] = m[q];
+            c[q][1] = c[q][2] = c[q][3] = 0;
+        }
+        for (int s = 0; s < kDistRadius; ++s) {
+#pragma unroll
+            for (int h = 0; h < kKinds; ++h) erode_x<W>(m + h * W);
+#pragma unroll
+            for (int q = 0; q < 2; ++q) S.a[tid][q] = m[q];
+            __syncthreads();
+#pragma unroll
+            for (int q = 0; q < 2; ++q) {
+                m[q] &= S.a[ym][q] & S.a[yp][q];
+                S.b[tid][q] = m[q];
+            }
+            __syncthreads();
+#pragma unroll
+            for (int q = 0; q < 2; ++q) {
+                m[q] &= S.b[zm][q] & S.b[zp][q];
+                uint64_t carry = m[q];
+#pragma unroll
+                for (int p = 0; p < 4; ++p) {
+                    const uint64_t t = c[q][p] & carry;
+                    c[q][p] ^= carry;
+                    carry = t;
+                }
+            }
+        }
+        const int oy = y - kDistRadius, oz = z - kDistRadius;
+        if (oy >= 0 && oy < 8 && oz >= 0 && oz < 8) {
+#pragma unroll
+            for (int q = 0; q < 2; ++q)
+#pragma unroll
+                for (int p = 0; p < 4; ++p) S.planes[oz * 8 + oy][h0 + q / W][p][q % W] = c[q][p];
+        }
+    }
+    __syncthreads();
+    // one row of the tile per wave, a brick per lane
+    const int lane = tid & 63;
+    for (int o = __builtin_amdgcn_readfirstlane(tid >> 6); o < 64; o += kDistThreads / 64) {
+        const int by = ty * 8 + (o & 7), bz = tz * 8 + (o >> 3);
+        if (by >= nb || bz >= nb) continue;
+#pragma unroll
+        for (int w = 0; w < W; ++w) {
+            unsigned d = 0;
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+#pragma unroll
+                for (int p = 0; p < 4; ++p)
+                    d |= (unsigned)((S.planes[o][h][p][w] >> lane) & 1ull) << (4 * h + p);
+            if (w * 64 + lane < nb) dist[((int64_t)bz * nb + by) * nb + w * 64 + lane] = (uint8_t)d;
+        }
+    }
+}
+template <int W>
+__global__ __launch_bounds__(kDistThreads) void brick_dist_kernel(const unsigned long long* free_bits, uint8_t* dist,
+                                                                  int nb)
+{
+    __shared__ DistRows<W> S;
+    brick_dist_tile<W>(free_bits, dist, nb, blockIdx.x, S);
+}
+// The same for every fused volume of a tick (workgroups stride over the tiles).
+__global__ __launch_bounds__(kDistThreads) void brick_dist_batch_kernel(const BatchHeader* hd, const FuseJob* jobs)
+{
+    __shared__ union {
+        DistRows<1> one;
+        DistRows<2> two;
+    } S;
+    const int tiles = hd->dist_tiles, njobs = hd->n_fuse;
+    for (int t = blockIdx.x; t < tiles; t += gridDim.x) {
+        const FuseJob& J = jobs[job_of(jobs, njobs, t, [](const FuseJob& x) { return x.dist_tile0; })];
+        if (J.a.nb <= 64) brick_dist_tile<1>(J.a.free_bits, J.a.dist, J.a.nb, t - J.dist_tile0, S.one);
+        else brick_dist_tile<2>(J.a.free_bits, J.a.dist, J.a.nb, t - J.dist_tile0, S.two);
+        __syncthreads();  // the planes have been read
+    }
+}
+int launch_brick_dist(const kf_volume* v, hipStream_t s)
+{
+    const unsigned blocks = (unsigned)dist_tiles(v->nb);
+    if (v->nb <= 64) brick_dist_kernel<1><<<blocks, kDistThreads, 0, s>>>(v->free_bits, v->dist, v->nb);
+    else brick_dist_kernel<2><<<blocks, kDistThreads, 0, s>>>(v->free_bits, v->dist, v->nb);
+    KF_LAUNCHED("brick_dist_kernel");
+    return KF_OK;
 }
 
 // z of each k slice: one lane, the host loop's repeated additions in order.
@@ -844,15 +970,15 @@ int for_each_slab(const kf_volume* v, bool to_volume, Fn&& host_side)
     if (st == KF_OK && to_volume) {
         const int64_t nbricks = (int64_t)v->nb * v->nb * v->nb;
         const unsigned b = (unsigned)((nbricks + 3) / 4);
-        const int nsuper = v->ns * v->ns * v->ns;
-        super_reset_kernel<<<(nsuper + 255) / 256, 256>>>(v->super_key, nsuper);
+        const int64_t words = (int64_t)free_words(v->nb);
+        free_reset_kernel<<<(unsigned)((words + 255) / 256), 256>>>(v->free_bits, words);
         if (v->format == KF_VOXEL_F32)
-            brick_bound_kernel<KF_VOXEL_F32><<<b, 256>>>(v->f, v->brick_key, nbricks, v->n, v->nb, v->ns, v->super_key);
+            free_bits_kernel<KF_VOXEL_F32><<<b, 256>>>(v->f, v->free_bits, nbricks, v->n, v->nb);
         else
-            brick_bound_kernel<KF_VOXEL_SNORM16_U8><<<b, 256>>>(v->f, v->brick_key, nbricks, v->n, v->nb, v->ns,
-                                                                v->super_key);
+            free_bits_kernel<KF_VOXEL_SNORM16_U8><<<b, 256>>>(v->f, v->free_bits, nbricks, v->n, v->nb);
+        if ((st = launch_brick_dist(v, nullptr))) return st;
         hipError_t e = hipDeviceSynchronize();
-        if (e != hipSuccess) st = fail_hip(e, "brick_bound_kernel");
+        if (e != hipSuccess) st = fail_hip(e, "free_bits_kernel");
     }
     return st;
 }
@@ -881,9 +1007,8 @@ FuseArgs fuse_args(const float* depth, int w, int h, const kf_volume* v, const f
     a.f = v->f;
     a.wt = v->w;
     a.touched = v->touched;
-    a.brick_key = v->brick_key;
-    a.super_key = v->super_key;
-    a.ns = v->ns;
+    a.free_bits = v->free_bits;
+    a.dist = v->dist;
     a.cull = is_pinhole(K) ? 1 : 0;
     const double W = (double)w, H = (double)h;
     const double pn[4] = {std::hypot((double)K[0], (double)K[6]), std::hypot((double)K[0], W - (double)K[6]),
@@ -906,6 +1031,9 @@ int launch_fuse_batch(const BatchHeader* hd, const FuseJob* jobs, unsigned cull_
     if (mid) KF_HIP(hipEventRecord(mid, s));
     fuse_batch_list_kernel<<<list_blocks, 64 * kFuseWaves, 0, s>>>(hd, jobs);
     KF_LAUNCHED("fuse_batch_list_kernel");
+    // three workgroups of nine waves fit a CU
+    brick_dist_batch_kernel<<<768, kDistThreads, 0, s>>>(hd, jobs);
+    KF_LAUNCHED("brick_dist_batch_kernel");
     return KF_OK;
 }
 
@@ -974,21 +1102,18 @@ int launch_fuse(const float* depth, int w, int h, kf_volume* v, const float* K, 
     KF_LAUNCHED("fuse_list_kernel");
     if (list_events) KF_HIP(hipEventRecord(list_events[1], s));
     v->fuse_launches += 1;
-    return KF_OK;
+    return launch_brick_dist(v, s);
 }
 
 int launch_initialize(kf_volume* v, float f, float wt, hipStream_t s)
 {
     int64_t count = (int64_t)v->n * v->n * v->n;
     unsigned blocks = (unsigned)std::min<int64_t>((count + 255) / 256, 65536);
-    const int64_t nbricks = (int64_t)v->nb * v->nb * v->nb;
-    const int nsuper = v->ns * v->ns * v->ns;
     if (v->format == KF_VOXEL_F32)
-        init_kernel<KF_VOXEL_F32><<<blocks, 256, 0, s>>>(v->f, v->w, count, f, wt, v->brick_key, nbricks, v->super_key,
-                                                         nsuper);
+        init_kernel<KF_VOXEL_F32><<<blocks, 256, 0, s>>>(v->f, v->w, count, f, wt, v->free_bits, v->dist, v->nb);
     else
-        init_kernel<KF_VOXEL_SNORM16_U8><<<blocks, 256, 0, s>>>(v->f, v->w, count, f, wt, v->brick_key, nbricks,
-                                                                v->super_key, nsuper);
+        init_kernel<KF_VOXEL_SNORM16_U8><<<blocks, 256, 0, s>>>(v->f, v->w, count, f, wt, v->free_bits, v->dist,
+                                                                v->nb);
     KF_LAUNCHED("init_kernel");
     return KF_OK;
 }
@@ -1009,7 +1134,6 @@ int volume_create(int n, float width_m, float mue_m, int format, hipStream_t s, 
     kf_volume* v = new kf_volume();
     v->n = n;
     v->nb = n / 8;
-    v->ns = (v->nb + 7) / 8;
     v->format = format;
     v->width = width_m;
     v->res = width_m / (float)(n - 1);  // voxel_grid.h:43
@@ -1024,8 +1148,8 @@ int volume_create(int n, float width_m, float mue_m, int format, hipStream_t s, 
         (e = hipMalloc(&v->touched, sizeof(unsigned long long) * kFuseBlocks)) != hipSuccess ||
         (e = hipMemsetAsync(v->touched, 0, sizeof(unsigned long long) * kFuseBlocks, s)) != hipSuccess ||
         (e = hipMalloc(&v->brick_list, sizeof(int) * (size_t)v->nb * v->nb * v->nb)) != hipSuccess ||
-        (e = hipMalloc(&v->brick_key, sizeof(int) * (size_t)v->nb * v->nb * v->nb)) != hipSuccess ||
-        (e = hipMalloc(&v->super_key, sizeof(int) * (size_t)v->ns * v->ns * v->ns)) != hipSuccess ||
+        (e = hipMalloc(&v->free_bits, sizeof(unsigned long long) * free_words(v->nb))) != hipSuccess ||
+        (e = hipMalloc(&v->dist, (size_t)v->nb * v->nb * v->nb)) != hipSuccess ||
         (e = hipMalloc(&v->list_count, 2 * sizeof(unsigned int))) != hipSuccess ||
         (e = hipMemsetAsync(v->list_count, 0, 2 * sizeof(unsigned int), s)) != hipSuccess) {
         kf_volume_destroy(v);
@@ -1082,8 +1206,8 @@ int kf_volume_destroy(kf_volume* v)
     (void)hipFree(v->zt);
     (void)hipFree(v->touched);
     (void)hipFree(v->brick_list);
-    (void)hipFree(v->brick_key);
-    (void)hipFree(v->super_key);
+    (void)hipFree(v->free_bits);
+    (void)hipFree(v->dist);
     (void)hipFree(v->list_count);
     (void)hipFree(v->dmax);
     (void)hipFree(v->ray_list);

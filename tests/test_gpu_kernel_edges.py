@@ -58,3 +58,43 @@ def test_preprocess_edges_bit_exact(kf, oracle32, w, h, levels, mirrored, normal
         same(vp[l].download(), v, f"vertex L{l}")
         if normals:
             same(npm[l].download(), oracle32.create_normal_map(v), f"normal L{l}")
+
+
+# Sparse volumes: free space with scattered voxels on either side of the two values that matter to a
+# march (0.991 on large steps, 0 on small ones), so rays run through boxes of free bricks of every size
+# and end, shorten their step or graze at their faces.  n = 8: one brick; 40 and 136: rows that are no
+# multiple of the 8-brick tiles; 528: rows of more than 64 bricks.  4 m and n a power of two take the
+# march's exact texel coordinates, the others its divisions.
+@pytest.mark.parametrize("n,L,mue", [(8, 2.0, 0.05), (40, 2.5, 0.05), (64, 4.0, 0.1), (128, 4.0, 0.02),
+                                     (136, 3.0, 0.03), (528, 5.0, 0.03)])
+@pytest.mark.parametrize("density", [2e-5, 1e-3])
+def test_raycast_sparse_volume_bit_exact(kf, oracle32, n, L, mue, density):
+    w, h = 64, 48
+    rng = np.random.default_rng(n)
+    F = np.full(n ** 3, 1.0, np.float32)
+    F[rng.random(n ** 3, np.float32) < 0.3 * min(1.0, 64 / n)] = 2.0  # unobserved
+    hits = rng.integers(0, n ** 3, max(4, int(density * n ** 3)))
+    F[hits] = rng.choice(np.array([0.992, 0.9909, 0.98, 0.3, 0.0, -0.01, -0.6, -1.0], np.float32), hits.size)
+    slab = F.reshape(n, n, n)
+    slab[-1 - n // 5:, :, :] *= -1.0  # something to end at
+    grid = kf.VoxelGrid(L, n, mue=mue)
+    grid.upload(F, np.ones(n ** 3, np.float32))
+    sensor = kf.Sensor(60.0, 60.0, w / 2 - 0.5, h / 2 - 0.5)
+    vm, nm = kf.GridMap(w, h, 4), kf.GridMap(w, h, 4)
+    init = np.zeros((h, w, 4), np.float32)
+    init[..., 3] = -2
+    for k, (eye, turn) in enumerate([((0.1 * L, -0.05 * L, -0.45 * L), 0.0), ((-0.6 * L, 0.0, 0.1 * L), 1.2),
+                                     ((0.0, 0.0, 0.0), 0.7)]):
+        pose = np.eye(4, dtype=np.float64)
+        pose[0, 0] = pose[2, 2] = np.cos(turn)
+        pose[0, 2], pose[2, 0] = np.sin(turn), -np.sin(turn)
+        pose[:3, 3] = eye
+        sensor.set_pose(pose.T.reshape(-1).astype(np.float32))
+        announce(f"raycast sparse n {n} L {L} mue {mue} density {density} pose {k}")
+        vm.upload(init)
+        nm.upload(init)
+        kf.kernel.raycast(grid, sensor, vm, nm, 0)
+        rv, rn = oracle32.raycast(F, n, L, mue, sensor.get_pose(), sensor.get_inverse_intr(0), w, h, init.copy(),
+                                  init.copy())
+        same(vm.download(), rv, f"vertex pose {k}")
+        same(nm.download(), rn, f"normal pose {k}")
