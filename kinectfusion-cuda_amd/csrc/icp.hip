@@ -4,10 +4,10 @@
 // One iteration = two launches:
 //   reduce   : 256 lanes x 4 pixels per workgroup.  Each lane associates its
 //              pixels (icp.cu:7-82) and accumulates the 27 unique terms of the
-//              normal equations (21 of A^T A, 6 of A^T b) in registers, either
-//              plainly in FP32 or compensated (TwoSum, Kahan-Babuska-Neumaier);
-//              then a 64-lane shuffle tree, an LDS pass over the 4 waves, and
-//              one partial row per workgroup.  A and b are never materialised.
+//              normal equations (21 of A^T A, 6 of A^T b) in FP32 registers;
+//              then a 64-lane shuffle tree and an LDS pass over the 4 waves, in
+//              FP32 or (the compensated form) in FP64, and one partial row per
+//              workgroup.  A and b are never materialised.
 //   finalize : one workgroup sums the partial rows in a fixed order (so the
 //              result is deterministic), solves the 6x6 system with an FP64
 //              Cholesky, applies the pose update (icp.cpp:65-87) and the early
@@ -34,9 +34,21 @@ namespace {
 constexpr int kThreads = 256;
 constexpr int kPixPerThread = 4;  // pixels per lane, at most (see icp_pix_for)
 constexpr int kTerms = 27;
-// partial layout (component-major): [0,27) sums, [27,54) compensations, 54 count
-constexpr int kCountSlot = 54;
-
+// The type the lanes' sums are added up in: FP32, or FP64 for the compensated
+// form.  An FP64 addition issues at the rate of an FP32 one here, so it takes one
+// instruction where FP32 sums that carry their rounding errors (TwoSum) take
+// eight, and rounds at 2^-53.  Association of a tick of 64 sessions, sums with their
+// errors -> FP64: 640x480 (4 pixels per lane) 247 -> 235 us, 320x240 (one) 117 -> 96;
+// a whole compensated frame of 640x480 into 256^3 416 -> 388 us.
+template <bool COMP>
+struct SumType {
+    using T = float;
+};
+template <>
+struct SumType<true> {
+    using T = double;
+};
+// Partial rows (component-major, of SumType): [0,27) sums, 27 the inlier count.
 
 // icp.cu:7-82 split in two: what a pixel needs that does not depend on the
 // pose (its vertex and its live normal, device_helper.cuh:81-110) and the
@@ -163,26 +175,14 @@ __device__ __forceinline__ bool icp_row(const IcpArgs& a, int u, int v, const fl
     return icp_pixel_row(a, icp_pixel_in(a, u, v), Rc, tc, M, tp, row, b);
 }
 
-// (s1, c1) += (s2, c2)
-__device__ __forceinline__ void comp_merge(float& s1, float& c1, float s2, float c2)
+// Adds a pixel's row to the lane's FP32 sums of A^T A (upper triangle) and
+// A^T b, each product fused into its sum (one rounding instead of two).  A lane
+// sums at most kPixPerThread rows, so its few roundings are small against the
+// total; the compensated form takes every addition after that (lanes, waves,
+// workgroups: block_reduce_store and the partial-row sums) in FP64, where
+// nearly all of the additions happen.
+__device__ __forceinline__ void accumulate(float* s, const float* row, float b)
 {
-    float t = s1 + s2;
-    float bp = t - s1;
-    float e = (s1 - (t - bp)) + (s2 - bp);
-    s1 = t;
-    c1 = (c1 + c2) + e;
-}
-
-template <bool COMP>
-// Adds a pixel's row to the lane's sums of A^T A (upper triangle) and A^T b,
-// each product fused into its sum (one rounding instead of two).  A lane sums
-// at most kPixPerThread rows, so its few roundings are small against the
-// total; the compensated form carries the rounding errors of every addition
-// after that (lanes, waves, workgroups: block_reduce_store and the partial-row
-// sums), where nearly all of the additions happen.
-__device__ __forceinline__ void accumulate(float* s, float* c, const float* row, float b)
-{
-    (void)c;
     int q = 0;
 #pragma unroll
     for (int p = 0; p < 6; ++p)
@@ -192,75 +192,68 @@ __device__ __forceinline__ void accumulate(float* s, float* c, const float* row,
     for (int p = 0; p < 6; ++p) s[21 + p] = fmaf(row[p], b, s[21 + p]);
 }
 
-// One halving step of the lane reduction: the first n/2 entries of s (and c)
-// become, on the lane with the step's bit clear, its first half plus the
-// partner's copy and, on the other lane, its second half plus the partner's
-// copy; the compensated merge takes the lower lane's operand first.
-template <bool COMP, int N, int OFF>
-__device__ __forceinline__ void halve_swap(float* s, float* c)
+// The lane exchanges of kf_device.hpp for both sum types.
+template <int CTRL>
+__device__ __forceinline__ float sum_partner(float v)
+{
+    return dpp_partner<CTRL>(v);
+}
+template <int CTRL>
+__device__ __forceinline__ double sum_partner(double v)
+{
+    return __hiloint2double(dpp_partner<CTRL>(__double2hiint(v)), dpp_partner<CTRL>(__double2loint(v)));
+}
+template <int OFF>
+__device__ __forceinline__ void sum_swap(float a, float b, float& lo, float& hi)
+{
+    swap_pair<OFF>(a, b, lo, hi);
+}
+template <int OFF>
+__device__ __forceinline__ void sum_swap(double a, double b, double& lo, double& hi)
+{
+    float l0, l1, h0, h1;
+    swap_pair<OFF>(__int_as_float(__double2loint(a)), __int_as_float(__double2loint(b)), l0, h0);
+    swap_pair<OFF>(__int_as_float(__double2hiint(a)), __int_as_float(__double2hiint(b)), l1, h1);
+    lo = __hiloint2double(__float_as_int(l1), __float_as_int(l0));
+    hi = __hiloint2double(__float_as_int(h1), __float_as_int(h0));
+}
+// Sum over the 64 lanes, in every lane (the same pairing as wave_reduce).
+template <class T>
+__device__ __forceinline__ T wave_total(T v)
+{
+    T lo, hi;
+    sum_swap<32>(v, v, lo, hi);
+    v = lo + hi;
+    sum_swap<16>(v, v, lo, hi);
+    v = lo + hi;
+    v = v + sum_partner<kDppRowMirror>(v);
+    v = v + sum_partner<kDppRowHalfMirror>(v);
+    v = v + sum_partner<kDppXor2>(v);
+    return v + sum_partner<kDppXor1>(v);
+}
+
+// One halving step of the lane reduction: the first n/2 entries of s become, on
+// the lane with the step's bit clear, its first half plus the partner's copy
+// and, on the other lane, its second half plus the partner's copy.
+template <int N, int OFF, class T>
+__device__ __forceinline__ void halve_swap(T* s)
 {
 #pragma unroll
     for (int i = 0; i < N / 2; ++i) {
-        float lo, hi;
-        swap_pair<OFF>(s[i], s[N / 2 + i], lo, hi);
-        if (COMP) {
-            float clo, chi;
-            swap_pair<OFF>(c[i], c[N / 2 + i], clo, chi);
-            comp_merge(lo, clo, hi, chi);
-            s[i] = lo;
-            c[i] = clo;
-        } else {
-            s[i] = lo + hi;
-        }
+        T lo, hi;
+        sum_swap<OFF>(s[i], s[N / 2 + i], lo, hi);
+        s[i] = lo + hi;
     }
 }
-template <bool COMP, int N, int CTRL>
-__device__ __forceinline__ void halve_dpp(float* s, float* c, bool upper)
+template <int N, int CTRL, class T>
+__device__ __forceinline__ void halve_dpp(T* s, bool upper)
 {
 #pragma unroll
     for (int i = 0; i < N / 2; ++i) {
-        const float send = upper ? s[i] : s[N / 2 + i];
-        const float keep = upper ? s[N / 2 + i] : s[i];
-        const float recv = dpp_partner<CTRL>(send);
-        if (COMP) {
-            const float csend = upper ? c[i] : c[N / 2 + i];
-            const float ckeep = upper ? c[N / 2 + i] : c[i];
-            const float crecv = dpp_partner<CTRL>(csend);
-            float ls = upper ? recv : keep, lc = upper ? crecv : ckeep;
-            comp_merge(ls, lc, upper ? keep : recv, upper ? ckeep : crecv);
-            s[i] = ls;
-            c[i] = lc;
-        } else {
-            s[i] = keep + recv;
-        }
+        const T send = upper ? s[i] : s[N / 2 + i];
+        const T keep = upper ? s[N / 2 + i] : s[i];
+        s[i] = keep + sum_partner<CTRL>(send);
     }
-}
-// The compensated form: lane 0 holds the total (the lower lane's operand first
-// in every merge).
-__device__ __forceinline__ void wave_comp_sum(float& s, float& c)
-{
-    const int lane = threadIdx.x & 63;
-    float lo, hi, clo, chi;
-    swap_pair<32>(s, s, lo, hi);
-    swap_pair<32>(c, c, clo, chi);
-    comp_merge(lo, clo, hi, chi);
-    swap_pair<16>(lo, lo, s, hi);
-    swap_pair<16>(clo, clo, c, chi);
-    comp_merge(s, c, hi, chi);
-#define KF_DPP_MERGE(CTRL, BIT)                                                  \
-    {                                                                            \
-        const bool up = (lane & (BIT)) != 0;                                     \
-        const float rs = dpp_partner<CTRL>(s), rc = dpp_partner<CTRL>(c);        \
-        float ls = up ? rs : s, lc = up ? rc : c;                                \
-        comp_merge(ls, lc, up ? s : rs, up ? c : rc);                            \
-        s = ls;                                                                  \
-        c = lc;                                                                  \
-    }
-    KF_DPP_MERGE(kDppRowMirror, 8)
-    KF_DPP_MERGE(kDppRowHalfMirror, 4)
-    KF_DPP_MERGE(kDppXor2, 2)
-    KF_DPP_MERGE(kDppXor1, 1)
-#undef KF_DPP_MERGE
 }
 
 // Reduces the lane values of a workgroup and writes one partial row.  The 27
@@ -268,61 +261,36 @@ __device__ __forceinline__ void wave_comp_sum(float& s, float& c)
 // pad at 27 and one at the 7 -> 8 step): lane L ends with term
 // 14*b5 + 7*b4 + 4*b3 + 2*b2 + b1 of its bits, every pair (L, L^1) holding it
 // (each step keeps the first half on the lane whose step bit is clear).
-template <bool COMP>
-__device__ __forceinline__ void block_reduce_store(float* s_in, float* c_in, int cnt, float* partials, int stride,
-                                                   int row)
+// The first step exchanges the lanes' FP32 sums and widens them as it adds.
+template <class T>
+__device__ __forceinline__ void block_reduce_store(const float* s_in, int cnt, float* partials, int stride, int row)
 {
-    __shared__ float red[kThreads / 64][2 * kTerms + 1];
+    __shared__ T red[kThreads / 64][kTerms + 1];
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    float s[28], c[28];
+    T s[14];
 #pragma unroll
-    for (int q = 0; q < kTerms; ++q) {
-        s[q] = s_in[q];
-        c[q] = COMP ? c_in[q] : 0.0f;
+    for (int q = 0; q < 14; ++q) {
+        float lo, hi;
+        swap_pair<32>(s_in[q], q < 13 ? s_in[14 + q] : 0.0f, lo, hi);
+        s[q] = (T)lo + (T)hi;
     }
-    s[27] = c[27] = 0.0f;
-    halve_swap<COMP, 28, 32>(s, c);
-    halve_swap<COMP, 14, 16>(s, c);
-    s[7] = c[7] = 0.0f;
-    halve_dpp<COMP, 8, kDppRowMirror>(s, c, (lane & 8) != 0);
-    halve_dpp<COMP, 4, kDppRowHalfMirror>(s, c, (lane & 4) != 0);
-    halve_dpp<COMP, 2, kDppXor2>(s, c, (lane & 2) != 0);
-    {
-        // last step: both lanes of the pair add the same two operands, lower first
-        const bool upper = (lane & 1) != 0;
-        const float recv = dpp_partner<kDppXor1>(s[0]);
-        if (COMP) {
-            const float crecv = dpp_partner<kDppXor1>(c[0]);
-            float ls = upper ? recv : s[0], lc = upper ? crecv : c[0];
-            comp_merge(ls, lc, upper ? s[0] : recv, upper ? c[0] : crecv);
-            s[0] = ls;
-            c[0] = lc;
-        } else {
-            s[0] = s[0] + recv;
-        }
-    }
+    halve_swap<14, 16>(s);
+    s[7] = 0;
+    halve_dpp<8, kDppRowMirror>(s, (lane & 8) != 0);
+    halve_dpp<4, kDppRowHalfMirror>(s, (lane & 4) != 0);
+    halve_dpp<2, kDppXor2>(s, (lane & 2) != 0);
+    s[0] = s[0] + sum_partner<kDppXor1>(s[0]);  // both lanes of the pair add the same two operands
     cnt = wave_sum(cnt);
     const int sub = 4 * ((lane >> 3) & 1) + 2 * ((lane >> 2) & 1) + ((lane >> 1) & 1);
     const int q = 14 * ((lane >> 5) & 1) + 7 * ((lane >> 4) & 1) + sub;
-    if ((lane & 1) == 0 && sub < 7 && q < kTerms) {
-        red[wave][q] = s[0];
-        red[wave][kTerms + q] = COMP ? c[0] : 0.0f;
-    }
-    if (lane == 0) red[wave][2 * kTerms] = (float)cnt;
+    if ((lane & 1) == 0 && sub < 7 && q < kTerms) red[wave][q] = s[0];
+    if (lane == 0) red[wave][kTerms] = (T)cnt;
     __syncthreads();
-    if (threadIdx.x < kTerms) {
-        const int q = threadIdx.x;
-        float ss = red[0][q], cc = red[0][kTerms + q];
-        for (int wv = 1; wv < kThreads / 64; ++wv) {
-            if (COMP) comp_merge(ss, cc, red[wv][q], red[wv][kTerms + q]);
-            else ss = ss + red[wv][q];
-        }
-        partials[(int64_t)q * stride + row] = ss;
-        partials[(int64_t)(kTerms + q) * stride + row] = cc;
-    } else if (threadIdx.x == kTerms) {
-        float n = 0.0f;
-        for (int wv = 0; wv < kThreads / 64; ++wv) n = n + red[wv][2 * kTerms];
-        partials[(int64_t)kCountSlot * stride + row] = n;
+    if (threadIdx.x <= kTerms) {
+        const int t = threadIdx.x;
+        T ss = red[0][t];
+        for (int wv = 1; wv < kThreads / 64; ++wv) ss = ss + red[wv][t];
+        reinterpret_cast<T*>(partials)[(int64_t)t * stride + row] = ss;
     }
 }
 
@@ -396,9 +364,9 @@ __device__ void associate_reduce(const IcpArgs& a, const LanePixels<PIX>& lp, co
     m3t(pose + 12, Rt);
     m3m3(a.K, Rt, M);
     const float* tp = pose + 21;
-    float s[kTerms], c[kTerms];
+    float s[kTerms];
 #pragma unroll
-    for (int q = 0; q < kTerms; ++q) s[q] = c[q] = 0.0f;
+    for (int q = 0; q < kTerms; ++q) s[q] = 0.0f;
     int cnt = 0;
     PixelGather g[PIX];
 #pragma unroll
@@ -411,11 +379,11 @@ __device__ void associate_reduce(const IcpArgs& a, const LanePixels<PIX>& lp, co
         if (k >= pix) break;
         float row[6], b;
         if (icp_pixel_finish(a, lp.in[k], g[k], Rc, row, b)) {
-            accumulate<COMP>(s, c, row, b);
+            accumulate(s, row, b);
             ++cnt;
         }
     }
-    block_reduce_store<COMP>(s, c, cnt, a.partials, a.stride, block);
+    block_reduce_store<typename SumType<COMP>::T>(s, cnt, a.partials, a.stride, block);
 }
 
 template <bool COMP>
@@ -445,9 +413,9 @@ template <bool COMP>
 __global__ __launch_bounds__(kThreads) void ab_reduce_kernel(const float* A, const float* B, int64_t n,
                                                              float* partials, int stride)
 {
-    float s[kTerms], c[kTerms];
+    float s[kTerms];
 #pragma unroll
-    for (int q = 0; q < kTerms; ++q) s[q] = c[q] = 0.0f;
+    for (int q = 0; q < kTerms; ++q) s[q] = 0.0f;
     int cnt = 0;
 #pragma unroll
     for (int k = 0; k < kPixPerThread; ++k) {
@@ -457,13 +425,13 @@ __global__ __launch_bounds__(kThreads) void ab_reduce_kernel(const float* A, con
 #pragma unroll
         for (int p = 0; p < 6; ++p) row[p] = A[r * 6 + p];
         float b = B[r];
-        accumulate<COMP>(s, c, row, b);
+        accumulate(s, row, b);
         bool nz = b != 0.0f;
 #pragma unroll
         for (int p = 0; p < 6; ++p) nz = nz || row[p] != 0.0f;
         cnt += nz ? 1 : 0;
     }
-    block_reduce_store<COMP>(s, c, cnt, partials, stride, blockIdx.x);
+    block_reduce_store<typename SumType<COMP>::T>(s, cnt, partials, stride, blockIdx.x);
 }
 
 // icp.cu:7-82, writing the rows (kernel::constructIcpResiduals).
@@ -671,82 +639,70 @@ __device__ void pose_error(const float* R1, const float* t1, const float* R2, co
 
 // Sums the partial rows (fixed order) into 27 doubles + count in LDS.  Wave w
 // owns rows q = w, w + 4, ... (7 of the 28); lane l adds blocks l, l + 64, ...
-// in that order, then the lanes combine (wave_reduce / wave_comp_sum: lane 0
-// ends with the total, the lower lane's operand first).  The loads of all of a
+// in that order, then the lanes combine (wave_total).  The loads of all of a
 // wave's rows for a chunk of kRowHalves 64-block groups (RowChunk) are issued
 // before any is added, so a row set costs one memory round trip per 320 blocks
 // (a 640x480 level is 300); the first chunk can be loaded by the caller ahead
 // of other loads (sum_loaded_partials).
 constexpr int kRowsPerWave = (kTerms + 1 + 3) / 4;
 constexpr int kRowHalves = 5;
+template <class T>
 struct RowChunk {
-    float vs[kRowHalves][kRowsPerWave], vc[kRowHalves][kRowsPerWave];
+    T v[kRowHalves][kRowsPerWave];
 };
 // Needs nblocks > 0.  Lanes past the last block load the last block's entry
 // (no divergent branch around the loads, so none waits for another);
 // add_row_chunk skips them.  Groups wholly past the last block are not loaded
 // (a wave-uniform test).
-template <bool COMP>
-__device__ __forceinline__ void load_row_chunk(const float* partials, int stride, int nblocks, int b0, RowChunk& ch)
+template <class T>
+__device__ __forceinline__ void load_row_chunk(const float* partials, int stride, int nblocks, int b0, RowChunk<T>& ch)
 {
     static_assert(kThreads == 256 && 3 + 4 * (kRowsPerWave - 1) == kTerms, "four waves own rows 0..kTerms");
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const T* rows = reinterpret_cast<const T*>(partials);
 #pragma unroll
     for (int h = 0; h < kRowHalves; ++h) {
         if (h > 0 && b0 + 64 * h >= nblocks) break;
         const int b = min(b0 + 64 * h + lane, nblocks - 1);
 #pragma unroll
-        for (int k = 0; k < kRowsPerWave; ++k) {
-            const int q = wave + 4 * k;
-            const bool is_count = (q == kTerms);  // wave-uniform
-            ch.vs[h][k] = partials[(int64_t)(is_count ? kCountSlot : q) * stride + b];
-            ch.vc[h][k] = (COMP && !is_count) ? partials[(int64_t)(kTerms + q) * stride + b] : 0.0f;
-        }
+        for (int k = 0; k < kRowsPerWave; ++k) ch.v[h][k] = rows[(int64_t)(wave + 4 * k) * stride + b];
     }
 }
-template <bool COMP>
-__device__ __forceinline__ void add_row_chunk(int nblocks, int b0, const RowChunk& ch, float* s, float* c)
+template <class T>
+__device__ __forceinline__ void add_row_chunk(int nblocks, int b0, const RowChunk<T>& ch, T* s)
 {
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int lane = threadIdx.x & 63;
 #pragma unroll
     for (int h = 0; h < kRowHalves; ++h) {
         if (h > 0 && b0 + 64 * h >= nblocks) break;
         const int b = b0 + 64 * h + lane;
 #pragma unroll
-        for (int k = 0; k < kRowsPerWave; ++k) {
-            const int q = wave + 4 * k;
-            if (b < nblocks) {
-                if (COMP && q != kTerms) comp_merge(s[k], c[k], ch.vs[h][k], ch.vc[h][k]);
-                else s[k] = s[k] + ch.vs[h][k];
-            }
-        }
+        for (int k = 0; k < kRowsPerWave; ++k)
+            if (b < nblocks) s[k] = s[k] + ch.v[h][k];
     }
 }
 // `first` = load_row_chunk(partials, stride, nblocks, 0, first); nblocks > 0.
-template <bool COMP>
-__device__ void sum_loaded_partials(const float* partials, int stride, int nblocks, const RowChunk& first,
+template <class T>
+__device__ void sum_loaded_partials(const float* partials, int stride, int nblocks, const RowChunk<T>& first,
                                     double* tot, double* count)
 {
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    float s[kRowsPerWave], c[kRowsPerWave];
+    T s[kRowsPerWave];
 #pragma unroll
-    for (int k = 0; k < kRowsPerWave; ++k) s[k] = c[k] = 0.0f;
-    add_row_chunk<COMP>(nblocks, 0, first, s, c);
+    for (int k = 0; k < kRowsPerWave; ++k) s[k] = 0;
+    add_row_chunk(nblocks, 0, first, s);
     for (int b0 = 64 * kRowHalves; b0 < nblocks; b0 += 64 * kRowHalves) {
-        RowChunk ch;
-        load_row_chunk<COMP>(partials, stride, nblocks, b0, ch);
-        add_row_chunk<COMP>(nblocks, b0, ch, s, c);
+        RowChunk<T> ch;
+        load_row_chunk(partials, stride, nblocks, b0, ch);
+        add_row_chunk(nblocks, b0, ch, s);
     }
 #pragma unroll
     for (int k = 0; k < kRowsPerWave; ++k) {
         const int q = wave + 4 * k;
-        const bool is_count = (q == kTerms);
-        float sk = s[k], ck = c[k];
-        if (COMP && !is_count) wave_comp_sum(sk, ck);
-        else sk = wave_reduce(sk, [](float x, float y) { return x + y; });  // both lanes of a pair: same sum
+        const double t = (double)wave_total(s[k]);  // every lane: the same sum
         if (lane == 0) {
-            if (is_count) *count = (double)sk;
-            else tot[q] = COMP ? (double)sk + (double)ck : (double)sk;
+            if (q == kTerms) *count = t;  // wave-uniform
+            else tot[q] = t;
         }
     }
     __syncthreads();
@@ -754,9 +710,9 @@ __device__ void sum_loaded_partials(const float* partials, int stride, int nbloc
 template <bool COMP>
 __device__ void sum_partials(const float* partials, int stride, int nblocks, double* tot, double* count)
 {
-    RowChunk first = {};
-    if (nblocks > 0) load_row_chunk<COMP>(partials, stride, nblocks, 0, first);
-    sum_loaded_partials<COMP>(partials, stride, nblocks, first, tot, count);
+    RowChunk<typename SumType<COMP>::T> first = {};
+    if (nblocks > 0) load_row_chunk(partials, stride, nblocks, 0, first);
+    sum_loaded_partials(partials, stride, nblocks, first, tot, count);
 }
 
 // Pose update of one iteration from its FP64 solution (one lane): the float
@@ -894,14 +850,15 @@ __device__ __forceinline__ int level_flag(const int* v, int level)
 // the first chunk of the previous launch's partial rows.  Issued before the
 // pixel loads, so waiting for them does not wait for those (loads complete in
 // issue order).
+template <bool COMP>
 struct BeginLoads {
     int cw;
     float pw;
-    RowChunk rows;
+    RowChunk<typename SumType<COMP>::T> rows;
 };
 template <bool COMP>
 __device__ __forceinline__ void issue_begin_loads(const PoseState* st, const IcpCarry* cin, const float* pin,
-                                                  int prev_blocks, BeginLoads& bl)
+                                                  int prev_blocks, BeginLoads<COMP>& bl)
 {
     // every lane loads (indexes clamped; begin_iteration keeps the wanted
     // lanes' words), so no branch makes a load wait for the loads before it
@@ -911,7 +868,7 @@ __device__ __forceinline__ void issue_begin_loads(const PoseState* st, const Icp
     bl.pw = *(pi < 9 ? st->Rp + pi : st->tp + (pi - 9));
     // no branch around the row loads either: with no previous launch
     // (prev_blocks = 0) every lane reads pin[0], and nothing is summed
-    load_row_chunk<COMP>(pin, prev_blocks, max(prev_blocks, 1), 0, bl.rows);
+    load_row_chunk(pin, prev_blocks, max(prev_blocks, 1), 0, bl.rows);
 }
 
 // Phase B of a launch for one session: finish the previous iteration from
@@ -923,13 +880,13 @@ __device__ __forceinline__ void issue_begin_loads(const PoseState* st, const Icp
 // (prev_blocks is that launch's row count, known to the host; a sum nobody
 // needs is discarded), so no load waits for the carry.
 template <bool COMP>
-__device__ void begin_iteration(const BeginLoads& bl, PoseState* st, IcpCarry* cout, const float* pin,
+__device__ void begin_iteration(const BeginLoads<COMP>& bl, PoseState* st, IcpCarry* cout, const float* pin,
                                 int prev_blocks, int level, int blocks, bool first, float stop_angle, float stop_dist,
                                 float* pose, int* run, double* tot, double* count)
 {
     __shared__ IcpCarry carry;
     constexpr int kWords = (int)(sizeof(IcpCarry) / sizeof(int));
-    if (prev_blocks > 0) sum_loaded_partials<COMP>(pin, prev_blocks, prev_blocks, bl.rows, tot, count);
+    if (prev_blocks > 0) sum_loaded_partials(pin, prev_blocks, prev_blocks, bl.rows, tot, count);
     if (threadIdx.x < kWords) reinterpret_cast<int*>(&carry)[threadIdx.x] = bl.cw;
     else if (threadIdx.x >= 64 && threadIdx.x < 76) pose[12 + (threadIdx.x - 64)] = bl.pw;
     __syncthreads();
@@ -964,8 +921,8 @@ __global__ __launch_bounds__(kThreads) void icp_step_kernel(IcpArgs a, const Icp
     __shared__ double count;
     // phase A: the loads of phase B, then the pose-independent loads of this
     // lane's pixels (in flight during B)
-    BeginLoads bl;
-    issue_begin_loads<COMP>(a.st, cin, pin, prev_blocks, bl);
+    BeginLoads<COMP> bl;
+    issue_begin_loads(a.st, cin, pin, prev_blocks, bl);
     LaneLoads<PIX> ll;
     issue_lane_loads(a, ll, blockIdx.x, PIX);
     __builtin_amdgcn_sched_barrier(0);  // nothing of phase B moves above the pixel loads
@@ -1124,7 +1081,7 @@ __global__ __launch_bounds__(kThreads) void icp_batch_solve_kernel(const BatchHe
 }
 
 template <bool COMP>
-__global__ __launch_bounds__(kThreads) void icp_batch_assoc_kernel(const BatchHeader* hd, const IcpJob* jobs,
+__global__ __launch_bounds__(kThreads, 4) void icp_batch_assoc_kernel(const BatchHeader* hd, const IcpJob* jobs,
                                                                    int level)
 {
     __shared__ float pose[24];

@@ -156,7 +156,7 @@ int launch_raycast_levels(const kf_volume* v, const float* pose, const PoseState
                           hipStream_t s);
 
 // ---- ICP (icp.hip)
-constexpr int kPartialStride = 64;  // floats per block partial: 27 sums, 27 compensations, count
+constexpr int kPartialStride = 64;  // floats per block partial: 27 sums and the count, FP32 or FP64
 struct IcpArgs {
     const float4* V;
     const float4* TV;

@@ -98,3 +98,47 @@ def test_raycast_sparse_volume_bit_exact(kf, oracle32, n, L, mue, density):
                                   init.copy())
         same(vm.download(), rv, f"vertex pose {k}")
         same(nm.download(), rn, f"normal pose {k}")
+
+
+# (w, h): a map with one full stencil, one workgroup partly and just filled, one pixel over it, 64 and 65
+# partial rows (one and two per lane of the sum), and more rows than one round of loads takes (320)
+@pytest.mark.parametrize("w,h", [(2, 2), (33, 31), (32, 32), (41, 25), (256, 256), (260, 256), (1300, 260)])
+@pytest.mark.parametrize("comp", [False, True])
+def test_icp_reduce_edges(kf, w, h, comp):
+    """The fused reduction against the FP64 sums of the rows kf_construct_icp_residuals writes.  Every
+    product is fused into a lane's sum of at most 4 rows (4 roundings of 2^-24 of the sum of the
+    products' magnitudes); the plain form then rounds at each of 6 lane steps, 3 waves, ceil(rows / 64)
+    partial rows and 6 lane steps more, the compensated form adds in FP64."""
+    announce(f"kf_icp_reduce {w}x{h} compensated {comp}")
+    rng = np.random.default_rng(7 * w + h)
+    f = 1.2 * w
+    u, v = np.meshgrid(np.arange(w) + 0.5, np.arange(h) + 0.5)
+    z = 2.0 + 0.1 / w * rng.random((h, w))
+    V = np.stack([(u - w / 2) / f * z, (v - h / 2) / f * z, z, np.full((h, w), -1.0)], -1).astype(np.float32)
+    V[rng.random((h, w)) < 0.03] = (0, 0, 0, -2)
+    TV = V.copy()
+    TV[..., :3] += (0.02 * rng.random((h, w, 3)) - 0.01).astype(np.float32)
+    N = np.concatenate([0.2 * rng.random((h, w, 2)) - 0.1, np.ones((h, w, 1))], -1)
+    TN = np.concatenate([N / np.linalg.norm(N, axis=-1, keepdims=True), np.full((h, w, 1), -1.0)], -1)
+    TN = TN.astype(np.float32)
+    maps = []
+    for m in (V, TV, TN):
+        g = kf.GridMap(w, h, 4)
+        g.upload(m)
+        maps.append(g)
+    R, t = np.eye(3, dtype=np.float32).reshape(9), np.zeros(3, np.float32)
+    K = np.array([f, 0, 0, 0, f, 0, w / 2, h / 2, 1], np.float32)
+    th = float(np.deg2rad(60.0))
+    A, b = kf.DeviceArray((h * w, 6)), kf.DeviceArray((h * w,))
+    kf.kernel.construct_icp_residuals(*maps, R, t, R, t, K, 0.1, th, A, b)
+    rows = np.concatenate([A.download(), b.download()[:, None]], 1).astype(np.float64)
+    hits = int(np.any(rows[:, :6] != 0, axis=1).sum())
+    assert hits > 0
+    p, q = [np.concatenate([x, y]) for x, y in zip(np.triu_indices(6), (np.arange(6), np.full(6, 6)))]
+    prod = rows[:, p] * rows[:, q]
+    sums, inliers = kf.kernel.icp_reduce(*maps, R, t, R, t, K, 0.1, th, compensated=comp)
+    assert inliers == hits
+    blocks = -(-w * h // 1024)
+    roundings = 4 if comp else 4 + 6 + 3 + -(-blocks // 64) + 6
+    bound = 1.01 * roundings * 2.0 ** -24 * np.abs(prod).sum(0)
+    assert (np.abs(sums - prod.sum(0)) <= bound).all()
