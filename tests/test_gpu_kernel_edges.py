@@ -115,7 +115,9 @@ def test_icp_reduce_edges(kf, w, h, comp):
     u, v = np.meshgrid(np.arange(w) + 0.5, np.arange(h) + 0.5)
     z = 2.0 + 0.1 / w * rng.random((h, w))
     V = np.stack([(u - w / 2) / f * z, (v - h / 2) / f * z, z, np.full((h, w), -1.0)], -1).astype(np.float32)
-    V[rng.random((h, w)) < 0.03] = (0, 0, 0, -2)
+    holes = rng.random((h, w)) < 0.03
+    holes[:2, :2] = False  # at least one pixel keeps its row
+    V[holes] = (0, 0, 0, -2)
     TV = V.copy()
     TV[..., :3] += (0.02 * rng.random((h, w, 3)) - 0.01).astype(np.float32)
     N = np.concatenate([0.2 * rng.random((h, w, 2)) - 0.1, np.ones((h, w, 1))], -1)
