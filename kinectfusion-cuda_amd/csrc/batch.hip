@@ -53,6 +53,7 @@ struct Slot {
     void* host = nullptr;  // pinned copy of the table
     void* dev = nullptr;
     hipGraphExec_t exec = nullptr;
+    unsigned ray_blocks[2] = {0, 0};  // first-pass raycast workgroups per voxel format in exec
     // tick start, after each stage (preprocess, raycast, ICP, fuse); with per-kernel
     // timing also after the raycast's first pass (5) and after the fuse's brick cull (6)
     hipEvent_t ev[7] = {nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
@@ -66,7 +67,7 @@ struct Slot {
 
 const unsigned kCand[4][kCandidates] = {
     {2048, 4096, 8192, 16384},   // preprocess
-    {2048, 4096, 8192, 16384},   // raycast
+    {8192, 16384, 32768, 65536}, // raycast
     {256, 512, 1024, 2048},      // ICP steps
     {4096, 8192, 16384, 32768},  // fuse list
 };
@@ -111,8 +112,8 @@ struct kf_batch {
     Slot slot[2];
     int next = 0;
     unsigned* fuse_count = nullptr;
-    unsigned* ray_next = nullptr;  // 16 raycast tile counters + 2 deferred-ray counts
-    kf::DeferredRay* ray_list = nullptr;  // 2 x ray_cap deferred rays (per voxel format)
+    unsigned* ray_count = nullptr;  // 16 deferred-ray counts, kf::kCountStride apart
+    kf::DeferredRay* ray_list = nullptr;  // 2 x ray_cap deferred rays (per voxel format, 8 XCDs each)
     size_t ray_cap = 0;
     unsigned long long* fuse_list = nullptr;
     size_t list_cap = 0;
@@ -208,6 +209,32 @@ int drop_graphs(kf_batch* b)
     return KF_OK;
 }
 
+// 8x8 raycast tiles of a session's levels, each level's padded to 8 (one band per XCD).
+size_t ray_tiles_of(const Session& q, int levels)
+{
+    size_t tiles = 0;
+    for (int l = 0; l < levels; ++l) {
+        const size_t tx = (size_t)((q.cfg.frame_width >> l) + 7) / 8, ty = (size_t)((q.cfg.frame_height >> l) + 7) / 8;
+        tiles += (tx * ty + 7) & ~(size_t)7;
+    }
+    return tiles;
+}
+
+// First-pass raycast workgroups per voxel format: the shape's, or fewer where the
+// resident sessions have fewer tiles (to a power of two, so that sessions coming one
+// by one change it seldom), none for a format without sessions.
+void ray_grids(const kf_batch* b, const kf_batch_shape& sh, unsigned out[2])
+{
+    size_t tiles[2] = {0, 0};
+    for (const Session& q : b->sess)
+        if (q.used) tiles[q.cfg.voxel_format == KF_VOXEL_F32 ? 0 : 1] += ray_tiles_of(q, b->cfg.icp.levels);
+    for (int f = 0; f < 2; ++f) {
+        size_t g = tiles[f] ? 1024 : 0;
+        while (g && g < tiles[f]) g *= 2;
+        out[f] = (unsigned)std::min(g, (size_t)sh.raycast_blocks);
+    }
+}
+
 // Total bricks of the resident sessions: the fuse list never holds more.
 // Deferred raycast rays: room for every ray of the resident sessions, per
 // voxel format, up to kMaxDeferred (beyond it a lane marches its ray itself).
@@ -218,8 +245,7 @@ int ensure_ray_list(kf_batch* b)
     size_t need = 0;
     for (const Session& q : b->sess)
         if (q.used) {
-            const size_t w = (size_t)q.cfg.frame_width, h = (size_t)q.cfg.frame_height;
-            need += w * h + (w / 2) * (h / 2) + (w / 4) * (h / 4);
+            need += ray_tiles_of(q, 3) * 64;
         }
     need = std::min(need, kMaxDeferred);
     if (need <= b->ray_cap) return KF_OK;
@@ -267,7 +293,9 @@ int enqueue_tick(kf_batch* b, const Slot& sl, const kf_batch_shape& sh, hipEvent
     int st;
     if ((st = kf::launch_preprocess_batch(hd, pre, sh.preprocess_blocks, s))) return st;
     if (ev) KF_HIP(hipEventRecord(ev[1], s));
-    if ((st = kf::launch_raycast_batch(hd, ray, sh.raycast_blocks, s, fine ? ev[5] : nullptr))) return st;
+    unsigned ray_blocks[2];
+    ray_grids(b, sh, ray_blocks);
+    if ((st = kf::launch_raycast_batch(hd, ray, ray_blocks, s, fine ? ev[5] : nullptr))) return st;
     if (ev) KF_HIP(hipEventRecord(ev[2], s));
     const kf_icp_config& ic = b->cfg.icp;
     if ((st = kf::launch_icp_batch(hd, icp, ic.iters_per_layer, ic.levels, b->cfg.max_sessions, ic.compensated,
@@ -284,6 +312,7 @@ int capture(kf_batch* b, Slot& sl)
 {
     hipGraph_t g = nullptr;
     KF_HIP(hipStreamBeginCapture(b->s, hipStreamCaptureModeThreadLocal));
+    ray_grids(b, b->shape, sl.ray_blocks);
     int st = enqueue_tick(b, sl, b->shape, nullptr);
     hipError_t e = hipStreamEndCapture(b->s, &g);
     if (st) {
@@ -368,7 +397,7 @@ void default_shape(kf_batch_shape& s, const kf_batch_shape& given)
 {
     // the shapes the tuner picks for 64 sessions of 640x480 -> 512^3
     s.preprocess_blocks = given.preprocess_blocks ? given.preprocess_blocks : 8192;
-    s.raycast_blocks = given.raycast_blocks ? given.raycast_blocks : 8192;
+    s.raycast_blocks = given.raycast_blocks ? given.raycast_blocks : 65536;
     s.icp_blocks = given.icp_blocks ? given.icp_blocks : 1024;
     // the brick cull (not tuned): per 64 x 512^3 tick 0.18 ms at 4096 workgroups, 0.16 at 8192,
     // 0.15 at 16384
@@ -420,7 +449,7 @@ int kf_batch_destroy(kf_batch* b)
     for (Session& q : b->sess)
         if (q.used) free_session(q);
     (void)hipFree(b->fuse_count);
-    (void)hipFree(b->ray_next);
+    (void)hipFree(b->ray_count);
     (void)hipFree(b->ray_list);
     (void)hipFree(b->fuse_list);
     (void)hipFree(b->touched);
@@ -473,7 +502,7 @@ int kf_batch_create(const kf_batch_config* cfg, kf_stream_t stream, kf_batch** o
             if (!st && hipEventCreate(&ev) != hipSuccess) st = kf::fail(KF_ERR_HIP, "kf_batch_create events");
     }
     if (!st) st = alloc((void**)&b->fuse_count, sizeof(unsigned), nullptr);
-    if (!st) st = alloc((void**)&b->ray_next, 18 * sizeof(unsigned), nullptr);
+    if (!st) st = alloc((void**)&b->ray_count, 16 * kf::kCountStride * sizeof(unsigned), nullptr);
     if (!st) st = alloc((void**)&b->touched, sizeof(unsigned long long) * kMaxFuseBlocks, nullptr);
     if (!st) {
         hipError_t e = hipMemset(b->touched, 0, sizeof(unsigned long long) * kMaxFuseBlocks);
@@ -593,9 +622,9 @@ int kf_batch_tick(kf_batch* b, int n, const int* ids, const uint16_t* const* raw
     auto* fuse = reinterpret_cast<kf::FuseJob*>(base + b->off_fuse);
     memset(hd, 0, sizeof(*hd));
     hd->fuse_count = b->fuse_count;
-    hd->ray_next = b->ray_next;
+    hd->ray_count = b->ray_count;
     hd->ray_list = b->ray_list;
-    hd->ray_list_cap = (unsigned)b->ray_cap;
+    hd->ray_list_cap = (unsigned)(b->ray_cap / 8);
     hd->fuse_list = b->fuse_list;
     hd->touched = b->touched;
     const kf_icp_config& ic = b->cfg.icp;
@@ -672,7 +701,7 @@ int kf_batch_tick(kf_batch* b, int n, const int* ids, const uint16_t* const* raw
             Session& q = b->sess[ids[k]];
             if (q.frames == 0 || q.cfg.voxel_format != fmt) continue;
             const int w = q.cfg.frame_width, h = q.cfg.frame_height;
-            for (int l = 0; l < ic.levels; ++l) {
+            for (int l = ic.levels - 1; l >= 0; --l) {  // the coarse levels' tiles march longest
                 kf::RaycastJob& R = ray[n_ray++];
                 memset(&R, 0, sizeof(R));
                 R.vol = kf::raycast_volume(q.vol);
@@ -685,7 +714,7 @@ int kf_batch_tick(kf_batch* b, int n, const int* ids, const uint16_t* const* raw
                 R.L.h = h >> l;
                 R.L.tiles_x = (R.L.w + 7) / 8;
                 R.L.tile0 = ray_tiles;
-                ray_tiles += R.L.tiles_x * ((R.L.h + 7) / 8);
+                ray_tiles += (R.L.tiles_x * ((R.L.h + 7) / 8) + 7) & ~7;
             }
         }
     }
@@ -720,6 +749,12 @@ int kf_batch_tick(kf_batch* b, int n, const int* ids, const uint16_t* const* raw
         st = enqueue_tick(b, sl, b->shape, sl.ev, true);
         sl.fine = true;
     } else if (b->cfg.use_graph) {
+        unsigned need[2];
+        ray_grids(b, b->shape, need);
+        if (sl.exec && (need[0] > sl.ray_blocks[0] || need[1] > sl.ray_blocks[1])) {
+            (void)hipGraphExecDestroy(sl.exec);  // its last tick is done (retire)
+            sl.exec = nullptr;
+        }
         if (!sl.exec) st = capture(b, sl);
         if (!st) {
             KF_HIP(hipEventRecord(sl.ev[0], b->s));

@@ -13,12 +13,17 @@ int launch_down_sample(const float* in, int w_in, int h_in, float* out, hipStrea
 int launch_vertex_map(const float* depth, float4* out, int w, int h, const float* inv_k, hipStream_t s);
 int launch_normal_map(const float4* v, float4* out, int w, int h, hipStream_t s);
 
+// Counters that the waves of different XCDs add to lie this many words apart: a
+// returning atomic on a 128-byte line that the whole device shares completes one
+// in 11 ns.
+constexpr int kCountStride = 32;
+
 // ---- batch ticks (batch.hip): one table per tick in device memory, a header
 // followed by the job arrays of every stage.  Counts are per tick; the fuse
 // brick list, its counter and the touched slots belong to the batch.
 struct BatchHeader {
     int n_pre, pre_tiles, pyr_tiles;  // preprocess jobs, L0 16x16 tiles, L2 16x16 tiles
-    int n_ray, ray_tiles;             // raycast jobs (session x level), 8x8 tiles
+    int n_ray, ray_tiles;             // raycast jobs (session x level), 8x8 tiles, each job's padded to 8
     int n_ray_f32, ray_tiles_f32;     // the FP32-volume jobs come first: their count and tiles
     int n_icp, icp_blocks[3];         // ICP sessions, blocks per level
     int n_fuse;                       // fuse jobs
@@ -27,9 +32,9 @@ struct BatchHeader {
     unsigned* fuse_count;
     unsigned long long* fuse_list;    // job << 32 | brick of the job's volume
     unsigned long long* touched;
-    unsigned* ray_next;  // 16 tile counters (8 XCD bands x 2 voxel formats) and 2 deferred-ray
-                         // counts (per format), cleared by the first kernel
-    struct DeferredRay* ray_list;  // 2 x ray_list_cap deferred rays (F32 jobs, then snorm16 jobs)
+    unsigned* ray_count;  // 16 deferred-ray counts (8 XCDs of the F32 jobs, then of the snorm16 jobs),
+                          // kCountStride apart, cleared by the first kernel
+    struct DeferredRay* ray_list;  // 16 lists of ray_list_cap deferred rays, in the same order
     unsigned ray_list_cap;
 };
 
@@ -128,7 +133,7 @@ struct RaycastLevel {
     float Kinv[9];
     float4* vout;
     float4* nout;
-    int w, h, tiles_x, tile0;  // tile0: first global tile of this level
+    int w, h, tiles_x, tile0;  // tile0: first global tile of this level (batch ticks: a multiple of 8)
 };
 // A ray the per-lane march handed to the finishing pass: its march state
 // before the sample at t.
@@ -145,8 +150,10 @@ struct RaycastJob {
     RaycastLevel L;
 };
 RaycastVolume raycast_volume(const kf_volume* v);
-// mid (optional): an event recorded between the first pass and the finishing pass.
-int launch_raycast_batch(const BatchHeader* hd, const RaycastJob* jobs, unsigned blocks, hipStream_t s,
+// blocks: workgroups of the first pass per voxel format, 0 (no jobs of that format)
+// or a multiple of 8.  mid (optional): an event recorded between the first pass and
+// the finishing pass.
+int launch_raycast_batch(const BatchHeader* hd, const RaycastJob* jobs, const unsigned blocks[2], hipStream_t s,
                          hipEvent_t mid = nullptr);
 int launch_raycast(const kf_volume* v, const float* pose, const PoseState* dyn_state, const float* inv_k,
                    float4* vout, float4* nout, int w, int h, hipStream_t s);

@@ -334,16 +334,15 @@ __global__ __launch_bounds__(256) void pyramid_kernel(PreJob J)
 }
 
 // Many sessions per launch (batch ticks), persistent over the tick's tiles.
-// The first kernel also clears the tick's fuse-list counter and raycast tile
-// counters, which later passes of this tick use.
+// The first kernel also clears the tick's fuse-list counter and deferred-ray
+// counts, which later passes of this tick use.
 __global__ __launch_bounds__(256) void measure_batch_kernel(const BatchHeader* hd, const PreJob* jobs)
 {
     __shared__ BilateralTile tile;
     __shared__ float wave_max[4];
     if (blockIdx.x == 0 && threadIdx.y == 0) {
         if (threadIdx.x == 0) *hd->fuse_count = 0u;
-        hd->ray_next[threadIdx.x] = 0u;  // kTile == 16 tile counters
-        if (threadIdx.x < 2) hd->ray_next[16 + threadIdx.x] = 0u;  // deferred-ray counts
+        hd->ray_count[threadIdx.x * kCountStride] = 0u;  // kTile == 16 deferred-ray counts
     }
     const int tiles = hd->pre_tiles, njobs = hd->n_pre;
     for (int tl = blockIdx.x; tl < tiles; tl += gridDim.x) {

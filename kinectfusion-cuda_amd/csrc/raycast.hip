@@ -39,12 +39,18 @@ constexpr float kMargin = 0.01f;
 // the front when the wave took longer than the level's mean, else at the back,
 // so the tiles that marched longest start first (they made the kernel's tail
 // when they started late).  The mean is estimated from one wave in eight,
-// summed per level and XCD (one shared sum per level made every wave wait on
-// the same contended atomic).  Only the order changes, never a result.
+// summed per level and XCD.  Only the order changes, never a result.  What one
+// XCD's waves count with lies in 128 bytes of its own (kCountStride).
 struct TileOrderState {
-    unsigned ctr[2][3][8][2];         // [parity][level][XCD][front, back] appends
-    unsigned long long dur[3][3][8];  // [launch % 3][level][XCD] sum of sampled wave times
-    unsigned waves[3][3][8];          // [launch % 3][level][XCD] waves sampled
+    struct Appends {
+        unsigned ctr[3][2];  // [level][front, back] appends
+        unsigned pad[kCountStride - 6];
+    } ctr[2][8];             // [parity][XCD]
+    struct Times {
+        unsigned long long dur[3];  // [level] sum of sampled wave times
+        unsigned waves[3];          // [level] waves sampled
+        unsigned pad[kCountStride - 9];
+    } time[3][8];                   // [launch % 3][XCD]
 };
 struct RaycastArgs {
     RaycastVolume vol;
@@ -52,9 +58,9 @@ struct RaycastArgs {
     const PoseState* dyn;  // when set, the pose comes from dyn->pose
     RaycastLevel lv[3];
     int levels, tiles;
-    DeferredRay* rays;  // rays handed to the finishing pass (at most cap)
-    unsigned* count;    // their count for this launch
-    unsigned* clear;    // the count of the other launch parity, cleared for the next launch
+    DeferredRay* rays;  // rays handed to the finishing pass: 8 lists (XCDs) of at most cap
+    unsigned* count;    // their counts for this launch, kCountStride apart
+    unsigned* clear;    // the counts of the other launch parity, cleared for the next launch
     unsigned cap;
     const int* order_in;   // band slot of each workgroup, from the previous launch (null: g / 8)
     int* order_out;        // the same for the next launch (null: not recorded)
@@ -384,7 +390,9 @@ __device__ __forceinline__ void advance(float& t, float& prev_t, float step, int
 // of both steps' code; the boxes of free bricks leave 8 large-step and 7
 // small-step ones.  First + finishing pass: 64 frames of 640x480 from 512^3
 // snorm16 volumes 3.98 + 0.45 -> 3.14 + 0.28 ms, one frame from 512^3 FP32 105 + 22
-// -> 86 + 17 us, its coarsest level alone (160x120) 52 -> 30 us.
+// -> 86 + 17 us, its coarsest level alone (160x120) 52 -> 30 us.  With lists per
+// XCD instead of one for the launch (their counters in lines of their own) 66 + 11
+// us, and 2.36 + 0.27 ms (raycast_batch_kernel).
 template <int FMT, bool P2>
 __device__ __forceinline__ void raycast_pixel(const RaycastVolume& a, const float* pose, const RaycastLevel& L, int i,
                                               int j, bool in_image, const RayQueue& rq, int job)
@@ -657,16 +665,16 @@ __device__ __forceinline__ void record_order(const RaycastArgs& a, int l, int x,
     unsigned long long n = 0, sum = 0;
 #pragma unroll
     for (int q = 0; q < 8; ++q) {
-        n += o->waves[prev][l][q];
-        sum += o->dur[prev][l][q];
+        n += o->time[prev][q].waves[l];
+        sum += o->time[prev][q].dur[l];
     }
     const bool front = n == 0 || dur * n > sum;
-    unsigned* c = &o->ctr[1 - a.parity][l][x][front ? 0 : 1];
+    unsigned* c = &o->ctr[1 - a.parity][x].ctr[l][front ? 0 : 1];
     const int k = (int)atomicAdd(c, 1u);
     if (k < per) a.order_out[base + (front ? k : per - 1 - k) * 8 + x] = slot;
     if (dur != 0 && ((int)blockIdx.x / 8) % 8 == 0) {  // one workgroup in eight
-        atomicAdd(&o->dur[a.tri][l][x], dur);
-        atomicAdd(&o->waves[a.tri][l][x], 1u);
+        atomicAdd(&o->time[a.tri][x].dur[l], dur);
+        atomicAdd(&o->time[a.tri][x].waves[l], 1u);
     }
 }
 
@@ -678,14 +686,15 @@ __global__ __launch_bounds__(64, 5) void raycast_kernel(RaycastArgs a)
 {
     const unsigned long long t0 = wall_clock64();
     if (blockIdx.x == 0) {
-        if (threadIdx.x == 0) *a.clear = 0u;
-        if (a.ost) {
+        if (threadIdx.x < 8) a.clear[threadIdx.x * kCountStride] = 0u;
+        if (a.ost && threadIdx.x < 8) {
             // counters the next launch appends with, and the wave times of the launch after it
-            unsigned* c = &a.ost->ctr[a.parity][0][0][0];
-            if (threadIdx.x < 3 * 8 * 2) c[threadIdx.x] = 0u;
-            if (threadIdx.x < 3 * 8) {
-                (&a.ost->dur[(a.tri + 1) % 3][0][0])[threadIdx.x] = 0ull;
-                (&a.ost->waves[(a.tri + 1) % 3][0][0])[threadIdx.x] = 0u;
+            TileOrderState::Appends& c = a.ost->ctr[a.parity][threadIdx.x];
+            TileOrderState::Times& t = a.ost->time[(a.tri + 1) % 3][threadIdx.x];
+            for (int l = 0; l < 3; ++l) {
+                c.ctr[l][0] = c.ctr[l][1] = 0u;
+                t.dur[l] = 0ull;
+                t.waves[l] = 0u;
             }
         }
     }
@@ -705,7 +714,7 @@ __global__ __launch_bounds__(64, 5) void raycast_kernel(RaycastArgs a)
         const RaycastLevel& L = a.lv[l];
         const int i = (lt % L.tiles_x) * 8 + (threadIdx.x & 7);
         const int j = (lt / L.tiles_x) * 8 + (threadIdx.x >> 3);
-        const RayQueue rq{a.rays, a.count, a.cap, kSmallTrips};
+        const RayQueue rq{a.rays + (size_t)x * a.cap, a.count + x * kCountStride, a.cap, kSmallTrips};
         const float* pose = a.dyn ? a.dyn->pose : a.pose;
         if (a.vol.p2) raycast_pixel<FMT, true>(a.vol, pose, L, i, j, i < L.w && j < L.h, rq, l);
         else raycast_pixel<FMT, false>(a.vol, pose, L, i, j, i < L.w && j < L.h, rq, l);
@@ -727,17 +736,49 @@ constexpr unsigned kFinishWaves = 8192;
 constexpr unsigned kBatchFinishWaves = 65536;
 constexpr unsigned kFinishPer = 4;
 
+// The 8 lists of a launch as one: ray r is number r - start of list x.  Every
+// wave takes its rays from all lists alike, since a band of the image where the
+// rays graze the floor hands over many times the rays of another (each XCD's waves
+// on their own XCD's list: 16 instead of 11 us, 340 instead of 260 us in a tick of
+// 64 sessions).  The counts are read through the constant address space (scalar
+// loads; nothing writes them while a finishing pass runs).
+struct RayLists {
+    unsigned end[8];  // end[x]: rays of lists 0..x
+};
+__device__ __forceinline__ RayLists ray_lists(const unsigned* count, unsigned cap)
+{
+    typedef __attribute__((address_space(4))) const unsigned ConstCount;
+    RayLists r;
+    unsigned sum = 0;
+#pragma unroll
+    for (int x = 0; x < 8; ++x) {
+        const unsigned n = ((ConstCount*)count)[x * kCountStride];
+        sum += n < cap ? n : cap;
+        r.end[x] = sum;
+    }
+    return r;
+}
+__device__ __forceinline__ size_t ray_slot(const RayLists& l, unsigned cap, unsigned r)
+{
+    unsigned x = 0, start = 0;
+#pragma unroll
+    for (int q = 0; q < 7; ++q)
+        if (r >= l.end[q]) {
+            x = q + 1;
+            start = l.end[q];
+        }
+    return (size_t)x * cap + (r - start);
+}
+
 template <int FMT>
 __global__ __launch_bounds__(64 * kFinishPer) void raycast_finish_kernel(RaycastArgs a)
 {
-    typedef __attribute__((address_space(4))) const unsigned ConstCount;
     typedef __attribute__((address_space(4))) const DeferredRay ConstRay;
-    const unsigned total = *(ConstCount*)a.count;
-    const unsigned n = total < a.cap ? total : a.cap;
+    const RayLists lists = ray_lists(a.count, a.cap);
     const float* pose = a.dyn ? a.dyn->pose : a.pose;
     const unsigned w0 = blockIdx.x * kFinishPer + (unsigned)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    for (unsigned r = w0; r < n; r += gridDim.x * kFinishPer) {
-        ConstRay& cr = ((ConstRay*)a.rays)[r];
+    for (unsigned r = w0; r < lists.end[7]; r += gridDim.x * kFinishPer) {
+        ConstRay& cr = ((ConstRay*)a.rays)[ray_slot(lists, a.cap, r)];
         DeferredRay d;
         d.job = cr.job;
         d.px = cr.px;
@@ -748,6 +789,15 @@ __global__ __launch_bounds__(64 * kFinishPer) void raycast_finish_kernel(Raycast
         if (a.vol.p2) finish_ray<FMT, true>(a.vol, pose, a.lv[d.job], d);
         else finish_ray<FMT, false>(a.vol, pose, a.lv[d.job], d);
     }
+}
+
+// The handed-over rays of format FMT's tiles on XCD x.
+template <int FMT, class Header>
+__device__ __forceinline__ RayQueue ray_queue(const Header& hd, int x)
+{
+    const int k = (FMT == KF_VOXEL_F32 ? 0 : 8) + x;
+    return RayQueue{hd.ray_list + (size_t)k * hd.ray_list_cap, hd.ray_count + k * kCountStride, hd.ray_list_cap,
+                    kBatchSmallTrips};
 }
 
 // Field-wise copy of a job read through the constant address space.
@@ -773,60 +823,53 @@ __device__ __forceinline__ void copy_job(const CJ& j, RaycastVolume& vol, Raycas
     L.tile0 = j.L.tile0;
 }
 
-// Many sessions and levels per persistent launch, one launch per voxel format:
-// the jobs of format FMT are jobs[j0, j1), covering tiles [t0, t1) of the tick
-// (jobs[k] covers [jobs[k].L.tile0, jobs[k+1].L.tile0)).  March lengths vary
-// by an order of magnitude between tiles (rays grazing a surface take hundreds
-// of small steps), so tiles are claimed dynamically: the range is cut into 8
-// bands, workgroups on XCD x claim pairs of tiles of band x from its counter
-// (locality in that XCD's L2) and then help the other bands until all are done.
-constexpr int kClaim = 2;  // tiles per claim
-
+// Many sessions and levels per launch, one launch per voxel format: the jobs of
+// format FMT are jobs[j0, j1), their tiles padded to multiples of 8 and numbered
+// [t0, t1) (jobs[k] has [jobs[k].L.tile0, jobs[k+1].L.tile0)).  As in
+// raycast_kernel each job's tiles are cut into 8 bands, one per XCD, so every XCD
+// gets its share of every job and keeps a part of each volume in its L2;
+// workgroups on XCD x take the tiles of its bands in turn.
+//
+// March lengths vary by an order of magnitude between tiles, so a workgroup takes
+// few of them and the hardware's dispatch levels the load.  Waves that claimed
+// pairs of tiles from counters instead were bound by those: returning atomics of
+// the whole device on one 128-byte line complete one in 11 ns, and 8192 waves
+// that each look for work in all 8 bands make 65536 of them (0.74 ms) before a
+// launch of any size ends.  First pass, claimed -> dispatched: 64 sessions of
+// 640x480 from 512^3 snorm16 volumes 2.91 -> 2.36 ms, 16 uneven sessions 1.07 ->
+// 0.39; the tick of 64 with 16384, 32768, 65536 workgroups 7.94, 7.71, 7.64 ms.
 template <int FMT>
 __global__ __launch_bounds__(64) void raycast_batch_kernel(const BatchHeader* hd, const RaycastJob* jobs)
 {
-    const RayQueue rq{hd->ray_list + (FMT == KF_VOXEL_F32 ? 0u : hd->ray_list_cap),
-                      hd->ray_next + (FMT == KF_VOXEL_F32 ? 16 : 17), hd->ray_list_cap, kBatchSmallTrips};
+    const int x = (int)(blockIdx.x & 7);
     const int nf = hd->n_ray_f32, tf = hd->ray_tiles_f32;
     const int j0 = FMT == KF_VOXEL_F32 ? 0 : nf, j1 = FMT == KF_VOXEL_F32 ? nf : hd->n_ray;
     const int t0 = FMT == KF_VOXEL_F32 ? 0 : tf, t1 = FMT == KF_VOXEL_F32 ? tf : hd->ray_tiles;
-    if (t1 <= t0) return;
-    unsigned* next = hd->ray_next + (FMT == KF_VOXEL_F32 ? 0 : 8);
-    const int per = (t1 - t0 + 7) / 8;
-    const int xcd = (int)(blockIdx.x & 7);
+    const RayQueue rq = ray_queue<FMT>(*hd, x);
     // The table is read through the constant address space: it is never written
     // while the kernel runs, so its fields load with scalar loads into scalar
     // registers even after the kernel's stores (the vertex and normal maps).
     typedef __attribute__((address_space(4))) const RaycastJob ConstJob;
     ConstJob* cj = (ConstJob*)jobs;
-    for (int bi = 0; bi < 8; ++bi) {
-        const int band = (xcd + bi) & 7;
-        const int b0 = t0 + band * per, b1 = min(t1, b0 + per);
-        for (;;) {
-            int c = 0;
-            if (threadIdx.x == 0) c = (int)atomicAdd(&next[band], 1u);
-            c = __builtin_amdgcn_readlane(c, 0);
-            const int tc = b0 + c * kClaim;
-            if (tc >= b1) break;
-            for (int t = tc; t < min(b1, tc + kClaim); ++t) {
-                int lo = j0, hi = j1 - 1;
-                while (lo < hi) {
-                    const int mid = (lo + hi + 1) >> 1;
-                    if (cj[mid].L.tile0 <= t) lo = mid;
-                    else hi = mid - 1;
-                }
-                const int jb = __builtin_amdgcn_readfirstlane(lo);
-                RaycastVolume vol;
-                RaycastLevel L;
-                copy_job(cj[jb], vol, L);
-                const float* pose = cj[jb].pose;
-                const int lt = t - L.tile0;
-                const int i = (lt % L.tiles_x) * 8 + (threadIdx.x & 7);
-                const int j = (lt / L.tiles_x) * 8 + (threadIdx.x >> 3);
-                if (vol.p2) raycast_pixel<FMT, true>(vol, pose, L, i, j, i < L.w && j < L.h, rq, jb);
-                else raycast_pixel<FMT, false>(vol, pose, L, i, j, i < L.w && j < L.h, rq, jb);
-            }
+    for (int t = t0 + (int)(blockIdx.x & ~7u); t < t1; t += (int)gridDim.x) {
+        int lo = j0, hi = j1 - 1;
+        while (lo < hi) {
+            const int mid = (lo + hi + 1) >> 1;
+            if (cj[mid].L.tile0 <= t) lo = mid;
+            else hi = mid - 1;
         }
+        const int jb = __builtin_amdgcn_readfirstlane(lo);
+        RaycastVolume vol;
+        RaycastLevel L;
+        copy_job(cj[jb], vol, L);
+        const float* pose = cj[jb].pose;
+        const int tiles = L.tiles_x * ((L.h + 7) / 8);
+        const int lt = x * ((tiles + 7) / 8) + (t - L.tile0) / 8;
+        if (lt >= tiles) continue;  // padding of the last bands
+        const int i = (lt % L.tiles_x) * 8 + (threadIdx.x & 7);
+        const int j = (lt / L.tiles_x) * 8 + (threadIdx.x >> 3);
+        if (vol.p2) raycast_pixel<FMT, true>(vol, pose, L, i, j, i < L.w && j < L.h, rq, jb);
+        else raycast_pixel<FMT, false>(vol, pose, L, i, j, i < L.w && j < L.h, rq, jb);
     }
 }
 
@@ -838,23 +881,21 @@ __global__ __launch_bounds__(64 * kFinishPer) void raycast_batch_finish_kernel(c
 {
     typedef __attribute__((address_space(4))) const RaycastJob ConstJob;
     typedef __attribute__((address_space(4))) const BatchHeader ConstHeader;
-    typedef __attribute__((address_space(4))) const unsigned ConstCount;
     typedef __attribute__((address_space(4))) const DeferredRay ConstRay;
     ConstJob* cj = (ConstJob*)jobs;
-    ConstHeader* ch = (ConstHeader*)hd;
-    const unsigned cap = ch->ray_list_cap;
-    const unsigned total = *(ConstCount*)(ch->ray_next + (FMT == KF_VOXEL_F32 ? 16 : 17));
-    const unsigned n = total < cap ? total : cap;
-    ConstRay* rays = (ConstRay*)(ch->ray_list + (FMT == KF_VOXEL_F32 ? 0u : cap));
+    const RayQueue rq = ray_queue<FMT>(*(ConstHeader*)hd, 0);
+    const RayLists lists = ray_lists(rq.count, rq.cap);
+    ConstRay* rays = (ConstRay*)rq.rays;
     const unsigned w0 = blockIdx.x * kFinishPer + (unsigned)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    for (unsigned r = w0; r < n; r += gridDim.x * kFinishPer) {
+    for (unsigned r = w0; r < lists.end[7]; r += gridDim.x * kFinishPer) {
+        const size_t k = ray_slot(lists, rq.cap, r);
         DeferredRay d;
-        d.job = rays[r].job;
-        d.px = rays[r].px;
-        d.flags = rays[r].flags;
-        d.t = rays[r].t;
-        d.prev = rays[r].prev;
-        d.prev_t = rays[r].prev_t;
+        d.job = rays[k].job;
+        d.px = rays[k].px;
+        d.flags = rays[k].flags;
+        d.t = rays[k].t;
+        d.prev = rays[k].prev;
+        d.prev_t = rays[k].prev_t;
         RaycastVolume vol;
         RaycastLevel L;
         copy_job(cj[d.job], vol, L);
@@ -881,20 +922,29 @@ RaycastVolume raycast_volume(const kf_volume* v)
     return r;
 }
 
-// The two voxel formats use disjoint tile counters, ray-list halves and maps, so
-// both first passes run before both finishing passes.
-int launch_raycast_batch(const BatchHeader* hd, const RaycastJob* jobs, unsigned blocks, hipStream_t s, hipEvent_t mid)
+// The two voxel formats use disjoint ray lists and maps, so both first passes run
+// before both finishing passes.  A format without workgroups is not launched.
+int launch_raycast_batch(const BatchHeader* hd, const RaycastJob* jobs, const unsigned blocks[2], hipStream_t s,
+                         hipEvent_t mid)
 {
-    raycast_batch_kernel<KF_VOXEL_F32><<<blocks, 64, 0, s>>>(hd, jobs);
-    KF_LAUNCHED("raycast_batch_kernel");
-    raycast_batch_kernel<KF_VOXEL_SNORM16_U8><<<blocks, 64, 0, s>>>(hd, jobs);
-    KF_LAUNCHED("raycast_batch_kernel");
+    if (blocks[0]) {
+        raycast_batch_kernel<KF_VOXEL_F32><<<blocks[0], 64, 0, s>>>(hd, jobs);
+        KF_LAUNCHED("raycast_batch_kernel");
+    }
+    if (blocks[1]) {
+        raycast_batch_kernel<KF_VOXEL_SNORM16_U8><<<blocks[1], 64, 0, s>>>(hd, jobs);
+        KF_LAUNCHED("raycast_batch_kernel");
+    }
     if (mid) KF_HIP(hipEventRecord(mid, s));
-    raycast_batch_finish_kernel<KF_VOXEL_F32><<<kBatchFinishWaves / kFinishPer, 64 * kFinishPer, 0, s>>>(hd, jobs);
-    KF_LAUNCHED("raycast_batch_finish_kernel");
-    raycast_batch_finish_kernel<KF_VOXEL_SNORM16_U8><<<kBatchFinishWaves / kFinishPer, 64 * kFinishPer, 0, s>>>(
-        hd, jobs);
-    KF_LAUNCHED("raycast_batch_finish_kernel");
+    constexpr unsigned finish = kBatchFinishWaves / kFinishPer;
+    if (blocks[0]) {
+        raycast_batch_finish_kernel<KF_VOXEL_F32><<<finish, 64 * kFinishPer, 0, s>>>(hd, jobs);
+        KF_LAUNCHED("raycast_batch_finish_kernel");
+    }
+    if (blocks[1]) {
+        raycast_batch_finish_kernel<KF_VOXEL_SNORM16_U8><<<finish, 64 * kFinishPer, 0, s>>>(hd, jobs);
+        KF_LAUNCHED("raycast_batch_finish_kernel");
+    }
     return KF_OK;
 }
 
@@ -904,8 +954,8 @@ int launch_raycast_batch(const BatchHeader* hd, const RaycastJob* jobs, unsigned
 static int ensure_ray_list(const kf_volume* v, size_t rays, hipStream_t s)
 {
     if (!v->ray_count) {
-        KF_HIP(hipMalloc(&v->ray_count, 2 * sizeof(unsigned)));
-        KF_HIP(hipMemset(v->ray_count, 0, 2 * sizeof(unsigned)));
+        KF_HIP(hipMalloc(&v->ray_count, 2 * 8 * kCountStride * sizeof(unsigned)));
+        KF_HIP(hipMemset(v->ray_count, 0, 2 * 8 * kCountStride * sizeof(unsigned)));
     }
     if (v->ray_cap >= rays) return KF_OK;
     KF_HIP(hipStreamSynchronize(s));
@@ -939,10 +989,6 @@ int launch_raycast_levels(const kf_volume* v, const float* pose, const PoseState
                           const float (*inv_k)[9], float4* const* vout, float4* const* nout, int w0, int h0,
                           hipStream_t s)
 {
-    size_t rays = 0;
-    for (int l = 0; l < levels; ++l) rays += (size_t)(w0 >> l) * (size_t)(h0 >> l);
-    int st = ensure_ray_list(v, rays, s);
-    if (st) return st;
     RaycastArgs a{};
     a.vol = raycast_volume(v);
     if (pose) memcpy(a.pose, pose, sizeof(a.pose));
@@ -963,14 +1009,16 @@ int launch_raycast_levels(const kf_volume* v, const float* pose, const PoseState
     a.tiles = tiles;
     unsigned blocks = 0;
     for (int l = 0; l < levels; ++l) blocks += (unsigned)level_blocks(a, l);
-    st = ensure_tile_order(v, blocks, s);
+    // every ray of an XCD's workgroups has a place in its list
+    int st = ensure_ray_list(v, (size_t)blocks * 64, s);
+    if (!st) st = ensure_tile_order(v, blocks, s);
     if (st) return st;
     const int64_t launch = v->ray_launches++;
     const int parity = (int)(launch & 1);
     a.rays = static_cast<DeferredRay*>(v->ray_list);
-    a.count = v->ray_count + parity;
-    a.clear = v->ray_count + (1 - parity);
-    a.cap = (unsigned)v->ray_cap;
+    a.count = v->ray_count + parity * 8 * kCountStride;
+    a.clear = v->ray_count + (1 - parity) * 8 * kCountStride;
+    a.cap = (unsigned)(v->ray_cap / 8);
     // the order recorded by the previous launch is used when it was made for the same maps
     const int64_t key = ((int64_t)levels << 42) | ((int64_t)w0 << 21) | (int64_t)h0;
     a.order_in = v->order_key == key ? v->tile_order + (size_t)parity * v->order_cap : nullptr;

@@ -141,6 +141,29 @@ def test_skipped_ticks(kf, inputs):
         assert_same(got[k], ref, f"session {k} with skipped ticks")
 
 
+# (w, h): coarse levels of fewer tiles than XCDs, ragged tiles, several tiles per XCD
+@pytest.mark.parametrize("w,h", [(64, 48), (76, 52), (100, 76)])
+def test_sessions_of_another_format_join_a_captured_batch(kf, inputs, w, h):
+    """The raycast's workgroups follow the resident sessions: a session of the other voxel format, and a
+    larger one, join after ticks were captured."""
+    specs = [dict(w=w, h=h, n=64, L=3.0, fmt=1, seed=105), dict(w=w, h=h, n=64, L=3.0, fmt=0, seed=106), SESSIONS[0]]
+    ins = [make_inputs(kf, specs[0]), make_inputs(kf, specs[1]), inputs[0]]
+    first = [0, 2, 3]  # the tick each session joins at
+    b = kf.Batch(3, icp=icp_cfg(kf), use_graph=True)
+    ids = []
+    for t in range(TICKS):
+        announce(f"late sessions {w}x{h} tick {t}")
+        ids += [b.add(session_cfg(kf, specs[k], ins[k][0])) for k in range(3) if first[k] == t]
+        b.tick(ids, [ins[k][2].ptr.value + (t - first[k]) * specs[k]["w"] * specs[k]["h"] * 2 for k in range(len(ids))])
+    b.sync()
+    for k, sp in enumerate(specs):
+        ref = run_pipeline(kf, sp, ins[k], range(TICKS - first[k]))
+        got = dict(pose=b.pose(ids[k]), vol=b.volume_download(ids[k]),
+                   maps=[b.map(ids[k], which, l) for which in (2, 4, 5) for l in range(3)] + [b.map(ids[k], 0)])
+        assert_same(got, ref, f"session {k}")
+    b.close()
+
+
 def test_session_admission_and_errors(kf, inputs):
     b = kf.Batch(2, icp=icp_cfg(kf))
     seq = inputs[0][0]
