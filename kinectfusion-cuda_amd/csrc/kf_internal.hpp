@@ -88,17 +88,11 @@ struct kf_volume {
     int64_t fuse_launches = 0;
     size_t bytes = 0;
     // raycast scratch (grown on demand, also by raycasts through a const volume):
-    // deferred-ray list and its two launch-parity counters
+    // deferred rays (a list per XCD) and their counters of two launch parities
     mutable void* ray_list = nullptr;
     mutable unsigned* ray_count = nullptr;
     mutable size_t ray_cap = 0;
     mutable int64_t ray_launches = 0;
-    // first-pass dispatch order (tiles that took longest last time first):
-    // 2 launch parities x order_cap slots, and its counters and wave times
-    mutable int* tile_order = nullptr;
-    mutable void* order_state = nullptr;
-    mutable size_t order_cap = 0;
-    mutable int64_t order_key = -1;  // (levels, width, height) the stored order was made for
 };
 
 struct kf_icp {
