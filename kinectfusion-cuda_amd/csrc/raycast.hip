@@ -215,13 +215,14 @@ __device__ __forceinline__ int free_run(const BrickAt& b, float xa, float ya, fl
 // is appended to a list that a second pass finishes with a whole wave per ray,
 // so no wave of the first pass waits on one long ray.  The single-session
 // pass's tail bounds the frame; the batch's persistent pass is throughput-bound.
-// Large/small trips, first + finishing pass: one 640x480 frame into 512^3 (three
-// levels) 12/12 82 + 90 us, 16/16 87 + 24, 20/16 86 + 17, 24/24 103 + 15, 32/32
-// 120 + 14; 64 such frames in a tick (small trips) 12 3.26 + 2.10 ms, 16 3.06 +
-// 0.61, 24 3.11 + 0.54, 32 3.14 + 0.28, 40 3.18 + 0.21.
-constexpr int kLargeTrips = 20;
-constexpr int kSmallTrips = 16;
-constexpr int kBatchSmallTrips = 32;
+// Small trips, first + finishing pass: one 640x480 frame (three levels) into 512^3
+// FP32 12 59 + 15 us, 14 62 + 11, 16 65 + 10, into 256^3 snorm16 53 + 32, 57 + 27,
+// 60 + 22, 8 of either 50 + 100 and more; 64 frames in a tick 16 2.11 + 0.41 ms, 20
+// 2.18 + 0.37, 24 2.22 + 0.33, 28 2.31 + 0.30.  Large trips: 16 to 32 alike, but 16
+// gives the batch's finishing pass 0.1 ms more.
+constexpr int kLargeTrips = 24;
+constexpr int kSmallTrips = 14;
+constexpr int kBatchSmallTrips = 20;
 
 __device__ __forceinline__ float lane_bcast(float v, int lane)
 {
@@ -366,9 +367,11 @@ __device__ __forceinline__ void advance(float& t, float& prev_t, float step, int
 // of both steps' code; the boxes of free bricks leave 8 large-step and 7
 // small-step ones.  First + finishing pass: 64 frames of 640x480 from 512^3
 // snorm16 volumes 3.98 + 0.45 -> 3.14 + 0.28 ms, one frame from 512^3 FP32 105 + 22
-// -> 86 + 17 us, its coarsest level alone (160x120) 52 -> 30 us.  With lists per
-// XCD instead of one for the launch (their counters in lines of their own) 66 + 11
-// us, and 2.36 + 0.27 ms (raycast_batch_kernel).
+// -> 86 + 17 us, its coarsest level alone (160x120) 52 -> 30 us.  Lists per XCD
+// instead of one for the launch (their counters in lines of their own): 66 + 11 us,
+// and 2.36 + 0.27 ms (raycast_batch_kernel).  Small steps that enter a cell load its
+// corners along with the brick's distance, one round trip instead of two: 320x240
+// from 200^3 40 -> 37 us, 640x480 from 256^3 61 -> 60 us, 64 frames 2.24 -> 2.19 ms.
 template <int FMT, bool P2>
 __device__ __forceinline__ void raycast_pixel(const RaycastVolume& a, const float* pose, const RaycastLevel& L, int i,
                                               int j, bool in_image, const RayQueue& rq, int job)
@@ -445,13 +448,10 @@ __device__ __forceinline__ void raycast_pixel(const RaycastVolume& a, const floa
                         z = P2 ? za : tex(a, p.z) * nf - 0.5f;
             const float fx = floorf(x), fy = floorf(y), fz = floorf(z);
             if (fx != fi || fy != fj || fz != fk) {
+                // the corners and the brick's distance in one round trip: near a surface few
+                // samples are free
                 const BrickAt b = brick_at(a, xa, ya, za);
-                const float E = free_extent(a.dist[b.index] >> 4);
-                if (inside_box(b, xa, ya, za, E)) {
-                    prev_skipped = true;
-                    advance(t, prev_t, small, free_run(b, xa, ya, za, E, speed, 19.9f));
-                    continue;
-                }
+                const int dist = a.dist[b.index];
                 fi = fx;
                 fj = fy;
                 fk = fz;
@@ -459,6 +459,12 @@ __device__ __forceinline__ void raycast_pixel(const RaycastVolume& a, const floa
                 cell_offsets(a.nb, stencil_texel(a.n, x, y, z), q);
 #pragma unroll
                 for (int k = 0; k < 8; ++k) c[k] = voxel_at<FMT>(a.f, q[k]);
+                const float E = free_extent(dist >> 4);
+                if (inside_box(b, xa, ya, za, E)) {
+                    prev_skipped = true;
+                    advance(t, prev_t, small, free_run(b, xa, ya, za, E, speed, 19.9f));
+                    continue;
+                }
             }
             const float f = lerp_cell(c, x - fx, y - fy, z - fz);
             if (f < 0.0f) {
