@@ -36,6 +36,7 @@ struct Session {
     kf_volume* vol = nullptr;
     kf::PoseState* st = nullptr;
     kf::IcpCarry* carry = nullptr;
+    kf::IterPose* iter_pose = nullptr;
     float* partials = nullptr;
     int max_blocks = 0;
     float* depth_m = nullptr;
@@ -155,7 +156,7 @@ size_t maps_bytes(int w, int h)
 {
     size_t px = (size_t)w * h, b = 2 * sizeof(float) * px + sizeof(float) * kf::depth_max_floats(w, h);
     for (int l = 0; l < 3; ++l) b += 3 * sizeof(float4) * (size_t)(w >> l) * (h >> l);
-    return b + 2 * sizeof(kf::IcpCarry) + 2 * sizeof(float) * kf::kPartialStride * (size_t)kf::icp_blocks_for(w, h) +
+    return b + 2 * sizeof(kf::IcpCarry) + sizeof(kf::IterPose) + 2 * sizeof(float) * kf::kPartialStride * (size_t)kf::icp_blocks_for(w, h) +
            sizeof(kf::PoseState);
 }
 
@@ -187,6 +188,7 @@ void free_session(Session& q)
     kf_volume_destroy(q.vol);
     (void)hipFree(q.st);
     (void)hipFree(q.carry);
+    (void)hipFree(q.iter_pose);
     (void)hipFree(q.partials);
     (void)hipFree(q.depth_m);
     (void)hipFree(q.d0);
@@ -546,6 +548,7 @@ int kf_batch_add_session(kf_batch* b, const kf_session_config* c, int* id)
         st = alloc((void**)&q.st, sizeof(kf::PoseState), &q.bytes);
     }
     if (!st) st = alloc((void**)&q.carry, 2 * sizeof(kf::IcpCarry), &q.bytes);
+    if (!st) st = alloc((void**)&q.iter_pose, sizeof(kf::IterPose), &q.bytes);
     if (!st) st = alloc((void**)&q.partials, 2 * sizeof(float) * kf::kPartialStride * (size_t)q.max_blocks, &q.bytes);
     if (!st) st = alloc((void**)&q.depth_m, sizeof(float) * (size_t)w * h, &q.bytes);
     if (!st) st = alloc((void**)&q.d0, sizeof(float) * (size_t)w * h, &q.bytes);
@@ -673,6 +676,7 @@ int kf_batch_tick(kf_batch* b, int n, const int* ids, const uint16_t* const* raw
                 J.a.pix = kf::icp_pix_for((int64_t)(w >> l) * (h >> l));
                 J.a.stride = kf::icp_level_blocks(w >> l, h >> l);
                 J.carry = q.carry;
+                J.pose = q.iter_pose;
                 J.partials = q.partials;
                 J.max_blocks = q.max_blocks;
                 J.block0 = icp_blocks[l];

@@ -50,6 +50,13 @@ struct SumType<true> {
 };
 // Partial rows (component-major, of SumType): [0,27) sums, 27 the inlier count.
 
+// Element e of M = K R_prev^T (both column-major), in m3m3's order.
+__device__ __forceinline__ float projection_element(const float* K, const float* Rp, int e)
+{
+    const int c = e / 3, r = e % 3;
+    return (K[r] * Rp[c] + K[3 + r] * Rp[3 + c]) + K[6 + r] * Rp[6 + c];
+}
+
 // icp.cu:7-82 split in two: what a pixel needs that does not depend on the
 // pose (its vertex and its live normal, device_helper.cuh:81-110) and the
 // pose-dependent association, so the loads of the first part can be issued
@@ -59,19 +66,68 @@ struct PixelIn {
     v3 cr;       // live normal before normalization (device_helper.cuh:81-110's cross product)
     bool ok;     // vertex and normal valid
 };
-__device__ __forceinline__ PixelIn icp_pixel_from(const NormalStencil& ns)
+__device__ __forceinline__ PixelIn icp_pixel_from(float4 c, float4 r, float4 d, bool ok)
 {
     PixelIn in;
-    in.ok = ns.c.w == kValid;
-    in.vc = in.ok ? xyz(ns.c) : mk3(0.0f, 0.0f, 0.0f);
-    const v3 c = xyz(ns.c);
-    in.cr = cross3(sub3(xyz(ns.r), c), sub3(xyz(ns.d), c));  // normal_of before its normalize3
-    in.ok = in.ok && ns.r.w == kValid && ns.d.w == kValid;
+    in.vc = xyz(c);
+    in.cr = cross3(sub3(xyz(r), in.vc), sub3(xyz(d), in.vc));  // normal_of before its normalize3
+    in.ok = ok && c.w == kValid && r.w == kValid && d.w == kValid;
     return in;
 }
-__device__ __forceinline__ PixelIn icp_pixel_in(const IcpArgs& a, int u, int v)
+
+// The rejection tests decide a boolean only, so each is first decided from a
+// cheap approximation and evaluated exactly (the reference arithmetic, correctly
+// rounded square root and division) only when the approximation lies too close to
+// the threshold to decide: the decision is the exact one always.
+//
+// Projection, icp.cuh:40-49: the floor of p.x / p.z and p.y / p.z.  The quotients
+// from the hardware reciprocal (1 ulp) and the correctly rounded ones differ by
+// less than 2^-21 of their size, so inside the map by less than band = 2^-21
+// max(w, h): both have the same floor unless the former lies within band of an
+// integer.  Outside the map both floors are outside.  A p.z that the hardware
+// routine may flush takes the exact path.
+__device__ __forceinline__ void floor_quotients(v3 p, float band, float& fu, float& fv)
 {
-    return icp_pixel_from(load_normal_stencil(a.V, a.w, a.h, u, v));
+    const float r = __builtin_amdgcn_rcpf(p.z);
+    const float qx = p.x * r, qy = p.y * r;
+    fu = floorf(qx);
+    fv = floorf(qy);
+    const float off = fmaxf(fabsf((qx - fu) - 0.5f), fabsf((qy - fv) - 0.5f)), az = fabsf(p.z);
+    if (!(off <= 0.5f - band) || !(az >= 0x1p-100f && az <= 0x1p100f)) {
+        fu = floorf(p.x / p.z);
+        fv = floorf(p.y / p.z);
+    }
+}
+// Distance, icp.cuh:57-60: reject iff RN(sqrt(D)) > T, D = dot(v, v) (the
+// same bits on both paths).  D <= T^2 gives sqrt(D) <= T; D >= (T + ulp(T))^2
+// gives RN(sqrt(D)) > T.  lo and hi below bound those squares from inside
+// (lo <= T^2, hi >= T^2 (1 + 2^-21) > (T + ulp(T))^2); NaN takes the exact path.
+//
+// Angle, icp.cuh:63-70 in its cosine form (acos(d) > th <=> d >= -1 && d < cos
+// th), d = dot(normalize(Rc normalize(cr)), n).  The approximation da rotates cr
+// as it is and takes one normalization, with the hardware reciprocal square root
+// (1 ulp): it is within 2^-19 |n|_1 of the exact d, so a margin of 2^-16 |n|_1
+// decides; a squared length outside [2^-100, 2^100] (where the hardware routine
+// may flush or overflow) and NaN take the exact path.
+__device__ __forceinline__ bool pair_rejected(const IcpArgs& a, const float* Rc, v3 v, v3 cr, v3 n, bool live)
+{
+    const float D = dot3(v, v);
+    const float T2 = a.dist_thresh * a.dist_thresh;
+    const float lo = T2 * (1.0f - 0x1p-22f), hi = T2 * (1.0f + 0x1p-20f);
+    const v3 m = m3v(Rc, cr);
+    const float mq = dot3(m, m);
+    const float da = dot3(m, n) * __builtin_amdgcn_rsqf(mq);
+    const float del = 0x1p-16f * (fabsf(n.x) + fabsf(n.y) + fabsf(n.z));
+    const bool ranged = mq >= 0x1p-100f && mq <= 0x1p100f;
+    const float c = a.cos_thresh;
+    bool rejected = D >= hi || (ranged && da < c - del && da >= -1.0f + del);
+    const bool accepted = D <= lo && ranged && da >= c + del;
+    if (live && !rejected && !accepted) {
+        rejected = len3(v) > a.dist_thresh;
+        const float dd = dot3(normalize3(m3v(Rc, normalize3(cr))), n);
+        rejected = rejected || (dd >= -1.0f && dd < c);
+    }
+    return rejected;
 }
 
 // false = zero row (rejection reasons as icp.cu:29-70, evaluated in an order
@@ -81,78 +137,41 @@ __device__ __forceinline__ PixelIn icp_pixel_in(const IcpArgs& a, int u, int v)
 // issues the loads of its target vertex and normal (at an in-map index even
 // when the projection is off the map, so no branch surrounds the loads);
 // icp_pixel_finish applies the tests and builds the row.
-// The two rejection tests decide a boolean only, so each is first decided
-// from a cheap approximation and evaluated exactly (the reference arithmetic,
-// correctly rounded sqrt and division) only when the approximation lies too
-// close to the threshold to decide: the decision is the exact one always.
-//
-// Distance, icp.cuh:57-60: reject iff RN(sqrt(D)) > T, D = dot(v, v) (the
-// same bits on both paths).  D <= T^2 gives sqrt(D) <= T; D >= (T + ulp(T))^2
-// gives RN(sqrt(D)) > T.  lo and hi below bound those squares from inside
-// (lo <= T^2, hi >= T^2 (1 + 2^-21) > (T + ulp(T))^2); NaN takes the exact path.
-__device__ __forceinline__ bool distance_rejects(const IcpArgs& a, v3 v)
-{
-    const float D = dot3(v, v);
-    const float T2 = a.dist_thresh * a.dist_thresh;
-    const float lo = T2 * (1.0f - 0x1p-22f), hi = T2 * (1.0f + 0x1p-20f);
-    if (D >= hi) return true;
-    if (D <= lo) return false;
-    return len3(v) > a.dist_thresh;
-}
-// Angle, icp.cuh:63-70 in its cosine form (acos(d) > th <=> d >= -1 && d < cos
-// th), d = dot(normalize(Rc normalize(cr)), n).  The approximation takes both
-// normalizations with the hardware reciprocal square root (1 ulp); its d is
-// within 2^-19 |n|_1 of the exact d (measured worst case over 8M random
-// inputs with every rsq off by one ulp either way: 2^-21.8), so a margin of
-// 2^-16 |n|_1 decides; squared lengths outside [2^-100, 2^100] (where the
-// hardware routine may flush or overflow) and NaN take the exact path.
-__device__ __forceinline__ bool angle_rejects(const IcpArgs& a, v3 cr, const float* Rc, v3 n)
-{
-    const float q = dot3(cr, cr);
-    const v3 m = m3v(Rc, mul3s(cr, __builtin_amdgcn_rsqf(q)));
-    const float mq = dot3(m, m);
-    const float da = dot3(mul3s(m, __builtin_amdgcn_rsqf(mq)), n);
-    const float del = 0x1p-16f * (fabsf(n.x) + fabsf(n.y) + fabsf(n.z));
-    const bool ranged = q >= 0x1p-100f && q <= 0x1p100f && mq >= 0x1p-100f && mq <= 0x1p100f;
-    const float c = a.cos_thresh;
-    if (ranged) {
-        if (da >= c + del || da < -1.0f - del) return false;
-        if (da >= -1.0f + del && da < c - del) return true;
-    }
-    const float dd = dot3(normalize3(m3v(Rc, normalize3(cr))), n);
-    return dd >= -1.0f && dd < c;
-}
-
 struct PixelGather {
     v3 s;             // the vertex in the frame of the current estimate
     float4 tv, tn;    // target vertex and normal at the projection
     bool ok;          // the pixel is valid and projects into the map
 };
-__device__ __forceinline__ PixelGather icp_pixel_gather(const IcpArgs& a, const PixelIn& in, const float* Rc,
-                                                       const float* tc, const float* M, const float* tp)
+// SMALL: the map has at most kMaxMapPixels pixels, so a pixel's index is exact in
+// FP32 and its byte offset fits 32 bits (one register beside the map's address).
+template <bool SMALL>
+__device__ __forceinline__ PixelGather icp_pixel_gather(const IcpArgs& a, const PixelIn& in, const IterPose& P)
 {
     PixelGather g;
-    g.s = add3(m3v(Rc, in.vc), mk3(tc[0], tc[1], tc[2]));
+    g.s = add3(m3v(P.R, in.vc), mk3(P.t[0], P.t[1], P.t[2]));
     // icp.cuh:40-49: (K * R_prev^T) * (s - t_prev), floor of the perspective division
-    v3 p = m3v(M, sub3(g.s, mk3(tp[0], tp[1], tp[2])));
-    float fu = floorf(p.x / p.z), fv = floorf(p.y / p.z);
-    g.ok = in.ok && fu >= 0.0f && fv >= 0.0f && fu < (float)a.w && fv < (float)a.h;
-    const int64_t q = g.ok ? (int64_t)(int)fv * a.w + (int)fu : 0;
-    g.tv = a.TV[q];
-    g.tn = a.TN[q];
+    const v3 p = m3v(P.M, sub3(g.s, mk3(P.tp[0], P.tp[1], P.tp[2])));
+    const float wf = (float)a.w, hf = (float)a.h;
+    float fu, fv;
+    floor_quotients(p, 0x1p-21f * fmaxf(wf, hf), fu, fv);
+    g.ok = in.ok && fu >= 0.0f && fv >= 0.0f && fu < wf && fv < hf;
+    if (SMALL) {
+        const uint32_t o = g.ok ? (uint32_t)(int)fmaf(fv, wf, fu) * 16u : 0u;
+        g.tv = *reinterpret_cast<const float4*>(reinterpret_cast<const char*>(a.TV) + o);
+        g.tn = *reinterpret_cast<const float4*>(reinterpret_cast<const char*>(a.TN) + o);
+    } else {
+        const int64_t q = g.ok ? (int64_t)(int)fv * a.w + (int)fu : 0;
+        g.tv = a.TV[q];
+        g.tn = a.TN[q];
+    }
     return g;
 }
 __device__ __forceinline__ bool icp_pixel_finish(const IcpArgs& a, const PixelIn& in, const PixelGather& g,
                                                  const float* Rc, float* row, float& b)
 {
-    if (!g.ok) return false;
-    const float4 tv = g.tv, tn = g.tn;
-    const v3 s = g.s;
-    if (tv.w != kValid || tn.w != kValid) return false;
-    v3 d = xyz(tv);
-    if (distance_rejects(a, sub3(d, s))) return false;  // icp.cuh:57-60
-    v3 n = xyz(tn);
-    if (angle_rejects(a, in.cr, Rc, n)) return false;  // icp.cuh:63-70
+    const v3 s = g.s, d = xyz(g.tv), n = xyz(g.tn);
+    const bool live = g.ok && g.tv.w == kValid && g.tn.w == kValid;
+    if (pair_rejected(a, Rc, sub3(d, s), in.cr, n, live) || !live) return false;
     // icp.cuh:72-95
     row[0] = n.y * s.z - n.z * s.y;
     row[1] = n.z * s.x - n.x * s.z;
@@ -162,17 +181,6 @@ __device__ __forceinline__ bool icp_pixel_finish(const IcpArgs& a, const PixelIn
     row[5] = n.z;
     b = ((((n.x * d.x + n.y * d.y) + n.z * d.z) - n.x * s.x) - n.y * s.y) - n.z * s.z;
     return true;
-}
-__device__ __forceinline__ bool icp_pixel_row(const IcpArgs& a, const PixelIn& in, const float* Rc, const float* tc,
-                                              const float* M, const float* tp, float* row, float& b)
-{
-    return icp_pixel_finish(a, in, icp_pixel_gather(a, in, Rc, tc, M, tp), Rc, row, b);
-}
-
-__device__ __forceinline__ bool icp_row(const IcpArgs& a, int u, int v, const float* Rc, const float* tc,
-                                        const float* M, const float* tp, float* row, float& b)
-{
-    return icp_pixel_row(a, icp_pixel_in(a, u, v), Rc, tc, M, tp, row, b);
 }
 
 // Adds a pixel's row to the lane's FP32 sums of A^T A (upper triangle) and
@@ -261,7 +269,8 @@ __device__ __forceinline__ void halve_dpp(T* s, bool upper)
 // pad at 27 and one at the 7 -> 8 step): lane L ends with term
 // 14*b5 + 7*b4 + 4*b3 + 2*b2 + b1 of its bits, every pair (L, L^1) holding it
 // (each step keeps the first half on the lane whose step bit is clear).
-// The first step exchanges the lanes' FP32 sums and widens them as it adds.
+// The first step exchanges the lanes' FP32 sums and widens them as it adds.  cnt is
+// the wave's count.
 template <class T>
 __device__ __forceinline__ void block_reduce_store(const float* s_in, int cnt, float* partials, int stride, int row)
 {
@@ -280,7 +289,6 @@ __device__ __forceinline__ void block_reduce_store(const float* s_in, int cnt, f
     halve_dpp<4, kDppRowHalfMirror>(s, (lane & 4) != 0);
     halve_dpp<2, kDppXor2>(s, (lane & 2) != 0);
     s[0] = s[0] + sum_partner<kDppXor1>(s[0]);  // both lanes of the pair add the same two operands
-    cnt = wave_sum(cnt);
     const int sub = 4 * ((lane >> 3) & 1) + 2 * ((lane >> 2) & 1) + ((lane >> 1) & 1);
     const int q = 14 * ((lane >> 5) & 1) + 7 * ((lane >> 4) & 1) + sub;
     if ((lane & 1) == 0 && sub < 7 && q < kTerms) red[wave][q] = s[0];
@@ -300,40 +308,48 @@ template <int PIX = kPixPerThread>
 struct LanePixels {
     PixelIn in[PIX];
 };
-// Their vertex loads only (a pixel past the map reads as invalid), so the
-// loads can be in flight while the workgroup finishes the previous iteration.
+// Their vertex loads only, so the loads can be in flight while the workgroup
+// finishes the previous iteration.  ok: the pixel has a right and a lower neighbour.
 template <int PIX = kPixPerThread>
 struct LaneLoads {
-    NormalStencil ns[PIX];
+    float4 c[PIX], r[PIX], d[PIX];
+    bool ok[PIX];
 };
-// Column and row of pixel px of a w-wide map, px < kMaxMapPixels: px is exact
-// in FP32 and px * (1/w) is within one of px / w, so one correction each way
-// gives the quotient.
+// Column of pixel px of a w-wide map, px < kMaxMapPixels: px is exact in FP32 and
+// px * (1/w) is within one of px / w, so one correction each way gives the
+// quotient (and 24-bit products suffice).
 constexpr int kMaxMapPixels = 1 << 24;
-__device__ __forceinline__ void pixel_uv(int px, int w, float inv_w, int& u, int& v)
+__device__ __forceinline__ int pixel_column(int px, int w, float inv_w)
 {
-    v = (int)((float)px * inv_w);
-    u = px - v * w;
-    if (u < 0) {
-        u += w;
-        --v;
-    } else if (u >= w) {
-        u -= w;
-        ++v;
-    }
+    int u = px - (int)__umul24((unsigned)((float)px * inv_w), (unsigned)w);
+    if (u < 0) u += w;
+    else if (u >= w) u -= w;
+    return u;
 }
+// Only pixels up to `last` have a lower and (short of their row's end) a right
+// neighbour; a pixel past it loads the last one's, so no select surrounds a load,
+// and the three loads share one 32-bit offset.
 template <int PIX>
 __device__ __forceinline__ void issue_lane_loads(const IcpArgs& a, LaneLoads<PIX>& ll, int block, int pix)
 {
-    const int npx = a.w * a.h;  // <= kMaxMapPixels (checked on the host)
+    const int last = a.w * a.h - a.w - 2;  // w x h <= kMaxMapPixels (checked on the host)
+    const bool any = a.w > 1 && a.h > 1;   // uniform; else no pixel has both neighbours
     const float inv_w = 1.0f / (float)a.w;
+    const char* row0 = reinterpret_cast<const char*>(a.V);
+    const char* row1 = row0 + (size_t)a.w * 16;
 #pragma unroll
     for (int k = 0; k < PIX; ++k) {
         if (k >= pix) break;  // uniform
         const int px = (block * pix + k) * kThreads + (int)threadIdx.x;
-        int u = -1, v = -1;
-        if (px < npx) pixel_uv(px, a.w, inv_w, u, v);
-        ll.ns[k] = load_normal_stencil(a.V, a.w, a.h, u, v);
+        ll.ok[k] = any && px <= last && pixel_column(px, a.w, inv_w) + 1 < a.w;
+        if (!any) {
+            ll.c[k] = ll.r[k] = ll.d[k] = make_float4(0.0f, 0.0f, 0.0f, kInvalid);
+            continue;
+        }
+        const uint32_t o = (uint32_t)min(px, last) * 16u;
+        ll.c[k] = *reinterpret_cast<const float4*>(row0 + o);
+        ll.r[k] = *reinterpret_cast<const float4*>(row0 + o + 16);
+        ll.d[k] = *reinterpret_cast<const float4*>(row1 + o);
     }
 }
 template <int PIX>
@@ -342,7 +358,7 @@ __device__ __forceinline__ void finish_lane_pixels(const LaneLoads<PIX>& ll, Lan
 #pragma unroll
     for (int k = 0; k < PIX; ++k) {
         if (k >= pix) break;
-        lp.in[k] = icp_pixel_from(ll.ns[k]);
+        lp.in[k] = icp_pixel_from(ll.c[k], ll.r[k], ll.d[k], ll.ok[k]);
     }
 }
 template <int PIX>
@@ -353,35 +369,35 @@ __device__ __forceinline__ void load_lane_pixels(const IcpArgs& a, LanePixels<PI
     finish_lane_pixels(ll, lp, pix);
 }
 
-// pose: R (9), t (3), Rp (9), tp (3) of the iteration, in LDS.  Writes partial
-// row `block` of a.partials.
+// Associates the lane's pixels at the iteration's pose and writes partial row
+// `block` of a.partials.  Bound: the vector ALU (80-90 % busy in a batch tick).
+// With the projection's quotients taken approximately, one normalization less in
+// the angle test, offsets of 32 bits shared by a pixel's loads, the projection
+// matrix formed once instead of by every lane, the batch's pose in scalar registers
+// and counts by ballot, the association of a tick of 64 sessions takes 122 instead
+// of 141 us on average over its 19 iterations; sixteen uneven sessions 32 -> 25 us,
+// a frame 333 -> 321 us (512^3, plain) and 365 -> 347 us (256^3, compensated).
 template <bool COMP, int PIX>
-__device__ void associate_reduce(const IcpArgs& a, const LanePixels<PIX>& lp, const float* pose, int block, int pix)
+__device__ __forceinline__ void associate_reduce(const IcpArgs& a, const LanePixels<PIX>& lp, const IterPose& P,
+                                                 int block, int pix)
 {
-    const float* Rc = pose;
-    const float* tc = pose + 9;
-    float Rt[9], M[9];
-    m3t(pose + 12, Rt);
-    m3m3(a.K, Rt, M);
-    const float* tp = pose + 21;
     float s[kTerms];
 #pragma unroll
     for (int q = 0; q < kTerms; ++q) s[q] = 0.0f;
-    int cnt = 0;
+    int cnt = 0;  // of the wave
     PixelGather g[PIX];
 #pragma unroll
     for (int k = 0; k < PIX; ++k) {
         if (k >= pix) break;
-        g[k] = icp_pixel_gather(a, lp.in[k], Rc, tc, M, tp);
+        g[k] = icp_pixel_gather<true>(a, lp.in[k], P);
     }
 #pragma unroll
     for (int k = 0; k < PIX; ++k) {
         if (k >= pix) break;
         float row[6], b;
-        if (icp_pixel_finish(a, lp.in[k], g[k], Rc, row, b)) {
-            accumulate(s, row, b);
-            ++cnt;
-        }
+        const bool hit = icp_pixel_finish(a, lp.in[k], g[k], P.R, row, b);
+        cnt += __popcll(__ballot(hit));
+        if (hit) accumulate(s, row, b);
     }
     block_reduce_store<typename SumType<COMP>::T>(s, cnt, a.partials, a.stride, block);
 }
@@ -390,13 +406,13 @@ template <bool COMP>
 __device__ void reduce_body(const IcpArgs& a)
 {
     PoseState* st = a.st;
-    __shared__ float pose[24];
+    __shared__ IterPose pose;
     LanePixels<> lp;
     load_lane_pixels(a, lp, blockIdx.x, kPixPerThread);
-    if (threadIdx.x < 9) pose[threadIdx.x] = st->R[threadIdx.x];
-    else if (threadIdx.x < 12) pose[threadIdx.x] = st->t[threadIdx.x - 9];
-    else if (threadIdx.x < 21) pose[threadIdx.x] = st->Rp[threadIdx.x - 12];
-    else if (threadIdx.x < 24) pose[threadIdx.x] = st->tp[threadIdx.x - 21];
+    if (threadIdx.x < 9) pose.R[threadIdx.x] = st->R[threadIdx.x];
+    else if (threadIdx.x < 12) pose.t[threadIdx.x - 9] = st->t[threadIdx.x - 9];
+    else if (threadIdx.x < 21) pose.M[threadIdx.x - 12] = projection_element(a.K, st->Rp, threadIdx.x - 12);
+    else if (threadIdx.x < 24) pose.tp[threadIdx.x - 21] = st->tp[threadIdx.x - 21];
     __syncthreads();
     associate_reduce<COMP>(a, lp, pose, blockIdx.x, kPixPerThread);
 }
@@ -419,17 +435,19 @@ __global__ __launch_bounds__(kThreads) void ab_reduce_kernel(const float* A, con
     int cnt = 0;
 #pragma unroll
     for (int k = 0; k < kPixPerThread; ++k) {
-        int64_t r = ((int64_t)blockIdx.x * kPixPerThread + k) * kThreads + threadIdx.x;
-        if (r >= n) break;
-        float row[6];
+        const int64_t r = ((int64_t)blockIdx.x * kPixPerThread + k) * kThreads + threadIdx.x;
+        bool nz = false;
+        if (r < n) {
+            float row[6];
 #pragma unroll
-        for (int p = 0; p < 6; ++p) row[p] = A[r * 6 + p];
-        float b = B[r];
-        accumulate(s, row, b);
-        bool nz = b != 0.0f;
+            for (int p = 0; p < 6; ++p) row[p] = A[r * 6 + p];
+            const float b = B[r];
+            accumulate(s, row, b);
+            nz = b != 0.0f;
 #pragma unroll
-        for (int p = 0; p < 6; ++p) nz = nz || row[p] != 0.0f;
-        cnt += nz ? 1 : 0;
+            for (int p = 0; p < 6; ++p) nz = nz || row[p] != 0.0f;
+        }
+        cnt += __popcll(__ballot(nz));
     }
     block_reduce_store<typename SumType<COMP>::T>(s, cnt, partials, stride, blockIdx.x);
 }
@@ -438,14 +456,24 @@ __global__ __launch_bounds__(kThreads) void ab_reduce_kernel(const float* A, con
 __global__ __launch_bounds__(kThreads) void icp_rows_kernel(IcpArgs a, float* A, float* B)
 {
     const float* pose = reinterpret_cast<const float*>(a.partials);  // 24 floats by value (R, t, Rp, tp)
-    float Rt[9], M[9];
-    m3t(pose + 12, Rt);
-    m3m3(a.K, Rt, M);
+    IterPose P;
+#pragma unroll
+    for (int q = 0; q < 9; ++q) {
+        P.R[q] = pose[q];
+        P.M[q] = projection_element(a.K, pose + 12, q);
+    }
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+        P.t[q] = pose[9 + q];
+        P.tp[q] = pose[21 + q];
+    }
     int64_t px = (int64_t)blockIdx.x * kThreads + threadIdx.x;
     if (px >= (int64_t)a.w * a.h) return;
     int u = (int)(px % a.w), v = (int)(px / a.w);
     float row[6] = {0, 0, 0, 0, 0, 0}, b = 0.0f;
-    if (!icp_row(a, u, v, pose, pose + 9, M, pose + 21, row, b)) {
+    const NormalStencil ns = load_normal_stencil(a.V, a.w, a.h, u, v);
+    const PixelIn in = icp_pixel_from(ns.c, ns.r, ns.d, true);
+    if (!icp_pixel_finish(a, in, icp_pixel_gather<false>(a, in, P), P.R, row, b)) {
 #pragma unroll
         for (int p = 0; p < 6; ++p) row[p] = 0.0f;
         b = 0.0f;
@@ -882,14 +910,18 @@ __device__ __forceinline__ void issue_begin_loads(const PoseState* st, const Icp
 template <bool COMP>
 __device__ void begin_iteration(const BeginLoads<COMP>& bl, PoseState* st, IcpCarry* cout, const float* pin,
                                 int prev_blocks, int level, int blocks, bool first, float stop_angle, float stop_dist,
-                                float* pose, int* run, double* tot, double* count)
+                                const float* K, IterPose* pose, int* run, double* tot, double* count)
 {
     __shared__ IcpCarry carry;
+    __shared__ float Rp[9];
     constexpr int kWords = (int)(sizeof(IcpCarry) / sizeof(int));
     if (prev_blocks > 0) sum_loaded_partials(pin, prev_blocks, prev_blocks, bl.rows, tot, count);
     if (threadIdx.x < kWords) reinterpret_cast<int*>(&carry)[threadIdx.x] = bl.cw;
-    else if (threadIdx.x >= 64 && threadIdx.x < 76) pose[12 + (threadIdx.x - 64)] = bl.pw;
+    else if (threadIdx.x >= 64 && threadIdx.x < 73) Rp[threadIdx.x - 64] = bl.pw;
+    else if (threadIdx.x >= 73 && threadIdx.x < 76) pose->tp[threadIdx.x - 73] = bl.pw;
     __syncthreads();
+    if (threadIdx.x >= 64 && threadIdx.x < 73)  // while wave 0 solves
+        pose->M[threadIdx.x - 64] = projection_element(K, Rp, (int)threadIdx.x - 64);
     if (threadIdx.x < 64) {
         double xd[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
         const int rc = (carry.pending && carry.status == 0) ? chol6_wave(tot, xd) : 0;
@@ -901,8 +933,8 @@ __device__ void begin_iteration(const BeginLoads<COMP>& bl, PoseState* st, IcpCa
         c.pending = go;
         c.pending_level = level;
         c.pending_blocks = blocks;
-        for (int q = 0; q < 9; ++q) pose[q] = c.R[q];
-        for (int q = 0; q < 3; ++q) pose[9 + q] = c.t[q];
+        for (int q = 0; q < 9; ++q) pose->R[q] = c.R[q];
+        for (int q = 0; q < 3; ++q) pose->t[q] = c.t[q];
         *run = go;
         if (first) *cout = c;
         }
@@ -915,7 +947,7 @@ __global__ __launch_bounds__(kThreads) void icp_step_kernel(IcpArgs a, const Icp
                                                             const float* pin, int prev_blocks, float stop_angle,
                                                             float stop_dist)
 {
-    __shared__ float pose[24];
+    __shared__ IterPose pose;
     __shared__ int run;
     __shared__ double tot[kTerms];
     __shared__ double count;
@@ -928,7 +960,7 @@ __global__ __launch_bounds__(kThreads) void icp_step_kernel(IcpArgs a, const Icp
     __builtin_amdgcn_sched_barrier(0);  // nothing of phase B moves above the pixel loads
     // phase B: finish the previous iteration
     begin_iteration<COMP>(bl, a.st, cout, pin, prev_blocks, a.level, (int)gridDim.x, blockIdx.x == 0, stop_angle,
-                          stop_dist, pose, &run, tot, &count);
+                          stop_dist, a.K, &pose, &run, tot, &count);
     if (!run) return;
     // phase C: live normals, association + reduction of this iteration
     LanePixels<PIX> lp;
@@ -1057,6 +1089,12 @@ __global__ __launch_bounds__(kThreads) void icp_batch_solve_kernel(const BatchHe
         const bool pend = c->pending && c->status == 0;
         __syncthreads();  // every lane has read the carry before lane 0 rewrites it
         if (pend) sum_partials<COMP>(J.partials, c->pending_blocks, c->pending_blocks, tot, &count);
+        if (!final_) {  // of the association launch that follows
+            if (threadIdx.x >= 64 && threadIdx.x < 73)
+                J.pose->M[threadIdx.x - 64] = projection_element(J.a.K, st->Rp, (int)threadIdx.x - 64);
+            else if (threadIdx.x >= 73 && threadIdx.x < 76)
+                J.pose->tp[threadIdx.x - 73] = st->tp[threadIdx.x - 73];
+        }
         if (threadIdx.x < 64) {
             double xd[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
             const int rc = pend ? chol6_wave(tot, xd) : 0;
@@ -1065,6 +1103,8 @@ __global__ __launch_bounds__(kThreads) void icp_batch_solve_kernel(const BatchHe
                 IcpCarry cc = *c;
                 apply_solution(cc, rc, xd, sc, tot, count, st, true, stop_angle, stop_dist);
                 if (!final_) {
+                    for (int q = 0; q < 9; ++q) J.pose->R[q] = cc.R[q];
+                    for (int q = 0; q < 3; ++q) J.pose->t[q] = cc.t[q];
                     cc.pending = (cc.status == 0 && !level_flag(cc.level_done, level)) ? 1 : 0;
                     cc.pending_level = level;
                     cc.pending_blocks = J.a.stride;
@@ -1080,12 +1120,12 @@ __global__ __launch_bounds__(kThreads) void icp_batch_solve_kernel(const BatchHe
     }
 }
 
+// Four waves per SIMD (102 VGPRs); held to 96 for five it spills and takes 145 us
+// where this takes 122.
 template <bool COMP>
 __global__ __launch_bounds__(kThreads, 4) void icp_batch_assoc_kernel(const BatchHeader* hd, const IcpJob* jobs,
                                                                    int level)
 {
-    __shared__ float pose[24];
-    __shared__ int run;
     const int njobs = hd->n_icp, total = hd->icp_blocks[level];
     const int G = (int)gridDim.x;
     const int rank = xcd_rank((int)blockIdx.x, G);
@@ -1093,51 +1133,46 @@ __global__ __launch_bounds__(kThreads, 4) void icp_batch_assoc_kernel(const Batc
     int b = rank * chunk;
     const int end = min(total, b + chunk);
     if (b >= end) return;
-    // the table is never written while the kernel runs: scalar loads through
-    // the constant address space keep the job's fields in scalar registers
+    // the table, the carries and the iteration's poses are never written while the
+    // kernel runs: scalar loads through the constant address space keep them in
+    // scalar registers
     typedef __attribute__((address_space(4))) const IcpJob ConstJob;
+    typedef __attribute__((address_space(4))) const IcpCarry ConstCarry;
+    typedef __attribute__((address_space(4))) const IterPose ConstPose;
     ConstJob* cj = (ConstJob*)jobs;
     int j = job_of(jobs, njobs, b, [](const IcpJob& J) { return J.block0; });
-    int cur = -1;
     for (; b < end; ++b) {
         while (j + 1 < njobs && cj[j + 1].block0 <= b) ++j;
         j = __builtin_amdgcn_readfirstlane(j);
+        if (!((ConstCarry*)cj[j].carry)->pending) continue;
         IcpArgs a;
         a.V = cj[j].a.V;
         a.TV = cj[j].a.TV;
         a.TN = cj[j].a.TN;
         a.w = cj[j].a.w;
         a.h = cj[j].a.h;
-#pragma unroll
-        for (int q = 0; q < 9; ++q) a.K[q] = cj[j].a.K[q];
         a.dist_thresh = cj[j].a.dist_thresh;
         a.cos_thresh = cj[j].a.cos_thresh;
-        a.st = cj[j].a.st;
-        a.level = level;
         a.partials = cj[j].partials;
         a.stride = cj[j].a.stride;
         a.pix = cj[j].a.pix;
         const int lb = b - cj[j].block0;
         LanePixels<> lp;
         load_lane_pixels(a, lp, lb, a.pix);
-        if (j != cur) {
-            cur = j;
-            __syncthreads();  // the previous session's pose is no longer read
-            if (threadIdx.x == 0) {
-                const IcpCarry* c = cj[j].carry;
-                const PoseState* st = a.st;
-                for (int q = 0; q < 9; ++q) pose[q] = c->R[q];
-                for (int q = 0; q < 3; ++q) pose[9 + q] = c->t[q];
-                for (int q = 0; q < 9; ++q) pose[12 + q] = st->Rp[q];
-                for (int q = 0; q < 3; ++q) pose[21 + q] = st->tp[q];
-                run = c->pending;
-            }
-            __syncthreads();
-        } else {
-            __syncthreads();  // the previous block's reduction LDS is free again
+        ConstPose* cp = (ConstPose*)cj[j].pose;
+        IterPose P;
+#pragma unroll
+        for (int q = 0; q < 9; ++q) {
+            P.R[q] = cp->R[q];
+            P.M[q] = cp->M[q];
         }
-        if (!run) continue;
-        associate_reduce<COMP>(a, lp, pose, lb, a.pix);
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+            P.t[q] = cp->t[q];
+            P.tp[q] = cp->tp[q];
+        }
+        __syncthreads();  // the previous block's reduction LDS is free again
+        associate_reduce<COMP>(a, lp, P, lb, a.pix);
     }
 }
 

@@ -189,10 +189,16 @@ struct IcpCarry {
     int pending_blocks;  // partial-row count of that launch
     int pad[2];
 };
+// What the association of an iteration needs of its pose: the current estimate
+// R, t, the projection M = K R_prev^T and t_prev.
+struct IterPose {
+    float R[9], t[3], M[9], tp[3];
+};
 // One session at one level of a batched ICP launch.
 struct IcpJob {
     IcpArgs a;         // a.stride = the session's blocks at this level; a.partials unused
     IcpCarry* carry;   // 2 entries, by launch parity
+    IterPose* pose;    // of the iteration, written by its solve launch
     float* partials;   // 2 x kPartialStride x max_blocks, by launch parity
     int max_blocks;
     int block0;        // first block of this job in the launch

@@ -144,3 +144,41 @@ def test_icp_reduce_edges(kf, w, h, comp):
     roundings = 4 if comp else 4 + 6 + 3 + -(-blocks // 64) + 6
     bound = 1.01 * roundings * 2.0 ** -24 * np.abs(prod).sum(0)
     assert (np.abs(sums - prod.sum(0)) <= bound).all()
+
+
+@pytest.mark.parametrize("w,h", [(64, 48), (2, 300), (300, 2)])
+def test_projection_at_pixel_borders_bit_exact(kf, oracle32, w, h):
+    """A pixel's target is the floor of its projection, taken from approximate quotients except near
+    an integer: projections on the pixel borders and within 3 ulps of them, off the map, behind the
+    camera and at depths beyond the approximation's range, every row against the oracle's.  The
+    thresholds accept any target, so a wrong one shows."""
+    announce(f"projection at pixel borders {w}x{h}")
+    rng = np.random.default_rng(w)
+    z = (0.4 + 5.6 * rng.random((h, w))).astype(np.float32)
+    z[rng.random((h, w)) < 0.1] *= -1
+    scale = rng.choice([1.0, 1e-33, 1e33], size=(h, w), p=[0.9, 0.05, 0.05]).astype(np.float32)
+    z = z * scale
+    k, l = rng.integers(-2, w + 3, (h, w)), rng.integers(-2, h + 3, (h, w))
+    ulp = lambda: 1 + rng.integers(-3, 4, (h, w)).astype(np.float32) * np.float32(2.0 ** -23)  # noqa: E731
+    V = np.stack([k.astype(np.float32) * z * ulp(), l.astype(np.float32) * z * ulp(), z, np.full((h, w), -1.0)], -1)
+    V = V.astype(np.float32)
+    TV = np.concatenate([rng.standard_normal((h, w, 3)), np.full((h, w, 1), -1.0)], -1).astype(np.float32)
+    N = rng.standard_normal((h, w, 3))
+    TN = np.concatenate([N / np.linalg.norm(N, axis=-1, keepdims=True), np.full((h, w, 1), -1.0)], -1)
+    TN = TN.astype(np.float32)
+    maps = []
+    for m in (V, TV, TN):
+        g = kf.GridMap(w, h, 4)
+        g.upload(m)
+        maps.append(g)
+    R, t = np.eye(3, dtype=np.float32).reshape(9), np.zeros(3, np.float32)
+    K = np.eye(3, dtype=np.float32).reshape(9)
+    A, b = kf.DeviceArray((h * w, 6)), kf.DeviceArray((h * w,))
+    kf.kernel.construct_icp_residuals(*maps, R, t, R, t, K, 1e18, float(np.pi), A, b)
+    Ar, br = oracle32.construct_icp_residuals(V, TV, TN, R, t, R, t, K, 1e18, float(np.pi))
+    assert np.count_nonzero(np.any(Ar != 0, axis=1)) > 0.1 * w * h
+    same(A.download(), Ar, "A")
+    same(b.download(), br, "b")
+    # the fused reduction takes its targets by 32-bit offsets: the same rows are counted
+    _, inliers = kf.kernel.icp_reduce(*maps, R, t, R, t, K, 1e18, float(np.pi))
+    assert inliers == np.count_nonzero(np.any(Ar != 0, axis=1) | (br != 0))
