@@ -37,6 +37,7 @@ struct Session {
     kf::PoseState* st = nullptr;
     kf::IcpCarry* carry = nullptr;
     kf::IterPose* iter_pose = nullptr;
+    kf::PoseMirror* mirror = nullptr;  // its place in kf_batch::mirrors
     float* partials = nullptr;
     int max_blocks = 0;
     float* depth_m = nullptr;
@@ -84,9 +85,9 @@ __global__ void fill_invalid_kernel(float4* m, int64_t n)
 struct Pose32 {
     float m[32];  // pose, inverse pose
 };
-// A new session's PoseState (pose and its inverse, everything else zero) and
-// zeroed ICP carries.
-__global__ void pose_state_init_kernel(kf::PoseState* st, kf::IcpCarry* carry, Pose32 p)
+// A new session's PoseState (pose and its inverse, everything else zero), its
+// mirror and zeroed ICP carries.
+__global__ void pose_state_init_kernel(kf::PoseState* st, kf::IcpCarry* carry, kf::PoseMirror* mirror, Pose32 p)
 {
     if (threadIdx.x != 0) return;
     kf::PoseState z;
@@ -94,7 +95,9 @@ __global__ void pose_state_init_kernel(kf::PoseState* st, kf::IcpCarry* carry, P
     for (int q = 0; q < 16; ++q) {
         z.pose[q] = p.m[q];
         z.inv_pose[q] = p.m[16 + q];
+        mirror->pose[q] = p.m[q];
     }
+    z.mirror = mirror;
     *st = z;
     kf::IcpCarry c;
     memset(&c, 0, sizeof(c));
@@ -113,6 +116,7 @@ struct kf_batch {
     Slot slot[2];
     int next = 0;
     unsigned* fuse_count = nullptr;
+    kf::PoseMirror* mirrors = nullptr;  // pinned host memory, one per session
     unsigned* ray_count = nullptr;  // 16 deferred-ray counts, kf::kCountStride apart
     kf::DeferredRay* ray_list = nullptr;  // 2 x ray_cap deferred rays (per voxel format, 8 XCDs each)
     size_t ray_cap = 0;
@@ -452,6 +456,7 @@ int kf_batch_destroy(kf_batch* b)
         if (q.used) free_session(q);
     (void)hipFree(b->fuse_count);
     (void)hipFree(b->ray_count);
+    if (b->mirrors) (void)hipHostFree(b->mirrors);
     (void)hipFree(b->ray_list);
     (void)hipFree(b->fuse_list);
     (void)hipFree(b->touched);
@@ -506,6 +511,11 @@ int kf_batch_create(const kf_batch_config* cfg, kf_stream_t stream, kf_batch** o
     if (!st) st = alloc((void**)&b->fuse_count, sizeof(unsigned), nullptr);
     if (!st) st = alloc((void**)&b->ray_count, 16 * kf::kCountStride * sizeof(unsigned), nullptr);
     if (!st) st = alloc((void**)&b->touched, sizeof(unsigned long long) * kMaxFuseBlocks, nullptr);
+    if (!st) {
+        hipError_t e = hipHostMalloc(reinterpret_cast<void**>(&b->mirrors),
+                                     sizeof(kf::PoseMirror) * (size_t)cfg->max_sessions, hipHostMallocDefault);
+        if (e != hipSuccess) st = kf::fail_hip(e, "kf_batch_create poses");
+    }
     if (!st) {
         hipError_t e = hipMemset(b->touched, 0, sizeof(unsigned long long) * kMaxFuseBlocks);
         if (e == hipSuccess) e = hipMemset(b->fuse_count, 0, sizeof(unsigned));
@@ -569,7 +579,8 @@ int kf_batch_add_session(kf_batch* b, const kf_session_config* c, int* id)
         Pose32 p;
         memcpy(p.m, sensor.pose, sizeof(sensor.pose));
         memcpy(p.m + 16, sensor.inv_pose, sizeof(sensor.inv_pose));
-        pose_state_init_kernel<<<1, 64, 0, b->s>>>(q.st, q.carry, p);
+        q.mirror = b->mirrors + slot;
+        pose_state_init_kernel<<<1, 64, 0, b->s>>>(q.st, q.carry, q.mirror, p);
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) st = kf::fail_hip(e, "kf_batch_add_session state");
     }
@@ -813,7 +824,7 @@ int kf_batch_pose(kf_batch* b, int id, float pose[16])
     Session* q = session_of(b, id);
     if (!q || !pose) return kf::fail(KF_ERR_ARG, "kf_batch_pose: bad argument");
     KF_HIP(hipStreamSynchronize(b->s));
-    KF_HIP(hipMemcpy(pose, q->st->pose, sizeof(float) * 16, hipMemcpyDeviceToHost));
+    memcpy(pose, q->mirror->pose, sizeof(float) * 16);
     return KF_OK;
 }
 
@@ -932,7 +943,7 @@ int kf_batch_session_restore(kf_batch* b, int id, const char* path)
         if ((st = kf_sensor_set_pose(&sensor, pose))) return st;
         memcpy(p.m + 16, sensor.inv_pose, sizeof(sensor.inv_pose));
     }
-    pose_state_init_kernel<<<1, 64, 0, b->s>>>(q->st, q->carry, p);
+    pose_state_init_kernel<<<1, 64, 0, b->s>>>(q->st, q->carry, q->mirror, p);
     KF_LAUNCHED("pose_state_init_kernel");
     KF_HIP(hipStreamSynchronize(b->s));
     q->frames = frames;

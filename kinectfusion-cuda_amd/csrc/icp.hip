@@ -21,6 +21,7 @@
 #include <string.h>
 
 #include <algorithm>
+#include <atomic>
 #include <mutex>
 #include <vector>
 
@@ -51,7 +52,7 @@ struct SumType<true> {
 // Partial rows (component-major, of SumType): [0,27) sums, 27 the inlier count.
 
 // Element e of M = K R_prev^T (both column-major), in m3m3's order.
-__device__ __forceinline__ float projection_element(const float* K, const float* Rp, int e)
+__host__ __device__ __forceinline__ float projection_element(const float* K, const float* Rp, int e)
 {
     const int c = e / 3, r = e % 3;
     return (K[r] * Rp[c] + K[3 + r] * Rp[3 + c]) + K[6 + r] * Rp[6 + c];
@@ -424,11 +425,16 @@ __global__ __launch_bounds__(kThreads) void icp_reduce_kernel(IcpArgs a)
     reduce_body<COMP>(a);
 }
 
-// Rows of a given A (n x 6 row-major) and b (LinearLeastSquares::solve).
+// Rows of a given A (n x 6 row-major) and b (LinearLeastSquares::solve).  The first
+// workgroup clears what the solve that follows reports.
 template <bool COMP>
 __global__ __launch_bounds__(kThreads) void ab_reduce_kernel(const float* A, const float* B, int64_t n,
-                                                             float* partials, int stride)
+                                                             float* partials, int stride, PoseState* st)
 {
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        st->status = st->sticky_status = 0;
+        for (int q = 0; q < 6; ++q) st->last_x[q] = 0.0f;
+    }
     float s[kTerms];
 #pragma unroll
     for (int q = 0; q < kTerms; ++q) s[q] = 0.0f;
@@ -453,20 +459,8 @@ __global__ __launch_bounds__(kThreads) void ab_reduce_kernel(const float* A, con
 }
 
 // icp.cu:7-82, writing the rows (kernel::constructIcpResiduals).
-__global__ __launch_bounds__(kThreads) void icp_rows_kernel(IcpArgs a, float* A, float* B)
+__global__ __launch_bounds__(kThreads) void icp_rows_kernel(IcpArgs a, IterPose P, float* A, float* B)
 {
-    const float* pose = reinterpret_cast<const float*>(a.partials);  // 24 floats by value (R, t, Rp, tp)
-    IterPose P;
-#pragma unroll
-    for (int q = 0; q < 9; ++q) {
-        P.R[q] = pose[q];
-        P.M[q] = projection_element(a.K, pose + 12, q);
-    }
-#pragma unroll
-    for (int q = 0; q < 3; ++q) {
-        P.t[q] = pose[9 + q];
-        P.tp[q] = pose[21 + q];
-    }
     int64_t px = (int64_t)blockIdx.x * kThreads + threadIdx.x;
     if (px >= (int64_t)a.w * a.h) return;
     int u = (int)(px % a.w), v = (int)(px / a.w);
@@ -1010,6 +1004,13 @@ __device__ void commit_state(PoseState* st, const IcpCarry& c)
     for (int l = 0; l < 4; ++l) st->level_done[l] = c.level_done[l];
     st->iterations = c.iterations;
     st->status = c.status;
+    PoseMirror* out = st->mirror;
+    if (out) {
+        for (int q = 0; q < 9; ++q) out->R[q] = c.R[q];
+        for (int q = 0; q < 3; ++q) out->t[q] = c.t[q];
+        out->status = c.status;
+        out->iterations = c.iterations;
+    }
     if (c.status != 0) {
         if (st->sticky_status == 0) st->sticky_status = c.status;
         st->frame_skip_fuse = 1;
@@ -1021,6 +1022,8 @@ __device__ void commit_state(PoseState* st, const IcpCarry& c)
     P[3] = P[7] = P[11] = 0.0f;
     for (int r = 0; r < 3; ++r) P[12 + r] = c.t[r];
     P[15] = 1.0f;
+    if (out)
+        for (int q = 0; q < 16; ++q) out->pose[q] = P[q];
     float* I = st->inv_pose;
     for (int cc = 0; cc < 3; ++cc)
         for (int r = 0; r < 3; ++r) I[cc * 4 + r] = c.R[r * 3 + cc];
@@ -1241,9 +1244,9 @@ static IcpArgs level_args(const kf_icp* icp, const IcpLevel& L, int l)
     return a;
 }
 
-// Enqueues the iteration launches; `events` (optional) receives one event
-// after every launch.  Returns the number of launches in *launches.
-static int enqueue_steps(kf_icp* icp, const IcpLevel* levels, int n_levels, hipStream_t s, hipEvent_t* events,
+// Enqueues the iteration launches and the commit; `before_commit` (optional) is
+// recorded between them.  Returns the number of iterations in *launches.
+static int enqueue_steps(kf_icp* icp, const IcpLevel* levels, int n_levels, hipStream_t s, hipEvent_t before_commit,
                          int* launches)
 {
     const float sa = icp->cfg.iteration_stop_thresh_angle, sd = icp->cfg.iteration_stop_thresh_distance;
@@ -1262,9 +1265,9 @@ static int enqueue_steps(kf_icp* icp, const IcpLevel* levels, int n_levels, hipS
             step<<<blocks, kThreads, 0, s>>>(a, carry_of(icp, k), carry_of(icp, k + 1), partials_of(icp, k + 1),
                                              prev_blocks, sa, sd);
             KF_LAUNCHED("icp_step_kernel");
-            if (events) KF_HIP(hipEventRecord(events[k], s));
             prev_blocks = blocks;
         }
+    if (before_commit) KF_HIP(hipEventRecord(before_commit, s));
     if (icp->cfg.compensated)
         icp_commit_kernel<true><<<1, kThreads, 0, s>>>(icp->state, carry_of(icp, k), partials_of(icp, k + 1), sa, sd);
     else
@@ -1319,12 +1322,6 @@ constexpr int kNoAllocMaxBlocks = (int)((kNoAllocMaxEquations + kThreads * kPixP
 constexpr size_t kNoAllocStateBytes = (sizeof(PoseState) + 255) & ~(size_t)255;
 constexpr size_t kNoAllocBytes = kNoAllocStateBytes + sizeof(float) * kPartialStride * kNoAllocMaxBlocks;
 
-__global__ void noalloc_clear_state_kernel(PoseState* st)
-{
-    int* w = reinterpret_cast<int*>(st);
-    for (size_t q = threadIdx.x; q < sizeof(PoseState) / sizeof(int); q += blockDim.x) w[q] = 0;
-}
-
 __global__ void noalloc_result_kernel(const PoseState* st, float* x, int* status)
 {
     if (threadIdx.x < 6) x[threadIdx.x] = st->last_x[threadIdx.x];
@@ -1334,26 +1331,34 @@ __global__ void noalloc_result_kernel(const PoseState* st, float* x, int* status
 }  // namespace kf
 
 static __device__ __align__(256) unsigned char scratch[kf::kNoAllocBytes];
+// A second one, for the calls that wait (kf_solve_normal_equations): a call that finds
+// it in use by another thread allocates instead.
+static __device__ __align__(256) unsigned char solve_scratch[kf::kNoAllocBytes];
 
 namespace {
 
-// The device address of this GPU's `scratch`, looked up once per device.
-int noalloc_scratch(char** out)
+constexpr int kMaxDevices = 64;
+std::atomic<bool> solve_scratch_used[kMaxDevices];
+
+// The device address of this GPU's `scratch` or `solve_scratch`, looked up once per device.
+int scratch_address(bool solve, char** out, int* device)
 {
-    constexpr int kMaxDevices = 64;
     static std::mutex mu;
-    static char* ptr[kMaxDevices] = {};
+    static char* ptr[2][kMaxDevices] = {};
     int dev = 0;
     KF_HIP(hipGetDevice(&dev));
     if (dev < 0 || dev >= kMaxDevices) return kf::fail(KF_ERR_ARG, "solve (no allocation): device index out of range");
     std::lock_guard<std::mutex> lock(mu);
-    if (!ptr[dev]) {
+    char*& known = ptr[solve ? 1 : 0][dev];
+    if (!known) {
         void* p = nullptr;
-        hipError_t e = hipGetSymbolAddress(&p, HIP_SYMBOL(scratch));
+        hipError_t e = solve ? hipGetSymbolAddress(&p, HIP_SYMBOL(solve_scratch))
+                             : hipGetSymbolAddress(&p, HIP_SYMBOL(scratch));
         if (e != hipSuccess) return kf::fail_hip(e, "solve (no allocation): scratch address");
-        ptr[dev] = static_cast<char*>(p);
+        known = static_cast<char*>(p);
     }
-    *out = ptr[dev];
+    *out = known;
+    *device = dev;
     return KF_OK;
 }
 
@@ -1372,39 +1377,30 @@ int kf_construct_icp_residuals(const float* vertex_map, const float* target_vert
         !prev_transl || !cur_rot || !cur_transl || !intrinsics)
         return kf::fail(KF_ERR_ARG, "constructIcpResiduals: bad argument");
     hipStream_t s = kf::stream_of(stream);
-    // the pose travels by value through a 24-float staging block
-    float pose[24];
-    memcpy(pose, cur_rot, 9 * sizeof(float));
-    memcpy(pose + 9, cur_transl, 3 * sizeof(float));
-    memcpy(pose + 12, prev_rot, 9 * sizeof(float));
-    memcpy(pose + 21, prev_transl, 3 * sizeof(float));
-    float* dpose = nullptr;
-    KF_HIP(hipMalloc(&dpose, sizeof(pose)));
+    kf::IterPose P;  // passed by value
+    memcpy(P.R, cur_rot, sizeof(P.R));
+    memcpy(P.t, cur_transl, sizeof(P.t));
+    for (int e = 0; e < 9; ++e) P.M[e] = kf::projection_element(intrinsics, prev_rot, e);
+    memcpy(P.tp, prev_transl, sizeof(P.tp));
     kf::IcpArgs a{};
     a.V = reinterpret_cast<const float4*>(vertex_map);
     a.TV = reinterpret_cast<const float4*>(target_vertex_map);
     a.TN = reinterpret_cast<const float4*>(target_normal_map);
     a.w = w;
     a.h = h;
-    memcpy(a.K, intrinsics, sizeof(a.K));
     a.dist_thresh = distance_thresh;
     a.cos_thresh = (float)cos((double)angle_thresh);
-    a.partials = dpose;
     kf::CallTimer t(elapsed_ms, s);
-    int st = KF_OK;
-    hipError_t e = hipMemcpyAsync(dpose, pose, sizeof(pose), hipMemcpyHostToDevice, s);
-    if (e != hipSuccess) st = kf::fail_hip(e, "constructIcpResiduals pose copy");
-    if (st == KF_OK) st = t.start();
+    int st = t.start();
     if (st == KF_OK) {
         const unsigned blocks = (unsigned)(((int64_t)w * h + kf::kThreads - 1) / kf::kThreads);
-        kf::icp_rows_kernel<<<blocks, kf::kThreads, 0, s>>>(a, mat_a, vec_b);
-        e = hipGetLastError();
+        kf::icp_rows_kernel<<<blocks, kf::kThreads, 0, s>>>(a, P, mat_a, vec_b);
+        const hipError_t e = hipGetLastError();
         if (e != hipSuccess) st = kf::fail_hip(e, "icp_rows_kernel");
     }
     if (st == KF_OK) st = t.finish();
-    e = hipStreamSynchronize(s);
+    const hipError_t e = hipStreamSynchronize(s);
     if (st == KF_OK && e != hipSuccess) st = kf::fail_hip(e, "constructIcpResiduals");
-    (void)hipFree(dpose);
     return st;
 }
 
@@ -1412,7 +1408,6 @@ int kf_construct_icp_residuals(const float* vertex_map, const float* target_vert
 static int reduce_to_state(kf::PoseState** st_out, float** partials_out, int blocks)
 {
     KF_HIP(hipMalloc(st_out, sizeof(kf::PoseState)));
-    KF_HIP(hipMemset(*st_out, 0, sizeof(kf::PoseState)));
     KF_HIP(hipMalloc(partials_out, sizeof(float) * kf::kPartialStride * (size_t)(blocks > 0 ? blocks : 1)));
     return KF_OK;
 }
@@ -1426,11 +1421,20 @@ int kf_solve_normal_equations(const float* mat_a, const float* vec_b, unsigned i
     const int blocks = kf::blocks_for(n_equations);
     kf::PoseState* st = nullptr;
     float* partials = nullptr;
-    int rc = reduce_to_state(&st, &partials, blocks);
+    char* base = nullptr;
+    int dev = 0, rc = KF_OK;
+    const bool shared = n_equations <= kf::kNoAllocMaxEquations && scratch_address(true, &base, &dev) == KF_OK &&
+                        !solve_scratch_used[dev].exchange(true, std::memory_order_acquire);
+    if (shared) {
+        st = reinterpret_cast<kf::PoseState*>(base);
+        partials = reinterpret_cast<float*>(base + kf::kNoAllocStateBytes);
+    } else {
+        rc = reduce_to_state(&st, &partials, blocks);
+    }
     kf::CallTimer t(elapsed_ms, s);
     if (rc == KF_OK) rc = t.start();
     if (rc == KF_OK) {
-        kf::ab_reduce_kernel<false><<<blocks, kf::kThreads, 0, s>>>(mat_a, vec_b, n_equations, partials, blocks);
+        kf::ab_reduce_kernel<false><<<blocks, kf::kThreads, 0, s>>>(mat_a, vec_b, n_equations, partials, blocks, st);
         kf::icp_finalize_kernel<false><<<1, kf::kThreads, 0, s>>>(st, partials, blocks, blocks, 0, 0.0f, 0.0f, 1);
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) rc = kf::fail_hip(e, "solve kernels");
@@ -1445,9 +1449,15 @@ int kf_solve_normal_equations(const float* mat_a, const float* vec_b, unsigned i
     if (rc == KF_OK) {
         for (int q = 0; q < 6; ++q) result[q] = hs.last_x[q];
         if (hs.status) rc = kf::fail(hs.status, kf_status_string(hs.status));
+    } else {
+        (void)hipStreamSynchronize(s);  // nothing uses the working memory past this call
     }
-    (void)hipFree(st);
-    (void)hipFree(partials);
+    if (shared) {
+        solve_scratch_used[dev].store(false, std::memory_order_release);
+    } else {
+        (void)hipFree(st);
+        (void)hipFree(partials);
+    }
     return rc;
 }
 
@@ -1459,14 +1469,14 @@ int kf_solve_normal_equations_noalloc(const float* mat_a, const float* vec_b, un
     if (n_equations > kf::kNoAllocMaxEquations)
         return kf::fail(KF_ERR_ARG, "solve (no allocation): more than 2^22 equations");
     char* base = nullptr;
-    int rc = noalloc_scratch(&base);
+    int dev = 0;
+    int rc = scratch_address(false, &base, &dev);
     if (rc) return rc;
     auto* st = reinterpret_cast<kf::PoseState*>(base);
     auto* partials = reinterpret_cast<float*>(base + kf::kNoAllocStateBytes);
     hipStream_t s = kf::stream_of(stream);
     const int blocks = kf::blocks_for(n_equations);
-    kf::noalloc_clear_state_kernel<<<1, 256, 0, s>>>(st);
-    kf::ab_reduce_kernel<false><<<blocks, kf::kThreads, 0, s>>>(mat_a, vec_b, n_equations, partials, blocks);
+    kf::ab_reduce_kernel<false><<<blocks, kf::kThreads, 0, s>>>(mat_a, vec_b, n_equations, partials, blocks, st);
     kf::icp_finalize_kernel<false><<<1, kf::kThreads, 0, s>>>(st, partials, blocks, blocks, 0, 0.0f, 0.0f, 1);
     kf::noalloc_result_kernel<<<1, 64, 0, s>>>(st, result_dev, status_dev);
     KF_HIP(hipGetLastError());
@@ -1556,10 +1566,21 @@ int kf_icp_create(const kf_icp_config* config, kf_icp** out)
         (e = hipMemset(icp->state, 0, sizeof(kf::PoseState))) != hipSuccess ||
         (e = hipMalloc(&icp->carry, 2 * sizeof(kf::IcpCarry))) != hipSuccess ||
         (e = hipMemset(icp->carry, 0, 2 * sizeof(kf::IcpCarry))) != hipSuccess ||
-        (e = hipMalloc(&icp->partials, 2 * sizeof(float) * kf::kPartialStride * (size_t)icp->max_blocks)) != hipSuccess) {
+        (e = hipMalloc(&icp->partials, 2 * sizeof(float) * kf::kPartialStride * (size_t)icp->max_blocks)) != hipSuccess ||
+        (e = hipHostMalloc(reinterpret_cast<void**>(&icp->mirror), sizeof(kf::PoseMirror), hipHostMallocDefault)) !=
+            hipSuccess ||
+        (e = hipMemcpy(&icp->state->mirror, &icp->mirror, sizeof(icp->mirror), hipMemcpyHostToDevice)) != hipSuccess) {
         kf_icp_destroy(icp);
         return kf::fail_hip(e, "kf_icp_create");
     }
+    memset(icp->mirror, 0, sizeof(*icp->mirror));
+    // the first two are for timing only: no system-scope cache write-back when they complete
+    for (int q = 0; q < 3; ++q)
+        if ((e = hipEventCreateWithFlags(&icp->ev[q], q < 2 ? hipEventDisableSystemFence : hipEventDefault)) !=
+            hipSuccess) {
+            kf_icp_destroy(icp);
+            return kf::fail_hip(e, "kf_icp_create");
+        }
     *out = icp;
     return KF_OK;
 }
@@ -1567,6 +1588,9 @@ int kf_icp_create(const kf_icp_config* config, kf_icp** out)
 int kf_icp_destroy(kf_icp* icp)
 {
     if (!icp) return KF_OK;
+    for (hipEvent_t v : icp->ev)
+        if (v) (void)hipEventDestroy(v);
+    if (icp->mirror) (void)hipHostFree(icp->mirror);
     (void)hipFree(icp->state);
     (void)hipFree(icp->carry);
     (void)hipFree(icp->partials);
@@ -1590,31 +1614,23 @@ int kf_icp_compute_pose(kf_icp* icp, const float* const vertex_pyr[], const floa
         lv[l].h = icp->cfg.height >> l;
         memcpy(lv[l].K, sensor->intr[l], sizeof(lv[l].K));
     }
-    // Events after every launch (ICP::getExecutionTimes): times[0] = the iteration
-    // launches (association, reduction and the solve of the previous iteration),
-    // times[1] = the final solve and commit.
-    int total = 0;
-    for (int l = 0; l < icp->cfg.levels; ++l) total += icp->cfg.iters_per_layer[l];
-    std::vector<hipEvent_t> ev((size_t)total + 2, nullptr);
-    int rc = KF_OK;
-    for (auto& e : ev)
-        if (rc == KF_OK && hipEventCreate(&e) != hipSuccess) rc = kf::fail(KF_ERR_HIP, "ICP event create");
-    if (rc == KF_OK) rc = kf::launch_icp_begin(icp, sensor->pose, s);
-    if (rc == KF_OK && hipEventRecord(ev[0], s) != hipSuccess) rc = kf::fail(KF_ERR_HIP, "ICP event record");
+    // ICP::getExecutionTimes: times[0] = the iteration launches (association, reduction
+    // and the solve of the previous iteration), times[1] = the final solve and commit.
+    int rc = kf::launch_icp_begin(icp, sensor->pose, s);
+    if (rc == KF_OK && hipEventRecord(icp->ev[0], s) != hipSuccess) rc = kf::fail(KF_ERR_HIP, "ICP event record");
     int k = 0;
-    if (rc == KF_OK) rc = kf::enqueue_steps(icp, lv, icp->cfg.levels, s, ev.data() + 1, &k);
-    if (rc == KF_OK && hipEventRecord(ev.back(), s) != hipSuccess) rc = kf::fail(KF_ERR_HIP, "ICP event record");
-    kf::PoseState hs;
+    if (rc == KF_OK) rc = kf::enqueue_steps(icp, lv, icp->cfg.levels, s, icp->ev[1], &k);
+    if (rc == KF_OK && hipEventRecord(icp->ev[2], s) != hipSuccess) rc = kf::fail(KF_ERR_HIP, "ICP event record");
     if (rc == KF_OK) {
-        hipError_t e = hipMemcpyAsync(&hs, icp->state, sizeof(hs), hipMemcpyDeviceToHost, s);
-        if (e == hipSuccess) e = hipStreamSynchronize(s);
+        const hipError_t e = hipStreamSynchronize(s);
         if (e != hipSuccess) rc = kf::fail_hip(e, "ICP readback");
     }
     if (rc == KF_OK) {
+        const kf::PoseMirror& hs = *icp->mirror;
         icp->times[0] = icp->times[1] = 0.0f;
-        if (k > 0) (void)hipEventElapsedTime(&icp->times[0], ev[0], ev[k]);
-        (void)hipEventElapsedTime(&icp->times[1], ev[k], ev.back());
-        if (elapsed_ms) (void)hipEventElapsedTime(elapsed_ms, ev[0], ev.back());
+        if (k > 0) (void)hipEventElapsedTime(&icp->times[0], icp->ev[0], icp->ev[1]);
+        (void)hipEventElapsedTime(&icp->times[1], icp->ev[1], icp->ev[2]);
+        if (elapsed_ms) (void)hipEventElapsedTime(elapsed_ms, icp->ev[0], icp->ev[2]);
         icp->last_iterations = hs.iterations;
         // the last good estimate (the commit does not run on failure)
         float P[16] = {0};
@@ -1625,8 +1641,6 @@ int kf_icp_compute_pose(kf_icp* icp, const float* const vertex_pyr[], const floa
         memcpy(pose_out, P, sizeof(P));
         if (hs.status) rc = kf::fail(hs.status, kf_status_string(hs.status));
     }
-    for (auto& e : ev)
-        if (e) (void)hipEventDestroy(e);
     return rc;
 }
 

@@ -50,6 +50,14 @@ private:
     hipEvent_t a_ = nullptr, b_ = nullptr;
 };
 
+// What a finished ICP leaves in pinned host memory (written by its commit, read by
+// the host after the stream: no copy and no second wait to read a pose).
+struct PoseMirror {
+    float pose[16];      // PoseState::pose
+    float R[9], t[3];    // the last estimate, also of a failed ICP
+    int status, iterations;
+};
+
 // Device-resident ICP / pose state shared by the ICP loop, the raycast and the
 // fuse of a frame, so a whole frame runs without host round-trips.
 struct alignas(256) PoseState {
@@ -67,6 +75,7 @@ struct alignas(256) PoseState {
     double last_sums[27];
     long long last_inliers;
     float last_x[6];
+    PoseMirror* mirror;  // may be null
 };
 
 }  // namespace kf
@@ -102,6 +111,8 @@ struct kf_icp {
     void* carry = nullptr;           // device, 2 x IcpCarry (double-buffered by launch parity)
     float* partials = nullptr;       // device, 2 x [kPartialStride][max_blocks]
     int max_blocks = 0;
+    kf::PoseMirror* mirror = nullptr;  // pinned host memory, state->mirror
+    hipEvent_t ev[3] = {nullptr, nullptr, nullptr};  // of a computePose: start, last iteration, end
     float times[2] = {0, 0};
     int last_iterations = 0;
 };

@@ -145,6 +145,8 @@ int kf_pipeline_create(const kf_pipeline_config* cfg, kf_stream_t stream, kf_pip
         memset(&hs, 0, sizeof(hs));
         memcpy(hs.pose, sensor.pose, sizeof(hs.pose));
         memcpy(hs.inv_pose, sensor.inv_pose, sizeof(hs.inv_pose));
+        hs.mirror = p->icp->mirror;
+        memcpy(hs.mirror->pose, sensor.pose, sizeof(hs.mirror->pose));
         hipError_t he = hipMemcpy(p->icp->state, &hs, sizeof(hs), hipMemcpyHostToDevice);
         if (he != hipSuccess) st = kf::fail_hip(he, "kf_pipeline_create state");
     }
@@ -249,7 +251,7 @@ int kf_pipeline_pose(kf_pipeline* p, float pose[16])
 {
     if (!p || !pose) return kf::fail(KF_ERR_ARG, "kf_pipeline_pose: null argument");
     KF_HIP(hipStreamSynchronize(p->s));
-    KF_HIP(hipMemcpy(pose, p->icp->state->pose, sizeof(float) * 16, hipMemcpyDeviceToHost));
+    memcpy(pose, p->icp->mirror->pose, sizeof(float) * 16);
     return KF_OK;
 }
 
@@ -307,7 +309,7 @@ int kf_pipeline_render(kf_pipeline* p, const float pose[16], int shading, uint32
         memcpy(P, pose, sizeof(P));
     } else {
         KF_HIP(hipStreamSynchronize(p->s));
-        KF_HIP(hipMemcpy(P, p->icp->state->pose, sizeof(P), hipMemcpyDeviceToHost));
+        memcpy(P, p->icp->mirror->pose, sizeof(P));
     }
     const kf_volume* v = p->vis ? p->vis : p->vol;
     int st = kf::launch_raycast(v, P, nullptr, p->Ki[0], p->rv, p->rn, w, h, p->s);
