@@ -18,6 +18,7 @@
 #include <algorithm>
 #include <type_traits>
 #include <cmath>
+#include <thread>
 #include <vector>
 
 #include "kf_device.hpp"
@@ -712,42 +713,42 @@ __global__ __launch_bounds__(256) void init_kernel(void* f, void* wt, int64_t co
     }
 }
 
-// Raw interchange <-> bricked planes, for the 8 z-slices of brick layer bk.
-// slab: interleaved (f, w) floats, x fastest, n*n*8 voxels.
+// Raw interchange <-> bricked planes, for `count` voxels from q0 in the
+// interchange's order (x fastest, then y and z).  slab: their interleaved (f, w)
+// floats, in pinned host memory: the kernels move them over the host link themselves
+// (8 bytes a lane, 512 contiguous bytes a wave).
 template <int FMT>
-__global__ __launch_bounds__(256) void slab_to_volume(const float* __restrict__ slab, void* f, void* wt, int n, int nb,
-                                                      int bk)
+__global__ __launch_bounds__(256) void slab_to_volume(const float2* __restrict__ slab, void* f, void* wt, int n, int nb,
+                                                      int64_t q0, int64_t count)
 {
-    int64_t q = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    int64_t per = (int64_t)n * n * 8;
-    if (q >= per) return;
-    int i = (int)(q % n), j = (int)((q / n) % n), k = bk * 8 + (int)(q / ((int64_t)n * n));
-    int64_t d = brick_index(nb, i, j, k);
-    float fv = slab[2 * q], wv = slab[2 * q + 1];
+    const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (e >= count) return;
+    const int64_t q = q0 + e, row = q / n;
+    const int i = (int)(q - row * n), k = (int)(row / n), j = (int)(row - (int64_t)k * n);
+    const int64_t d = brick_index(nb, i, j, k);
+    const float2 fw = slab[e];
     if (FMT == KF_VOXEL_F32) {
-        static_cast<float*>(f)[d] = fv;
-        static_cast<float*>(wt)[d] = wv;
+        static_cast<float*>(f)[d] = fw.x;
+        static_cast<float*>(wt)[d] = fw.y;
     } else {
-        static_cast<int16_t*>(f)[d] = snorm_encode(fv);
-        static_cast<uint8_t*>(wt)[d] = (uint8_t)rintf(fminf(fmaxf(wv, 0.0f), 255.0f));
+        static_cast<int16_t*>(f)[d] = snorm_encode(fw.x);
+        static_cast<uint8_t*>(wt)[d] = (uint8_t)rintf(fminf(fmaxf(fw.y, 0.0f), 255.0f));
     }
 }
 template <int FMT>
-__global__ __launch_bounds__(256) void volume_to_slab(float* __restrict__ slab, const void* f, const void* wt, int n,
-                                                      int nb, int bk)
+__global__ __launch_bounds__(256) void volume_to_slab(float2* __restrict__ slab, const void* f, const void* wt, int n,
+                                                      int nb, int64_t q0, int64_t count)
 {
-    int64_t q = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    int64_t per = (int64_t)n * n * 8;
-    if (q >= per) return;
-    int i = (int)(q % n), j = (int)((q / n) % n), k = bk * 8 + (int)(q / ((int64_t)n * n));
-    int64_t d = brick_index(nb, i, j, k);
-    if (FMT == KF_VOXEL_F32) {
-        slab[2 * q] = static_cast<const float*>(f)[d];
-        slab[2 * q + 1] = static_cast<const float*>(wt)[d];
-    } else {
-        slab[2 * q] = snorm_decode(static_cast<const int16_t*>(f)[d]);
-        slab[2 * q + 1] = (float)static_cast<const uint8_t*>(wt)[d];
-    }
+    const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (e >= count) return;
+    const int64_t q = q0 + e, row = q / n;
+    const int i = (int)(q - row * n), k = (int)(row / n), j = (int)(row - (int64_t)k * n);
+    const int64_t d = brick_index(nb, i, j, k);
+    if (FMT == KF_VOXEL_F32)
+        slab[e] = make_float2(static_cast<const float*>(f)[d], static_cast<const float*>(wt)[d]);
+    else
+        slab[e] = make_float2(snorm_decode(static_cast<const int16_t*>(f)[d]),
+                              (float)static_cast<const uint8_t*>(wt)[d]);
 }
 
 // Every free bit set (before free_bits_kernel clears the others).
@@ -934,39 +935,106 @@ bool is_pinhole(const float* K)
            K[4] > 0.0f;
 }
 
-// Moves the volume through host memory one brick layer (8 z-slices) at a time.
+// Moves voxels [q0, q1) between the volume and the host's side through two pinned
+// chunks in turn, so the host fills or empties one while a kernel moves the other.
+// host_side(q, count, chunk): reads or writes `count` voxels from q.
+constexpr int64_t kChunkVoxels = 1 << 18;  // 2 MiB
 template <class Fn>
-int for_each_slab(const kf_volume* v, bool to_volume, Fn&& host_side)
+int move_voxels(const kf_volume* v, bool to_volume, int64_t q0, int64_t q1, float2* pinned, const hipEvent_t* ev,
+                Fn&& host_side)
 {
-    const int64_t per = (int64_t)v->n * v->n * 8;
-    float* dslab = nullptr;
-    std::vector<float> hslab((size_t)per * 2);
-    KF_HIP(hipMalloc(&dslab, sizeof(float) * per * 2));
-    int st = KF_OK;
-    const unsigned blocks = (unsigned)((per + 255) / 256);
-    for (int bk = 0; bk < v->nb && st == KF_OK; ++bk) {
-        if (to_volume) {
-            st = host_side(bk, hslab.data());
-            if (st != KF_OK) break;
-            hipError_t e = hipMemcpy(dslab, hslab.data(), sizeof(float) * per * 2, hipMemcpyHostToDevice);
-            if (e != hipSuccess) { st = fail_hip(e, "volume upload copy"); break; }
-            if (v->format == KF_VOXEL_F32)
-                slab_to_volume<KF_VOXEL_F32><<<blocks, 256>>>(dslab, v->f, v->w, v->n, v->nb, bk);
-            else
-                slab_to_volume<KF_VOXEL_SNORM16_U8><<<blocks, 256>>>(dslab, v->f, v->w, v->n, v->nb, bk);
-            e = hipDeviceSynchronize();
-            if (e != hipSuccess) { st = fail_hip(e, "slab_to_volume"); break; }
-        } else {
-            if (v->format == KF_VOXEL_F32)
-                volume_to_slab<KF_VOXEL_F32><<<blocks, 256>>>(dslab, v->f, v->w, v->n, v->nb, bk);
-            else
-                volume_to_slab<KF_VOXEL_SNORM16_U8><<<blocks, 256>>>(dslab, v->f, v->w, v->n, v->nb, bk);
-            hipError_t e = hipMemcpy(hslab.data(), dslab, sizeof(float) * per * 2, hipMemcpyDeviceToHost);
-            if (e != hipSuccess) { st = fail_hip(e, "volume download copy"); break; }
-            st = host_side(bk, hslab.data());
+    const auto launch = [&](int64_t q, int b) -> int {
+        const int64_t count = std::min(kChunkVoxels, q1 - q);
+        const unsigned blocks = (unsigned)((count + 255) / 256);
+        float2* slab = pinned + b * kChunkVoxels;
+        const bool f32 = v->format == KF_VOXEL_F32;
+        if (to_volume && f32)
+            slab_to_volume<KF_VOXEL_F32><<<blocks, 256>>>(slab, v->f, v->w, v->n, v->nb, q, count);
+        else if (to_volume)
+            slab_to_volume<KF_VOXEL_SNORM16_U8><<<blocks, 256>>>(slab, v->f, v->w, v->n, v->nb, q, count);
+        else if (f32)
+            volume_to_slab<KF_VOXEL_F32><<<blocks, 256>>>(slab, v->f, v->w, v->n, v->nb, q, count);
+        else
+            volume_to_slab<KF_VOXEL_SNORM16_U8><<<blocks, 256>>>(slab, v->f, v->w, v->n, v->nb, q, count);
+        KF_LAUNCHED("volume transfer");
+        KF_HIP(hipEventRecord(ev[b], nullptr));
+        return KF_OK;
+    };
+    int st = KF_OK, b = 0;
+    if (!to_volume && q0 < q1) st = launch(q0, 0);
+    for (int64_t q = q0; q < q1 && st == KF_OK; q += kChunkVoxels, b ^= 1) {
+        const int64_t count = std::min(kChunkVoxels, q1 - q);
+        if (!to_volume && q + kChunkVoxels < q1) st = launch(q + kChunkVoxels, b ^ 1);
+        // the chunk's last kernel is done (an event never recorded counts as done)
+        if (st == KF_OK) {
+            const hipError_t e = hipEventSynchronize(ev[b]);
+            if (e != hipSuccess) st = fail_hip(e, "volume transfer");
         }
+        if (st == KF_OK) st = host_side(q, count, pinned + b * kChunkVoxels);
+        if (st == KF_OK && to_volume) st = launch(q, b);
     }
-    (void)hipFree(dslab);
+    return st;
+}
+
+// The volume to or from the host.  `parallel`: host_side may run for several chunks
+// at once, on threads of this call, each moving a part of the volume through chunks
+// of its own: one core copies at a quarter of the host link's rate.  Small volumes
+// are not worth the threads (about 50 us each).  A 256^3 FP32 volume from the host
+// and back (268 MB), through one pageable layer, its staged copy and a device copy in
+// turn -> now: 24.1 -> 6.2 ms, 43 GB/s.
+template <class Fn>
+int move_volume(const kf_volume* v, bool to_volume, bool parallel, Fn&& host_side)
+{
+    constexpr int kMovers = 4;
+    const int64_t total = (int64_t)v->n * v->n * v->n;
+    const int movers = parallel ? (int)std::min<int64_t>(kMovers, std::max<int64_t>(1, total / (2 * kChunkVoxels))) : 1;
+    float2* pinned = nullptr;
+    hipEvent_t ev[2 * kMovers] = {};
+    KF_HIP(hipHostMalloc(reinterpret_cast<void**>(&pinned), sizeof(float2) * 2 * kChunkVoxels * movers,
+                         hipHostMallocDefault));
+    int st = KF_OK;
+    for (int k = 0; k < 2 * movers && st == KF_OK; ++k) {
+        const hipError_t e = hipEventCreateWithFlags(&ev[k], hipEventDisableTiming);
+        if (e != hipSuccess) st = fail_hip(e, "volume transfer events");
+    }
+    if (st == KF_OK) {
+        int device = 0;
+        (void)hipGetDevice(&device);
+        int status[kMovers] = {};
+        std::string message[kMovers];
+        const auto part = [&](int k) {  // whole chunks each
+            const int64_t chunks = (total + kChunkVoxels - 1) / kChunkVoxels;
+            const int64_t q0 = chunks * k / movers * kChunkVoxels;
+            const int64_t q1 = std::min(total, chunks * (k + 1) / movers * kChunkVoxels);
+            status[k] = move_voxels(v, to_volume, q0, q1, pinned + 2 * kChunkVoxels * k, ev + 2 * k, host_side);
+        };
+        std::vector<std::thread> threads;
+        int started = 1;
+        try {
+            threads.reserve(kMovers);
+            for (; started < movers; ++started) {
+                const int k = started;
+                threads.emplace_back([&, k] {
+                    const hipError_t e = hipSetDevice(device);
+                    if (e != hipSuccess) status[k] = fail_hip(e, "volume transfer");
+                    else part(k);
+                    if (status[k]) message[k] = kf_last_error();  // the thread's own
+                });
+            }
+        } catch (const std::exception&) {
+            // no more threads: this one moves the rest
+        }
+        part(0);
+        for (int k = started; k < movers; ++k) part(k);
+        for (std::thread& t : threads) t.join();
+        for (int k = 0; k < movers && st == KF_OK; ++k)
+            if (status[k]) st = message[k].empty() ? status[k] : fail(status[k], message[k]);
+        const hipError_t e = hipDeviceSynchronize();
+        if (st == KF_OK && e != hipSuccess) st = fail_hip(e, "volume transfer");
+    }
+    for (hipEvent_t e : ev)
+        if (e) (void)hipEventDestroy(e);
+    (void)hipHostFree(pinned);
     if (st == KF_OK && to_volume) {
         const int64_t nbricks = (int64_t)v->nb * v->nb * v->nb;
         const unsigned b = (unsigned)((nbricks + 3) / 4);
@@ -1272,9 +1340,8 @@ int kf_volume_download(const kf_volume* v, float* fw_host)
 {
     if (!v || !fw_host) return kf::fail(KF_ERR_ARG, "kf_volume_download: null argument");
     KF_HIP(hipDeviceSynchronize());
-    const int64_t per = (int64_t)v->n * v->n * 8;
-    return kf::for_each_slab(v, false, [&](int bk, float* slab) {
-        memcpy(fw_host + (size_t)bk * per * 2, slab, sizeof(float) * per * 2);
+    return kf::move_volume(v, false, true, [&](int64_t q, int64_t count, float2* chunk) {
+        memcpy(fw_host + (size_t)q * 2, chunk, sizeof(float2) * (size_t)count);
         return (int)KF_OK;
     });
 }
@@ -1283,9 +1350,8 @@ int kf_volume_upload(kf_volume* v, const float* fw_host)
 {
     if (!v || !fw_host) return kf::fail(KF_ERR_ARG, "kf_volume_upload: null argument");
     KF_HIP(hipDeviceSynchronize());
-    const int64_t per = (int64_t)v->n * v->n * 8;
-    return kf::for_each_slab(v, true, [&](int bk, float* slab) {
-        memcpy(slab, fw_host + (size_t)bk * per * 2, sizeof(float) * per * 2);
+    return kf::move_volume(v, true, true, [&](int64_t q, int64_t count, float2* chunk) {
+        memcpy(chunk, fw_host + (size_t)q * 2, sizeof(float2) * (size_t)count);
         return (int)KF_OK;
     });
 }
@@ -1297,11 +1363,10 @@ int kf_volume_save(const kf_volume* v, const char* path)
     FILE* fp = fopen(path, "wb");
     if (!fp) return kf::fail(KF_ERR_IO, std::string("kf_volume_save: cannot open ") + path);
     KF_HIP(hipDeviceSynchronize());
-    const int64_t per = (int64_t)v->n * v->n * 8;
-    int st = kf::for_each_slab(v, false, [&](int, float* slab) {
-        size_t want = (size_t)per * 2;
-        return fwrite(slab, sizeof(float), want, fp) == want ? (int)KF_OK
-                                                              : kf::fail(KF_ERR_IO, "kf_volume_save: short write");
+    int st = kf::move_volume(v, false, false, [&](int64_t, int64_t count, float2* chunk) {
+        return fwrite(chunk, sizeof(float2), (size_t)count, fp) == (size_t)count
+                   ? (int)KF_OK
+                   : kf::fail(KF_ERR_IO, "kf_volume_save: short write");
     });
     if (fclose(fp) != 0 && st == KF_OK) st = kf::fail(KF_ERR_IO, "kf_volume_save: close failed");
     return st;
@@ -1314,11 +1379,10 @@ int kf_volume_load(kf_volume* v, const char* path)
     FILE* fp = fopen(path, "rb");
     if (!fp) return kf::fail(KF_ERR_IO, std::string("kf_volume_load: cannot open ") + path);
     KF_HIP(hipDeviceSynchronize());
-    const int64_t per = (int64_t)v->n * v->n * 8;
-    int st = kf::for_each_slab(v, true, [&](int, float* slab) {
-        size_t want = (size_t)per * 2;
-        return fread(slab, sizeof(float), want, fp) == want ? (int)KF_OK
-                                                             : kf::fail(KF_ERR_IO, "kf_volume_load: short file");
+    int st = kf::move_volume(v, true, false, [&](int64_t, int64_t count, float2* chunk) {
+        return fread(chunk, sizeof(float2), (size_t)count, fp) == (size_t)count
+                   ? (int)KF_OK
+                   : kf::fail(KF_ERR_IO, "kf_volume_load: short file");
     });
     fclose(fp);
     return st;

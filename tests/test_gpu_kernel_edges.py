@@ -182,3 +182,36 @@ def test_projection_at_pixel_borders_bit_exact(kf, oracle32, w, h):
     # the fused reduction takes its targets by 32-bit offsets: the same rows are counted
     _, inliers = kf.kernel.icp_reduce(*maps, R, t, R, t, K, 1e18, float(np.pi))
     assert inliers == np.count_nonzero(np.any(Ar != 0, axis=1) | (br != 0))
+
+
+# one chunk, one thread with two chunks and a remainder, two threads, four threads with a remainder
+@pytest.mark.parametrize("n", [8, 72, 104, 136])
+@pytest.mark.parametrize("fmt", [0, 1])
+def test_volume_to_host_and_back(kf, tmp_path, n, fmt):
+    """Every voxel arrives where it left: random values uploaded, downloaded, saved, loaded into another
+    volume and drawn alike (the precision form's values are representable: codes and whole counts)."""
+    announce(f"volume transfer {n}^3 format {fmt}")
+    rng = np.random.default_rng(n)
+    if fmt == 0:
+        F, W = rng.standard_normal((2, n, n, n)).astype(np.float32)
+    else:
+        F = rng.integers(-32767, 32768, (n, n, n)).astype(np.float32) * (np.float32(1) / np.float32(32767))
+        W = rng.integers(0, 129, (n, n, n)).astype(np.float32)
+    fw = np.ascontiguousarray(np.stack([F, W], -1))
+    p = lambda a: a.ctypes.data_as(C.c_void_p)  # noqa: E731
+    a, b = [kf.VoxelGrid(3.0, n, mue=0.03, voxel_format=fmt) for _ in range(2)]
+    kf.check(kf.lib().kf_volume_upload(a.h, p(fw)))
+    back = np.zeros_like(fw)
+    kf.check(kf.lib().kf_volume_download(a.h, p(back)))
+    np.testing.assert_array_equal(back.view(np.uint32), fw.view(np.uint32))
+    path = str(tmp_path / "v.bin").encode()
+    kf.check(kf.lib().kf_volume_save(a.h, path))
+    np.testing.assert_array_equal(np.fromfile(path.decode(), np.uint32), fw.view(np.uint32).reshape(-1))
+    kf.check(kf.lib().kf_volume_load(b.h, path))
+    kf.check(kf.lib().kf_volume_download(b.h, p(back)))
+    np.testing.assert_array_equal(back.view(np.uint32), fw.view(np.uint32))
+    with open(path.decode(), "r+b") as f:
+        f.truncate(fw.nbytes - 8)
+    assert kf.lib().kf_volume_load(b.h, path) == kf.KF_ERR_IO
+    a.close()
+    b.close()
