@@ -42,7 +42,7 @@ struct Session {
     int max_blocks = 0;
     float* depth_m = nullptr;
     float* d0 = nullptr;
-    float* dmax = nullptr;
+    float2* drange = nullptr;
     float4* v[3] = {nullptr, nullptr, nullptr};
     float4* pv[3] = {nullptr, nullptr, nullptr};
     float4* pn[3] = {nullptr, nullptr, nullptr};
@@ -158,7 +158,7 @@ size_t volume_meta_bytes(int n)
 
 size_t maps_bytes(int w, int h)
 {
-    size_t px = (size_t)w * h, b = 2 * sizeof(float) * px + sizeof(float) * kf::depth_max_floats(w, h);
+    size_t px = (size_t)w * h, b = 2 * sizeof(float) * px + sizeof(float2) * kf::depth_range_tiles(w, h);
     for (int l = 0; l < 3; ++l) b += 3 * sizeof(float4) * (size_t)(w >> l) * (h >> l);
     return b + 2 * sizeof(kf::IcpCarry) + sizeof(kf::IterPose) + 2 * sizeof(float) * kf::kPartialStride * (size_t)kf::icp_blocks_for(w, h) +
            sizeof(kf::PoseState);
@@ -196,7 +196,7 @@ void free_session(Session& q)
     (void)hipFree(q.partials);
     (void)hipFree(q.depth_m);
     (void)hipFree(q.d0);
-    (void)hipFree(q.dmax);
+    (void)hipFree(q.drange);
     for (int l = 0; l < 3; ++l) {
         (void)hipFree(q.v[l]);
         (void)hipFree(q.pv[l]);
@@ -405,9 +405,9 @@ void default_shape(kf_batch_shape& s, const kf_batch_shape& given)
     s.preprocess_blocks = given.preprocess_blocks ? given.preprocess_blocks : 8192;
     s.raycast_blocks = given.raycast_blocks ? given.raycast_blocks : 65536;
     s.icp_blocks = given.icp_blocks ? given.icp_blocks : 1024;
-    // the brick cull (not tuned): per 64 x 512^3 tick 0.18 ms at 4096 workgroups, 0.16 at 8192,
-    // 0.15 at 16384
-    s.cull_blocks = given.cull_blocks ? given.cull_blocks : 16384;
+    // the brick cull (not tuned): per 64 x 512^3 tick 107 us at 4096 workgroups, 98 at 8192, 111 at
+    // 16384, 148 at 32768
+    s.cull_blocks = given.cull_blocks ? given.cull_blocks : 8192;
     s.fuse_blocks = given.fuse_blocks ? given.fuse_blocks : 16384;
 }
 
@@ -562,7 +562,7 @@ int kf_batch_add_session(kf_batch* b, const kf_session_config* c, int* id)
     if (!st) st = alloc((void**)&q.partials, 2 * sizeof(float) * kf::kPartialStride * (size_t)q.max_blocks, &q.bytes);
     if (!st) st = alloc((void**)&q.depth_m, sizeof(float) * (size_t)w * h, &q.bytes);
     if (!st) st = alloc((void**)&q.d0, sizeof(float) * (size_t)w * h, &q.bytes);
-    if (!st) st = alloc((void**)&q.dmax, sizeof(float) * kf::depth_max_floats(w, h), &q.bytes);
+    if (!st) st = alloc((void**)&q.drange, sizeof(float2) * kf::depth_range_tiles(w, h), &q.bytes);
     for (int l = 0; l < 3 && !st; ++l) {
         const size_t px = (size_t)(w >> l) * (h >> l);
         if ((st = alloc((void**)&q.v[l], sizeof(float4) * px, &q.bytes))) break;
@@ -645,7 +645,7 @@ int kf_batch_tick(kf_batch* b, int n, const int* ids, const uint16_t* const* raw
     const float cos_th = (float)cos((double)ic.angle_thresh);
     int ray_tiles = 0, pre_tiles = 0, pyr_tiles = 0;
     int icp_blocks[3] = {0, 0, 0};
-    unsigned bricks = 0;
+    unsigned groups = 0;
     int dist_tiles = 0;
     int n_ray = 0, n_icp = 0;
     for (int k = 0; k < n; ++k) {
@@ -656,7 +656,7 @@ int kf_batch_tick(kf_batch* b, int n, const int* ids, const uint16_t* const* raw
         P.raw = raw[k];
         P.depth_m = q.depth_m;
         P.d0 = q.d0;
-        P.dmax = q.dmax;
+        P.drange = q.drange;
         for (int l = 0; l < 3; ++l) P.v[l] = q.v[l];
         P.w = w;
         P.h = h;
@@ -698,12 +698,11 @@ int kf_batch_tick(kf_batch* b, int n, const int* ids, const uint16_t* const* raw
         kf::FuseJob& F = fuse[k];
         memset(&F, 0, sizeof(F));
         F.a = kf::fuse_args(q.depth_m, w, h, q.vol, q.K[0], nullptr, q.st);
-        F.a.dmax = q.dmax;
-        F.brick0 = bricks;
+        F.a.drange = q.drange;
+        F.group0 = groups;
         F.dist_tile0 = dist_tiles;
         dist_tiles += kf::dist_tiles(q.cfg.volume_n / 8);
-        const unsigned nb = (unsigned)(q.cfg.volume_n / 8);
-        bricks += nb * nb * nb;
+        groups += kf::fuse_groups(q.cfg.volume_n / 8);
     }
     // raycast jobs of the tracking sessions, FP32 volumes first (one launch per format)
     for (int pass = 0; pass < 2; ++pass) {
@@ -741,7 +740,7 @@ int kf_batch_tick(kf_batch* b, int n, const int* ids, const uint16_t* const* raw
     hd->n_icp = n_icp;
     for (int l = 0; l < 3; ++l) hd->icp_blocks[l] = icp_blocks[l];
     hd->n_fuse = n;
-    hd->fuse_bricks = bricks;
+    hd->fuse_groups = groups;
     hd->dist_tiles = dist_tiles;
 
     // ---- launch

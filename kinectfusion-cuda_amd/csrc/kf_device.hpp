@@ -242,6 +242,19 @@ __device__ __forceinline__ float wave_max(float v)
 {
     return wave_reduce(v, [](float a, float b) { return fmaxf(a, b); });
 }
+// The max of m and the min of l over the 16 lanes of a row, in every lane.
+__device__ __forceinline__ float2 row_range(float m, float l)
+{
+    m = fmaxf(m, dpp_partner<kDppRowMirror>(m));
+    l = fminf(l, dpp_partner<kDppRowMirror>(l));
+    m = fmaxf(m, dpp_partner<kDppRowHalfMirror>(m));
+    l = fminf(l, dpp_partner<kDppRowHalfMirror>(l));
+    m = fmaxf(m, dpp_partner<kDppXor2>(m));
+    l = fminf(l, dpp_partner<kDppXor2>(l));
+    m = fmaxf(m, dpp_partner<kDppXor1>(m));
+    l = fminf(l, dpp_partner<kDppXor1>(l));
+    return make_float2(m, l);
+}
 __device__ __forceinline__ int wave_sum(int v)
 {
     const auto r32 = __builtin_amdgcn_permlane32_swap((unsigned)v, (unsigned)v, false, false);

@@ -92,8 +92,8 @@ struct kf_volume {
     uint8_t* dist = nullptr;                  // per-brick free distances, formed from free_bits
     int* brick_list = nullptr;              // visible bricks of the current fuse
     unsigned int* list_count = nullptr;     // list lengths, double-buffered by launch parity
-    float* dmax = nullptr;                  // max valid depth per 16x16 and per 64x64 pixel tile
-    size_t dmax_cap = 0;                    // floats allocated for dmax
+    float2* drange = nullptr;               // depth range per 16x16 and per 64x64 pixel tile (FuseArgs::drange)
+    size_t drange_cap = 0;                  // tiles allocated for drange
     int64_t fuse_launches = 0;
     size_t bytes = 0;
     // raycast scratch (grown on demand, also by raycasts through a const volume):

@@ -27,7 +27,7 @@ struct BatchHeader {
     int n_ray_f32, ray_tiles_f32;     // the FP32-volume jobs come first: their count and tiles
     int n_icp, icp_blocks[3];         // ICP sessions, blocks per level
     int n_fuse;                       // fuse jobs
-    unsigned fuse_bricks;             // bricks over all fuse jobs
+    unsigned fuse_groups;             // cubes of 4x4x4 bricks over all fuse jobs
     int dist_tiles;                   // free-distance tiles over all fuse jobs
     unsigned* fuse_count;
     unsigned long long* fuse_list;    // job << 32 | brick of the job's volume
@@ -44,7 +44,7 @@ struct PreJob {
     const uint16_t* raw;
     float* depth_m;
     float* d0;         // bilateral-filtered level 0
-    float* dmax;       // tile-max maps of depth_m (FuseArgs::dmax layout; optional)
+    float2* drange;    // tile depth ranges of depth_m (FuseArgs::drange layout; optional)
     float4* v[3];      // camera-space vertex maps
     float4* n[3];      // camera-space normal maps (all levels or none)
     float* d12[2];     // one session: filtered depth of levels 1 and 2 (optional)
@@ -84,22 +84,24 @@ struct FuseArgs {
     // |(fy, h - cy)|, rounded up (they scale the bounding-sphere radius)
     float plane_norm[4];
     int format;   // kf_voxel_format
-    // occlusion test: max valid depth per 16x16 tile (tx16 x ty16) followed by
-    // the max per 64x64 tile (tx64 x ty64); null = frustum test only
-    const float* dmax;
+    // occlusion and free-space tests: (max valid depth, min depth) per 16x16 tile (tx16 x
+    // ty16) followed by the same per 64x64 tile (tx64 x ty64), an invalid depth counting
+    // as 0 in both; null = frustum test only
+    const float2* drange;
     int tx16, ty16, tx64, ty64;
 };
-// Floats of the tile-max maps of a w x h depth map.
-inline size_t depth_max_floats(int w, int h)
+// Tiles of the depth ranges of a w x h depth map.
+inline size_t depth_range_tiles(int w, int h)
 {
     return (size_t)((w + 15) / 16) * ((h + 15) / 16) + (size_t)((w + 63) / 64) * ((h + 63) / 64);
 }
 struct FuseJob {
     FuseArgs a;       // a.dyn set: the session's committed pose
-    unsigned brick0;  // first global brick index of this job
+    unsigned group0;  // first global cube (4x4x4 bricks) of this job
     int dist_tile0;   // first 8x8-row tile of this job's free distances
 };
 // Workgroups of one volume's free distances: one per 8x8 rows of bricks.
+inline unsigned fuse_groups(int nb) { return (unsigned)((nb + 3) / 4) * ((nb + 3) / 4) * ((nb + 3) / 4); }
 inline size_t free_words(int nb) { return (size_t)nb * nb * 2 * (nb > 64 ? 2 : 1); }
 inline int dist_tiles(int nb) { return ((nb + 7) / 8) * ((nb + 7) / 8); }
 FuseArgs fuse_args(const float* depth, int w, int h, const kf_volume* v, const float* K, const float* inv_pose,
@@ -110,12 +112,12 @@ int launch_fuse_batch(const BatchHeader* hd, const FuseJob* jobs, unsigned cull_
 // inv_pose: by-value world->camera matrix; dyn_state (may be null) overrides it
 // with PoseState::inv_pose and skips the launch's work when the frame failed.
 // list_events (optional): two events recorded around the brick-list kernel alone.
-// dmax_ready: the volume's tile-max maps (volume_depth_max) already hold this
+// drange_ready: the volume's tile depth ranges (volume_depth_range) already hold this
 // depth map's (the measurement pass wrote them).
 int launch_fuse(const float* depth, int w, int h, kf_volume* v, const float* K, const float* inv_pose,
-                const PoseState* dyn_state, hipStream_t s, hipEvent_t* list_events, bool dmax_ready);
-// The volume's tile-max map buffer sized for w x h (grown if needed); null on failure.
-float* volume_depth_max(kf_volume* v, int w, int h, hipStream_t s);
+                const PoseState* dyn_state, hipStream_t s, hipEvent_t* list_events, bool drange_ready);
+// The volume's tile depth range buffer sized for w x h (grown if needed); null on failure.
+float2* volume_depth_range(kf_volume* v, int w, int h, hipStream_t s);
 int launch_initialize(kf_volume* v, float f, float wt, hipStream_t s);
 // kf_volume_create without the host wait: initialisation is enqueued on `s`.
 int volume_create(int n, float width_m, float mue_m, int format, hipStream_t s, kf_volume** out);

@@ -148,11 +148,11 @@ __global__ __launch_bounds__(256) void vertex_kernel(const float* __restrict__ d
 
 // ---- the measurement step in two launches (one session or many).
 // Pass 1, per level-0 16x16 tile lt of job J: raw codes -> metres in LDS (the
-// fuse input is written back, with the tile's max valid depth when J.dmax is
+// fuse input is written back, with the tile's depth range when J.drange is
 // set), bilateral filter, level-0 vertex map.
 // UNMIRROR: row j of the frame is read right to left (measurement.cu:22-25).
 template <bool UNMIRROR>
-__device__ __forceinline__ void measure_tile(const PreJob& J, int lt, BilateralTile& tile, float* wave_max)
+__device__ __forceinline__ void measure_tile(const PreJob& J, int lt, BilateralTile& tile, float2* wave_range)
 {
     const int t = threadIdx.y * kTile + threadIdx.x;
     const int i0 = (lt % J.tiles_x) * kTile - 3, j0 = (lt / J.tiles_x) * kTile - 3;
@@ -165,49 +165,50 @@ __device__ __forceinline__ void measure_tile(const PreJob& J, int lt, BilateralT
     }
     __syncthreads();
     const int i = i0 + 3 + threadIdx.x, j = j0 + 3 + threadIdx.y;
-    float dv = 0.0f;  // this pixel's contribution to the tile's max valid depth
+    float dv = 0.0f, dl = __int_as_float(0x7f800000);  // this pixel's part of the tile's range
     if (i < J.w && j < J.h) {
         const int64_t q = (int64_t)j * J.w + i;
         const float dm = tile[threadIdx.y + 3][threadIdx.x + 3];
         J.depth_m[q] = dm;
-        dv = is_depth_valid(dm) ? dm : 0.0f;
+        dv = dl = is_depth_valid(dm) ? dm : 0.0f;
         const float d = bilateral_at(tile, threadIdx.x, threadIdx.y);
         J.d0[q] = d;
         J.v[0][q] = vertex_at(d, i, j, J.Kinv[0]);
     }
-    if (!J.dmax) return;
-    dv = kf::wave_max(dv);  // (wave_max below is the LDS array)
-    if ((t & 63) == 0) wave_max[t >> 6] = dv;
+    if (!J.drange) return;
+    dv = wave_max(dv);
+    dl = wave_min(dl);
+    if ((t & 63) == 0) wave_range[t >> 6] = make_float2(dv, dl);
     __syncthreads();
-    if (t == 0) J.dmax[lt] = fmaxf(fmaxf(wave_max[0], wave_max[1]), fmaxf(wave_max[2], wave_max[3]));
+    if (t == 0) {
+        const float2 a = wave_range[0], b = wave_range[1], c = wave_range[2], d = wave_range[3];
+        J.drange[lt] = make_float2(fmaxf(fmaxf(a.x, b.x), fmaxf(c.x, d.x)), fminf(fminf(a.y, b.y), fminf(c.y, d.y)));
+    }
 }
 
-// The max valid depth of 64x64 level-0 region (rx, ry) from its 16x16 tiles',
+// The depth range of 64x64 level-0 region (rx, ry) from its 16x16 tiles',
 // by one wave (each row of 16 lanes reads the 16 tiles; past the last tile row
 // or column they repeat it).
-__device__ __forceinline__ void region_max(const PreJob& J, int rx, int ry)
+__device__ __forceinline__ void region_range(const PreJob& J, int rx, int ry)
 {
     const int lane = (threadIdx.y * kTile + threadIdx.x) & 63;
     const int tx16 = J.tiles_x, ty16 = (J.h + 15) / 16;
     const int qx = min(rx * 4 + (lane & 3), tx16 - 1), qy = min(ry * 4 + ((lane >> 2) & 3), ty16 - 1);
-    float m = J.dmax[qy * tx16 + qx];
-    m = fmaxf(m, dpp_partner<kDppRowMirror>(m));
-    m = fmaxf(m, dpp_partner<kDppRowHalfMirror>(m));
-    m = fmaxf(m, dpp_partner<kDppXor2>(m));
-    m = fmaxf(m, dpp_partner<kDppXor1>(m));
-    if (lane == 0) J.dmax[tx16 * ty16 + ry * ((J.w + 63) / 64) + rx] = m;
+    const float2 e = J.drange[qy * tx16 + qx];
+    const float2 r = row_range(e.x, e.y);
+    if (lane == 0) J.drange[tx16 * ty16 + ry * ((J.w + 63) / 64) + rx] = r;
 }
 
 // Pass 2 of many sessions (3 levels, no normals), one thread per level-2 pixel
 // of level-2 tile lt: its 4x4 level-0 block (the frame's width is a multiple of
 // 4, so each row is one 16-byte load) gives 4 level-1 depths (downSample) and
 // those the level-2 depth; vertex maps of both levels.  A workgroup covers a
-// 64x64 level-0 region and also writes its max valid depth.  Bound: HBM.
+// 64x64 level-0 region and also writes its depth range.  Bound: HBM.
 __device__ __forceinline__ void pyramid_tile(const PreJob& J, int lt)
 {
     const int t = threadIdx.y * kTile + threadIdx.x;
     const int rx = lt % J.ptiles_x, ry = lt / J.ptiles_x;
-    if (t < 64) region_max(J, rx, ry);
+    if (t < 64) region_range(J, rx, ry);
     const int i2 = rx * kTile + threadIdx.x, j2 = ry * kTile + threadIdx.y;
     const int w1 = J.w >> 1, w2 = J.w >> 2;
     if (i2 >= w2 || j2 >= (J.h >> 2)) return;
@@ -274,7 +275,7 @@ __device__ __forceinline__ void pyramid_region(const PreJob& J, int lt, PyramidT
         const bool in = x0 + x < J.w && y0 + y < J.h;
         T.d0[y][x] = in ? J.d0[(int64_t)(y0 + y) * J.w + (x0 + x)] : 0.0f;
     }
-    if (J.dmax && !(rx & 1) && !(ry & 1) && t >= 192) region_max(J, rx >> 1, ry >> 1);
+    if (J.drange && !(rx & 1) && !(ry & 1) && t >= 192) region_range(J, rx >> 1, ry >> 1);
     __syncthreads();
     if (normals) {
 #pragma unroll
@@ -324,8 +325,8 @@ template <bool UNMIRROR>
 __global__ __launch_bounds__(256) void measure_kernel(PreJob J)
 {
     __shared__ BilateralTile tile;
-    __shared__ float wave_max[4];
-    measure_tile<UNMIRROR>(J, blockIdx.x, tile, wave_max);
+    __shared__ float2 wave_range[4];
+    measure_tile<UNMIRROR>(J, blockIdx.x, tile, wave_range);
 }
 __global__ __launch_bounds__(256) void pyramid_kernel(PreJob J)
 {
@@ -339,7 +340,7 @@ __global__ __launch_bounds__(256) void pyramid_kernel(PreJob J)
 __global__ __launch_bounds__(256) void measure_batch_kernel(const BatchHeader* hd, const PreJob* jobs)
 {
     __shared__ BilateralTile tile;
-    __shared__ float wave_max[4];
+    __shared__ float2 wave_range[4];
     if (blockIdx.x == 0 && threadIdx.y == 0) {
         if (threadIdx.x == 0) *hd->fuse_count = 0u;
         hd->ray_count[threadIdx.x * kCountStride] = 0u;  // kTile == 16 deferred-ray counts
@@ -347,7 +348,7 @@ __global__ __launch_bounds__(256) void measure_batch_kernel(const BatchHeader* h
     const int tiles = hd->pre_tiles, njobs = hd->n_pre;
     for (int tl = blockIdx.x; tl < tiles; tl += gridDim.x) {
         const PreJob& J = jobs[job_of(jobs, njobs, tl, [](const PreJob& x) { return x.tile0; })];
-        measure_tile<false>(J, tl - J.tile0, tile, wave_max);
+        measure_tile<false>(J, tl - J.tile0, tile, wave_range);
     }
 }
 
@@ -413,7 +414,7 @@ int launch_measure(PreJob& J, hipStream_t s)
     else measure_kernel<false><<<tiles, dim3(kTile, kTile), 0, s>>>(J);
     KF_LAUNCHED("measure_kernel");
     // pass 2 has work for a pyramid, normals or the 64x64 tile maxima
-    if (J.levels > 1 || J.n[0] || J.dmax) {
+    if (J.levels > 1 || J.n[0] || J.drange) {
         const int regions = ((J.w + kRegion - 1) / kRegion) * ((J.h + kRegion - 1) / kRegion);
         pyramid_kernel<<<(unsigned)regions, dim3(kTile, kTile), 0, s>>>(J);
         KF_LAUNCHED("pyramid_kernel");

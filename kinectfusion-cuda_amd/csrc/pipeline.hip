@@ -173,7 +173,7 @@ int kf_pipeline_frame(kf_pipeline* p, const uint16_t* raw)
     int st;
     kf::PoseState* state = p->icp->state;
     // the two-pass measurement: metres, bilateral, pyramid, vertex maps and the
-    // fuse's tile-max maps (depthFrameToVertexPyramid, kinect_fusion.cpp:116-135).
+    // fuse's tile depth ranges (depthFrameToVertexPyramid, kinect_fusion.cpp:116-135).
     // ICP computes the live normals itself, so the normal pyramid is only built
     // when a caller asks for it.
     kf::PreJob J;
@@ -181,8 +181,8 @@ int kf_pipeline_frame(kf_pipeline* p, const uint16_t* raw)
     J.raw = raw;
     J.depth_m = p->depth_m;
     J.d0 = p->dpyr[0];
-    J.dmax = kf::volume_depth_max(p->vol, w, h, s);
-    if (!J.dmax) return kf::fail(KF_ERR_OOM, "kf_pipeline_frame: depth tile-max maps");
+    J.drange = kf::volume_depth_range(p->vol, w, h, s);
+    if (!J.drange) return kf::fail(KF_ERR_OOM, "kf_pipeline_frame: depth tile maps");
     for (int l = 0; l < p->levels; ++l) J.v[l] = p->vpyr[l];
     J.d12[0] = p->dpyr[1];
     J.d12[1] = p->dpyr[2];

@@ -215,3 +215,43 @@ def test_volume_to_host_and_back(kf, tmp_path, n, fmt):
     assert kf.lib().kf_volume_load(b.h, path) == kf.KF_ERR_IO
     a.close()
     b.close()
+
+
+@pytest.mark.parametrize("n,w,h", [(200, 320, 240), (96, 200, 148)])
+def test_free_bricks_bit_exact(kf, oracle32, n, w, h):
+    """Bricks in free space are updated without projecting their voxels: a wall seen over an object
+    that comes and goes, with holes, infinite and NaN depths, into a volume that holds random codes and
+    counts (127 and 128 among them) in places, against the oracle voxel by voxel."""
+    announce(f"free bricks n {n} {w}x{h}")
+    L, mue = 2.0, 0.03
+    rng = np.random.default_rng(n)
+    Fq, Wq = oracle32.new_volume_q(n)
+    some = rng.random((n // 8,) * 3) < 0.3
+    some = np.repeat(np.repeat(np.repeat(some, 8, 0), 8, 1), 8, 2).reshape(-1)
+    Fq[some] = rng.choice(np.array([32767, 32767, 32767, 20000, -500], np.int16), int(some.sum()))
+    Wq[some] = rng.choice(np.array([1, 5, 127, 128], np.uint8), int(some.sum()))
+    inv = np.float32(1) / np.float32(32767)
+    F = np.where(Fq == -32768, np.float32(2), Fq.astype(np.float32) * inv)
+    fw = np.ascontiguousarray(np.stack([F, Wq.astype(np.float32)], -1))
+    grid = kf.VoxelGrid(L, n, mue=mue, voxel_format=kf.KF_VOXEL_SNORM16_U8)
+    kf.check(kf.lib().kf_volume_upload(grid.h, fw.ctypes.data_as(C.c_void_p)))
+    sensor = kf.Sensor(0.82 * w, 0.82 * w, w / 2 - 0.5, h / 2 - 0.5)
+    dm = kf.GridMap(w, h)
+    touched = 0
+    for f in range(4):
+        d = (1.9 + 0.1 * np.sin(np.arange(w) / 17.0)[None, :] + 0.05 * rng.random((h, w))).astype(np.float32)
+        if f % 2:
+            d[h // 4:h // 2, w // 4:w // 2] = 0.9
+        d[rng.random((h, w)) < 2e-4] = 0.0
+        d[3 * h // 4, : w // 3] = np.inf
+        d[h - 9, w // 2] = np.nan
+        pose = np.eye(4, dtype=np.float32)
+        pose[3, :3] = (0.02 * f, 0.01 * f, -1.35)  # column-major
+        sensor.set_pose(pose.reshape(-1))
+        dm.upload(d)
+        kf.kernel.fuse(dm, grid, sensor)
+        touched += oracle32.fuse_q(Fq, Wq, n, L, mue, d, sensor.get_inverse_pose(), sensor.get_intr(0))
+    Fg, Wg = grid.download()
+    np.testing.assert_array_equal(Wg.reshape(-1), Wq.astype(np.float32))
+    np.testing.assert_array_equal(Fg.reshape(-1), np.where(Fq == -32768, np.float32(2), Fq.astype(np.float32) * inv))
+    assert grid.touched_total() == touched > 0.1 * n ** 3
