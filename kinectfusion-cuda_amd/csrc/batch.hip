@@ -70,7 +70,7 @@ struct Slot {
 const unsigned kCand[4][kCandidates] = {
     {2048, 4096, 8192, 16384},   // preprocess
     {8192, 16384, 32768, 65536}, // raycast
-    {256, 512, 1024, 2048},      // ICP steps
+    {256, 512, 1280, 4096},      // ICP steps
     {4096, 8192, 16384, 32768},  // fuse list
 };
 
@@ -404,7 +404,7 @@ void default_shape(kf_batch_shape& s, const kf_batch_shape& given)
     // the shapes the tuner picks for 64 sessions of 640x480 -> 512^3
     s.preprocess_blocks = given.preprocess_blocks ? given.preprocess_blocks : 8192;
     s.raycast_blocks = given.raycast_blocks ? given.raycast_blocks : 65536;
-    s.icp_blocks = given.icp_blocks ? given.icp_blocks : 1024;
+    s.icp_blocks = given.icp_blocks ? given.icp_blocks : 1280;
     // the brick cull (not tuned): per 64 x 512^3 tick 107 us at 4096 workgroups, 98 at 8192, 111 at
     // 16384, 148 at 32768
     s.cull_blocks = given.cull_blocks ? given.cull_blocks : 8192;

@@ -330,27 +330,30 @@ __device__ __forceinline__ int pixel_column(int px, int w, float inv_w)
 // Only pixels up to `last` have a lower and (short of their row's end) a right
 // neighbour; a pixel past it loads the last one's, so no select surrounds a load,
 // and the three loads share one 32-bit offset.
-template <int PIX>
-__device__ __forceinline__ void issue_lane_loads(const IcpArgs& a, LaneLoads<PIX>& ll, int block, int pix)
+__device__ __forceinline__ void issue_pixel_loads(const IcpArgs& a, int px, float4& c, float4& r, float4& d, bool& ok)
 {
     const int last = a.w * a.h - a.w - 2;  // w x h <= kMaxMapPixels (checked on the host)
     const bool any = a.w > 1 && a.h > 1;   // uniform; else no pixel has both neighbours
     const float inv_w = 1.0f / (float)a.w;
     const char* row0 = reinterpret_cast<const char*>(a.V);
     const char* row1 = row0 + (size_t)a.w * 16;
+    ok = any && px <= last && pixel_column(px, a.w, inv_w) + 1 < a.w;
+    if (!any) {
+        c = r = d = make_float4(0.0f, 0.0f, 0.0f, kInvalid);
+        return;
+    }
+    const uint32_t o = (uint32_t)min(px, last) * 16u;
+    c = *reinterpret_cast<const float4*>(row0 + o);
+    r = *reinterpret_cast<const float4*>(row0 + o + 16);
+    d = *reinterpret_cast<const float4*>(row1 + o);
+}
+template <int PIX>
+__device__ __forceinline__ void issue_lane_loads(const IcpArgs& a, LaneLoads<PIX>& ll, int block, int pix)
+{
 #pragma unroll
     for (int k = 0; k < PIX; ++k) {
         if (k >= pix) break;  // uniform
-        const int px = (block * pix + k) * kThreads + (int)threadIdx.x;
-        ll.ok[k] = any && px <= last && pixel_column(px, a.w, inv_w) + 1 < a.w;
-        if (!any) {
-            ll.c[k] = ll.r[k] = ll.d[k] = make_float4(0.0f, 0.0f, 0.0f, kInvalid);
-            continue;
-        }
-        const uint32_t o = (uint32_t)min(px, last) * 16u;
-        ll.c[k] = *reinterpret_cast<const float4*>(row0 + o);
-        ll.r[k] = *reinterpret_cast<const float4*>(row0 + o + 16);
-        ll.d[k] = *reinterpret_cast<const float4*>(row1 + o);
+        issue_pixel_loads(a, (block * pix + k) * kThreads + (int)threadIdx.x, ll.c[k], ll.r[k], ll.d[k], ll.ok[k]);
     }
 }
 template <int PIX>
@@ -1123,10 +1126,15 @@ __global__ __launch_bounds__(kThreads) void icp_batch_solve_kernel(const BatchHe
     }
 }
 
-// Four waves per SIMD (102 VGPRs); held to 96 for five it spills and takes 145 us
-// where this takes 122.
+// A lane takes its pixels one after the other, the next one's loads issued ahead, so
+// that few registers (84) hold them and other waves fill the waits: with its four
+// pixels' loads in flight together the kernel held 102 and had four waves per SIMD.
+// Five workgroups per CU resident, as many launched.  On average over the 19 iterations
+// of a tick of 64 sessions 145 -> 136 us (216 of those at 640x480, whose maps come at
+// 4.4 TB/s), of 16 uneven sessions 26.8 -> 26.3; nothing issued ahead (70 registers,
+// six waves) 136.6 and 26.6, two pixels at a time (96) 139.5 and 27.3.
 template <bool COMP>
-__global__ __launch_bounds__(kThreads, 4) void icp_batch_assoc_kernel(const BatchHeader* hd, const IcpJob* jobs,
+__global__ __launch_bounds__(kThreads, 5) void icp_batch_assoc_kernel(const BatchHeader* hd, const IcpJob* jobs,
                                                                    int level)
 {
     const int njobs = hd->n_icp, total = hd->icp_blocks[level];
@@ -1160,8 +1168,6 @@ __global__ __launch_bounds__(kThreads, 4) void icp_batch_assoc_kernel(const Batc
         a.stride = cj[j].a.stride;
         a.pix = cj[j].a.pix;
         const int lb = b - cj[j].block0;
-        LanePixels<> lp;
-        load_lane_pixels(a, lp, lb, a.pix);
         ConstPose* cp = (ConstPose*)cj[j].pose;
         IterPose P;
 #pragma unroll
@@ -1174,8 +1180,27 @@ __global__ __launch_bounds__(kThreads, 4) void icp_batch_assoc_kernel(const Batc
             P.t[q] = cp->t[q];
             P.tp[q] = cp->tp[q];
         }
+        float s[kTerms];
+#pragma unroll
+        for (int q = 0; q < kTerms; ++q) s[q] = 0.0f;
+        int cnt = 0;  // of the wave
+        int px = lb * a.pix * kThreads + (int)threadIdx.x;
+        float4 c, r, d;
+        bool ok;
+        issue_pixel_loads(a, px, c, r, d, ok);
+#pragma unroll 1
+        for (int k = 0; k < a.pix; ++k) {
+            const PixelIn in = icp_pixel_from(c, r, d, ok);
+            px += kThreads;
+            if (k + 1 < a.pix) issue_pixel_loads(a, px, c, r, d, ok);
+            const PixelGather g = icp_pixel_gather<true>(a, in, P);
+            float row[6], rb;
+            const bool hit = icp_pixel_finish(a, in, g, P.R, row, rb);
+            cnt += __popcll(__ballot(hit));
+            if (hit) accumulate(s, row, rb);
+        }
         __syncthreads();  // the previous block's reduction LDS is free again
-        associate_reduce<COMP>(a, lp, P, lb, a.pix);
+        block_reduce_store<typename SumType<COMP>::T>(s, cnt, a.partials, a.stride, lb);
     }
 }
 
