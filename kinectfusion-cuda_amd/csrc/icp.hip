@@ -18,6 +18,7 @@
 // cublasSgemv, copies 42 floats to the host and solves with Eigen's FP32 LLT,
 // with a host synchronisation per iteration.
 #include <math.h>
+#include <stddef.h>
 #include <string.h>
 
 #include <algorithm>
@@ -481,20 +482,18 @@ __global__ __launch_bounds__(kThreads) void icp_rows_kernel(IcpArgs a, IterPose 
 }
 
 // ---- FP64 6x6 Cholesky solve, unblocked, in the column order of Eigen's LLT
-// (3rd/eigen/Eigen/src/Cholesky/LLT.h:306-326), by one wave: lane r < 6
-// holds row r of A (from the 27 sums) and of L; column k is finished by its
-// lanes and its values are broadcast with readlane:
-//   D = A(k,k) - sum_j<k L(k,j)^2,   i(k) = 1 / sqrt(D),   L(k,k) = D i(k),
+// (3rd/eigen/Eigen/src/Cholesky/LLT.h:306-326):
+//   D = A(k,k) - sum_j<k L(k,j)^2,   i(k) = 1 / sqrt(D),
 //   L(r,k) = (A(r,k) - sum_j<k L(r,j) L(k,j)) * i(k),
 //   y(r) = (b(r) - sum_j<r L(r,j) y(j)) * i(r),
 //   x(r) = (y(r) - sum_j>r L(j,r) x(j)) * i(r)
 // (a reciprocal square root and multiplications instead of a square root and
 // divisions by L(r,r), and fused multiply-adds in the sums: each value moves
 // by a few ulp of FP64, far below the FP32 pose it feeds, and the FP64 square
-// roots and divisions leave the dependent chain).  No lane holds the whole matrix (a one-lane FP64 solve
-// would set the register budget of every kernel that embeds it).
-// Called by all 64 lanes of a wave; returns 0 or the failing column + 1 and
-// the solution in x (the same values in every lane).
+// roots and divisions leave the dependent chain).  Every lane forms the whole matrix
+// from the sums in LDS: the solve is one chain of dependent FP64 operations, and rows
+// spread over lanes added a lane broadcast to each of its links.
+// Returns 0 or the failing column + 1 and the solution in x.
 __device__ __forceinline__ double bcast(double v, int lane)
 {
     const long long b = __double_as_longlong(v);
@@ -506,53 +505,36 @@ __device__ __forceinline__ double bcast(double v, int lane)
 // index of A(p, q), p <= q, among the 21 sums: rows of the upper triangle
 __device__ __forceinline__ int sym_index(int p, int q) { return p * 6 - (p * (p - 1)) / 2 + (q - p); }
 
-__device__ int chol6_wave(const double* tot, double* x)
+__device__ __forceinline__ int chol6(const double* tot, double* x)
 {
-    const int lane = threadIdx.x & 63;
-    const int r = lane < 6 ? lane : 5;  // lanes >= 6 shadow row 5; their values are never read
-    double a[6], Lr[6], inv[6];
-#pragma unroll
-    for (int c = 0; c < 6; ++c) {
-        a[c] = tot[sym_index(min(r, c), max(r, c))];
-        Lr[c] = 0.0;
-    }
-    // each diagonal entry's reciprocal square root is taken once per column;
-    // the column below it and both substitutions multiply by it, so the
-    // substitutions' twelve dependent steps are multiplications, not divisions
+    double L[6][6], inv[6], y[6];
 #pragma unroll
     for (int k = 0; k < 6; ++k) {
-        double d = a[k];
+        double d = tot[sym_index(k, k)];
 #pragma unroll
-        for (int j = 0; j < k; ++j) d = fma(-Lr[j], Lr[j], d);
-        d = bcast(d, k);
+        for (int j = 0; j < k; ++j) d = fma(-L[k][j], L[k][j], d);
         if (!(d > 0.0)) return k + 1;
         inv[k] = rsqrt(d);  // 1/sqrt, within 2 ulp of FP64
-        d = d * inv[k];
-        double Lk[6];
 #pragma unroll
-        for (int j = 0; j < k; ++j) Lk[j] = bcast(Lr[j], k);
-        if (r == k) {
-            Lr[k] = d;
-        } else if (r > k) {
-            double v = a[k];
+        for (int r = k + 1; r < 6; ++r) {
+            double v = tot[sym_index(k, r)];
 #pragma unroll
-            for (int j = 0; j < k; ++j) v = fma(-Lr[j], Lk[j], v);
-            Lr[k] = v * inv[k];
+            for (int j = 0; j < k; ++j) v = fma(-L[r][j], L[k][j], v);
+            L[r][k] = v * inv[k];
         }
     }
-    double y[6];
 #pragma unroll
     for (int q = 0; q < 6; ++q) {
-        double v = tot[21 + r];
+        double v = tot[21 + q];
 #pragma unroll
-        for (int j = 0; j < q; ++j) v = fma(-Lr[j], y[j], v);
-        y[q] = bcast(v, q) * inv[q];
+        for (int j = 0; j < q; ++j) v = fma(-L[q][j], y[j], v);
+        y[q] = v * inv[q];
     }
 #pragma unroll
     for (int q = 5; q >= 0; --q) {
         double v = y[q];
 #pragma unroll
-        for (int j = q + 1; j < 6; ++j) v = fma(-bcast(Lr[q], j), x[j], v);
+        for (int j = q + 1; j < 6; ++j) v = fma(-L[j][q], x[j], v);
         x[q] = v * inv[q];
     }
     return 0;
@@ -604,20 +586,12 @@ __device__ __forceinline__ void sincos_small(double x, double* sn, double* cs)
 struct SinCos3 {
     double sh, ch, sp, cp, sb, cb;
 };
-__device__ __forceinline__ SinCos3 angle_sincos(const float* x)
-{
-    SinCos3 a;
-    sincos_small(x[1], &a.sh, &a.ch);
-    sincos_small(x[0], &a.sp, &a.cp);
-    sincos_small(x[2], &a.sb, &a.cb);
-    return a;
-}
-// The same by lanes 0, 1, 2 of a wave, from the FP64 solution xd (every lane
-// of the wave calls it and receives all six values).
-__device__ __forceinline__ SinCos3 angle_sincos_wave(const double* xd)
+// Formed by lanes 0, 1, 2 of a wave, from the float update x (every lane of the wave
+// calls it and receives all six values).
+__device__ __forceinline__ SinCos3 angle_sincos_wave(const float* x)
 {
     const int lane = threadIdx.x & 63;
-    const float ang = lane == 0 ? (float)xd[1] : (lane == 1 ? (float)xd[0] : (float)xd[2]);
+    const float ang = lane == 0 ? x[1] : (lane == 1 ? x[0] : x[2]);
     double sn, cs;
     sincos_small(ang, &sn, &cs);
     SinCos3 a;
@@ -630,27 +604,24 @@ __device__ __forceinline__ SinCos3 angle_sincos_wave(const double* xd)
     return a;
 }
 
-__device__ void update_pose(float* Rm, float* t, const float* x, const SinCos3& a)
+// The updated pose, a float per lane: lane 3 c + r < 9 holds R(r, c), lanes 9 to 11 t.
+// v: the same of the pose before.
+__device__ __forceinline__ float update_pose_wave(float v, const float* x, const SinCos3& a)
 {
     const double sh = a.sh, ch = a.ch, sp = a.sp, cp = a.cp, sb = a.sb, cb = a.cb;
     double Ri[9];
     Ri[0] = ch * cb + sh * sp * sb;  Ri[1] = sb * cp;  Ri[2] = -sh * cb + ch * sp * sb;
     Ri[3] = -ch * sb + sh * sp * cb; Ri[4] = cb * cp;  Ri[5] = sb * sh + ch * sp * cb;
     Ri[6] = sh * cp;                 Ri[7] = -sp;      Ri[8] = ch * cp;
-    double Rn[9], tn[3];
-    for (int c = 0; c < 3; ++c)
-        for (int r = 0; r < 3; ++r) {
-            double s = 0;
-            for (int q = 0; q < 3; ++q) s += Ri[r * 3 + q] * (double)Rm[c * 3 + q];
-            Rn[c * 3 + r] = s;
-        }
-    for (int r = 0; r < 3; ++r) {
-        double s = 0;
-        for (int q = 0; q < 3; ++q) s += Ri[r * 3 + q] * (double)t[q];
-        tn[r] = s + (double)x[3 + r];
+    const int lane = threadIdx.x & 63, r = lane % 3, col = min(lane - r, 9);
+    double s = 0;
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+        const double e = r == 0 ? Ri[q] : (r == 1 ? Ri[3 + q] : Ri[6 + q]);
+        s += e * (double)__shfl(v, col + q);
     }
-    for (int q = 0; q < 9; ++q) Rm[q] = (float)Rn[q];
-    for (int q = 0; q < 3; ++q) t[q] = (float)tn[q];
+    const float xt = r == 0 ? x[3] : (r == 1 ? x[4] : x[5]);
+    return (float)(lane < 9 ? s : s + (double)xt);
 }
 
 // general_helper.cpp:11-21
@@ -740,40 +711,18 @@ __device__ void sum_partials(const float* partials, int stride, int nblocks, dou
     sum_loaded_partials(partials, stride, nblocks, first, tot, count);
 }
 
-// Pose update of one iteration from its FP64 solution (one lane): the float
-// update x, the pose update (icp.cpp:65-87) and the early-stop test
-// (icp.cpp:45-53).  Returns 0 or KF_ERR_NONFINITE; *done = early stop.
-__device__ int pose_step(const double* xd, const SinCos3& sc, float* R, float* t, float stop_angle,
-                         float stop_dist, float* x, bool* done)
-{
-    bool finite = true;
-    for (int q = 0; q < 6; ++q) {
-        x[q] = (float)xd[q];
-        finite = finite && isfinite(x[q]);
-    }
-    *done = false;
-    if (!finite) return KF_ERR_NONFINITE;
-    float Rprev[9], tprev[3], err[2];
-    for (int q = 0; q < 9; ++q) Rprev[q] = R[q];
-    for (int q = 0; q < 3; ++q) tprev[q] = t[q];
-    update_pose(R, t, x, sc);
-    pose_error(Rprev, tprev, R, t, err);
-    *done = err[0] < stop_angle && err[1] < stop_dist;
-    return KF_OK;
-}
-
-// mode 0: ICP iteration (solve + pose update + early stop); mode 1: solve only.
-// Executed by every lane of one workgroup.
+// The solution of the sums of partial rows (LinearLeastSquares::solve), recorded in the
+// PoseState.  Executed by every lane of one workgroup.
 template <bool COMP>
-__device__ void finalize_body(PoseState* st, const float* partials, int stride, int nblocks, int level,
-                              float stop_angle, float stop_dist, int mode)
+__global__ __launch_bounds__(kThreads) void icp_finalize_kernel(PoseState* st, const float* partials, int stride,
+                                                                int nblocks)
 {
     __shared__ double tot[kTerms];
     __shared__ double count;
     sum_partials<COMP>(partials, stride, nblocks, tot, &count);
     if (threadIdx.x >= 64) return;
     double xd[6];
-    const int rc = chol6_wave(tot, xd);
+    const int rc = chol6(tot, xd);
     if (threadIdx.x != 0) return;
     for (int q = 0; q < kTerms; ++q) st->last_sums[q] = tot[q];
     st->last_inliers = (long long)count;
@@ -783,36 +732,17 @@ __device__ void finalize_body(PoseState* st, const float* partials, int stride, 
         st->frame_skip_fuse = 1;
         return;
     }
-    float x[6];
     bool finite = true;
     for (int q = 0; q < 6; ++q) {
-        x[q] = (float)xd[q];
-        finite = finite && isfinite(x[q]);
-        st->last_x[q] = x[q];
+        const float x = (float)xd[q];
+        finite = finite && isfinite(x);
+        st->last_x[q] = x;
     }
     if (!finite) {
         if (st->status == 0) st->status = KF_ERR_NONFINITE;
         if (st->sticky_status == 0) st->sticky_status = KF_ERR_NONFINITE;
         st->frame_skip_fuse = 1;
-        return;
     }
-    if (mode != 0) return;
-    float Rprev[9], tprev[3], err[2];
-    for (int q = 0; q < 9; ++q) Rprev[q] = st->R[q];
-    for (int q = 0; q < 3; ++q) tprev[q] = st->t[q];
-    update_pose(st->R, st->t, x, angle_sincos(x));
-    pose_error(Rprev, tprev, st->R, st->t, err);
-    st->iterations = st->iterations + 1;
-    if (err[0] < stop_angle && err[1] < stop_dist) st->level_done[level] = 1;
-}
-
-template <bool COMP>
-__global__ __launch_bounds__(kThreads) void icp_finalize_kernel(PoseState* st, const float* partials, int stride,
-                                                                int nblocks, int level, float stop_angle,
-                                                                float stop_dist, int mode)
-{
-    if (mode == 0 && (st->status != 0 || st->level_done[level])) return;
-    finalize_body<COMP>(st, partials, stride, nblocks, level, stop_angle, stop_dist, mode);
 }
 
 // ---- the device-resident coarse-to-fine loop: one launch per iteration.
@@ -822,47 +752,76 @@ __global__ __launch_bounds__(kThreads) void icp_finalize_kernel(PoseState* st, c
 // and the partial rows are double-buffered by launch parity, so no workgroup
 // reads what another workgroup of the same launch writes.
 
-// Applies the solve of the pending iteration of `c` (thread 0): rc and xd from
-// chol6_wave, tot/count the sums it was solved from.
-__device__ void apply_solution(IcpCarry& c, int rc, const double* xd, const SinCos3& sc, const double* tot,
-                               double count,
-                               PoseState* st, bool record, float stop_angle, float stop_dist)
+// The carried state as a wave holds it: lane l has word l of the IcpCarry.
+constexpr int kCarryWords = (int)(sizeof(IcpCarry) / sizeof(int));
+constexpr int kWordStatus = (int)(offsetof(IcpCarry, status) / sizeof(int));
+constexpr int kWordDone = (int)(offsetof(IcpCarry, level_done) / sizeof(int));
+constexpr int kWordIterations = (int)(offsetof(IcpCarry, iterations) / sizeof(int));
+constexpr int kWordPending = (int)(offsetof(IcpCarry, pending) / sizeof(int));
+constexpr int kWordPendingLevel = (int)(offsetof(IcpCarry, pending_level) / sizeof(int));
+constexpr int kWordPendingBlocks = (int)(offsetof(IcpCarry, pending_blocks) / sizeof(int));
+static_assert(offsetof(IcpCarry, R) == 0 && offsetof(IcpCarry, t) == 36 && kWordStatus == 12 && kCarryWords <= 64,
+              "the pose is the first twelve words");
+__device__ __forceinline__ bool carry_pending(int word)
 {
-    if (!c.pending || c.status != 0) return;
-    float x[6] = {0, 0, 0, 0, 0, 0};
-    bool done = false;
-    if (rc) rc = KF_ERR_NOT_PD;
-    else rc = pose_step(xd, sc, c.R, c.t, stop_angle, stop_dist, x, &done);
-    if (rc) {
-        c.status = rc;
-    } else {
-        c.iterations += 1;
-        // c.level_done[c.pending_level] = 1 without a dynamic index (keeps c in registers)
+    return __builtin_amdgcn_readlane(word, kWordPending) != 0 && __builtin_amdgcn_readlane(word, kWordStatus) == 0;
+}
+
+// Applies the pending iteration of a carried state, solved from tot (icp.cpp:65-87, the
+// early-stop test icp.cpp:45-53), by one wave; `record`: keeps the solve in st as well.
+// Without a pending iteration the state stays as it is.
+__device__ __forceinline__ int finish_iteration(int word, const double* tot, double count, PoseState* st, bool record,
+                                                float stop_angle, float stop_dist)
+{
+    if (!carry_pending(word)) return word;  // uniform
+    const int lane = threadIdx.x & 63;
+    double xd[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+    int rc = chol6(tot, xd) ? KF_ERR_NOT_PD : KF_OK;
+    float x[6];
+    bool finite = true;
 #pragma unroll
-        for (int l = 0; l < 4; ++l)
-            if (done && l == c.pending_level) c.level_done[l] = 1;
+    for (int q = 0; q < 6; ++q) {
+        x[q] = rc ? 0.0f : (float)xd[q];
+        finite = finite && isfinite(x[q]);
     }
+    if (!finite) rc = KF_ERR_NONFINITE;
     if (record) {
-        for (int q = 0; q < kTerms; ++q) st->last_sums[q] = tot[q];
-        st->last_inliers = (long long)count;
-        for (int q = 0; q < 6; ++q) st->last_x[q] = x[q];
-    }
-}
-
-// Wave 0 solves the pending iteration of cin (if any) from tot; every lane of
-// the wave gets rc and xd.
-__device__ __forceinline__ int solve_pending(const IcpCarry* cin, const double* tot, double* xd)
-{
-    if (!(cin->pending && cin->status == 0)) return 0;
-    return chol6_wave(tot, xd);
-}
-
-__device__ __forceinline__ int level_flag(const int* v, int level)
-{
-    int r = 0;
+        if (lane < kTerms) st->last_sums[lane] = tot[lane];
+        else if (lane == kTerms) st->last_inliers = (long long)count;
 #pragma unroll
-    for (int l = 0; l < 4; ++l) r = (l == level) ? v[l] : r;
-    return r;
+        for (int q = 0; q < 6; ++q)
+            if (lane == 32 + q) st->last_x[q] = x[q];
+    }
+    if (rc) return lane == kWordStatus ? rc : word;
+    const float next = update_pose_wave(__int_as_float(word), x, angle_sincos_wave(x));
+    // an error is at least 0: below a threshold of 0 or less it never is
+    if (stop_angle > 0.0f && stop_dist > 0.0f) {  // uniform
+        float was[12], is[12], err[2];
+#pragma unroll
+        for (int q = 0; q < 12; ++q) {
+            was[q] = __int_as_float(__builtin_amdgcn_readlane(word, q));
+            is[q] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(next), q));
+        }
+        pose_error(was, was + 9, is, is + 9, err);
+        if (err[0] < stop_angle && err[1] < stop_dist &&
+            lane == kWordDone + __builtin_amdgcn_readlane(word, kWordPendingLevel))
+            word = 1;
+    }
+    if (lane < 12) word = __float_as_int(next);
+    if (lane == kWordIterations) word += 1;
+    return word;
+}
+
+// Opens an iteration at `level`: the state with its pending fields, and whether the
+// session iterates.
+__device__ __forceinline__ int open_iteration(int word, int level, int blocks, bool* run)
+{
+    const int lane = threadIdx.x & 63;
+    *run = __builtin_amdgcn_readlane(word, kWordStatus) == 0 && !__builtin_amdgcn_readlane(word, kWordDone + level);
+    if (lane == kWordPending) word = *run ? 1 : 0;
+    if (lane == kWordPendingLevel) word = level;
+    if (lane == kWordPendingBlocks) word = blocks;
+    return word;
 }
 
 // Phase B of a launch for one session: finish the previous iteration from
@@ -887,8 +846,7 @@ __device__ __forceinline__ void issue_begin_loads(const PoseState* st, const Icp
 {
     // every lane loads (indexes clamped; begin_iteration keeps the wanted
     // lanes' words), so no branch makes a load wait for the loads before it
-    constexpr int kWords = (int)(sizeof(IcpCarry) / sizeof(int));
-    bl.cw = reinterpret_cast<const int*>(cin)[min((int)threadIdx.x & 63, kWords - 1)];
+    bl.cw = reinterpret_cast<const int*>(cin)[min((int)threadIdx.x & 63, kCarryWords - 1)];
     const int pi = min((int)threadIdx.x & 63, 11);
     bl.pw = *(pi < 9 ? st->Rp + pi : st->tp + (pi - 9));
     // no branch around the row loads either: with no previous launch
@@ -909,32 +867,21 @@ __device__ void begin_iteration(const BeginLoads<COMP>& bl, PoseState* st, IcpCa
                                 int prev_blocks, int level, int blocks, bool first, float stop_angle, float stop_dist,
                                 const float* K, IterPose* pose, int* run, double* tot, double* count)
 {
-    __shared__ IcpCarry carry;
     __shared__ float Rp[9];
-    constexpr int kWords = (int)(sizeof(IcpCarry) / sizeof(int));
     if (prev_blocks > 0) sum_loaded_partials(pin, prev_blocks, prev_blocks, bl.rows, tot, count);
-    if (threadIdx.x < kWords) reinterpret_cast<int*>(&carry)[threadIdx.x] = bl.cw;
-    else if (threadIdx.x >= 64 && threadIdx.x < 73) Rp[threadIdx.x - 64] = bl.pw;
+    if (threadIdx.x >= 64 && threadIdx.x < 73) Rp[threadIdx.x - 64] = bl.pw;
     else if (threadIdx.x >= 73 && threadIdx.x < 76) pose->tp[threadIdx.x - 73] = bl.pw;
     __syncthreads();
     if (threadIdx.x >= 64 && threadIdx.x < 73)  // while wave 0 solves
         pose->M[threadIdx.x - 64] = projection_element(K, Rp, (int)threadIdx.x - 64);
     if (threadIdx.x < 64) {
-        double xd[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
-        const int rc = (carry.pending && carry.status == 0) ? chol6_wave(tot, xd) : 0;
-        const SinCos3 sc = angle_sincos_wave(xd);
-        if (threadIdx.x == 0) {
-        IcpCarry c = carry;
-        apply_solution(c, rc, xd, sc, tot, *count, st, first, stop_angle, stop_dist);
-        const int go = (c.status == 0 && !level_flag(c.level_done, level)) ? 1 : 0;
-        c.pending = go;
-        c.pending_level = level;
-        c.pending_blocks = blocks;
-        for (int q = 0; q < 9; ++q) pose->R[q] = c.R[q];
-        for (int q = 0; q < 3; ++q) pose->t[q] = c.t[q];
-        *run = go;
-        if (first) *cout = c;
-        }
+        int word = finish_iteration(bl.cw, tot, *count, st, first, stop_angle, stop_dist);
+        bool go;
+        word = open_iteration(word, level, blocks, &go);
+        if (threadIdx.x < 9) pose->R[threadIdx.x] = __int_as_float(word);
+        else if (threadIdx.x < 12) pose->t[threadIdx.x - 9] = __int_as_float(word);
+        if (threadIdx.x == 0) *run = go ? 1 : 0;
+        if (first && threadIdx.x < kCarryWords) reinterpret_cast<int*>(cout)[threadIdx.x] = word;
     }
     __syncthreads();
 }
@@ -999,69 +946,59 @@ __global__ void icp_begin_kernel(PoseState* st, IcpCarry* c0, Pose16 pose, int f
 
 // Commits the carried estimate as the sensor pose (Sensor::setPose,
 // kinect_fusion.cpp:146-161, sensor.h:30-34); on failure the previous pose is
-// kept and the frame is not fused.  One lane.
-__device__ void commit_state(PoseState* st, const IcpCarry& c)
+// kept and the frame is not fused.  By one wave; lane l holds word l of the state.
+__device__ __forceinline__ void commit_state(PoseState* st, int word)
 {
-    for (int q = 0; q < 9; ++q) st->R[q] = c.R[q];
-    for (int q = 0; q < 3; ++q) st->t[q] = c.t[q];
-    for (int l = 0; l < 4; ++l) st->level_done[l] = c.level_done[l];
-    st->iterations = c.iterations;
-    st->status = c.status;
+    const int lane = threadIdx.x & 63;
+    const float v = __int_as_float(word);
+    const int status = __builtin_amdgcn_readlane(word, kWordStatus);
+    const int iterations = __builtin_amdgcn_readlane(word, kWordIterations);
     PoseMirror* out = st->mirror;
+    const int r = lane % 3, c = lane / 3;  // lanes 0..8: element (r, c) of R; 9..11: t
+    if (lane < 9) st->R[lane] = v;
+    else if (lane < 12) st->t[r] = v;
+    else if (lane >= kWordDone && lane < kWordDone + 4) st->level_done[lane - kWordDone] = word;
+    else if (lane == kWordIterations) st->iterations = iterations;
+    else if (lane == kWordStatus) st->status = status;
     if (out) {
-        for (int q = 0; q < 9; ++q) out->R[q] = c.R[q];
-        for (int q = 0; q < 3; ++q) out->t[q] = c.t[q];
-        out->status = c.status;
-        out->iterations = c.iterations;
+        if (lane < 9) out->R[lane] = v;
+        else if (lane < 12) out->t[r] = v;
+        else if (lane == kWordIterations) out->iterations = iterations;
+        else if (lane == kWordStatus) out->status = status;
     }
-    if (c.status != 0) {
-        if (st->sticky_status == 0) st->sticky_status = c.status;
-        st->frame_skip_fuse = 1;
+    if (status != 0) {
+        if (lane == 0) {
+            if (st->sticky_status == 0) st->sticky_status = status;
+            st->frame_skip_fuse = 1;
+        }
         return;
     }
-    float* P = st->pose;
-    for (int cc = 0; cc < 3; ++cc)
-        for (int r = 0; r < 3; ++r) P[cc * 4 + r] = c.R[cc * 3 + r];
-    P[3] = P[7] = P[11] = 0.0f;
-    for (int r = 0; r < 3; ++r) P[12 + r] = c.t[r];
-    P[15] = 1.0f;
-    if (out)
-        for (int q = 0; q < 16; ++q) out->pose[q] = P[q];
-    float* I = st->inv_pose;
-    for (int cc = 0; cc < 3; ++cc)
-        for (int r = 0; r < 3; ++r) I[cc * 4 + r] = c.R[r * 3 + cc];
-    I[3] = I[7] = I[11] = 0.0f;
-    for (int r = 0; r < 3; ++r) {
-        double sum = 0;
-        for (int q = 0; q < 3; ++q) sum += (double)c.R[r * 3 + q] * (double)c.t[q];
-        I[12 + r] = (float)(-sum);
+    // the pose, its last row 0 0 0 1, and its inverse R^T, -R^T t
+    double sum = 0;
+#pragma unroll
+    for (int q = 0; q < 3; ++q) sum += (double)__shfl(v, r * 3 + q) * (double)__shfl(v, 9 + q);
+    const bool top = lane < 12;
+    const int e = lane < 15 ? (lane - 12) * 4 + 3 : 15;  // lanes 12..15: elements 3, 7, 11, 15
+    const float p = top ? v : (lane == 15 ? 1.0f : 0.0f);
+    if (lane < 16) {
+        st->pose[top ? c * 4 + r : e] = p;
+        if (out) out->pose[top ? c * 4 + r : e] = p;
+        st->inv_pose[lane < 9 ? r * 4 + c : (top ? c * 4 + r : e)] = lane < 9 || !top ? p : (float)(-sum);
     }
-    I[15] = 1.0f;
 }
 
 // Finishes the last iteration and commits the estimate.
 template <bool COMP>
-__device__ void commit_body(PoseState* st, const IcpCarry* cin, const float* pin, float stop_angle, float stop_dist,
-                            double* tot, double* count)
-{
-    if (cin->pending && cin->status == 0) sum_partials<COMP>(pin, cin->pending_blocks, cin->pending_blocks, tot, count);
-    if (threadIdx.x >= 64) return;
-    double xd[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
-    const int rc = solve_pending(cin, tot, xd);
-    const SinCos3 sc = angle_sincos_wave(xd);
-    if (threadIdx.x != 0) return;
-    IcpCarry c = *cin;
-    apply_solution(c, rc, xd, sc, tot, *count, st, true, stop_angle, stop_dist);
-    commit_state(st, c);
-}
-
-template <bool COMP>
 __global__ __launch_bounds__(kThreads) void icp_commit_kernel(PoseState* st, const IcpCarry* cin, const float* pin,
-                                                              float stop_angle, float stop_dist)
+                                                              int prev_blocks, float stop_angle, float stop_dist)
 {
     __shared__ double tot[kTerms];
     __shared__ double count;
-    commit_body<COMP>(st, cin, pin, stop_angle, stop_dist, tot, &count);
+    const int word = reinterpret_cast<const int*>(cin)[min((int)threadIdx.x & 63, kCarryWords - 1)];
+    // summed whether or not an iteration is pending, so no load waits for the state
+    if (prev_blocks > 0) sum_partials<COMP>(pin, prev_blocks, prev_blocks, tot, &count);
+    if (threadIdx.x >= 64) return;
+    commit_state(st, finish_iteration(word, tot, count, st, true, stop_angle, stop_dist));
 }
 
 // ---- the same loop for many sessions per launch (batch ticks).  Each
@@ -1090,11 +1027,13 @@ __global__ __launch_bounds__(kThreads) void icp_batch_solve_kernel(const BatchHe
     __shared__ double count;
     for (int q = blockIdx.x; q < hd->n_icp; q += gridDim.x) {
         const IcpJob& J = jobs[q];
-        IcpCarry* c = J.carry;
         PoseState* st = J.a.st;
-        const bool pend = c->pending && c->status == 0;
-        __syncthreads();  // every lane has read the carry before lane 0 rewrites it
-        if (pend) sum_partials<COMP>(J.partials, c->pending_blocks, c->pending_blocks, tot, &count);
+        int word = reinterpret_cast<const int*>(J.carry)[min((int)threadIdx.x & 63, kCarryWords - 1)];
+        __syncthreads();  // every wave has read the carry before wave 0 rewrites it, and the previous sums
+        if (carry_pending(word)) {
+            const int blocks = __builtin_amdgcn_readlane(word, kWordPendingBlocks);
+            sum_partials<COMP>(J.partials, blocks, blocks, tot, &count);
+        }
         if (!final_) {  // of the association launch that follows
             if (threadIdx.x >= 64 && threadIdx.x < 73)
                 J.pose->M[threadIdx.x - 64] = projection_element(J.a.K, st->Rp, (int)threadIdx.x - 64);
@@ -1102,27 +1041,18 @@ __global__ __launch_bounds__(kThreads) void icp_batch_solve_kernel(const BatchHe
                 J.pose->tp[threadIdx.x - 73] = st->tp[threadIdx.x - 73];
         }
         if (threadIdx.x < 64) {
-            double xd[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
-            const int rc = pend ? chol6_wave(tot, xd) : 0;
-            const SinCos3 sc = angle_sincos_wave(xd);
-            if (threadIdx.x == 0) {
-                IcpCarry cc = *c;
-                apply_solution(cc, rc, xd, sc, tot, count, st, true, stop_angle, stop_dist);
-                if (!final_) {
-                    for (int q = 0; q < 9; ++q) J.pose->R[q] = cc.R[q];
-                    for (int q = 0; q < 3; ++q) J.pose->t[q] = cc.t[q];
-                    cc.pending = (cc.status == 0 && !level_flag(cc.level_done, level)) ? 1 : 0;
-                    cc.pending_level = level;
-                    cc.pending_blocks = J.a.stride;
-                    *c = cc;
-                } else {
-                    cc.pending = 0;
-                    *c = cc;
-                    commit_state(st, cc);
-                }
+            word = finish_iteration(word, tot, count, st, true, stop_angle, stop_dist);
+            if (!final_) {
+                bool run;
+                word = open_iteration(word, level, J.a.stride, &run);
+                if (threadIdx.x < 9) J.pose->R[threadIdx.x] = __int_as_float(word);
+                else if (threadIdx.x < 12) J.pose->t[threadIdx.x - 9] = __int_as_float(word);
+            } else {
+                commit_state(st, word);
+                if (threadIdx.x == kWordPending) word = 0;
             }
+            if (threadIdx.x < kCarryWords) reinterpret_cast<int*>(J.carry)[threadIdx.x] = word;
         }
-        __syncthreads();
     }
 }
 
@@ -1294,9 +1224,9 @@ static int enqueue_steps(kf_icp* icp, const IcpLevel* levels, int n_levels, hipS
         }
     if (before_commit) KF_HIP(hipEventRecord(before_commit, s));
     if (icp->cfg.compensated)
-        icp_commit_kernel<true><<<1, kThreads, 0, s>>>(icp->state, carry_of(icp, k), partials_of(icp, k + 1), sa, sd);
+        icp_commit_kernel<true><<<1, kThreads, 0, s>>>(icp->state, carry_of(icp, k), partials_of(icp, k + 1), prev_blocks, sa, sd);
     else
-        icp_commit_kernel<false><<<1, kThreads, 0, s>>>(icp->state, carry_of(icp, k), partials_of(icp, k + 1), sa, sd);
+        icp_commit_kernel<false><<<1, kThreads, 0, s>>>(icp->state, carry_of(icp, k), partials_of(icp, k + 1), prev_blocks, sa, sd);
     KF_LAUNCHED("icp_commit_kernel");
     if (launches) *launches = k;
     return KF_OK;
@@ -1460,7 +1390,7 @@ int kf_solve_normal_equations(const float* mat_a, const float* vec_b, unsigned i
     if (rc == KF_OK) rc = t.start();
     if (rc == KF_OK) {
         kf::ab_reduce_kernel<false><<<blocks, kf::kThreads, 0, s>>>(mat_a, vec_b, n_equations, partials, blocks, st);
-        kf::icp_finalize_kernel<false><<<1, kf::kThreads, 0, s>>>(st, partials, blocks, blocks, 0, 0.0f, 0.0f, 1);
+        kf::icp_finalize_kernel<false><<<1, kf::kThreads, 0, s>>>(st, partials, blocks, blocks);
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) rc = kf::fail_hip(e, "solve kernels");
     }
@@ -1502,7 +1432,7 @@ int kf_solve_normal_equations_noalloc(const float* mat_a, const float* vec_b, un
     hipStream_t s = kf::stream_of(stream);
     const int blocks = kf::blocks_for(n_equations);
     kf::ab_reduce_kernel<false><<<blocks, kf::kThreads, 0, s>>>(mat_a, vec_b, n_equations, partials, blocks, st);
-    kf::icp_finalize_kernel<false><<<1, kf::kThreads, 0, s>>>(st, partials, blocks, blocks, 0, 0.0f, 0.0f, 1);
+    kf::icp_finalize_kernel<false><<<1, kf::kThreads, 0, s>>>(st, partials, blocks, blocks);
     kf::noalloc_result_kernel<<<1, 64, 0, s>>>(st, result_dev, status_dev);
     KF_HIP(hipGetLastError());
     return KF_OK;
@@ -1549,10 +1479,10 @@ int kf_icp_reduce(const float* vertex_map, const float* target_vertex_map, const
     if (rc == KF_OK) {
         if (compensated) {
             kf::icp_reduce_kernel<true><<<blocks, kf::kThreads, 0, s>>>(a);
-            kf::icp_finalize_kernel<true><<<1, kf::kThreads, 0, s>>>(st, partials, blocks, blocks, 0, 0, 0, 1);
+            kf::icp_finalize_kernel<true><<<1, kf::kThreads, 0, s>>>(st, partials, blocks, blocks);
         } else {
             kf::icp_reduce_kernel<false><<<blocks, kf::kThreads, 0, s>>>(a);
-            kf::icp_finalize_kernel<false><<<1, kf::kThreads, 0, s>>>(st, partials, blocks, blocks, 0, 0, 0, 1);
+            kf::icp_finalize_kernel<false><<<1, kf::kThreads, 0, s>>>(st, partials, blocks, blocks);
         }
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) rc = kf::fail_hip(e, "kf_icp_reduce kernels");
