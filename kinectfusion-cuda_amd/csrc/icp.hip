@@ -912,36 +912,14 @@ __global__ __launch_bounds__(kThreads) void icp_step_kernel(IcpArgs a, const Icp
     associate_reduce<COMP>(a, lp, pose, blockIdx.x, PIX);
 }
 
-// Starts a frame's ICP: the working and previous poses are the sensor pose
-// (icp.cpp:27-29); from `pose` when given by value, else from st->pose.
+// Starts a frame's ICP from a pose given by value.
 struct Pose16 {
     float m[16];
 };
-__device__ void begin_state(PoseState* st, IcpCarry* c0)
+__global__ __launch_bounds__(64) void icp_begin_kernel(PoseState* st, IcpCarry* c0, Pose16 pose)
 {
-    const float* P = st->pose;
-    float Rm[9] = {P[0], P[1], P[2], P[4], P[5], P[6], P[8], P[9], P[10]};
-    IcpCarry c;
-    for (int q = 0; q < 9; ++q) st->R[q] = st->Rp[q] = c.R[q] = Rm[q];
-    for (int q = 0; q < 3; ++q) st->t[q] = st->tp[q] = c.t[q] = P[12 + q];
-    st->status = 0;
-    for (int l = 0; l < 4; ++l) st->level_done[l] = c.level_done[l] = 0;
-    st->iterations = 0;
-    st->frame_skip_fuse = 0;
-    c.status = 0;
-    c.iterations = 0;
-    c.pending = 0;
-    c.pending_level = 0;
-    c.pending_blocks = 0;
-    c.pad[0] = c.pad[1] = 0;
-    *c0 = c;
-}
-__global__ void icp_begin_kernel(PoseState* st, IcpCarry* c0, Pose16 pose, int from_value)
-{
-    if (threadIdx.x != 0) return;
-    if (from_value)
-        for (int q = 0; q < 16; ++q) st->pose[q] = pose.m[q];
-    begin_state(st, c0);
+    if (threadIdx.x < 16) st->pose[threadIdx.x] = pose.m[threadIdx.x];
+    icp_begin_state(st, c0, pose.m);
 }
 
 // Commits the carried estimate as the sensor pose (Sensor::setPose,
@@ -1010,10 +988,10 @@ __global__ __launch_bounds__(kThreads) void icp_commit_kernel(PoseState* st, con
 // launch.  Partial rows are indexed by the session's own block number and
 // summed in that order, so a session's result does not depend on the mix and
 // equals the single-session loop's.
-__global__ void icp_batch_begin_kernel(const BatchHeader* hd, const IcpJob* jobs)
+__global__ __launch_bounds__(64) void icp_batch_begin_kernel(const BatchHeader* hd, const IcpJob* jobs)
 {
-    const int q = blockIdx.x * blockDim.x + threadIdx.x;
-    if (q < hd->n_icp) begin_state(jobs[q].a.st, jobs[q].carry);
+    for (int q = blockIdx.x; q < hd->n_icp; q += gridDim.x)
+        icp_begin_state(jobs[q].a.st, jobs[q].carry, jobs[q].a.st->pose);
 }
 
 // final = 0: finish the pending iteration and open `level`; final = 1: finish
@@ -1172,11 +1150,13 @@ static float* partials_of(kf_icp* icp, int k)
     return icp->partials + (size_t)(k & 1) * kPartialStride * (size_t)icp->max_blocks;
 }
 
+IcpCarry* icp_first_carry(kf_icp* icp) { return carry_of(icp, 0); }
+
 int launch_icp_begin(kf_icp* icp, const float* pose16, hipStream_t s)
 {
-    Pose16 p{};
-    if (pose16) memcpy(p.m, pose16, sizeof(p.m));
-    icp_begin_kernel<<<1, 64, 0, s>>>(icp->state, carry_of(icp, 0), p, pose16 ? 1 : 0);
+    Pose16 p;
+    memcpy(p.m, pose16, sizeof(p.m));
+    icp_begin_kernel<<<1, 64, 0, s>>>(icp->state, carry_of(icp, 0), p);
     KF_LAUNCHED("icp_begin_kernel");
     return KF_OK;
 }
@@ -1241,7 +1221,7 @@ int launch_icp_batch(const BatchHeader* hd, const IcpJob* jobs, const int* iters
                      int compensated, float stop_angle, float stop_dist, unsigned step_blocks, hipStream_t s)
 {
     if (max_sessions <= 0) return KF_OK;
-    icp_batch_begin_kernel<<<(unsigned)((max_sessions + 63) / 64), 64, 0, s>>>(hd, jobs);
+    icp_batch_begin_kernel<<<(unsigned)std::min(max_sessions, 1024), 64, 0, s>>>(hd, jobs);
     KF_LAUNCHED("icp_batch_begin_kernel");
     const IcpJob* level_jobs[3] = {jobs, jobs + max_sessions, jobs + 2 * max_sessions};
     const unsigned sb = (unsigned)std::min(max_sessions, 1024);

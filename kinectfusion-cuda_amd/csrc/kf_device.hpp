@@ -255,6 +255,18 @@ __device__ __forceinline__ float2 row_range(float m, float l)
     l = fminf(l, dpp_partner<kDppXor1>(l));
     return make_float2(m, l);
 }
+// The depth range of the 64x64 pixel region (rx, ry) of a w x h map from its 16x16
+// tiles' (FuseArgs::drange), by one wave (each row of 16 lanes reads the 16 tiles; past
+// the last tile row or column they repeat it).
+__device__ __forceinline__ void region_range(float2* drange, int w, int h, int rx, int ry)
+{
+    const int lane = (threadIdx.y * blockDim.x + threadIdx.x) & 63;
+    const int tx16 = (w + 15) / 16, ty16 = (h + 15) / 16;
+    const int qx = min(rx * 4 + (lane & 3), tx16 - 1), qy = min(ry * 4 + ((lane >> 2) & 3), ty16 - 1);
+    const float2 e = drange[qy * tx16 + qx];
+    const float2 r = row_range(e.x, e.y);
+    if (lane == 0) drange[tx16 * ty16 + ry * ((w + 63) / 64) + rx] = r;
+}
 __device__ __forceinline__ int wave_sum(int v)
 {
     const auto r32 = __builtin_amdgcn_permlane32_swap((unsigned)v, (unsigned)v, false, false);

@@ -51,6 +51,7 @@ struct PreJob {
     int w, h;
     int levels;        // one session: 1..3, w and h divisible by 2^(levels - 1); a batch tick's jobs have 3
     int unmirror;      // one session: nonzero reads row j of the frame right to left
+    int late_regions;  // one session: drange's 64x64 ranges are formed later (RaycastSide)
     float scale;
     float Kinv[3][9];
     int tile0, tiles_x;    // level-0 16x16 tiles of this job
@@ -159,10 +160,19 @@ int launch_raycast_batch(const BatchHeader* hd, const RaycastJob* jobs, const un
                          hipEvent_t mid = nullptr);
 int launch_raycast(const kf_volume* v, const float* pose, const PoseState* dyn_state, const float* inv_k,
                    float4* vout, float4* nout, int w, int h, hipStream_t s);
+// What a frame needs between its measurement and its tracking, done beside the
+// finishing pass by waves that seldom get a ray (a launch of its own takes 5 us): the
+// ICP's start and the 64x64 depth ranges of the w x h frame.
+struct RaycastSide {
+    PoseState* begin;  // null: nothing to do
+    struct IcpCarry* carry;
+    float2* drange;
+    int w, h;
+};
 // All pyramid levels in one launch (level l is w0 >> l by h0 >> l).
 int launch_raycast_levels(const kf_volume* v, const float* pose, const PoseState* dyn_state, int levels,
                           const float (*inv_k)[9], float4* const* vout, float4* const* nout, int w0, int h0,
-                          hipStream_t s);
+                          hipStream_t s, const RaycastSide* side = nullptr);
 
 // ---- ICP (icp.hip)
 constexpr int kPartialStride = 64;  // floats per block partial: 27 sums and the count, FP32 or FP64
@@ -196,6 +206,27 @@ struct IcpCarry {
 struct IterPose {
     float R[9], t[3], M[9], tp[3];
 };
+// Starts a frame's ICP by one wave: the working and previous poses are the sensor pose
+// (icp.cpp:27-29), P (st->pose or the same by value).
+__device__ __forceinline__ void icp_begin_state(PoseState* st, IcpCarry* c0, const float* P)
+{
+    constexpr int kWords = (int)(sizeof(IcpCarry) / sizeof(int));
+    const int lane = threadIdx.x & 63, r = lane % 3, c = lane / 3;
+    int word = 0;  // of the carried state
+    if (lane < 12) {  // R column by column, then t
+        const float v = P[c * 4 + r];
+        word = __float_as_int(v);
+        if (lane < 9) st->R[lane] = st->Rp[lane] = v;
+        else st->t[r] = st->tp[r] = v;
+    } else if (lane < 16) {
+        st->level_done[lane - 12] = 0;
+    } else if (lane == 16) {
+        st->status = 0;
+        st->iterations = 0;
+        st->frame_skip_fuse = 0;
+    }
+    if (lane < kWords) reinterpret_cast<int*>(c0)[lane] = word;
+}
 // One session at one level of a batched ICP launch.
 struct IcpJob {
     IcpArgs a;         // a.stride = the session's blocks at this level; a.partials unused
@@ -219,9 +250,10 @@ int icp_blocks_for(int w, int h);    // the most of icp_level_blocks over the th
 // Enqueues the whole coarse-to-fine loop on `s` with the state on the device,
 // ending with the commit of the estimate into state->pose / inv_pose.
 int launch_icp_loop(kf_icp* icp, const IcpLevel* levels, int n_levels, hipStream_t s);
-// begin: starts the frame's ICP from state->pose (or from pose16 if given);
+// begin: starts the frame's ICP from pose16 (from state->pose: RaycastSide);
 // launch_icp_loop then enqueues one launch per iteration and the final commit.
 int launch_icp_begin(kf_icp* icp, const float* pose16, hipStream_t s);
+IcpCarry* icp_first_carry(kf_icp* icp);  // the state the first launch reads
 // Batched: begin, then steps k = 0.. over the levels coarse to fine, then commit.
 int launch_icp_batch(const BatchHeader* hd, const IcpJob* jobs, const int* iters, int levels, int max_sessions,
                      int compensated, float stop_angle, float stop_dist, unsigned step_blocks, hipStream_t s);

@@ -48,8 +48,8 @@ typedef float BilateralTile[kTile + 6][kTile + 6 + 1];
 // One column of taps.  CENTRE: the column holding the pixel itself, whose tap
 // has weight exp(0) = 1; 0 * centre makes it NaN for a centre that is not
 // finite, as its inf - inf would.
-template <bool CENTRE>
-__device__ __forceinline__ void bilateral_column(const BilateralTile& tile, int tx, int ty, int x, float center,
+template <bool CENTRE, class Window>
+__device__ __forceinline__ void bilateral_column(const Window& tile, int tx, int ty, int x, float center,
                                                  float& norm, float& acc)
 {
     const float cx = (float)(x * x) * -0.0625f;
@@ -69,7 +69,8 @@ __device__ __forceinline__ void bilateral_column(const BilateralTile& tile, int 
         acc = acc + f * cur;
     }
 }
-__device__ __forceinline__ float bilateral_at(const BilateralTile& tile, int tx, int ty)
+template <class Window>
+__device__ __forceinline__ float bilateral_at(const Window& tile, int tx, int ty)
 {
     const float center = tile[ty + 3][tx + 3];
     float norm = 0.0f, acc = 0.0f;
@@ -186,19 +187,6 @@ __device__ __forceinline__ void measure_tile(const PreJob& J, int lt, BilateralT
     }
 }
 
-// The depth range of 64x64 level-0 region (rx, ry) from its 16x16 tiles',
-// by one wave (each row of 16 lanes reads the 16 tiles; past the last tile row
-// or column they repeat it).
-__device__ __forceinline__ void region_range(const PreJob& J, int rx, int ry)
-{
-    const int lane = (threadIdx.y * kTile + threadIdx.x) & 63;
-    const int tx16 = J.tiles_x, ty16 = (J.h + 15) / 16;
-    const int qx = min(rx * 4 + (lane & 3), tx16 - 1), qy = min(ry * 4 + ((lane >> 2) & 3), ty16 - 1);
-    const float2 e = J.drange[qy * tx16 + qx];
-    const float2 r = row_range(e.x, e.y);
-    if (lane == 0) J.drange[tx16 * ty16 + ry * ((J.w + 63) / 64) + rx] = r;
-}
-
 // Pass 2 of many sessions (3 levels, no normals), one thread per level-2 pixel
 // of level-2 tile lt: its 4x4 level-0 block (the frame's width is a multiple of
 // 4, so each row is one 16-byte load) gives 4 level-1 depths (downSample) and
@@ -208,7 +196,7 @@ __device__ __forceinline__ void pyramid_tile(const PreJob& J, int lt)
 {
     const int t = threadIdx.y * kTile + threadIdx.x;
     const int rx = lt % J.ptiles_x, ry = lt / J.ptiles_x;
-    if (t < 64) region_range(J, rx, ry);
+    if (t < 64) region_range(J.drange, J.w, J.h, rx, ry);
     const int i2 = rx * kTile + threadIdx.x, j2 = ry * kTile + threadIdx.y;
     const int w1 = J.w >> 1, w2 = J.w >> 2;
     if (i2 >= w2 || j2 >= (J.h >> 2)) return;
@@ -248,10 +236,11 @@ __device__ __forceinline__ void pyramid_tile(const PreJob& J, int lt)
 // against one launch per level and map: kf_preprocess with normals 160x120
 // 30.9 -> 12.2 us, 640x480 30.0 -> 18.5 us, 1276x716 53.8 -> 33.7 us.
 constexpr int kRegion = 32;
+template <int R>
 struct PyramidTile {
-    float d0[kRegion + 4][kRegion + 5];
-    float d1[kRegion / 2 + 2][kRegion / 2 + 3];
-    float d2[kRegion / 4 + 1][kRegion / 4 + 1];
+    float d0[R + 4][R + 5];
+    float d1[R / 2 + 2][R / 2 + 3];
+    float d2[R / 4 + 1][R / 4 + 1];
 };
 template <class Row>
 __device__ __forceinline__ float4 normal_from_depths(const Row& d, int x, int y, int i, int j, const float* ki)
@@ -263,36 +252,29 @@ __device__ __forceinline__ float4 normal_from_depths(const Row& d, int x, int y,
     return normal_of(s);
 }
 
-__device__ __forceinline__ void pyramid_region(const PreJob& J, int lt, PyramidTile& T)
+// The normals and coarser levels of the RxR region at (x0, y0), whose filtered depths
+// (with the halo, when normals are asked for) are in T.d0.
+template <int R>
+__device__ __forceinline__ void region_levels(const PreJob& J, int x0, int y0, PyramidTile<R>& T)
 {
     const int t = threadIdx.y * kTile + threadIdx.x;
-    const int rtx = (J.w + kRegion - 1) / kRegion, rx = lt % rtx, ry = lt / rtx;
-    const int x0 = rx * kRegion, y0 = ry * kRegion;
     const bool normals = J.n[0] != nullptr;
-    const int halo = normals ? 4 : 0, e0 = kRegion + halo;
-    for (int q = t; q < e0 * e0; q += kTile * kTile) {
-        const int y = q / e0, x = q - y * e0;
-        const bool in = x0 + x < J.w && y0 + y < J.h;
-        T.d0[y][x] = in ? J.d0[(int64_t)(y0 + y) * J.w + (x0 + x)] : 0.0f;
-    }
-    if (J.drange && !(rx & 1) && !(ry & 1) && t >= 192) region_range(J, rx >> 1, ry >> 1);
-    __syncthreads();
     if (normals) {
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const int x = t & 31, y = (t >> 5) + 8 * q, i = x0 + x, j = y0 + y;
+        for (int q = 0; q < R * R / (kTile * kTile); ++q) {
+            const int e = t + q * kTile * kTile, x = e % R, y = e / R, i = x0 + x, j = y0 + y;
             if (i < J.w && j < J.h) J.n[0][(int64_t)j * J.w + i] = normal_from_depths(T.d0, x, y, i, j, J.Kinv[0]);
         }
     }
     if (J.levels < 2) return;  // uniform
-    const int w1 = J.w >> 1, h1 = J.h >> 1, e1 = kRegion / 2 + (normals ? 2 : 0);
+    const int w1 = J.w >> 1, h1 = J.h >> 1, e1 = R / 2 + (normals ? 2 : 0);
     for (int q = t; q < e1 * e1; q += kTile * kTile) {
         const int y = q / e1, x = q - y * e1;
         T.d1[y][x] = down4(T.d0[2 * y][2 * x], T.d0[2 * y][2 * x + 1], T.d0[2 * y + 1][2 * x], T.d0[2 * y + 1][2 * x + 1]);
     }
     __syncthreads();
-    {
-        const int x = threadIdx.x, y = threadIdx.y, i = x0 / 2 + x, j = y0 / 2 + y;
+    if (t < R * R / 4) {
+        const int x = t % (R / 2), y = t / (R / 2), i = x0 / 2 + x, j = y0 / 2 + y;
         if (i < w1 && j < h1) {
             const int64_t q = (int64_t)j * w1 + i;
             const float d = T.d1[y][x];
@@ -302,14 +284,14 @@ __device__ __forceinline__ void pyramid_region(const PreJob& J, int lt, PyramidT
         }
     }
     if (J.levels < 3) return;
-    const int w2 = J.w >> 2, h2 = J.h >> 2, e2 = kRegion / 4 + (normals ? 1 : 0);
+    const int w2 = J.w >> 2, h2 = J.h >> 2, e2 = R / 4 + (normals ? 1 : 0);
     if (t < e2 * e2) {
         const int y = t / e2, x = t - y * e2;
         T.d2[y][x] = down4(T.d1[2 * y][2 * x], T.d1[2 * y][2 * x + 1], T.d1[2 * y + 1][2 * x], T.d1[2 * y + 1][2 * x + 1]);
     }
     __syncthreads();
-    if (t < 64) {
-        const int x = t & 7, y = t >> 3, i = x0 / 4 + x, j = y0 / 4 + y;
+    if (t < R * R / 16) {
+        const int x = t % (R / 4), y = t / (R / 4), i = x0 / 4 + x, j = y0 / 4 + y;
         if (i < w2 && j < h2) {
             const int64_t q = (int64_t)j * w2 + i;
             const float d = T.d2[y][x];
@@ -318,6 +300,73 @@ __device__ __forceinline__ void pyramid_region(const PreJob& J, int lt, PyramidT
             if (normals) J.n[2][q] = normal_from_depths(T.d2, x, y, i, j, J.Kinv[2]);
         }
     }
+}
+
+__device__ __forceinline__ void pyramid_region(const PreJob& J, int lt, PyramidTile<kRegion>& T)
+{
+    const int t = threadIdx.y * kTile + threadIdx.x;
+    const int rtx = (J.w + kRegion - 1) / kRegion, rx = lt % rtx, ry = lt / rtx;
+    const int x0 = rx * kRegion, y0 = ry * kRegion;
+    const int e0 = kRegion + (J.n[0] ? 4 : 0);
+    for (int q = t; q < e0 * e0; q += kTile * kTile) {
+        const int y = q / e0, x = q - y * e0;
+        const bool in = x0 + x < J.w && y0 + y < J.h;
+        T.d0[y][x] = in ? J.d0[(int64_t)(y0 + y) * J.w + (x0 + x)] : 0.0f;
+    }
+    if (J.drange && !(rx & 1) && !(ry & 1) && t >= 192) region_range(J.drange, J.w, J.h, rx >> 1, ry >> 1);
+    __syncthreads();
+    region_levels(J, x0, y0, T);
+}
+
+// Both passes in one, per 16x16 tile lt.  Without normals a tile's coarser levels need
+// its own pixels only.  With normals it filters the halo they need again (20x20 pixels
+// for 16x16), which costs less than a second launch while the launches bound the call:
+// up to kOnePassNormals pixels.  Measured, two passes -> one: with normals 160x120 12.3
+// -> 9.5 us, 320x240 13.0 -> 10.5, 480x360 15.4 -> 14.4, 520x388 17.1 -> 17.5, 1276x716
+// 35 -> 45; without 160x120 8.9 -> 5.6, 640x480 14.4 -> 11.0, 1920x1080 55 -> 52.
+constexpr int kOnePassNormals = 180000;
+struct OnePassTile {
+    float window[kTile + 4 + 6][kTile + 4 + 6 + 1];
+    PyramidTile<kTile> pyramid;
+    float wave_max[4];
+};
+template <bool UNMIRROR>
+__device__ __forceinline__ void one_pass_tile(const PreJob& J, int lt, OnePassTile& S)
+{
+    const int t = threadIdx.y * kTile + threadIdx.x;
+    const int x0 = (lt % J.tiles_x) * kTile, y0 = (lt / J.tiles_x) * kTile;
+    const int e0 = kTile + (J.n[0] ? 4 : 0), ew = e0 + 6;
+    for (int q = t; q < ew * ew; q += kTile * kTile) {
+        const int ly = q / ew, lx = q - ly * ew;
+        int gi = clampi(x0 - 3 + lx, 0, J.w - 1);
+        const int gj = clampi(y0 - 3 + ly, 0, J.h - 1);
+        if (UNMIRROR) gi = J.w - 1 - gi;
+        S.window[ly][lx] = half_rne(J.raw[(int64_t)gj * J.w + gi]) * J.scale;
+    }
+    __syncthreads();
+    for (int q = t; q < e0 * e0; q += kTile * kTile) {
+        const int y = q / e0, x = q - y * e0, i = x0 + x, j = y0 + y;
+        const bool in = i < J.w && j < J.h;
+        const float d = in ? bilateral_at(S.window, x, y) : 0.0f;
+        S.pyramid.d0[y][x] = d;
+        if (in && x < kTile && y < kTile) {
+            const int64_t p = (int64_t)j * J.w + i;
+            J.depth_m[p] = S.window[y + 3][x + 3];
+            J.d0[p] = d;
+            J.v[0][p] = vertex_at(d, i, j, J.Kinv[0]);
+        }
+    }
+    if (J.drange) {
+        const int i = x0 + threadIdx.x, j = y0 + threadIdx.y;
+        const float dm = S.window[threadIdx.y + 3][threadIdx.x + 3];
+        const float m = wave_max(i < J.w && j < J.h && is_depth_valid(dm) ? dm : 0.0f);
+        if ((t & 63) == 0) S.wave_max[t >> 6] = m;
+    }
+    __syncthreads();
+    // the max only: one session's cull does not read the min
+    if (J.drange && t == 0)
+        J.drange[lt] = make_float2(fmaxf(fmaxf(S.wave_max[0], S.wave_max[1]), fmaxf(S.wave_max[2], S.wave_max[3])), 0.0f);
+    region_levels(J, x0, y0, S.pyramid);
 }
 
 // One session: one workgroup per tile, the job by value.
@@ -330,8 +379,14 @@ __global__ __launch_bounds__(256) void measure_kernel(PreJob J)
 }
 __global__ __launch_bounds__(256) void pyramid_kernel(PreJob J)
 {
-    __shared__ PyramidTile T;
+    __shared__ PyramidTile<kRegion> T;
     pyramid_region(J, blockIdx.x, T);
+}
+template <bool UNMIRROR>
+__global__ __launch_bounds__(256) void measure_one_pass_kernel(PreJob J)
+{
+    __shared__ OnePassTile S;
+    one_pass_tile<UNMIRROR>(J, blockIdx.x, S);
 }
 
 // Many sessions per launch (batch ticks), persistent over the tick's tiles.
@@ -410,11 +465,18 @@ int launch_measure(PreJob& J, hipStream_t s)
 {
     J.tiles_x = (J.w + kTile - 1) / kTile;
     const unsigned tiles = (unsigned)(J.tiles_x * ((J.h + kTile - 1) / kTile));
+    const bool second = J.levels > 1 || J.n[0];
+    if (second && (!J.drange || J.late_regions) && (!J.n[0] || (int64_t)J.w * J.h <= kOnePassNormals)) {
+        if (J.unmirror) measure_one_pass_kernel<true><<<tiles, dim3(kTile, kTile), 0, s>>>(J);
+        else measure_one_pass_kernel<false><<<tiles, dim3(kTile, kTile), 0, s>>>(J);
+        KF_LAUNCHED("measure_one_pass_kernel");
+        return KF_OK;
+    }
     if (J.unmirror) measure_kernel<true><<<tiles, dim3(kTile, kTile), 0, s>>>(J);
     else measure_kernel<false><<<tiles, dim3(kTile, kTile), 0, s>>>(J);
     KF_LAUNCHED("measure_kernel");
     // pass 2 has work for a pyramid, normals or the 64x64 tile maxima
-    if (J.levels > 1 || J.n[0] || J.drange) {
+    if (second || J.drange) {
         const int regions = ((J.w + kRegion - 1) / kRegion) * ((J.h + kRegion - 1) / kRegion);
         pyramid_kernel<<<(unsigned)regions, dim3(kTile, kTile), 0, s>>>(J);
         KF_LAUNCHED("pyramid_kernel");

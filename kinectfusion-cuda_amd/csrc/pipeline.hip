@@ -192,6 +192,7 @@ int kf_pipeline_frame(kf_pipeline* p, const uint16_t* raw)
     J.unmirror = p->cfg.unmirror;
     J.scale = p->cfg.depth_scale;
     memcpy(J.Kinv, p->Ki, sizeof(J.Kinv));
+    J.late_regions = p->frame > 0;  // the raycast forms them
     if ((st = kf::launch_measure(J, s))) return st;
     p->normals_fresh = false;
     if (p->frame == 0) {
@@ -204,7 +205,8 @@ int kf_pipeline_frame(kf_pipeline* p, const uint16_t* raw)
     } else {
         if (p->timing) KF_HIP(hipEventRecord(ev[1], s));
         // raycastTsdf (kinect_fusion.cpp:137-144) at the previous pose
-        if ((st = kf::launch_raycast_levels(p->vol, nullptr, state, p->levels, p->Ki, p->pv, p->pn, w, h, s)))
+        const kf::RaycastSide side{state, kf::icp_first_carry(p->icp), J.drange, w, h};
+        if ((st = kf::launch_raycast_levels(p->vol, nullptr, state, p->levels, p->Ki, p->pv, p->pn, w, h, s, &side)))
             return st;
         if (p->timing) KF_HIP(hipEventRecord(ev[2], s));
         // computePose (kinect_fusion.cpp:146-161)
@@ -213,7 +215,6 @@ int kf_pipeline_frame(kf_pipeline* p, const uint16_t* raw)
             lv[l] = kf::IcpLevel{p->vpyr[l], p->pv[l], p->pn[l], w >> l, h >> l, {0}};
             memcpy(lv[l].K, p->K[l], sizeof(lv[l].K));
         }
-        if ((st = kf::launch_icp_begin(p->icp, nullptr, s))) return st;
         if ((st = kf::launch_icp_loop(p->icp, lv, p->levels, s))) return st;
         if (p->timing) KF_HIP(hipEventRecord(ev[3], s));
     }

@@ -42,6 +42,7 @@ struct RaycastArgs {
     unsigned* count;    // their counts for this launch, kCountStride apart
     unsigned* clear;    // the counts of the other launch parity, cleared for the next launch
     unsigned cap;
+    RaycastSide side;
 };
 
 
@@ -717,6 +718,13 @@ __global__ __launch_bounds__(64 * kFinishPer) void raycast_finish_kernel(Raycast
     const RayLists lists = ray_lists(a.count, a.cap);
     const float* pose = a.dyn ? a.dyn->pose : a.pose;
     const unsigned w0 = blockIdx.x * kFinishPer + (unsigned)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (a.side.begin) {  // the last waves
+        const unsigned waves = gridDim.x * kFinishPer, back = waves - 1 - w0;
+        const unsigned rx = (unsigned)(a.side.w + 63) / 64, ry = (unsigned)(a.side.h + 63) / 64;
+        if (back == 0) icp_begin_state(a.side.begin, a.side.carry, a.side.begin->pose);
+        for (unsigned r = back; r < rx * ry; r += waves)
+            region_range(a.side.drange, a.side.w, a.side.h, (int)(r % rx), (int)(r / rx));
+    }
     for (unsigned r = w0; r < lists.end[7]; r += gridDim.x * kFinishPer) {
         ConstRay& cr = ((ConstRay*)a.rays)[ray_slot(lists, a.cap, r)];
         DeferredRay d;
@@ -909,12 +917,13 @@ static int ensure_ray_list(const kf_volume* v, size_t rays, hipStream_t s)
 
 int launch_raycast_levels(const kf_volume* v, const float* pose, const PoseState* dyn_state, int levels,
                           const float (*inv_k)[9], float4* const* vout, float4* const* nout, int w0, int h0,
-                          hipStream_t s)
+                          hipStream_t s, const RaycastSide* side)
 {
     RaycastArgs a{};
     a.vol = raycast_volume(v);
     if (pose) memcpy(a.pose, pose, sizeof(a.pose));
     a.dyn = dyn_state;
+    if (side) a.side = *side;
     a.levels = levels;
     int tiles = 0;
     for (int l = 0; l < levels; ++l) {

@@ -255,3 +255,10 @@ def test_free_bricks_bit_exact(kf, oracle32, n, w, h):
     np.testing.assert_array_equal(Wg.reshape(-1), Wq.astype(np.float32))
     np.testing.assert_array_equal(Fg.reshape(-1), np.where(Fq == -32768, np.float32(2), Fq.astype(np.float32) * inv))
     assert grid.touched_total() == touched > 0.1 * n ** 3
+
+
+# either side of the largest frame whose normals are formed in one pass (180000 pixels), and one whose
+# maps without normals are
+@pytest.mark.parametrize("w,h,normals", [(480, 372, 1), (484, 372, 1), (644, 484, 0)])
+def test_preprocess_one_or_two_passes(kf, oracle32, w, h, normals):
+    test_preprocess_edges_bit_exact(kf, oracle32, w, h, 3, 1, normals)
