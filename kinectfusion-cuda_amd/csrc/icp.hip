@@ -711,36 +711,38 @@ __device__ void sum_partials(const float* partials, int stride, int nblocks, dou
     sum_loaded_partials(partials, stride, nblocks, first, tot, count);
 }
 
+// What a solve leaves in pinned host memory for a caller that waits.
+struct SolveResult {
+    float x[6];
+    int status;
+};
+
 // The solution of the sums of partial rows (LinearLeastSquares::solve), recorded in the
-// PoseState.  Executed by every lane of one workgroup.
+// PoseState and, when given, in `out`.  Executed by every lane of one workgroup.
 template <bool COMP>
 __global__ __launch_bounds__(kThreads) void icp_finalize_kernel(PoseState* st, const float* partials, int stride,
-                                                                int nblocks)
+                                                                int nblocks, SolveResult* out)
 {
     __shared__ double tot[kTerms];
     __shared__ double count;
     sum_partials<COMP>(partials, stride, nblocks, tot, &count);
     if (threadIdx.x >= 64) return;
-    double xd[6];
-    const int rc = chol6(tot, xd);
+    double xd[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+    int rc = chol6(tot, xd) ? KF_ERR_NOT_PD : KF_OK;
     if (threadIdx.x != 0) return;
     for (int q = 0; q < kTerms; ++q) st->last_sums[q] = tot[q];
     st->last_inliers = (long long)count;
-    if (rc != 0) {
-        if (st->status == 0) st->status = KF_ERR_NOT_PD;
-        if (st->sticky_status == 0) st->sticky_status = KF_ERR_NOT_PD;
-        st->frame_skip_fuse = 1;
-        return;
-    }
-    bool finite = true;
+    const bool solved = rc == KF_OK;
     for (int q = 0; q < 6; ++q) {
-        const float x = (float)xd[q];
-        finite = finite && isfinite(x);
-        st->last_x[q] = x;
+        const float x = solved ? (float)xd[q] : 0.0f;
+        if (solved && !isfinite(x)) rc = KF_ERR_NONFINITE;
+        if (solved) st->last_x[q] = x;
+        if (out) out->x[q] = x;
     }
-    if (!finite) {
-        if (st->status == 0) st->status = KF_ERR_NONFINITE;
-        if (st->sticky_status == 0) st->sticky_status = KF_ERR_NONFINITE;
+    if (out) out->status = rc;
+    if (rc != KF_OK) {
+        if (st->status == 0) st->status = rc;
+        if (st->sticky_status == 0) st->sticky_status = rc;
         st->frame_skip_fuse = 1;
     }
 }
@@ -1274,6 +1276,20 @@ namespace {
 
 constexpr int kMaxDevices = 64;
 std::atomic<bool> solve_scratch_used[kMaxDevices];
+// Where a solve with solve_scratch leaves its result: 28 bytes of pinned host memory per
+// GPU, allocated at its first use and, like the scratch, held until the process ends.
+// Null where it could not be had (the result is copied then).  Called by the scratch's
+// holder only.
+kf::SolveResult* solve_result(int dev)
+{
+    static kf::SolveResult* ptr[kMaxDevices] = {};
+    if (!ptr[dev] && hipHostMalloc(reinterpret_cast<void**>(&ptr[dev]), sizeof(kf::SolveResult), hipHostMallocDefault) !=
+                         hipSuccess) {
+        (void)hipGetLastError();
+        ptr[dev] = nullptr;
+    }
+    return ptr[dev];
+}
 
 // The device address of this GPU's `scratch` or `solve_scratch`, looked up once per device.
 int scratch_address(bool solve, char** out, int* device)
@@ -1357,10 +1373,12 @@ int kf_solve_normal_equations(const float* mat_a, const float* vec_b, unsigned i
     kf::PoseState* st = nullptr;
     float* partials = nullptr;
     char* base = nullptr;
+    kf::SolveResult* pinned = nullptr;
     int dev = 0, rc = KF_OK;
     const bool shared = n_equations <= kf::kNoAllocMaxEquations && scratch_address(true, &base, &dev) == KF_OK &&
                         !solve_scratch_used[dev].exchange(true, std::memory_order_acquire);
     if (shared) {
+        pinned = solve_result(dev);
         st = reinterpret_cast<kf::PoseState*>(base);
         partials = reinterpret_cast<float*>(base + kf::kNoAllocStateBytes);
     } else {
@@ -1370,20 +1388,28 @@ int kf_solve_normal_equations(const float* mat_a, const float* vec_b, unsigned i
     if (rc == KF_OK) rc = t.start();
     if (rc == KF_OK) {
         kf::ab_reduce_kernel<false><<<blocks, kf::kThreads, 0, s>>>(mat_a, vec_b, n_equations, partials, blocks, st);
-        kf::icp_finalize_kernel<false><<<1, kf::kThreads, 0, s>>>(st, partials, blocks, blocks);
+        kf::icp_finalize_kernel<false><<<1, kf::kThreads, 0, s>>>(st, partials, blocks, blocks, pinned);
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) rc = kf::fail_hip(e, "solve kernels");
     }
     if (rc == KF_OK) rc = t.finish();
-    kf::PoseState hs;
+    kf::SolveResult r{};
     if (rc == KF_OK) {
-        hipError_t e = hipMemcpyAsync(&hs, st, sizeof(hs), hipMemcpyDeviceToHost, s);
+        kf::PoseState hs;
+        hipError_t e = pinned ? hipSuccess : hipMemcpyAsync(&hs, st, sizeof(hs), hipMemcpyDeviceToHost, s);
         if (e == hipSuccess) e = hipStreamSynchronize(s);
-        if (e != hipSuccess) rc = kf::fail_hip(e, "solve readback");
+        if (e != hipSuccess) {
+            rc = kf::fail_hip(e, "solve readback");
+        } else if (pinned) {
+            r = *pinned;
+        } else {
+            memcpy(r.x, hs.last_x, sizeof(r.x));
+            r.status = hs.status;
+        }
     }
     if (rc == KF_OK) {
-        for (int q = 0; q < 6; ++q) result[q] = hs.last_x[q];
-        if (hs.status) rc = kf::fail(hs.status, kf_status_string(hs.status));
+        for (int q = 0; q < 6; ++q) result[q] = r.x[q];
+        if (r.status) rc = kf::fail(r.status, kf_status_string(r.status));
     } else {
         (void)hipStreamSynchronize(s);  // nothing uses the working memory past this call
     }
@@ -1412,7 +1438,7 @@ int kf_solve_normal_equations_noalloc(const float* mat_a, const float* vec_b, un
     hipStream_t s = kf::stream_of(stream);
     const int blocks = kf::blocks_for(n_equations);
     kf::ab_reduce_kernel<false><<<blocks, kf::kThreads, 0, s>>>(mat_a, vec_b, n_equations, partials, blocks, st);
-    kf::icp_finalize_kernel<false><<<1, kf::kThreads, 0, s>>>(st, partials, blocks, blocks);
+    kf::icp_finalize_kernel<false><<<1, kf::kThreads, 0, s>>>(st, partials, blocks, blocks, nullptr);
     kf::noalloc_result_kernel<<<1, 64, 0, s>>>(st, result_dev, status_dev);
     KF_HIP(hipGetLastError());
     return KF_OK;
@@ -1459,10 +1485,10 @@ int kf_icp_reduce(const float* vertex_map, const float* target_vertex_map, const
     if (rc == KF_OK) {
         if (compensated) {
             kf::icp_reduce_kernel<true><<<blocks, kf::kThreads, 0, s>>>(a);
-            kf::icp_finalize_kernel<true><<<1, kf::kThreads, 0, s>>>(st, partials, blocks, blocks);
+            kf::icp_finalize_kernel<true><<<1, kf::kThreads, 0, s>>>(st, partials, blocks, blocks, nullptr);
         } else {
             kf::icp_reduce_kernel<false><<<blocks, kf::kThreads, 0, s>>>(a);
-            kf::icp_finalize_kernel<false><<<1, kf::kThreads, 0, s>>>(st, partials, blocks, blocks);
+            kf::icp_finalize_kernel<false><<<1, kf::kThreads, 0, s>>>(st, partials, blocks, blocks, nullptr);
         }
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) rc = kf::fail_hip(e, "kf_icp_reduce kernels");

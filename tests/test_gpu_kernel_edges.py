@@ -262,3 +262,35 @@ def test_free_bricks_bit_exact(kf, oracle32, n, w, h):
 @pytest.mark.parametrize("w,h,normals", [(480, 372, 1), (484, 372, 1), (644, 484, 0)])
 def test_preprocess_one_or_two_passes(kf, oracle32, w, h, normals):
     test_preprocess_edges_bit_exact(kf, oracle32, w, h, 3, 1, normals)
+
+
+def test_solve_from_several_threads(kf):
+    """One call at a time has the fixed working memory and the pinned result, the others allocate: every
+    thread gets its own system's solution, bit for bit the one it gets alone, and its own status."""
+    import threading
+
+    announce("solve from four threads")
+    rng = np.random.default_rng(3)
+    lib, sets = kf.lib(), []
+    for n in (7, 1000, 5000, 70000):
+        A, b = rng.standard_normal((n, 6)).astype(np.float32), rng.standard_normal(n).astype(np.float32)
+        sets.append([kf.DeviceArray.from_host(A), kf.DeviceArray.from_host(b), n])
+    sets[1][0] = kf.DeviceArray.from_host(np.zeros((1000, 6), np.float32))  # not positive definite
+
+    def solve(s):
+        x = np.full(6, 9.0, np.float32)
+        return lib.kf_solve_normal_equations(s[0].ptr, s[1].ptr, s[2], x.ctypes.data_as(C.c_void_p), None, None), x
+
+    alone = [solve(s) for s in sets]
+    assert [r[0] for r in alone] == [0, kf.KF_ERR_NOT_PD, 0, 0] and (alone[1][1] == 0).all()
+    got = [[] for _ in sets]
+    threads = [threading.Thread(target=lambda k=k: got[k].extend(solve(sets[k]) for _ in range(50))) for k in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for k in range(4):
+        assert len(got[k]) == 50
+        for rc, x in got[k]:
+            assert rc == alone[k][0]
+            np.testing.assert_array_equal(x, alone[k][1])
