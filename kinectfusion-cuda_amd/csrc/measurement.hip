@@ -48,8 +48,8 @@ typedef float BilateralTile[kTile + 6][kTile + 6 + 1];
 // One column of taps.  CENTRE: the column holding the pixel itself, whose tap
 // has weight exp(0) = 1; 0 * centre makes it NaN for a centre that is not
 // finite, as its inf - inf would.
-template <bool CENTRE, class Window>
-__device__ __forceinline__ void bilateral_column(const Window& tile, int tx, int ty, int x, float center,
+template <bool CENTRE>
+__device__ __forceinline__ void bilateral_column(const BilateralTile& tile, int tx, int ty, int x, float center,
                                                  float& norm, float& acc)
 {
     const float cx = (float)(x * x) * -0.0625f;
@@ -69,8 +69,7 @@ __device__ __forceinline__ void bilateral_column(const Window& tile, int tx, int
         acc = acc + f * cur;
     }
 }
-template <class Window>
-__device__ __forceinline__ float bilateral_at(const Window& tile, int tx, int ty)
+__device__ __forceinline__ float bilateral_at(const BilateralTile& tile, int tx, int ty)
 {
     const float center = tile[ty + 3][tx + 3];
     float norm = 0.0f, acc = 0.0f;
@@ -148,22 +147,30 @@ __global__ __launch_bounds__(256) void vertex_kernel(const float* __restrict__ d
 }
 
 // ---- the measurement step in two launches (one session or many).
+// The metres of the 22x22 window at (i0, j0), clamped to the image's edges.
+// UNMIRROR: row j of the frame is read right to left (measurement.cu:22-25).
+template <bool UNMIRROR>
+__device__ __forceinline__ void fill_window(const PreJob& J, int i0, int j0, BilateralTile& tile)
+{
+    for (int q = threadIdx.y * kTile + threadIdx.x; q < (kTile + 6) * (kTile + 6); q += kTile * kTile) {
+        const int ly = q / (kTile + 6), lx = q % (kTile + 6);
+        int gi = clampi(i0 + lx, 0, J.w - 1);
+        const int gj = clampi(j0 + ly, 0, J.h - 1);
+        if (UNMIRROR) gi = J.w - 1 - gi;
+        tile[ly][lx] = half_rne(J.raw[(int64_t)gj * J.w + gi]) * J.scale;
+    }
+}
+
 // Pass 1, per level-0 16x16 tile lt of job J: raw codes -> metres in LDS (the
 // fuse input is written back, with the tile's depth range when J.drange is
 // set), bilateral filter, level-0 vertex map.
-// UNMIRROR: row j of the frame is read right to left (measurement.cu:22-25).
 template <bool UNMIRROR>
 __device__ __forceinline__ void measure_tile(const PreJob& J, int lt, BilateralTile& tile, float2* wave_range)
 {
     const int t = threadIdx.y * kTile + threadIdx.x;
     const int i0 = (lt % J.tiles_x) * kTile - 3, j0 = (lt / J.tiles_x) * kTile - 3;
     __syncthreads();  // the previous tile's reads of the window are over
-    for (int q = t; q < (kTile + 6) * (kTile + 6); q += kTile * kTile) {
-        int ly = q / (kTile + 6), lx = q % (kTile + 6);
-        int gi = clampi(i0 + lx, 0, J.w - 1), gj = clampi(j0 + ly, 0, J.h - 1);
-        if (UNMIRROR) gi = J.w - 1 - gi;
-        tile[ly][lx] = half_rne(J.raw[(int64_t)gj * J.w + gi]) * J.scale;
-    }
+    fill_window<UNMIRROR>(J, i0, j0, tile);
     __syncthreads();
     const int i = i0 + 3 + threadIdx.x, j = j0 + 3 + threadIdx.y;
     float dv = 0.0f, dl = __int_as_float(0x7f800000);  // this pixel's part of the tile's range
@@ -219,23 +226,23 @@ __device__ __forceinline__ void pyramid_tile(const PreJob& J, int lt)
     J.v[2][(int64_t)j2 * w2 + i2] = vertex_at(d2, i2, j2, J.Kinv[2]);
 }
 
-// Pass 2 of one session, per 32x32 level-0 region lt: the depths of levels 1 and 2
+// Pass 2 of one session, per RxR level-0 region lt: the depths of levels 1 and 2
 // (downSample), their vertex maps and, when J.n is set, the normals of every
 // level, all from the region's filtered depths in LDS.  A normal needs its right
 // and lower neighbour (device_helper.cuh:81-110): one more column and row per
-// level, so 36x36 level-0 depths feed 18x18 of level 1 and 9x9 of level 2, and
+// level, so (for R = 32) 36x36 level-0 depths feed 18x18 of level 1 and 9x9 of level 2, and
 // the neighbours' vertices are formed again from those depths (15 operations)
 // instead of read back (48 bytes).  Depths outside the image are 0 here, which
 // makes their vertices invalid as device_helper.cuh:43-50 has it.
 //
-// Bound: launch and memory latency.  32x32 regions give a 640x480 frame 300
-// workgroups; the 64x64 ones above (80) leave most of the chip idle.  Many
-// sessions fill the chip either way, and there the regions' barriers cost: 64
-// frames of 640x480 took 109 us by regions, 50 us by the form above (73 us with
-// its depths read one by one).  Measured
-// against one launch per level and map: kf_preprocess with normals 160x120
-// 30.9 -> 12.2 us, 640x480 30.0 -> 18.5 us, 1276x716 53.8 -> 33.7 us.
-constexpr int kRegion = 32;
+// Bound: launch and memory latency.  16x16 regions give a 640x480 frame 1200
+// workgroups, 32x32 ones 300, which leave the chip half idle but read less halo:
+// kf_preprocess with normals by 32x32 -> 16x16 regions 484x372 16.2 -> 13.8 us, 640x480
+// 19.0 -> 17.0, 800x600 24.6 -> 23.3, 1276x716 35.9 -> 35.5, 1920x1080 65.5 -> 68.5, so
+// frames up to kSmallRegions pixels take 16x16.  Many sessions fill the chip either
+// way, and there the regions' barriers cost: 64 frames of 640x480 took 109 us by
+// regions, 50 us by the form above (73 us with its depths read one by one).
+constexpr int kSmallRegions = 600000;
 template <int R>
 struct PyramidTile {
     float d0[R + 4][R + 5];
@@ -302,31 +309,31 @@ __device__ __forceinline__ void region_levels(const PreJob& J, int x0, int y0, P
     }
 }
 
-__device__ __forceinline__ void pyramid_region(const PreJob& J, int lt, PyramidTile<kRegion>& T)
+template <int R>
+__device__ __forceinline__ void pyramid_region(const PreJob& J, int lt, PyramidTile<R>& T)
 {
     const int t = threadIdx.y * kTile + threadIdx.x;
-    const int rtx = (J.w + kRegion - 1) / kRegion, rx = lt % rtx, ry = lt / rtx;
-    const int x0 = rx * kRegion, y0 = ry * kRegion;
-    const int e0 = kRegion + (J.n[0] ? 4 : 0);
+    const int rtx = (J.w + R - 1) / R, rx = lt % rtx, ry = lt / rtx;
+    const int x0 = rx * R, y0 = ry * R;
+    const int e0 = R + (J.n[0] ? 4 : 0);
     for (int q = t; q < e0 * e0; q += kTile * kTile) {
         const int y = q / e0, x = q - y * e0;
         const bool in = x0 + x < J.w && y0 + y < J.h;
         T.d0[y][x] = in ? J.d0[(int64_t)(y0 + y) * J.w + (x0 + x)] : 0.0f;
     }
-    if (J.drange && !(rx & 1) && !(ry & 1) && t >= 192) region_range(J.drange, J.w, J.h, rx >> 1, ry >> 1);
+    constexpr int k64 = 64 / R;
+    if (J.drange && rx % k64 == 0 && ry % k64 == 0 && t >= 192)
+        region_range(J.drange, J.w, J.h, rx / k64, ry / k64);
     __syncthreads();
     region_levels(J, x0, y0, T);
 }
 
-// Both passes in one, per 16x16 tile lt.  Without normals a tile's coarser levels need
-// its own pixels only.  With normals it filters the halo they need again (20x20 pixels
-// for 16x16), which costs less than a second launch while the launches bound the call:
-// up to kOnePassNormals pixels.  Measured, two passes -> one: with normals 160x120 12.3
-// -> 9.5 us, 320x240 13.0 -> 10.5, 480x360 15.4 -> 14.4, 520x388 17.1 -> 17.5, 1276x716
-// 35 -> 45; without 160x120 8.9 -> 5.6, 640x480 14.4 -> 11.0, 1920x1080 55 -> 52.
-constexpr int kOnePassNormals = 180000;
+// Both passes in one for a frame without normals, per 16x16 tile lt: its coarser levels
+// need its own pixels only.  Two passes -> one: 160x120 8.9 -> 5.6 us, 640x480 14.4 ->
+// 11.0, 1920x1080 55 -> 52.  (With normals the tile would filter their halo again:
+// 160x120 9.5 us in two passes, 9.6 in one, 400x300 10.8 and 11.1, 1276x716 35 and 45.)
 struct OnePassTile {
-    float window[kTile + 4 + 6][kTile + 4 + 6 + 1];
+    BilateralTile window;
     PyramidTile<kTile> pyramid;
     float wave_max[4];
 };
@@ -335,31 +342,21 @@ __device__ __forceinline__ void one_pass_tile(const PreJob& J, int lt, OnePassTi
 {
     const int t = threadIdx.y * kTile + threadIdx.x;
     const int x0 = (lt % J.tiles_x) * kTile, y0 = (lt / J.tiles_x) * kTile;
-    const int e0 = kTile + (J.n[0] ? 4 : 0), ew = e0 + 6;
-    for (int q = t; q < ew * ew; q += kTile * kTile) {
-        const int ly = q / ew, lx = q - ly * ew;
-        int gi = clampi(x0 - 3 + lx, 0, J.w - 1);
-        const int gj = clampi(y0 - 3 + ly, 0, J.h - 1);
-        if (UNMIRROR) gi = J.w - 1 - gi;
-        S.window[ly][lx] = half_rne(J.raw[(int64_t)gj * J.w + gi]) * J.scale;
-    }
+    fill_window<UNMIRROR>(J, x0 - 3, y0 - 3, S.window);
     __syncthreads();
-    for (int q = t; q < e0 * e0; q += kTile * kTile) {
-        const int y = q / e0, x = q - y * e0, i = x0 + x, j = y0 + y;
-        const bool in = i < J.w && j < J.h;
-        const float d = in ? bilateral_at(S.window, x, y) : 0.0f;
-        S.pyramid.d0[y][x] = d;
-        if (in && x < kTile && y < kTile) {
-            const int64_t p = (int64_t)j * J.w + i;
-            J.depth_m[p] = S.window[y + 3][x + 3];
-            J.d0[p] = d;
-            J.v[0][p] = vertex_at(d, i, j, J.Kinv[0]);
-        }
+    const int i = x0 + threadIdx.x, j = y0 + threadIdx.y;
+    const bool in = i < J.w && j < J.h;
+    const float dm = S.window[threadIdx.y + 3][threadIdx.x + 3];
+    const float d = in ? bilateral_at(S.window, threadIdx.x, threadIdx.y) : 0.0f;
+    S.pyramid.d0[threadIdx.y][threadIdx.x] = d;
+    if (in) {
+        const int64_t q = (int64_t)j * J.w + i;
+        J.depth_m[q] = dm;
+        J.d0[q] = d;
+        J.v[0][q] = vertex_at(d, i, j, J.Kinv[0]);
     }
     if (J.drange) {
-        const int i = x0 + threadIdx.x, j = y0 + threadIdx.y;
-        const float dm = S.window[threadIdx.y + 3][threadIdx.x + 3];
-        const float m = wave_max(i < J.w && j < J.h && is_depth_valid(dm) ? dm : 0.0f);
+        const float m = wave_max(in && is_depth_valid(dm) ? dm : 0.0f);
         if ((t & 63) == 0) S.wave_max[t >> 6] = m;
     }
     __syncthreads();
@@ -377,9 +374,10 @@ __global__ __launch_bounds__(256) void measure_kernel(PreJob J)
     __shared__ float2 wave_range[4];
     measure_tile<UNMIRROR>(J, blockIdx.x, tile, wave_range);
 }
+template <int R>
 __global__ __launch_bounds__(256) void pyramid_kernel(PreJob J)
 {
-    __shared__ PyramidTile<kRegion> T;
+    __shared__ PyramidTile<R> T;
     pyramid_region(J, blockIdx.x, T);
 }
 template <bool UNMIRROR>
@@ -465,8 +463,7 @@ int launch_measure(PreJob& J, hipStream_t s)
 {
     J.tiles_x = (J.w + kTile - 1) / kTile;
     const unsigned tiles = (unsigned)(J.tiles_x * ((J.h + kTile - 1) / kTile));
-    const bool second = J.levels > 1 || J.n[0];
-    if (second && (!J.drange || J.late_regions) && (!J.n[0] || (int64_t)J.w * J.h <= kOnePassNormals)) {
+    if (J.levels > 1 && !J.n[0] && (!J.drange || J.late_regions)) {
         if (J.unmirror) measure_one_pass_kernel<true><<<tiles, dim3(kTile, kTile), 0, s>>>(J);
         else measure_one_pass_kernel<false><<<tiles, dim3(kTile, kTile), 0, s>>>(J);
         KF_LAUNCHED("measure_one_pass_kernel");
@@ -475,10 +472,12 @@ int launch_measure(PreJob& J, hipStream_t s)
     if (J.unmirror) measure_kernel<true><<<tiles, dim3(kTile, kTile), 0, s>>>(J);
     else measure_kernel<false><<<tiles, dim3(kTile, kTile), 0, s>>>(J);
     KF_LAUNCHED("measure_kernel");
-    // pass 2 has work for a pyramid, normals or the 64x64 tile maxima
-    if (second || J.drange) {
-        const int regions = ((J.w + kRegion - 1) / kRegion) * ((J.h + kRegion - 1) / kRegion);
-        pyramid_kernel<<<(unsigned)regions, dim3(kTile, kTile), 0, s>>>(J);
+    // pass 2 has work for a pyramid, normals or the 64x64 depth ranges
+    if (J.levels > 1 || J.n[0] || J.drange) {
+        const int r = (int64_t)J.w * J.h <= kSmallRegions ? 16 : 32;
+        const unsigned regions = (unsigned)(((J.w + r - 1) / r) * ((J.h + r - 1) / r));
+        if (r == 16) pyramid_kernel<16><<<regions, dim3(kTile, kTile), 0, s>>>(J);
+        else pyramid_kernel<32><<<regions, dim3(kTile, kTile), 0, s>>>(J);
         KF_LAUNCHED("pyramid_kernel");
     }
     return KF_OK;

@@ -257,9 +257,9 @@ def test_free_bricks_bit_exact(kf, oracle32, n, w, h):
     assert grid.touched_total() == touched > 0.1 * n ** 3
 
 
-# either side of the largest frame whose normals are formed in one pass (180000 pixels), and one whose
-# maps without normals are
-@pytest.mark.parametrize("w,h,normals", [(480, 372, 1), (484, 372, 1), (644, 484, 0)])
+# either side of the largest frame whose normals are formed by 16x16 regions (600000 pixels), and maps
+# without normals, formed in one pass
+@pytest.mark.parametrize("w,h,normals", [(960, 624, 1), (964, 624, 1), (644, 484, 0)])
 def test_preprocess_one_or_two_passes(kf, oracle32, w, h, normals):
     test_preprocess_edges_bit_exact(kf, oracle32, w, h, 3, 1, normals)
 
