@@ -107,7 +107,7 @@ class Events:
 
 def batched(args, kfusion, stream):
     """Sessions of 640x480 depth into 512^3 snorm16 + uint8 volumes over 4 m cubes (session s:
-    seed 100 + s) in the precision form's arithmetic (Kahan-compensated FP32 ICP sums, FP64
+    seed 100 + s) in the precision form's arithmetic (FP32 lane sums added up in FP64, FP64
     solve), advanced together: one tick = one frame of every session, each stage one launch across
     all sessions, each tick one hipGraph launch.  Launch shapes come from the autotuner during the
     untimed ticks.  After the timed ticks, --batch-stage-ticks more ticks run kernel by kernel
@@ -198,7 +198,7 @@ def batched(args, kfusion, stream):
     out = {"value": round(fps, 3), "unit": "frames/s", "sessions": S, "ticks_timed": args.batch_steps,
            "ms_per_tick": round(gpu_ms / args.batch_steps, 4), "max_tick_ms": round(mx, 4),
            "workload": f"{S} sessions x 640x480 -> 512^3 snorm16+u8 over 4 m cubes, seeds 100..{99 + S}, "
-                       "ICP 10/5/4 with Kahan-compensated FP32 sums and FP64 solve, one hipGraph per tick",
+                       "ICP 10/5/4 with FP32 lane sums added up in FP64 and an FP64 solve, one hipGraph per tick",
            "dtype": "snorm16/u8 volume, f32 compute", "launch_shape": shape, "autotuned": tuned,
            "hbm_per_session_gb": round(sb / 1e9, 3), "icp_failures": failed,
            "final_pose_err_vs_truth": {"trans_m_max": round(max(errs), 5),
@@ -336,7 +336,7 @@ def serving(args, kfusion, shape, batched_fps):
             "peak_resident_gb": round(st["peak_resident_bytes"] / 1e9, 2), "hbm_budget_gb": budget / 1e9,
             "icp_failed_sessions": int(st["failed_frames"]),
             "workload": f"{S} sessions x 640x480, volumes {{256..768}}^3 snorm16+u8 (seed 99), Poisson 30 Hz "
-                        f"+-10 % jitter (seed 7), {args.serve_frames} frames each, 200 GB budget, Kahan ICP sums",
+                        f"+-10 % jitter (seed 7), {args.serve_frames} frames each, 200 GB budget, ICP sums added up in FP64",
             "volume_sizes": [int(x) for x in sizes],
             "saturated": {"frames_per_s": round(sat["frames_per_s"], 3), "frames": int(sat["frames"]),
                           "mean_frames_per_tick": round(sat["mean_frames_per_tick"], 2),
@@ -384,7 +384,7 @@ PREC_FRAMES, PREC_N, PREC_L = 30, 256, 3.0
 
 def precision_run(kfusion):
     """The precision form on its own workload: seed-1 frames, 640x480 -> 256^3 snorm16 + uint8
-    counts over a 3 m cube, Kahan-compensated ICP sums and FP64 solve, 30 frames.  Returns what the
+    counts over a 3 m cube, ICP sums added up in FP64 and FP64 solve, 30 frames.  Returns what the
     CPU leg compares with the FP64 oracle of the same algorithm: every frame's pose, the final
     volume and the predicted vertex maps."""
     import numpy as np
@@ -466,7 +466,7 @@ def cpu_leg(result, args, seq, raws, n, L, mue, plain_model, batch_models, prec)
         both = (prec["W"] > 0) & (W64 > 0)
         dF = np.abs(prec["F"].astype(np.float64) - F64)[both]
         out = {"workload": f"seed-1 frames, 640x480 -> {PREC_N}^3 snorm16 + uint8 counts over "
-                           f"{PREC_L:g} m, Kahan-compensated ICP sums, FP64 solve, {PREC_FRAMES} frames",
+                           f"{PREC_L:g} m, ICP sums added up in FP64, FP64 solve, {PREC_FRAMES} frames",
                "reference": "FP64 oracle of the same algorithm (count weights, unquantised F), run independently",
                "icp_status": int(prec["status"]),
                "pose_max_rot_rad": float(f"{max(rot):.3g}"), "pose_max_trans_m": float(f"{max(trans):.3g}"),
@@ -627,7 +627,7 @@ def main():
                    "final_pose_err_vs_truth": {"trans_m": round(float(np.abs(pose[12:15] - gt[12:15]).max()), 5),
                                                "rot_deg": round(rot_err_deg(pose, gt), 4)}},
         "roofline": {"bound": "hbm", "kernel": "fuse_list_kernel<F32> (voxel sweep; the brick cull and depth "
-                                               "tile-max are two short launches before it)",
+                                               "tile ranges are two short launches before it)",
                      "achieved": round(achieved, 2), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": traffic,
                      "traffic_source": "recorded: rocprofv3 FETCH_SIZE + WRITE_SIZE per dispatch scaled by a known "

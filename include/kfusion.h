@@ -192,7 +192,7 @@ typedef struct kf_icp_config {
     float angle_thresh;                  /* radians */
     float iteration_stop_thresh_angle;   /* poseError chord (general_helper.cpp:11-21); 0 disables */
     float iteration_stop_thresh_distance;/* metres; 0 disables */
-    int compensated;                     /* 0: FP32 tree sums; 1: Kahan-compensated FP32 sums */
+    int compensated;                     /* 0: FP32 tree sums; 1: compensated (lane sums added up in FP64) */
 } kf_icp_config;
 typedef struct kf_icp kf_icp;
 /* ICP::ICP / ~ICP (icp.cpp:12-23). */
