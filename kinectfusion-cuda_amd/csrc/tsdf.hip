@@ -1088,7 +1088,7 @@ int move_voxels(const kf_volume* v, bool to_volume, int64_t q0, int64_t q1, floa
         else
             volume_to_slab<KF_VOXEL_SNORM16_U8><<<blocks, 256>>>(slab, v->f, v->w, v->n, v->nb, q, count);
         KF_LAUNCHED("volume transfer");
-        KF_HIP(hipEventRecord(ev[b], nullptr));
+        if (ev[b]) KF_HIP(hipEventRecord(ev[b], nullptr));
         return KF_OK;
     };
     int st = KF_OK, b = 0;
@@ -1096,9 +1096,10 @@ int move_voxels(const kf_volume* v, bool to_volume, int64_t q0, int64_t q1, floa
     for (int64_t q = q0; q < q1 && st == KF_OK; q += kChunkVoxels, b ^= 1) {
         const int64_t count = std::min(kChunkVoxels, q1 - q);
         if (!to_volume && q + kChunkVoxels < q1) st = launch(q + kChunkVoxels, b ^ 1);
-        // the chunk's last kernel is done (an event never recorded counts as done)
-        if (st == KF_OK) {
-            const hipError_t e = hipEventSynchronize(ev[b]);
+        // the chunk's last kernel is done (an event never recorded counts as done; a volume
+        // of one chunk has no events)
+        if (st == KF_OK && (ev[b] || !to_volume)) {
+            const hipError_t e = ev[b] ? hipEventSynchronize(ev[b]) : hipStreamSynchronize(nullptr);
             if (e != hipSuccess) st = fail_hip(e, "volume transfer");
         }
         if (st == KF_OK) st = host_side(q, count, pinned + b * kChunkVoxels);
@@ -1121,10 +1122,11 @@ int move_volume(const kf_volume* v, bool to_volume, bool parallel, Fn&& host_sid
     const int movers = parallel ? (int)std::min<int64_t>(kMovers, std::max<int64_t>(1, total / (2 * kChunkVoxels))) : 1;
     float2* pinned = nullptr;
     hipEvent_t ev[2 * kMovers] = {};
-    KF_HIP(hipHostMalloc(reinterpret_cast<void**>(&pinned), sizeof(float2) * 2 * kChunkVoxels * movers,
-                         hipHostMallocDefault));
+    // a volume of one chunk (up to 64^3) needs no second one
+    const int64_t slots = total <= kChunkVoxels ? total : 2 * kChunkVoxels * movers;
+    KF_HIP(hipHostMalloc(reinterpret_cast<void**>(&pinned), sizeof(float2) * (size_t)slots, hipHostMallocDefault));
     int st = KF_OK;
-    for (int k = 0; k < 2 * movers && st == KF_OK; ++k) {
+    for (int k = 0; k < 2 * movers && total > kChunkVoxels && st == KF_OK; ++k) {
         const hipError_t e = hipEventCreateWithFlags(&ev[k], hipEventDisableTiming);
         if (e != hipSuccess) st = fail_hip(e, "volume transfer events");
     }
@@ -1160,12 +1162,7 @@ int move_volume(const kf_volume* v, bool to_volume, bool parallel, Fn&& host_sid
         for (std::thread& t : threads) t.join();
         for (int k = 0; k < movers && st == KF_OK; ++k)
             if (status[k]) st = message[k].empty() ? status[k] : fail(status[k], message[k]);
-        const hipError_t e = hipDeviceSynchronize();
-        if (st == KF_OK && e != hipSuccess) st = fail_hip(e, "volume transfer");
     }
-    for (hipEvent_t e : ev)
-        if (e) (void)hipEventDestroy(e);
-    (void)hipHostFree(pinned);
     if (st == KF_OK && to_volume) {
         const int64_t nbricks = (int64_t)v->nb * v->nb * v->nb;
         const unsigned b = (unsigned)((nbricks + 3) / 4);
@@ -1175,10 +1172,13 @@ int move_volume(const kf_volume* v, bool to_volume, bool parallel, Fn&& host_sid
             free_bits_kernel<KF_VOXEL_F32><<<b, 256>>>(v->f, v->free_bits, nbricks, v->n, v->nb);
         else
             free_bits_kernel<KF_VOXEL_SNORM16_U8><<<b, 256>>>(v->f, v->free_bits, nbricks, v->n, v->nb);
-        if ((st = launch_brick_dist(v, nullptr))) return st;
-        hipError_t e = hipDeviceSynchronize();
-        if (e != hipSuccess) st = fail_hip(e, "free_bits_kernel");
+        st = launch_brick_dist(v, nullptr);
     }
+    const hipError_t e = hipDeviceSynchronize();  // nothing uses the chunks past this line
+    if (st == KF_OK && e != hipSuccess) st = fail_hip(e, "volume transfer");
+    for (hipEvent_t x : ev)
+        if (x) (void)hipEventDestroy(x);
+    (void)hipHostFree(pinned);
     return st;
 }
 
