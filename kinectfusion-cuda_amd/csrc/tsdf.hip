@@ -396,17 +396,18 @@ __device__ __forceinline__ void z_terms(const float* ip, const float* zk, float4
 // Pass 1: one lane per brick; bricks whose bounding sphere meets the view
 // frustum are appended to `list`, one atomic per workgroup.  The list length
 // lives in count[parity]; this pass also clears count[1 - parity], which the
-// previous launch used, for the next launch.
+// previous launch used, for the next launch (also when its own frame is not
+// fused: the next launch appends to that count from zero).
 constexpr int kCullThreads = 1024;
 
 __global__ __launch_bounds__(kCullThreads) void fuse_cull_kernel(FuseArgs a, int64_t nbricks, int* list,
                                                                  unsigned int* count, int parity)
 {
+    if (blockIdx.x == 0 && threadIdx.x == 0) count[1 - parity] = 0u;
     if (a.dyn && a.dyn->frame_skip_fuse) return;
     __shared__ float ip[16];
     __shared__ unsigned int wave_base[kCullThreads / 64 + 1];
     load_inv_pose(a, ip);
-    if (blockIdx.x == 0 && threadIdx.x == 0) count[1 - parity] = 0u;
     for (int k = blockIdx.x * kCullThreads + threadIdx.x; k < a.n; k += gridDim.x * kCullThreads) z_terms(ip, a.zk, a.zt, k);
     const int64_t brick = (int64_t)blockIdx.x * kCullThreads + threadIdx.x;
     bool vis = false;
