@@ -253,14 +253,14 @@ struct ColumnPlanes<KF_VOXEL_SNORM16_U8> {
 };
 
 // The precision form's update of voxel kl by f: unit weight per observation, count
-// capped at 128.
+// capped at 128 (an upload or a reset may have stored any count up to 255).
 __device__ __forceinline__ void update_voxel(ColumnPlanes<KF_VOXEL_SNORM16_U8>& v, int kl, float f,
                                              const float* inv_count, float& fmin, float& fk0)
 {
     const int wc = v.count(kl);
     const float Wv = (float)wc;
     float Fv = snorm_decode(v.code(kl));
-    Fv = div_by_exact_reciprocal(Fv * Wv + f, Wv + 1.0f, inv_count[wc + 1]);
+    Fv = div_by_exact_reciprocal(Fv * Wv + f, Wv + 1.0f, inv_count[wc]);
     const int16_t qf = snorm_encode(Fv);
     v.set(kl, qf, wc < 128 ? wc + 1 : 128);
     const float written = snorm_decode(qf);
@@ -276,7 +276,7 @@ __device__ __forceinline__ void update_voxel(ColumnPlanes<KF_VOXEL_SNORM16_U8>& 
 // division only near an integer (the decisions are the exact quotient's).
 // Update (tsdf.cu:47-69): f = min(1, diff / mue) from the exact reciprocal of
 // mue; the precision form divides by the observation count + 1 with the exact
-// reciprocal of 1..129 from inv_count (LDS); every value written is the one the
+// reciprocal of 1..256 from inv_count (LDS); every value written is the one the
 // plain quotients give.  fmin takes the smallest value written, fk0 the value
 // written to voxel 0 (the brick's k = 0 plane).  The column's planes are read
 // when any of its voxels passes the depth test (after the depth gathers) and
@@ -370,11 +370,12 @@ __device__ __forceinline__ int fuse_column(const FuseArgs& a, v3 col, const floa
     return cnt;
 }
 
-// Exact reciprocals 1/k, k = 0..129 (entry 0 unused), for the count update.
-constexpr int kInvCount = 130;
+// Exact reciprocals for the count update: entry c is 1 / (c + 1), for every count
+// a uint8 holds.
+constexpr int kInvCount = 256;
 __device__ __forceinline__ void fill_inv_count(float* t)
 {
-    for (int k = threadIdx.x; k < kInvCount; k += blockDim.x) t[k] = k ? 1.0f / (float)k : 0.0f;
+    for (int c = threadIdx.x; c < kInvCount; c += blockDim.x) t[c] = 1.0f / (float)(c + 1);
     __syncthreads();
 }
 

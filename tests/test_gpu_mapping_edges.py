@@ -1,9 +1,11 @@
 """Mapping through every route that fuses or draws a volume (single calls, the frame loop, batch ticks):
 frames that are not fused, uploaded states, volumes of more than 64 bricks a side."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
-from gpu_util import announce, small_sequence
+from gpu_util import announce, decode_q, small_sequence
 
 pytestmark = pytest.mark.gpu
 
@@ -28,6 +30,17 @@ def make_batch(kf, seq, n, fmt, iters=(4, 3, 2), sessions=1, **kw):
     b = kf.Batch(sessions, icp=kf.IcpConfig(iters, w, h, 0.1, TH, compensated=True), **kw)
     cfg = kf.SessionConfig(w, h, seq.fx, seq.fy, seq.cx, seq.cy, 1e-3, n, seq.L, 0.03, fmt, seq.pose(0))
     return b, [b.add(cfg) for _ in range(sessions)]
+
+
+def upload(kf, handle, F, W):
+    fw = np.ascontiguousarray(np.stack([F, W.astype(np.float32)], -1))
+    kf.check(kf.lib().kf_volume_upload(handle, fw.ctypes.data_as(C.c_void_p)))
+
+
+def batch_volume(kf, b, sid):
+    v = C.c_void_p()
+    kf.check(kf.lib().kf_batch_volume(b.h, sid, C.byref(v)))
+    return v
 
 
 # blank frames between the others: none, one, two in a row, two apart
@@ -74,3 +87,40 @@ def test_frames_that_are_not_fused(kf, blanks, fmt):
                 np.testing.assert_array_equal(maps(m, l).view(np.uint32), ref.map(m, l).view(np.uint32), err_msg=what)
     for x in (ref, gp, b):
         x.close()
+
+
+def test_every_count_a_volume_can_hold(kf, oracle32):
+    """A snorm16 volume may be uploaded with any count up to 255: the update divides by the count + 1
+    and stores at most 128, alike in a single fuse and in a batch's, against the oracle voxel by voxel.
+    (Without iterations a batch's session keeps its pose.)"""
+    announce("counts 0 to 255")
+    seq = small_sequence(seed=12, n_frames=1, w=160, h=120, L=3.0)
+    raw = seq.frames(0, 1)[0]
+    n, frames = 64, 3
+    rng = np.random.default_rng(12)
+    Fq = rng.integers(-32768, 32768, n ** 3).astype(np.int16)
+    Fq[rng.random(n ** 3) < 0.3] = 32767
+    Wq = rng.integers(0, 256, n ** 3).astype(np.uint8)
+    grid = kf.VoxelGrid(seq.L, n, mue=0.03, voxel_format=kf.KF_VOXEL_SNORM16_U8)
+    b, (sid,) = make_batch(kf, seq, n, 1, iters=(0, 0, 0))
+    upload(kf, grid.h, decode_q(Fq), Wq)
+    upload(kf, batch_volume(kf, b, sid), decode_q(Fq), Wq)
+    dev = kf.DeviceArray.from_host(raw)
+    d = oracle32.convert_to_depth_meters(raw, 1e-3)
+    dm = kf.GridMap(seq.width, seq.height)
+    dm.upload(d)
+    sensor = kf.Sensor(seq.fx, seq.fy, seq.cx, seq.cy)
+    sensor.set_pose(seq.pose(0))
+    above = Wq > 128
+    before = Wq.copy()
+    for f in range(frames):
+        kf.kernel.fuse(dm, grid, sensor)
+        b.tick([sid], [dev.ptr.value])
+        oracle32.fuse_q(Fq, Wq, n, seq.L, 0.03, d, sensor.get_inverse_pose(), sensor.get_intr(0))
+    assert b.status(sid) == 0
+    assert np.count_nonzero(above & (Wq != before)) > 1000  # voxels above 128 that the frames met
+    for what, (F, W) in [("single", grid.download()), ("batch", b.volume_download(sid))]:
+        np.testing.assert_array_equal(W, Wq.astype(np.float32), err_msg=what)
+        np.testing.assert_array_equal(F, decode_q(Fq), err_msg=what)
+    grid.close()
+    b.close()
