@@ -164,13 +164,26 @@ size_t maps_bytes(int w, int h)
            sizeof(kf::PoseState);
 }
 
+// 8x8 raycast tiles of a w x h frame's levels, each level's padded to 8 (one band per XCD).
+size_t ray_tiles_of(int w, int h, int levels)
+{
+    size_t tiles = 0;
+    for (int l = 0; l < levels; ++l) {
+        const size_t tx = (size_t)((w >> l) + 7) / 8, ty = (size_t)((h >> l) + 7) / 8;
+        tiles += (tx * ty + 7) & ~(size_t)7;
+    }
+    return tiles;
+}
+// Places a w x h frame's rays take in the deferred-ray list of its voxel format.
+size_t ray_places_of(int w, int h) { return ray_tiles_of(w, h, 3) * 64; }
+
 }  // namespace
 
 size_t kf::batch_shared_bytes(const kf_session_config* c)
 {
-    const size_t nb = (size_t)c->volume_n / 8, w = (size_t)c->frame_width, h = (size_t)c->frame_height;
-    const size_t rays = w * h + (w / 2) * (h / 2) + (w / 4) * (h / 4);
-    return 2 * (sizeof(unsigned long long) * nb * nb * nb + 2 * sizeof(kf::DeferredRay) * rays);
+    const size_t nb = (size_t)c->volume_n / 8;
+    return 2 * (sizeof(unsigned long long) * nb * nb * nb +
+                2 * sizeof(kf::DeferredRay) * ray_places_of(c->frame_width, c->frame_height));
 }
 
 namespace {
@@ -215,17 +228,6 @@ int drop_graphs(kf_batch* b)
     return KF_OK;
 }
 
-// 8x8 raycast tiles of a session's levels, each level's padded to 8 (one band per XCD).
-size_t ray_tiles_of(const Session& q, int levels)
-{
-    size_t tiles = 0;
-    for (int l = 0; l < levels; ++l) {
-        const size_t tx = (size_t)((q.cfg.frame_width >> l) + 7) / 8, ty = (size_t)((q.cfg.frame_height >> l) + 7) / 8;
-        tiles += (tx * ty + 7) & ~(size_t)7;
-    }
-    return tiles;
-}
-
 // First-pass raycast workgroups per voxel format: the shape's, or fewer where the
 // resident sessions have fewer tiles (to a power of two, so that sessions coming one
 // by one change it seldom), none for a format without sessions.
@@ -233,7 +235,9 @@ void ray_grids(const kf_batch* b, const kf_batch_shape& sh, unsigned out[2])
 {
     size_t tiles[2] = {0, 0};
     for (const Session& q : b->sess)
-        if (q.used) tiles[q.cfg.voxel_format == KF_VOXEL_F32 ? 0 : 1] += ray_tiles_of(q, b->cfg.icp.levels);
+        if (q.used)
+            tiles[q.cfg.voxel_format == KF_VOXEL_F32 ? 0 : 1] +=
+                ray_tiles_of(q.cfg.frame_width, q.cfg.frame_height, b->cfg.icp.levels);
     for (int f = 0; f < 2; ++f) {
         size_t g = tiles[f] ? 1024 : 0;
         while (g && g < tiles[f]) g *= 2;
@@ -241,7 +245,6 @@ void ray_grids(const kf_batch* b, const kf_batch_shape& sh, unsigned out[2])
     }
 }
 
-// Total bricks of the resident sessions: the fuse list never holds more.
 // Deferred raycast rays: room for every ray of the resident sessions, per
 // voxel format, up to kMaxDeferred (beyond it a lane marches its ray itself).
 constexpr size_t kMaxDeferred = size_t(1) << 21;
@@ -250,9 +253,7 @@ int ensure_ray_list(kf_batch* b)
 {
     size_t need = 0;
     for (const Session& q : b->sess)
-        if (q.used) {
-            need += ray_tiles_of(q, 3) * 64;
-        }
+        if (q.used) need += ray_places_of(q.cfg.frame_width, q.cfg.frame_height);
     need = std::min(need, kMaxDeferred);
     if (need <= b->ray_cap) return KF_OK;
     need = std::min(std::max(need, 2 * b->ray_cap), kMaxDeferred);
@@ -265,6 +266,7 @@ int ensure_ray_list(kf_batch* b)
     return st;
 }
 
+// Total bricks of the resident sessions: the fuse list never holds more.
 int ensure_list(kf_batch* b)
 {
     int rs = ensure_ray_list(b);
