@@ -746,6 +746,12 @@ int kf_batch_tick(kf_batch* b, int n, const int* ids, const uint16_t* const* raw
     hd->dist_tiles = dist_tiles;
 
     // ---- launch
+    // a tick's fuse forms the free distances; only a kf_fuse into a session's volume
+    // leaves them to the next raycast
+    for (int k = 0; k < n; ++k) {
+        const kf_volume* v = b->sess[ids[k]].vol;
+        if ((v->dist_stale || v->fuse_captured) && (st = kf::refresh_free_distances(v, b->s))) return st;
+    }
     if (b->tuning) {
         const int cand = b->tune_tick % kCandidates;
         kf_batch_shape sh = b->shape;

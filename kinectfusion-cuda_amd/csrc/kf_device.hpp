@@ -333,12 +333,12 @@ __device__ __forceinline__ int grid_index(int x, int y, int z, int m)
 // matters: non-negative corners and weights give a non-negative value in any
 // rounding.
 //
-// Free distances: from these bits every fuse forms, per brick and kind of step,
-// how many bricks (Chebyshev) it is away from the nearest brick that is not
-// free, at most kDistMax.  With distance D >= 1 every brick within D - 1 of this
-// one is free, so the box of bricks around it holds no first corner of a stencil
-// that matters (outside the volume counts as free: stencils clamp into the edge
-// bricks).
+// Free distances: from these bits the first raycast after a fuse (in a batch's tick
+// the fuse) forms, per brick and kind of step, how many bricks (Chebyshev) it is away
+// from the nearest brick that is not free, at most kDistMax.  With distance D >= 1
+// every brick within D - 1 of this one is free, so the box of bricks around it holds
+// no first corner of a stencil that matters (outside the volume counts as free:
+// stencils clamp into the edge bricks).
 constexpr float kSkipBound = 0.991f;
 constexpr int kDistRadius = 8, kDistMax = kDistRadius + 1;  // in a byte, low 4 bits: large steps, high 4: small
 // The word of bit x & 63 of brick (x, y, z), kind h (0: large steps, 1: small):

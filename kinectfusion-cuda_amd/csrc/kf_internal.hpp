@@ -90,6 +90,8 @@ struct kf_volume {
     unsigned long long* touched = nullptr;  // per-workgroup counts of fused voxels (summed on read)
     unsigned long long* free_bits = nullptr;  // per-brick free bits (raycast skipping)
     uint8_t* dist = nullptr;                  // per-brick free distances, formed from free_bits
+    mutable bool dist_stale = false;          // a fuse ran since they were formed
+    bool fuse_captured = false;               // a captured graph fuses: its replays are not seen here
     int* brick_list = nullptr;              // visible bricks of the current fuse
     unsigned int* list_count = nullptr;     // list lengths, double-buffered by launch parity
     float2* drange = nullptr;               // depth range per 16x16 and per 64x64 pixel tile (FuseArgs::drange)

@@ -117,6 +117,9 @@ int launch_fuse_batch(const BatchHeader* hd, const FuseJob* jobs, unsigned cull_
 // depth map's (the measurement pass wrote them).
 int launch_fuse(const float* depth, int w, int h, kf_volume* v, const float* K, const float* inv_pose,
                 const PoseState* dyn_state, hipStream_t s, hipEvent_t* list_events, bool drange_ready);
+// Forms the volume's free distances on `s` if a fuse may have changed the free bits
+// since they were formed: every raycast's first step.
+int refresh_free_distances(const kf_volume* v, hipStream_t s);
 // The volume's tile depth range buffer sized for w x h (grown if needed); null on failure.
 float2* volume_depth_range(kf_volume* v, int w, int h, hipStream_t s);
 int launch_initialize(kf_volume* v, float f, float wt, hipStream_t s);

@@ -941,7 +941,8 @@ int launch_raycast_levels(const kf_volume* v, const float* pose, const PoseState
     unsigned blocks = 0;
     for (int l = 0; l < levels; ++l) blocks += (unsigned)level_blocks(a, l);
     // every ray of an XCD's workgroups has a place in its list
-    const int st = ensure_ray_list(v, (size_t)blocks * 64, s);
+    int st = ensure_ray_list(v, (size_t)blocks * 64, s);
+    if (st == KF_OK) st = refresh_free_distances(v, s);
     if (st) return st;
     const int parity = (int)(v->ray_launches++ & 1);
     a.rays = static_cast<DeferredRay*>(v->ray_list);

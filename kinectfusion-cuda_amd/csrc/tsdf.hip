@@ -1051,6 +1051,15 @@ int launch_brick_dist(const kf_volume* v, hipStream_t s)
     KF_LAUNCHED("brick_dist_kernel");
     return KF_OK;
 }
+// Whether work enqueued on `s` goes into a graph (the query fails for the null stream
+// while another stream is captured: taken as yes).
+bool stream_captures(hipStream_t s)
+{
+    hipStreamCaptureStatus c = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &c) == hipSuccess) return c != hipStreamCaptureStatusNone;
+    (void)hipGetLastError();
+    return true;
+}
 
 // z of each k slice: one lane, the host loop's repeated additions in order.
 __global__ void z_table_kernel(float* zk, int n, float half, float res)
@@ -1175,6 +1184,7 @@ int move_volume(const kf_volume* v, bool to_volume, bool parallel, Fn&& host_sid
         else
             free_bits_kernel<KF_VOXEL_SNORM16_U8><<<b, 256>>>(v->f, v->free_bits, nbricks, v->n, v->nb);
         st = launch_brick_dist(v, nullptr);
+        if (st == KF_OK) v->dist_stale = false;
     }
     const hipError_t e = hipDeviceSynchronize();  // nothing uses the chunks past this line
     if (st == KF_OK && e != hipSuccess) st = fail_hip(e, "volume transfer");
@@ -1279,6 +1289,8 @@ int launch_fuse(const float* depth, int w, int h, kf_volume* v, const float* K, 
 {
     float2* drange = volume_depth_range(v, w, h, s);
     if (!drange) return fail(KF_ERR_OOM, "fuse: depth tile maps");
+    if (stream_captures(s)) v->fuse_captured = true;
+    else v->dist_stale = true;
     FuseArgs a = fuse_args(depth, w, h, v, K, inv_pose, dyn_state);
     a.drange = drange;
     if (!drange_ready) {
@@ -1303,7 +1315,20 @@ int launch_fuse(const float* depth, int w, int h, kf_volume* v, const float* K, 
     KF_LAUNCHED("fuse_list_kernel");
     if (list_events) KF_HIP(hipEventRecord(list_events[1], s));
     v->fuse_launches += 1;
-    return launch_brick_dist(v, s);
+    return KF_OK;
+}
+
+// A fuse leaves the distances to the raycast that needs them (kf_fuse of 640x480 with
+// them in every fuse -> now: 512^3 FP32 39.8 -> 32.0 us, 200^3 snorm16 24.7 -> 17.5).  A
+// captured fuse may run again without a call here and a captured raycast after any
+// fuse, so those always have the step.
+int refresh_free_distances(const kf_volume* v, hipStream_t s)
+{
+    const bool captures = stream_captures(s);
+    if (!v->dist_stale && !v->fuse_captured && !captures) return KF_OK;
+    const int st = launch_brick_dist(v, s);
+    if (st == KF_OK && !captures) v->dist_stale = false;
+    return st;
 }
 
 int launch_initialize(kf_volume* v, float f, float wt, hipStream_t s)

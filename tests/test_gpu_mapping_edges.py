@@ -124,3 +124,171 @@ def test_every_count_a_volume_can_hold(kf, oracle32):
         np.testing.assert_array_equal(F, decode_q(Fq), err_msg=what)
     grid.close()
     b.close()
+
+
+# ---- the free distances a raycast skips by are formed at the first raycast after a fuse
+WALL = dict(n=96, L=2.0, w=160, h=120)
+
+
+def wall_scene(kf):
+    """A camera 0.35 m in front of a 2 m cube and three depth maps of a wall through it: alone, and with
+    a box in front of it on the left or on the right (0.9 m away, in what the wall's frames saw as free)."""
+    w, h = WALL["w"], WALL["h"]
+    sensor = kf.Sensor(0.82 * w, 0.82 * w, w / 2 - 0.5, h / 2 - 0.5)
+    pose = np.eye(4, dtype=np.float32)
+    pose[3, 2] = -1.35  # column-major
+    sensor.set_pose(pose.reshape(-1))
+    wall = (1.9 + 0.1 * np.sin(np.arange(w) / 17.0)[None, :] + np.zeros((h, 1))).astype(np.float32)
+    left, right = wall.copy(), wall.copy()
+    left[h // 4:h // 2, w // 8:w // 3] = 0.9
+    right[h // 3:2 * h // 3, 2 * w // 3:5 * w // 6] = 0.9
+    return sensor, pose.reshape(-1), [wall, left, right]
+
+
+def empty_maps(kf):
+    init = np.zeros((WALL["h"], WALL["w"], 4), np.float32)
+    init[..., 3] = -2
+    maps = [kf.GridMap(WALL["w"], WALL["h"], 4) for _ in range(2)]
+    for m in maps:
+        m.upload(init)
+    return maps
+
+
+def redrawn(kf, handle, fmt, sensor):
+    """The maps of a new volume holding the same voxels: its distances come from the voxels."""
+    n = WALL["n"]
+    fw = np.empty((n ** 3, 2), np.float32)
+    kf.check(kf.lib().kf_volume_download(handle, fw.ctypes.data_as(C.c_void_p)))
+    grid = kf.VoxelGrid(WALL["L"], n, mue=0.03, voxel_format=fmt)
+    kf.check(kf.lib().kf_volume_upload(grid.h, fw.ctypes.data_as(C.c_void_p)))
+    maps = empty_maps(kf)
+    kf.kernel.raycast(grid, sensor, *maps, 0)
+    grid.close()
+    return [m.download() for m in maps]
+
+
+def assert_drawn(got, want, box, what):
+    """box: how many of the pixels show the box rather than the wall (0: none)."""
+    for g, r in zip(got, want):
+        np.testing.assert_array_equal(g.view(np.uint32), r.view(np.uint32), err_msg=what)
+    near = np.count_nonzero((want[0][..., 3] == -1) & (want[0][..., 2] < -0.3))
+    assert near == 0 if box == 0 else near > box, (what, near)
+
+
+class Graph:
+    """What `record` enqueues on the stream, as a graph."""
+
+    def __init__(self, kf, stream, record):
+        self.lib, self.s, self.exec = kf.lib(), stream, C.c_void_p()
+        g = C.c_void_p()
+        assert self.lib.hipStreamBeginCapture(stream, 0) == 0
+        record()
+        assert self.lib.hipStreamEndCapture(stream, C.byref(g)) == 0
+        assert self.lib.hipGraphInstantiate(C.byref(self.exec), g, None, None, C.c_size_t(0)) == 0
+        assert self.lib.hipGraphDestroy(g) == 0
+
+    def replay(self):
+        assert self.lib.hipGraphLaunch(self.exec, self.s) == 0
+        assert self.lib.hipStreamSynchronize(self.s) == 0
+
+    def close(self):
+        assert self.lib.hipGraphExecDestroy(self.exec) == 0
+
+
+@pytest.mark.parametrize("route", ["eager", "captured fuses", "captured raycasts"])
+@pytest.mark.parametrize("fmt", [0, 1])
+def test_raycast_after_any_fuse(kf, route, fmt):
+    """Boxes that appear where earlier frames saw free space are drawn, whether the fuses, the raycasts or
+    neither run from a graph that was captured before.  (Graphs hold launches in pairs: the counters of a
+    launch are cleared by the one after it.)"""
+    sensor, _, depths = wall_scene(kf)
+    lib, n = kf.lib(), WALL["n"]
+    grid = kf.VoxelGrid(WALL["L"], n, mue=0.03, voxel_format=fmt)
+    stream = C.c_void_p()
+    kf.check(lib.kf_stream_create(C.byref(stream)))
+    dm = kf.GridMap(WALL["w"], WALL["h"])
+    maps = empty_maps(kf)
+    sp = C.byref(sensor.s)
+
+    def fuses(times=8):
+        for _ in range(times):
+            kf.check(lib.kf_fuse(dm.ptr, dm.width, dm.height, grid.h, sp, stream, None))
+
+    def casts():
+        for _ in range(2):
+            kf.check(lib.kf_raycast(grid.h, sp, maps[0].ptr, maps[1].ptr, dm.width, dm.height, 0, stream, None))
+
+    dm.upload(depths[0])
+    fuses(2)
+    casts()
+    kf.check(lib.kf_stream_synchronize(stream))
+    graph = None
+    if route != "eager":
+        graph = Graph(kf, stream, fuses if route == "captured fuses" else casts)
+    for k, times in enumerate([1, 4, 20]):  # left, right, left: each time enough to outweigh what was seen before
+        announce(f"raycast after fuses, {route}, format {fmt}, step {k}")
+        dm.upload(depths[1 + k % 2])
+        for _ in range(times):
+            graph.replay() if route == "captured fuses" else fuses()
+        kf.check(lib.kf_stream_synchronize(stream))
+        graph.replay() if route == "captured raycasts" else casts()
+        kf.check(lib.kf_stream_synchronize(stream))
+        want = redrawn(kf, grid.h, fmt, sensor)
+        assert_drawn([m.download() for m in maps], want, 100, f"{route} step {k}")
+    if graph:
+        graph.close()
+    grid.close()
+    kf.check(lib.kf_stream_destroy(stream))
+
+
+@pytest.mark.parametrize("route", ["batch", "loop", "visualisation volume"])
+@pytest.mark.parametrize("fmt", [0, 1])
+def test_next_frame_after_a_single_fuse(kf, route, fmt):
+    """A program's own kf_fuse into the volume of a batch's session or of the frame loop is seen by the
+    next frame's predicted maps, and a volume that is only fused into is drawn as it is when it is
+    rendered.  Without iterations the pose stays."""
+    sensor, pose, depths = wall_scene(kf)
+    lib, n, w, h = kf.lib(), WALL["n"], WALL["w"], WALL["h"]
+    raw = kf.DeviceArray.from_host((1000.0 * depths[0]).astype(np.uint16))
+    dm = kf.GridMap(w, h)
+    icp = kf.IcpConfig((0, 0, 0), w, h, 0.1, TH)
+    fx, cx, cy = 0.82 * w, w / 2 - 0.5, h / 2 - 0.5
+    handle = C.c_void_p()
+    if route == "batch":
+        b = kf.Batch(1, icp=icp)
+        sid = b.add(kf.SessionConfig(w, h, fx, fx, cx, cy, 1e-3, n, WALL["L"], 0.03, fmt, pose))
+        handle = batch_volume(kf, b, sid)
+        frame, get, end = lambda: b.tick([sid], [raw.ptr.value]), lambda m: b.map(sid, m), b
+    else:
+        vis = (n, WALL["L"], 0.03) if route == "visualisation volume" else None
+        p = kf.Pipeline(w, h, fx, fx, cx, cy, 1e-3, n, WALL["L"], 0.03, voxel_format=fmt, initial_pose=pose, icp=icp,
+                        vis_volume=vis)
+        kf.check(lib.kf_pipeline_volume(p.h, C.byref(handle)))
+        frame, get, end = lambda: p.frame(raw.ptr.value), p.map, p
+    for k in range(3):
+        announce(f"single fuse between frames, {route}, format {fmt}, step {k}")
+        frame()
+        kf.check(lib.kf_device_synchronize())
+        if route == "visualisation volume":
+            # both volumes saw the same frames: the picture is the tracking volume's
+            img = p.render(shading=False)
+            maps = empty_maps(kf)
+            kf.check(lib.kf_raycast(handle, C.byref(sensor.s), maps[0].ptr, maps[1].ptr, w, h, 0, None, None))
+            want = redrawn(kf, handle, fmt, sensor)
+            assert_drawn([m.download() for m in maps], want, 0, f"{route} {k}")
+            drawn = kf.DeviceArray((h, w), np.uint32)
+            inv = np.ascontiguousarray(np.eye(3, dtype=np.float32).reshape(9))
+            kf.check(lib.kf_render_normals(maps[1].ptr, w, h, inv.ctypes.data_as(C.c_void_p), drawn.ptr, None, None))
+            kf.check(lib.kf_device_synchronize())
+            np.testing.assert_array_equal(img, drawn.download())
+            assert len(np.unique(img)) > 10
+            continue
+        dm.upload(depths[1 + k % 2])
+        for _ in range((6, 40, 200)[k]):  # enough to outweigh what was seen before
+            kf.check(lib.kf_fuse(dm.ptr, w, h, handle, C.byref(sensor.s), None, None))
+        kf.check(lib.kf_device_synchronize())
+        want = redrawn(kf, handle, fmt, sensor)
+        frame()
+        kf.check(lib.kf_device_synchronize())
+        assert_drawn([get(4), get(5)], want, 100, f"{route} {k}")
+    end.close()
