@@ -292,3 +292,101 @@ def test_next_frame_after_a_single_fuse(kf, route, fmt):
         kf.check(lib.kf_device_synchronize())
         assert_drawn([get(4), get(5)], want, 100, f"{route} {k}")
     end.close()
+
+
+# ---- a batch's sweep of bricks in free space
+def free_space_bricks(raw_m, n, L, mue, K, cam_z):
+    """Bricks (x, y, z) that a camera at (0, 0, cam_z), unturned, certainly updates whole by f = 1: the box
+    around the brick's bounding sphere lies in the image with a pixel to spare, the sphere lies between
+    the distance limits, and the smallest depth of the 16x16 tiles (64x64 where the box is 48 pixels or
+    more) the box touches is more than mue and 2 mm behind it."""
+    h, w = raw_m.shape
+    d = np.where(np.isfinite(raw_m) & (raw_m > 0), raw_m, 0.0).astype(np.float64)
+
+    def tile_min(s):
+        th, tw = -(-h // s), -(-w // s)
+        return np.array([[d[y * s:(y + 1) * s, x * s:(x + 1) * s].min() for x in range(tw)] for y in range(th)])
+
+    mins = {16: tile_min(16), 64: tile_min(64)}
+    res, r = L / (n - 1), 3.5 * 3 ** 0.5 * L / (n - 1) * 1.01 + 1e-4
+    c = -L / 2 + (8 * np.arange(n // 8) + 3.5) * res
+    out = np.zeros((n // 8,) * 3, bool)
+    for k, z in enumerate(c - cam_z):
+        lo, hi = z - r, z + r
+        if lo <= 0.402 or hi >= 5.998:
+            continue
+        for j, y in enumerate(c):
+            for i, x in enumerate(c):
+                u = [K[0] * f(a / q for q in (lo, hi)) + K[6] + m for f, a, m in ((min, x - r, -2), (max, x + r, 2))]
+                v = [K[4] * f(a / q for q in (lo, hi)) + K[7] + m for f, a, m in ((min, y - r, -2), (max, y + r, 2))]
+                if u[0] < 0 or v[0] < 0 or u[1] > w - 1 or v[1] > h - 1:
+                    continue
+                size = max(u[1] - u[0], v[1] - v[0])
+                s = 16 if size < 46 else 64
+                if size >= 190:
+                    continue
+                t = mins[s][int(v[0]) // s:int(v[1]) // s + 1, int(u[0]) // s:int(u[1]) // s + 1]
+                out[i, j, k] = t.min() - hi >= mue + 2e-3
+    return out
+
+
+@pytest.mark.parametrize("n,w,h", [(200, 320, 240), (96, 200, 148)])
+@pytest.mark.parametrize("graph", [False, True])
+def test_free_space_sweep_bit_exact(kf, oracle32, n, w, h, graph):
+    """A batch updates bricks in free space without projecting their voxels, and only the counts of those
+    whose every code is 1: a wall seen over a box that comes and goes, with holes and infinite depths, into
+    a volume of uploaded codes and counts (126 to 128 and above among them), so that bricks of every kind
+    lie in free space; voxels, fused-voxel counts and the maps drawn from them against the oracle.  (The
+    single fuse of the same frames has no such path.)"""
+    L, mue, cam_z = 2.0, 0.03, -1.35
+    rng = np.random.default_rng(n)
+    nb = n // 8
+    blow = lambda a: np.repeat(np.repeat(np.repeat(a, 8, 0), 8, 1), 8, 2).reshape(-1)  # noqa: E731
+    kind = rng.integers(0, 4, (nb, nb, nb))  # [z, y, x] bricks: untouched, all 1, mixed codes, mixed codes below 0.991
+    Fq, Wq = oracle32.new_volume_q(n)
+    every = blow(kind)
+    for k, codes in [(1, [32767]), (2, [32767, 32767, 32767, 32766, 32471]), (3, [32767, 20000, 3, 0, -500, -32768])]:
+        at = every == k
+        Fq[at] = rng.choice(np.array(codes, np.int16), int(at.sum()))
+        Wq[at] = rng.choice(np.array([0, 1, 5, 126, 127, 128, 129, 200, 255], np.uint8), int(at.sum()))
+    sensor = kf.Sensor(0.82 * w, 0.82 * w, w / 2 - 0.5, h / 2 - 0.5)
+    pose = np.eye(4, dtype=np.float32)
+    pose[3, 2] = cam_z  # column-major
+    sensor.set_pose(pose.reshape(-1))
+    K, Ki = sensor.get_intr(0), sensor.get_inverse_intr(0)
+    b = kf.Batch(1, icp=kf.IcpConfig((0, 0, 0), w, h, 0.1, TH), use_graph=graph)
+    sid = b.add(kf.SessionConfig(w, h, 0.82 * w, 0.82 * w, w / 2 - 0.5, h / 2 - 0.5, 1e-3, n, L, mue,
+                                 kf.KF_VOXEL_SNORM16_U8, pose.reshape(-1)))
+    upload(kf, batch_volume(kf, b, sid), decode_q(Fq), Wq)
+    touched, seen = 0, np.zeros(4, int)
+    for f in range(5):
+        announce(f"free-space sweep n {n} {w}x{h} graph {graph} tick {f}")
+        raw = (1900 + 100 * np.sin(np.arange(w) / 17.0)[None, :] + 50 * rng.random((h, w))).astype(np.uint16)
+        if f % 2:
+            raw[h // 4:h // 2, w // 4:w // 2] = 900
+        raw[rng.random((h, w)) < 2e-4] = 0
+        raw[3 * h // 4, : w // 3] = 65535
+        d = oracle32.convert_to_depth_meters(raw, 1e-3)
+        free = free_space_bricks(d, n, L, mue, K, cam_z).transpose(2, 1, 0)
+        if f == 0:
+            for k in range(4):
+                seen[k] = np.count_nonzero(free & (kind == k))
+        want = None
+        if f:
+            init = np.zeros((h, w, 4), np.float32)
+            init[..., 3] = -2
+            want = oracle32.raycast_q(Fq, n, L, mue, sensor.get_pose(), Ki, w, h, init.copy(), init.copy())
+        dev = kf.DeviceArray.from_host(raw)
+        b.tick([sid], [dev.ptr.value])
+        b.sync()
+        touched += oracle32.fuse_q(Fq, Wq, n, L, mue, d, sensor.get_inverse_pose(), K)
+        if f:
+            for m, x in zip((4, 5), want):
+                np.testing.assert_array_equal(b.map(sid, m).view(np.uint32), x.view(np.uint32), err_msg=f"map {m} {f}")
+    assert b.status(sid) == 0
+    assert (seen > 0).all(), seen  # bricks of every kind met the free-space rule in the first tick
+    F, W = b.volume_download(sid)
+    np.testing.assert_array_equal(W, Wq.astype(np.float32))
+    np.testing.assert_array_equal(F, decode_q(Fq))
+    assert b.touched_total() == touched > 0.1 * n ** 3
+    b.close()
