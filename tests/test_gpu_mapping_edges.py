@@ -390,3 +390,57 @@ def test_free_space_sweep_bit_exact(kf, oracle32, n, w, h, graph):
     np.testing.assert_array_equal(F, decode_q(Fq))
     assert b.touched_total() == touched > 0.1 * n ** 3
     b.close()
+
+
+# ---- volumes of more than 64 bricks a side: two words of free bits per row of bricks
+@pytest.mark.parametrize("n", [520, 528])
+@pytest.mark.parametrize("fmt", [0, 1])
+def test_surface_between_bricks_63_and_64(kf, oracle32, n, fmt):
+    """A wall that crosses the plane between bricks 63 and 64 along x, fused where earlier frames saw free
+    space, through single fuses and a batch: every voxel and what is drawn against the oracle.  A free bit
+    that is not cleared in either word lets a raycast step over the wall."""
+    L, mue, w, h = 4.0, 0.03, 160, 120
+    # the camera at (-0.5, 0, 0) looks along +x: camera axes x, y, z are -z, y, x of the world
+    pose = np.zeros((4, 4), np.float32)
+    pose[0, 2], pose[1, 1], pose[2, 0], pose[3] = -1.0, 1.0, 1.0, (-0.5, 0.0, 0.0, 1.0)
+    sensor = kf.Sensor(131.25, 131.25, 79.5, 59.5)
+    sensor.set_pose(pose.reshape(-1))
+    K, Ki = sensor.get_intr(0), sensor.get_inverse_intr(0)
+    edge = int(round(1000 * (-L / 2 + 511.5 * L / (n - 1) + 0.5)))  # its depth in millimetres
+    u, v = np.meshgrid(np.arange(w), np.arange(h))
+    wall = (edge + 60 * np.sin(u / 23.0) * np.cos(v / 19.0)).astype(np.uint16)
+    frames = [np.full((h, w), 2900, np.uint16)] + [wall] * 3
+    cast, fuse = (oracle32.raycast_q, oracle32.fuse_q) if fmt else (oracle32.raycast, oracle32.fuse)
+    Fo, Wo = oracle32.new_volume_q(n) if fmt else oracle32.new_volume(n)
+    grid = kf.VoxelGrid(L, n, mue=mue, voxel_format=fmt)
+    b = kf.Batch(1, icp=kf.IcpConfig((0, 0, 0), w, h, 0.1, TH))
+    sid = b.add(kf.SessionConfig(w, h, 131.25, 131.25, 79.5, 59.5, 1e-3, n, L, mue, fmt, pose.reshape(-1)))
+    dm, maps = kf.GridMap(w, h), [kf.GridMap(w, h, 4) for _ in range(2)]
+    init = np.zeros((h, w, 4), np.float32)
+    init[..., 3] = -2
+    for f, raw in enumerate(frames):
+        announce(f"wall at bricks 63/64 n {n} format {fmt} frame {f}")
+        want = cast(Fo, n, L, mue, sensor.get_pose(), Ki, w, h, init.copy(), init.copy())
+        for m in maps:
+            m.upload(init)
+        kf.kernel.raycast(grid, sensor, *maps, 0)
+        dev = kf.DeviceArray.from_host(raw)
+        b.tick([sid], [dev.ptr.value])
+        b.sync()
+        for m, got, x in zip((4, 5), maps, want):
+            np.testing.assert_array_equal(got.download().view(np.uint32), x.view(np.uint32), err_msg=f"single {m} {f}")
+            if f:
+                np.testing.assert_array_equal(b.map(sid, m).view(np.uint32), x.view(np.uint32), err_msg=f"batch {m} {f}")
+        d = oracle32.convert_to_depth_meters(raw, 1e-3)
+        dm.upload(d)
+        kf.kernel.fuse(dm, grid, sensor)
+        fuse(Fo, Wo, n, L, mue, d, sensor.get_inverse_pose(), K)
+    hit = want[0][..., 3] == -1
+    brick = ((want[0][..., 0] + L / 2) / (L / (n - 1)) / 8).astype(int)
+    assert np.count_nonzero(hit & (brick == 63)) > 500 and np.count_nonzero(hit & (brick == 64)) > 500
+    F, W = (decode_q(Fo), Wo.astype(np.float32)) if fmt else (Fo, Wo)
+    for what, (x, y) in [("single", grid.download()), ("batch", b.volume_download(sid))]:
+        assert np.array_equal(x.view(np.uint32), F.view(np.uint32)), what
+        assert np.array_equal(y.view(np.uint32), W.view(np.uint32)), what
+    grid.close()
+    b.close()
