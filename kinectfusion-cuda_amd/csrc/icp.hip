@@ -108,10 +108,16 @@ __device__ __forceinline__ void floor_quotients(v3 p, float band, float& fu, flo
 // Angle, icp.cuh:63-70 in its cosine form (acos(d) > th <=> d >= -1 && d < cos
 // th), d = dot(normalize(Rc normalize(cr)), n).  The approximation da rotates cr
 // as it is and takes one normalization, with the hardware reciprocal square root
-// (1 ulp): it is within 2^-19 |n|_1 of the exact d (measured worst case over 8M
-// random rotations, normals and lengths with the reciprocal root off by one ulp
-// either way: 2^-21.3), so a margin of 2^-16 |n|_1 decides; a squared length outside [2^-100, 2^100] (where the hardware routine
-// may flush or overflow) and NaN take the exact path.
+// (1 ulp).  With u = 2^-24 and Rc a rotation: turning cr costs at most 3 sqrt(3) u
+// of its length (three products and two sums per component), its squared length 3 u
+// and the root of it half of that, the reciprocal root 2 u, the product with n 3 u and
+// the last product u, 12.7 u |n| in all; d has the same, one more normalization (3 u)
+// and a division per component, at most 17 u |n|: they differ by less than 30 u |n| <
+// 2^-19 |n|_1 (measured worst case over 8M random rotations, normals and lengths with
+// the reciprocal root off by one ulp either way: 2^-21.3).  A margin of 2^-16 |n|_1
+// decides, eight times that, so also for a matrix that is a rotation only roughly; a
+// squared length outside [2^-100, 2^100] (where the hardware routine may flush or
+// overflow) and NaN take the exact path.
 __device__ __forceinline__ bool pair_rejected(const IcpArgs& a, const float* Rc, v3 v, v3 cr, v3 n, bool live)
 {
     const float D = dot3(v, v);

@@ -444,3 +444,49 @@ def test_surface_between_bricks_63_and_64(kf, oracle32, n, fmt):
         assert np.array_equal(y.view(np.uint32), W.view(np.uint32)), what
     grid.close()
     b.close()
+
+
+@pytest.mark.parametrize("degrees", [5.0, 20.0, 60.0, 120.0])
+def test_angle_near_the_threshold_bit_exact(kf, oracle32, degrees):
+    """The angle test is decided from an approximation except near the threshold: target normals whose
+    cosine with the turned live normal lies 2^-25 to 2^-13 to either side of the threshold's, so inside,
+    at and outside the band that is evaluated exactly, every row against the oracle's."""
+    w, h = 64, 48
+    rng = np.random.default_rng(int(degrees))
+    f = 60.0
+    u, v = np.meshgrid(np.arange(w) + 0.5, np.arange(h) + 0.5)
+    z = 1.0 + 0.3 * rng.random((h, w))
+    V = np.stack([(u - w / 2) / f * z, (v - h / 2) / f * z, z, np.full((h, w), -1.0)], -1).astype(np.float32)
+    live = oracle32.create_normal_map(V)
+    th = float(np.float32(np.deg2rad(degrees)))
+    accepted = 0
+    for turn in range(3):
+        announce(f"angle near {degrees} degrees, rotation {turn}")
+        Q = np.linalg.qr(rng.standard_normal((3, 3)))[0]
+        Q *= np.sign(np.linalg.det(Q))
+        R = np.ascontiguousarray(Q.T.reshape(-1), np.float32)  # column-major
+        t = rng.standard_normal(3).astype(np.float32)
+        a = live[..., :3].astype(np.float64) @ R.reshape(3, 3).astype(np.float64)
+        a /= np.maximum(np.linalg.norm(a, axis=-1, keepdims=True), 1e-30)
+        side = np.cross(a, rng.standard_normal(a.shape))
+        side /= np.maximum(np.linalg.norm(side, axis=-1, keepdims=True), 1e-30)
+        c = np.cos(th) + rng.choice([-1.0, 1.0], (h, w)) * 2.0 ** rng.uniform(-25, -13, (h, w))
+        N = c[..., None] * a + np.sqrt(1 - c * c)[..., None] * side
+        TN = np.concatenate([N, np.full((h, w, 1), -1.0)], -1).astype(np.float32)
+        TV = np.concatenate([rng.standard_normal((h, w, 3)), np.full((h, w, 1), -1.0)], -1).astype(np.float32)
+        maps = []
+        for m in (V, TV, TN):
+            g = kf.GridMap(w, h, 4)
+            g.upload(m)
+            maps.append(g)
+        K = np.array([f, 0, 0, 0, f, 0, w / 2, h / 2, 1], np.float32)
+        A, b = kf.DeviceArray((h * w, 6)), kf.DeviceArray((h * w,))
+        kf.kernel.construct_icp_residuals(*maps, R, t, R, t, K, 1e18, th, A, b)
+        Ar, br = oracle32.construct_icp_residuals(V, TV, TN, R, t, R, t, K, 1e18, th)
+        np.testing.assert_array_equal(A.download().view(np.uint32), Ar.view(np.uint32))
+        np.testing.assert_array_equal(b.download().view(np.uint32), br.view(np.uint32))
+        hits = np.count_nonzero(np.any(Ar != 0, axis=1))
+        accepted += hits
+        _, inliers = kf.kernel.icp_reduce(*maps, R, t, R, t, K, 1e18, th)
+        assert inliers == hits
+    assert 0.2 < accepted / (3 * (w - 1) * (h - 1)) < 0.8
