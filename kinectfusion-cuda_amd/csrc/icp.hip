@@ -1,7 +1,7 @@
 // Projective point-to-plane ICP (project/src/icp.cu, icp.cuh, icp.cpp,
 // linear_least_squares.cpp), kept on the device for a whole frame.
 //
-// One iteration = two launches:
+// One iteration has two parts:
 //   reduce   : 256 lanes x 4 pixels per workgroup.  Each lane associates its
 //              pixels (icp.cu:7-82) and accumulates the 27 unique terms of the
 //              normal equations (21 of A^T A, 6 of A^T b) in FP32 registers;
@@ -12,8 +12,9 @@
 //              result is deterministic), solves the 6x6 system with an FP64
 //              Cholesky, applies the pose update (icp.cpp:65-87) and the early
 //              stop test (icp.cpp:45-53) to the device-resident PoseState.
-// The kernel boundary between the two launches is what makes every
-// workgroup's partial row visible to the finalize across the 8 XCDs' L2s.
+// The kernel boundary between them is what makes every workgroup's partial row
+// visible to the finalize across the 8 XCDs' L2s.  A frame's loop has one launch per
+// iteration: every workgroup of the next reduce does the finalize for itself first.
 // The reference instead writes A (N x 6) and b to HBM, runs cublasSgemm and
 // cublasSgemv, copies 42 floats to the host and solves with Eigen's FP32 LLT,
 // with a host synchronisation per iteration.
@@ -382,12 +383,14 @@ __device__ __forceinline__ void load_lane_pixels(const IcpArgs& a, LanePixels<PI
 }
 
 // Associates the lane's pixels at the iteration's pose and writes partial row
-// `block` of a.partials.  Bound: the vector ALU (80-90 % busy in a batch tick).
+// `block` of a.partials.  Bound: latency in a frame, whose launches have a wave or two
+// per SIMD; the vector ALU in a batch tick (0.91 busy at 320x240, 0.67 at 640x480,
+// where the maps' bytes come at 4.4 TB/s).
 // With the projection's quotients taken approximately, one normalization less in
 // the angle test, offsets of 32 bits shared by a pixel's loads, the projection
 // matrix formed once instead of by every lane, the batch's pose in scalar registers
-// and counts by ballot, the association of a tick of 64 sessions takes 122 instead
-// of 141 us on average over its 19 iterations; sixteen uneven sessions 32 -> 25 us,
+// and counts by ballot, the association of a tick of 64 sessions took 142 instead of
+// 154 us on average over its 19 iterations; sixteen uneven sessions 32 -> 25 us,
 // a frame 333 -> 321 us (512^3, plain) and 365 -> 347 us (256^3, compensated).
 template <bool COMP, int PIX>
 __device__ __forceinline__ void associate_reduce(const IcpArgs& a, const LanePixels<PIX>& lp, const IterPose& P,
@@ -1047,9 +1050,10 @@ __global__ __launch_bounds__(kThreads) void icp_batch_solve_kernel(const BatchHe
 // that few registers (84) hold them and other waves fill the waits: with its four
 // pixels' loads in flight together the kernel held 102 and had four waves per SIMD.
 // Five workgroups per CU resident, as many launched.  On average over the 19 iterations
-// of a tick of 64 sessions 145 -> 136 us (216 of those at 640x480, whose maps come at
-// 4.4 TB/s), of 16 uneven sessions 26.8 -> 26.3; nothing issued ahead (70 registers,
-// six waves) 136.6 and 26.6, two pixels at a time (96) 139.5 and 27.3.
+// of a tick of 64 sessions 141 -> 135 us (22 -> 20.5 at 160x120, 77 -> 68 at 320x240,
+// 221 -> 215 at 640x480, whose maps come at 4.4 TB/s), of 16 uneven sessions 26.8 ->
+// 26.3; nothing issued ahead (70 registers, six waves) took 0.5 us more of the one and
+// 0.3 of the other, two pixels at a time (96 registers) 3.5 and 1.
 template <bool COMP>
 __global__ __launch_bounds__(kThreads, 5) void icp_batch_assoc_kernel(const BatchHeader* hd, const IcpJob* jobs,
                                                                    int level)

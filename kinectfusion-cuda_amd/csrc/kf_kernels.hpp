@@ -101,9 +101,11 @@ struct FuseJob {
     unsigned group0;  // first global cube (4x4x4 bricks) of this job
     int dist_tile0;   // first 8x8-row tile of this job's free distances
 };
-// Workgroups of one volume's free distances: one per 8x8 rows of bricks.
+// Cubes of 4x4x4 bricks of a volume, those at its far faces cut off by them.
 inline unsigned fuse_groups(int nb) { return (unsigned)((nb + 3) / 4) * ((nb + 3) / 4) * ((nb + 3) / 4); }
+// Words of a volume's free bits (free_word).
 inline size_t free_words(int nb) { return (size_t)nb * nb * 2 * (nb > 64 ? 2 : 1); }
+// Workgroups of a volume's free distances: one per 8x8 rows of bricks.
 inline int dist_tiles(int nb) { return ((nb + 7) / 8) * ((nb + 7) / 8); }
 FuseArgs fuse_args(const float* depth, int w, int h, const kf_volume* v, const float* K, const float* inv_pose,
                    const PoseState* dyn_state);

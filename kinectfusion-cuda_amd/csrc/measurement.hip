@@ -2,9 +2,10 @@
 // depth codes -> metres, bilateral filter, depth pyramid, vertex and normal maps.
 //
 // Maps are plain row-major arrays in HBM (float depth, float4 vertex/normal with
-// validity in .w).  Every kernel is one thread per output pixel over 16x16
-// tiles (4 waves of 64), with bounds checks, so any frame size works (the
-// reference launches w/8 x h/8 blocks and skips the remainder).
+// validity in .w).  Every kernel takes 16x16 lanes (4 waves of 64) a workgroup, one
+// lane per output pixel of a 16x16 tile, or several per pixel of a larger region where
+// its comment says so, with bounds checks, so any frame size works (the reference
+// launches w/8 x h/8 blocks and skips the remainder).
 #include <string.h>
 
 #include "kf_device.hpp"
@@ -146,7 +147,10 @@ __global__ __launch_bounds__(256) void vertex_kernel(const float* __restrict__ d
     out[(int64_t)j * w + i] = vertex_at(depth[(int64_t)j * w + i], i, j, ki.m);
 }
 
-// ---- the measurement step in two launches (one session or many).
+// ---- the measurement step in one launch (one session's frame without normals, whose
+// 64x64 depth ranges are not asked for here: measure_one_pass_kernel), or in two (with
+// normals or ranges: measure_kernel and pyramid_kernel; many sessions:
+// measure_batch_kernel and pyramid_batch_kernel).  launch_measure chooses.
 // The metres of the 22x22 window at (i0, j0), clamped to the image's edges.
 // UNMIRROR: row j of the frame is read right to left (measurement.cu:22-25).
 template <bool UNMIRROR>
@@ -238,8 +242,9 @@ __device__ __forceinline__ void pyramid_tile(const PreJob& J, int lt)
 // Bound: launch and memory latency.  16x16 regions give a 640x480 frame 1200
 // workgroups, 32x32 ones 300, which leave the chip half idle but read less halo:
 // kf_preprocess with normals by 32x32 -> 16x16 regions 484x372 16.2 -> 13.8 us, 640x480
-// 19.0 -> 17.0, 800x600 24.6 -> 23.3, 1276x716 35.9 -> 35.5, 1920x1080 65.5 -> 68.5, so
-// frames up to kSmallRegions pixels take 16x16.  Many sessions fill the chip either
+// 19.0 -> 17.0, 800x600 24.6 -> 23.3, 1276x716 35.9 -> 35.5 (within the runs' spread),
+// 1920x1080 65.5 -> 68.5: frames up to kSmallRegions pixels take 16x16, the line lying
+// between the last size that gains (480000 pixels) and the one that does not (913616).  Many sessions fill the chip either
 // way, and there the regions' barriers cost: 64 frames of 640x480 took 109 us by
 // regions, 50 us by the form above (73 us with its depths read one by one).
 constexpr int kSmallRegions = 600000;

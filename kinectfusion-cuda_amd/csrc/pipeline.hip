@@ -172,8 +172,9 @@ int kf_pipeline_frame(kf_pipeline* p, const uint16_t* raw)
     }
     int st;
     kf::PoseState* state = p->icp->state;
-    // the two-pass measurement: metres, bilateral, pyramid, vertex maps and the
-    // fuse's tile depth ranges (depthFrameToVertexPyramid, kinect_fusion.cpp:116-135).
+    // the measurement: metres, bilateral, pyramid, vertex maps and the fuse's tile depth
+    // ranges (depthFrameToVertexPyramid, kinect_fusion.cpp:116-135), in one launch from
+    // the second frame on, whose 64x64 ranges the raycast forms.
     // ICP computes the live normals itself, so the normal pyramid is only built
     // when a caller asks for it.
     kf::PreJob J;
