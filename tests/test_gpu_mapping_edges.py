@@ -490,3 +490,41 @@ def test_angle_near_the_threshold_bit_exact(kf, oracle32, degrees):
         _, inliers = kf.kernel.icp_reduce(*maps, R, t, R, t, K, 1e18, th)
         assert inliers == hits
     assert 0.2 < accepted / (3 * (w - 1) * (h - 1)) < 0.8
+
+
+# voxels much longer than a step of the march: a box of free bricks holds many times the march's range
+@pytest.mark.parametrize("n,L,mue", [(8, 9000.0, 1e-3), (16, 2000.0, 0.03), (64, 400.0, 0.01), (128, 1024.0, 0.5)])
+def test_raycast_of_long_voxels_bit_exact(kf, oracle32, n, L, mue):
+    """Random voxels, drawn from places where the rays' few metres cross the plane where F changes sign, lie
+    in free space or behind the surface, against the oracle."""
+    w, h = 64, 48
+    rng = np.random.default_rng(n)
+    res = L / n
+    F = (0.992 + 0.008 * rng.random((n, n, n), np.float32)).astype(np.float32)
+    F[n // 2:] = -(0.2 + 0.8 * rng.random((n - n // 2, n, n), np.float32))  # z
+    F[n // 2 - 1] = 0.2 + 0.8 * rng.random((n, n), np.float32)
+    grid = kf.VoxelGrid(L, n, mue=mue)
+    grid.upload(F.reshape(-1), np.ones(n ** 3, np.float32))
+    sensor = kf.Sensor(60.0, 60.0, w / 2 - 0.5, h / 2 - 0.5)
+    maps = [kf.GridMap(w, h, 4) for _ in range(2)]
+    init = np.zeros((h, w, 4), np.float32)
+    init[..., 3] = -2
+    hits = 0
+    # F at the middle column between the voxel planes either side of the change of sign
+    col = F[n // 2 - 1:n // 2 + 1, n // 2 - 1:n // 2 + 1, n // 2 - 1:n // 2 + 1].mean((1, 2)).astype(np.float64)
+    zero = -0.5 * res + res * col[0] / (col[0] - col[1])
+    for k, z in enumerate([zero - 2.5, zero - 5.0, zero + 1.0, -0.3 * L, -0.5 * L - 1.0]):
+        pose = np.eye(4, dtype=np.float32)
+        pose[3, 2] = z  # column-major
+        sensor.set_pose(pose.reshape(-1))
+        announce(f"raycast of long voxels n {n} L {L} mue {mue} pose {k}")
+        for m in maps:
+            m.upload(init)
+        kf.kernel.raycast(grid, sensor, *maps, 0)
+        want = oracle32.raycast(F.reshape(-1), n, L, mue, sensor.get_pose(), sensor.get_inverse_intr(0), w, h,
+                                init.copy(), init.copy())
+        hits += np.count_nonzero(want[0][..., 3] == -1)
+        for m, x in zip(maps, want):
+            np.testing.assert_array_equal(m.download().view(np.uint32), x.view(np.uint32), err_msg=f"pose {k}")
+    assert hits > 500
+    grid.close()
