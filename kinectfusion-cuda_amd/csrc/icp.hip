@@ -104,7 +104,9 @@ __device__ __forceinline__ void floor_quotients(v3 p, float band, float& fu, flo
 // Distance, icp.cuh:57-60: reject iff RN(sqrt(D)) > T, D = dot(v, v) (the
 // same bits on both paths).  D <= T^2 gives sqrt(D) <= T; D >= (T + ulp(T))^2
 // gives RN(sqrt(D)) > T.  lo and hi below bound those squares from inside
-// (lo <= T^2, hi >= T^2 (1 + 2^-21) > (T + ulp(T))^2); NaN takes the exact path.
+// (lo <= T^2, hi >= T^2 (1 + 2^-21) > (T + ulp(T))^2); NaN takes the exact path.  A
+// negative T keeps its sign in the square (no length is at most T), a square of 0
+// accepts a length of 0 only, and an infinite D is never accepted unseen.
 //
 // Angle, icp.cuh:63-70 in its cosine form (acos(d) > th <=> d >= -1 && d < cos
 // th), d = dot(normalize(Rc normalize(cr)), n).  The approximation da rotates cr
@@ -122,15 +124,15 @@ __device__ __forceinline__ void floor_quotients(v3 p, float band, float& fu, flo
 __device__ __forceinline__ bool pair_rejected(const IcpArgs& a, const float* Rc, v3 v, v3 cr, v3 n, bool live)
 {
     const float D = dot3(v, v);
-    const float T2 = a.dist_thresh * a.dist_thresh;
-    const float lo = T2 * (1.0f - 0x1p-22f), hi = T2 * (1.0f + 0x1p-20f);
+    const float T2 = a.dist_thresh * fabsf(a.dist_thresh);
+    const float lo = fminf(T2 * (1.0f - 0x1p-22f), 0x1.fffffep127f), hi = T2 * (1.0f + 0x1p-20f);
     const v3 m = m3v(Rc, cr);
     const float mq = dot3(m, m);
     const float da = dot3(m, n) * __builtin_amdgcn_rsqf(mq);
     const float del = 0x1p-16f * (fabsf(n.x) + fabsf(n.y) + fabsf(n.z));
     const bool ranged = mq >= 0x1p-100f && mq <= 0x1p100f;
     const float c = a.cos_thresh;
-    bool rejected = D >= hi || (ranged && da < c - del && da >= -1.0f + del);
+    bool rejected = D > hi || (ranged && da < c - del && da >= -1.0f + del);
     const bool accepted = D <= lo && ranged && da >= c + del;
     if (live && !rejected && !accepted) {
         rejected = len3(v) > a.dist_thresh;

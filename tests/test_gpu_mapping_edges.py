@@ -528,3 +528,46 @@ def test_raycast_of_long_voxels_bit_exact(kf, oracle32, n, L, mue):
             np.testing.assert_array_equal(m.download().view(np.uint32), x.view(np.uint32), err_msg=f"pose {k}")
     assert hits > 500
     grid.close()
+
+
+@pytest.mark.parametrize("dist", [-1.0, -0.0, 0.0, 1e-25, 1e-3, 0.05, 1e18, 1e20, float("inf"), float("nan")])
+def test_any_distance_threshold_bit_exact(kf, oracle32, dist):
+    """The distance test takes any threshold: none is met by a length above it, a negative one by no
+    length at all, 0 by coincident points, an infinite one by every length; targets at, near and 1e20 m
+    from the vertices, some of them infinite or NaN, every row against the oracle's."""
+    w, h = 64, 48
+    rng = np.random.default_rng(7)
+    f = 60.0
+    u, v = np.meshgrid(np.arange(w) + 0.5, np.arange(h) + 0.5)
+    z = 1.0 + 0.1 * rng.random((h, w))
+    V = np.stack([(u - w / 2) / f * z, (v - h / 2) / f * z, z, np.full((h, w), -1.0)], -1).astype(np.float32)
+    TV = V.copy()
+    kind = rng.integers(0, 6, (h, w))
+    for k, size in [(1, 1e-4), (2, 0.05), (3, 3.0), (4, 1e20)]:
+        at = kind == k
+        TV[at, :3] += (size * rng.standard_normal((int(at.sum()), 3))).astype(np.float32)
+    odd = (kind == 5) & (rng.random((h, w)) < 0.2)
+    TV[odd, 0] = rng.choice(np.array([np.inf, -np.inf, np.nan], np.float32), int(odd.sum()))
+    N = np.concatenate([0.1 * rng.standard_normal((h, w, 2)), np.ones((h, w, 1))], -1)
+    TN = np.concatenate([N / np.linalg.norm(N, axis=-1, keepdims=True), np.full((h, w, 1), -1.0)], -1)
+    TN = TN.astype(np.float32)
+    maps = []
+    for m in (V, TV, TN):
+        g = kf.GridMap(w, h, 4)
+        g.upload(m)
+        maps.append(g)
+    R, t = np.eye(3, dtype=np.float32).reshape(9), np.zeros(3, np.float32)
+    K = np.array([f, 0, 0, 0, f, 0, w / 2, h / 2, 1], np.float32)
+    A, b = kf.DeviceArray((h * w, 6)), kf.DeviceArray((h * w,))
+    for degrees in (60.0, 180.0):
+        announce(f"distance threshold {dist}, {degrees} degrees")
+        th = float(np.float32(np.deg2rad(degrees)))
+        kf.kernel.construct_icp_residuals(*maps, R, t, R, t, K, dist, th, A, b)
+        Ar, br = oracle32.construct_icp_residuals(V, TV, TN, R, t, R, t, K, dist, th)
+        for got, want in ((A.download(), Ar), (b.download(), br)):
+            nan = np.isnan(want)
+            np.testing.assert_array_equal(np.isnan(got), nan)
+            np.testing.assert_array_equal(np.where(nan, 0, got.view(np.uint32)), np.where(nan, 0, want.view(np.uint32)))
+        kept = np.count_nonzero(np.any(Ar != 0, axis=1) | (br != 0))  # NaN differs from 0
+        _, inliers = kf.kernel.icp_reduce(*maps, R, t, R, t, K, dist, th)
+        assert inliers == kept
