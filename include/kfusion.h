@@ -246,7 +246,8 @@ int kf_pipeline_sync(kf_pipeline* p, int* status);
 int kf_pipeline_pose(kf_pipeline* p, float pose[16]);
 int kf_pipeline_volume(kf_pipeline* p, kf_volume** v);
 /* which: 0 unfiltered metres (level 0), 1 filtered depth, 2 vertex, 3 normal,
- *        4 predicted vertex, 5 predicted normal. */
+ *        4 predicted vertex, 5 predicted normal.  The map holds the last enqueued frame's values
+ * once the pipeline's stream has run (normals are formed on it by this call: wait after it). */
 int kf_pipeline_map(kf_pipeline* p, int which, int level, void** dev_ptr, int* w, int* h);
 /* Per-stage event timing (kinect_fusion.cpp:216-224 prints these averages). */
 int kf_pipeline_set_timing(kf_pipeline* p, int enabled);

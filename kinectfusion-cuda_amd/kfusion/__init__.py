@@ -465,6 +465,8 @@ class Pipeline:
         ch = 1 if which in (0, 1) else 4
         shape = (h.value, w.value) if ch == 1 else (h.value, w.value, ch)
         out = np.empty(shape, np.float32)
+        # the frames, and the normals that are formed on request, run on the pipeline's own stream
+        check(lib().kf_device_synchronize(), "map download")
         check(lib().kf_memcpy_d2h(_p(out), ptr, out.nbytes, None), "map download")
         return out
 

@@ -571,3 +571,24 @@ def test_any_distance_threshold_bit_exact(kf, oracle32, dist):
         kept = np.count_nonzero(np.any(Ar != 0, axis=1) | (br != 0))  # NaN differs from 0
         _, inliers = kf.kernel.icp_reduce(*maps, R, t, R, t, K, dist, th)
         assert inliers == kept
+
+
+def test_maps_of_a_loop_that_still_runs(kf, oracle32):
+    """Pipeline.map returns the last enqueued frame's map without a sync before it, also the normals, which
+    are formed when they are asked for: with frames in flight, the normals of the vertices, level by level."""
+    seq = small_sequence(seed=14, n_frames=4, w=640, h=480, L=4.0)
+    raws = seq.frames(0, 4)
+    dev = kf.DeviceArray.from_host(raws)
+    p = make_pipeline(kf, seq, 256, 0)
+    for rep in range(3):
+        announce(f"maps of a running loop {rep}")
+        for f in range(4):
+            p.frame(dev.ptr.value + f * raws[0].nbytes)
+        for l in range(3):
+            n, v = p.map(3, l), p.map(2, l)
+            d = p.map(1, l)
+            np.testing.assert_array_equal(n.view(np.uint32), oracle32.create_normal_map(v).view(np.uint32))
+            if l == 0:
+                want = oracle32.apply_bilateral_filter(oracle32.convert_to_depth_meters(raws[3], 1e-3))
+                np.testing.assert_array_equal(d.view(np.uint32), want.view(np.uint32))
+    p.close()
