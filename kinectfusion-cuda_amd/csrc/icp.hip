@@ -386,7 +386,7 @@ __device__ __forceinline__ void load_lane_pixels(const IcpArgs& a, LanePixels<PI
 
 // Associates the lane's pixels at the iteration's pose and writes partial row
 // `block` of a.partials.  Bound: latency in a frame, whose launches have a wave or two
-// per SIMD; the vector ALU in a batch tick (0.91 busy at 320x240, 0.67 at 640x480,
+// per SIMD; the vector ALU in a batch tick (0.91 busy at 320x240, 0.68 at 640x480,
 // where the maps' bytes come at 4.4 TB/s).
 // With the projection's quotients taken approximately, one normalization less in
 // the angle test, offsets of 32 bits shared by a pixel's loads, the projection
